@@ -243,7 +243,7 @@ def _prepare_module(c, r):
         return {"module": module, "inputs": (x, mask), "gradient": r.normal((b, s, h), torch.float16), "buffers": {}}
     net = r.fill(MBConv(c["channels"]).cuda().train(), std=None)
     shape = (c["batch"], c["channels"], c["size"], c["size"])
-    x = r.normal(shape).requires_grad_(True)
+    x = r.normal(shape, mean=0.5).requires_grad_(True)   # not centred: the running means are then well-conditioned outputs
     return {"module": _wrap(net, (x, ), training=True), "inputs": (x, ), "gradient": r.normal(shape),
             "buffers": {n: t for n, t in net.named_buffers() if t.dtype.is_floating_point}}
 
@@ -372,11 +372,10 @@ def work(case):
 def tolerance(case):
     """About four times the largest error of any output against the same computation in fp64, over all listed cases and
     forty drawn ones: fp16 encoders 6.5e-4 (largest single difference 4.3e-3), fp16 rows 2.9e-4 (9.6e-4), everything in
-    fp32 1.2e-6 (8.4e-6) but for BatchNorm in training, 5e-6 (1.4e-5; the shift gradient under the squeeze-excite gate is a
-    sum that cancels)."""
+    fp32 1.2e-6 (8.4e-6) but for BatchNorm in training, 5e-6 (2.5e-5; its scale and shift gradients are sums that cancel)."""
     kind, half = case["kind"], case.get("dtype", "f16") == "f16"
     if half and kind in ("encoder", "encoder_module"):
         return {"rel": 2.5e-3, "max": 1.8e-2}
     if half and kind == "rows":
         return {"rel": 1.2e-3, "max": 4e-3}
-    return {"rel": 2e-5, "max": 6e-5} if kind == "mbconv_module" else {"rel": 5e-6, "max": 3.5e-5}
+    return {"rel": 2e-5, "max": 1e-4} if kind == "mbconv_module" else {"rel": 5e-6, "max": 3.5e-5}
