@@ -484,6 +484,10 @@ int dmlhip_batchnorm_backward_act_f32(const void* dy, const void* x, const void*
  * with the interleaved loop: likewise. Products with row sums or K-concatenated operand pairs exist on the 128x128 tile
  * only: 5 and 7 run them with the interleaved loop, 4, 6, 8 and 9 leave them on the plain one. */
 void dmlhip_debug_force_gemm_config(int cfg);
+/* Pin the tile of the fp32 contraction kernel: 0 = 128x128, 1 = 64x64, 2 = 32x32 with K split over the wavefronts;
+ * -1 = chosen per problem (default). Operands that cannot be read 16 bytes at a time have no 128x128 form and run on 64x64.
+ * Per calling thread. */
+void dmlhip_debug_force_gemm_f32_tile(int tile);
 /* 0: the fp16 contractions stage their operands through registers instead of loading them straight into LDS;
  * 1 = default. */
 void dmlhip_debug_gemm_direct_lds(int on);
