@@ -25,6 +25,8 @@ SOURCES = [
     "gemm_f16.hip",
     "gemm_f16_pipe.hip",
     "gemm_f16_pipe_ilv.hip",
+    "gemm_f16_pipe_ragged.hip",
+    "gemm_f16_split.hip",
     "gemm_f32.hip",
     "conv.hip",
     "conv_fused.hip", "conv_backward.hip", "conv_implicit.hip",

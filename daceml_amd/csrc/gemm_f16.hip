@@ -365,6 +365,34 @@ int operand_mode(const void* p, int64_t rows, int64_t k, int64_t s_row, int64_t 
     return 2;
 }
 
+// The configuration with the least estimated time for a product whose 128 x 128 tiles leave (much of) a round of compute
+// units idle. Estimate: fixed + (rounds of resident workgroups - 1) * round + tiles per compute unit * K steps * step, in us,
+// fitted to 330 products of encoder layers (24 - 2048 tokens, 512 - 1024 wide, every operand layout); its choice is within
+// 1 % of the fastest configuration in the mean, 19 % at worst. Decided by it (us, 128-wide tiles / 64 x 64 / 32 x 32):
+// 128 x 1024 x 4096 19 / 15 / 9; 651 x 1024 x 4096 24 / 17 / 23; 651 x 4096 x 1024 11 / 19 / 24; the K-concatenated
+// 651 x 1024 x 3 * 1024 26 / 14 / 22.
+int choose_small(const dmlhip_gemm_desc* d, long long batch, int pairs, bool narrow, bool pipe) {
+    struct Est { int cfg, bm, bn, resident; double fixed, round, step; };
+    constexpr Est kEst[] = {{5, 128, 128, 1, 5.59, 5.36, 0.353}, {7, 128, 128, 2, 5.26, 5.36, 0.484},
+                            {9, 128, 64, 2, 3.22, 1.86, 0.326},  {10, 64, 64, 1, 4.51, 3.35, 0.182},
+                            {12, 32, 32, 2, 3.26, 1.81, 0.100}};
+    const double steps = (double)ceil_div(d->k, (int64_t)BK) * pairs;
+    int best = -1;
+    double best_us = 0;
+    for (const Est& e : kEst) {
+        if ((e.cfg == 9 && !narrow) || (e.cfg < 10 && !pipe)) continue;
+        // an fp32 result is the same bits whatever the tile: one accumulation chain in K order, which a split K is not
+        if (e.cfg >= 10 && d->out_dtype == DMLHIP_F32 && pipe) continue;
+        const double n = (double)ceil_div(ceil_div(d->m, (int64_t)e.bm) * ceil_div(d->n, (int64_t)e.bn) * batch, (int64_t)kCus);
+        const double us = e.fixed + (ceil(n / e.resident) - 1) * e.round + n * steps * e.step;
+        if (best < 0 || us < best_us) {
+            best = e.cfg;
+            best_us = us;
+        }
+    }
+    return best;
+}
+
 // Diagnostic switches (declared in the public header). Per calling thread, so that one thread pinning a configuration
 // does not change what other threads launch.
 thread_local int g_force_cfg = -1;  // pin the tile configuration
@@ -382,7 +410,7 @@ void dmlhip_debug_force_gemm_config(int cfg) { g_force_cfg = cfg; }
 void dmlhip_debug_gemm_direct_lds(int on) { g_direct_lds = on; }
 void dmlhip_debug_gemm_trace(void* buffer) { g_trace = (unsigned long long*)buffer; }
 static std::atomic<long long> g_grouped_single_launches{0};
-// Number of grouped calls that went out as ONE launch (tests check that grouping really happens).
+// Number of grouped calls of whole K steps that went out as ONE launch (tests check that grouping really happens).
 long long dmlhip_debug_grouped_single_launches() { return g_grouped_single_launches.load(); }
 
 struct GemmGroup {
@@ -471,29 +499,33 @@ static int run_gemm_f16(const dmlhip_gemm_desc* d, const void* a, const void* b,
     hipStream_t st = (hipStream_t)stream;
 
     int cfg = g_force_cfg;
-    // Both operands vector-loadable and K a whole number of steps: the fully pipelined kernel.
-    if (amode != 2 && d->k % BK == 0 && d->k > 0 && g_direct_lds &&
-        epilogue_kind(g, bias, residual, pre_out) != EPI_GENERAL_ACT) {
+    // Both operands vector-loadable and K a whole number of steps, or a weight gradient over any number of tokens: the fully
+    // pipelined kernel. The kernel with K split over the wavefronts takes any K.
+    const int ek = epilogue_kind(g, bias, residual, pre_out);
+    const bool ragged = d->k % BK != 0;
+    const bool vec = amode != 2 && d->k > 0 && g_direct_lds && ek != EPI_GENERAL_ACT;
+    const bool pipe = vec && (!ragged || (amode == 1 && bmode == 1 && ek == EPI_PLAIN && !g.ksum));
+    if (vec) {
+        auto blocks = [&](int bm, int bn) { return (long long)ceil_div(d->m, bm) * ceil_div(d->n, bn) * batch; };
+        const bool sums = g.asum || (grp && g.gasum[0]);
+        const bool extra = grp || asum;   // operand pairs / row sums: the 128 x 128 tile only
+        const long long t256 = blocks(256, 256), t128 = blocks(128, 128);
+        const long long slots256 = ceil_div(t256, (long long)kCus) * kCus, slots128 = ceil_div(t128, (long long)kCus) * kCus;
+        if (cfg < 0 && d->k >= 512 && !extra && t256 * 10 >= slots256 * 9) {
+            // Measured on MI355X, alone and inside the BERT layer (4096 x 4096 x 1024: 39 us against 45 - 54 us for
+            // every 128-wide tile; 8192^3: 1176 TFLOP/s): the 256 x 256 tile halves the bytes each compute unit
+            // pulls through L2 and LDS per MFMA, and the interleaved loop keeps its single wavefront per SIMD
+            // issuing MFMAs while transfers and fragment reads are in flight. Only when its tiles fill (nearly) every
+            // round of compute units: 192 tiles on 256 units lose more than the tile gains.
+            cfg = 4;
+        } else if (cfg < 0 && t128 < 2 * kCus && t128 * 10 < slots128 * 9) {
+            cfg = choose_small(d, batch, g.ksum ? g.groups : 1, !extra, pipe);
+        }
         if (cfg < 0) {
-            auto blocks = [&](int bm, int bn) { return (long long)ceil_div(d->m, bm) * ceil_div(d->n, bn) * batch; };
-            const bool extra = grp || asum;   // operand pairs / row sums: the 128 x 128 tile only
-            const long long t256 = blocks(256, 256), t128 = blocks(128, 128);
-            const long long slots256 = ceil_div(t256, (long long)kCus) * kCus;
             if (d->k < 512) {
                 // a handful of K steps (the batched products of an unfused attention): bound by the epilogue, where two
                 // resident workgroups per compute unit overlap one's stores with the other's loads
                 cfg = t128 > kCus ? 3 : 0;
-            } else if (!extra && t256 * 10 >= slots256 * 9) {
-                // Measured on MI355X, alone and inside the BERT layer (4096 x 4096 x 1024: 39 us against 45 - 54 us for
-                // every 128-wide tile; 8192^3: 1176 TFLOP/s): the 256 x 256 tile halves the bytes each compute unit
-                // pulls through L2 and LDS per MFMA, and the interleaved loop keeps its single wavefront per SIMD
-                // issuing MFMAs while transfers and fragment reads are in flight. Only when its tiles fill (nearly) every
-                // round of compute units: 192 tiles on 256 units lose more than the tile gains.
-                cfg = 4;
-            } else if (!extra && t128 <= kCus / 2) {
-                // few tiles and a long K (1024 x 1024 x 4096: 24 us against 29 - 38 us): the 128 x 64 tile doubles the
-                // workgroups, two of them per compute unit
-                cfg = 9;
             } else if (d->k <= 1024 && t128 >= 2 * kCus) {
                 // several rounds of short K loops (the grouped q / k / v projections: 768 tiles of 16 steps): with two
                 // LDS stages instead of four, two workgroups share a compute unit and one's epilogue and first loads
@@ -510,8 +542,13 @@ static int run_gemm_f16(const dmlhip_gemm_desc* d, const void* a, const void* b,
                 cfg = 5;
             }
         }
-        return launch_pipelined(g, (const _Float16*)a, (const _Float16*)b, c, bias, residual, pre_out, amode == 1 ? 4 : 3,
-                                bmode == 1 ? 4 : 3, cfg, batch, st);
+        const _Float16 *pa = (const _Float16*)a, *pb = (const _Float16*)b;
+        if (cfg >= 10 && (!sums || amode == 1))
+            return launch_split(g, pa, pb, c, bias, residual, pre_out, amode, bmode, cfg, batch, st);
+        if (pipe && ragged) return launch_pipelined_ragged(g, pa, pb, c, bias, residual, pre_out, cfg, batch, st);
+        if (pipe)
+            return launch_pipelined(g, pa, pb, c, bias, residual, pre_out, amode == 1 ? 4 : 3, bmode == 1 ? 4 : 3, cfg, batch, st);
+        if (g_force_cfg < 0) cfg = -1;
     }
     if (grp || asum) return DMLHIP_ERR_UNSUPPORTED;  // only the pipelined kernel takes pointer groups / makes row sums
     if (cfg < 0 || cfg > 2) {
@@ -532,14 +569,13 @@ static int run_gemm_f16(const dmlhip_gemm_desc* d, const void* a, const void* b,
     }
 }
 
-// Number of K splits worth taking for this problem (1 = none).
+// Number of K splits worth taking for this problem (1 = none): only where even 64 x 64 tiles leave half of the compute units
+// idle and K is long enough to pay for the second launch (512 x 512 x 16384: 64 workgroups of 256 K steps otherwise).
 static int split_k_factor(const dmlhip_gemm_desc* d) {
-    if (!d || d->m <= 0 || d->n <= 0 || d->k < 1024 || d->batch[0] != 1) return 1;
-    long long batch = d->batch[1] * d->batch[2];
-    const long long tiles = ceil_div(d->m, 128) * ceil_div(d->n, 128) * batch;
-    if (tiles > 128) return 1;
+    if (!d || d->m <= 0 || d->n <= 0 || d->k < 2048 || d->batch[0] != 1) return 1;
+    const long long tiles = ceil_div(d->m, 64) * ceil_div(d->n, 64) * d->batch[1] * d->batch[2];
     int s = 1;
-    while (tiles * s * 2 <= 256 && d->k / (s * 2) >= 256 && d->k % (s * 2 * 64) == 0) s *= 2;
+    while (tiles * s * 2 <= kCus && d->k / (s * 2) >= 1024 && d->k % (s * 2 * BK) == 0) s *= 2;
     return s;
 }
 
@@ -616,7 +652,7 @@ int dmlhip_gemm_f16_grouped(const dmlhip_gemm_desc* d, int groups, const void* c
         p.a_stride_batch[0] = p.b_stride_batch[0] = p.c_stride_batch[0] = 0;   // the outer batch index selects the group
         GemmGroup grp = {groups, a, b, c, bias, false};
         const int e = run_gemm_f16(&p, a[0], b[0], c[0], bias ? bias[0] : nullptr, nullptr, nullptr, stream, &grp);
-        if (e == 0) ++g_grouped_single_launches;
+        if (e == 0 && d->k % BK == 0) ++g_grouped_single_launches;
         if (e != DMLHIP_ERR_UNSUPPORTED) return e;
     }
     for (int i = 0; i < groups; ++i)
@@ -664,7 +700,7 @@ int dmlhip_gemm_f16_grouped_asum(const dmlhip_gemm_desc* d, int groups, const vo
         } else {
             e = run_gemm_f16(d, a[0], b[0], c[0], nullptr, nullptr, nullptr, stream, nullptr, asum, asum_dtype == DMLHIP_F32);
         }
-        if (e == 0) ++g_grouped_single_launches;
+        if (e == 0 && d->k % BK == 0) ++g_grouped_single_launches;
         if (e != DMLHIP_ERR_UNSUPPORTED) return e;
     }
     // products and column sums of the stored [k, m] matrices one after the other
@@ -692,7 +728,7 @@ int dmlhip_gemm_f16_ksum(const dmlhip_gemm_desc* d, int groups, const void* cons
     if (same) {
         GemmGroup grp = {groups, a, b, nullptr, nullptr, true};
         const int e = run_gemm_f16(d, a[0], b[0], c, bias, residual, nullptr, stream, &grp);
-        if (e == 0) ++g_grouped_single_launches;
+        if (e == 0 && d->k % BK == 0) ++g_grouped_single_launches;
         if (e != DMLHIP_ERR_UNSUPPORTED) return e;
     }
     // one product after the other, accumulating in C (rounded to C's type in between)

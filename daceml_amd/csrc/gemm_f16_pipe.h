@@ -13,7 +13,7 @@
 //       c of K row k at slot c ^ ((k & 3) << 2); fragments are two ds_read_b64_tr_b16 — the LDS
 //       transpose read of gfx950 hands every lane four consecutive k of its row, which is exactly the
 //       MFMA operand layout, so no transpose is done in registers or in a separate pass.
-// Requirements (checked by the host): K % 64 == 0, 16-byte aligned bases and strides, rows % 8 == 0
+// Requirements (checked by the host): K % 64 == 0 (RAGGED: any K), 16-byte aligned bases and strides, rows % 8 == 0
 // for RC operands, 32-bit element offsets.
 #pragma once
 
@@ -28,6 +28,8 @@ namespace {
 // A stream owns one operand: where each lane's 16-byte DMA pieces come from, and where each lane
 // reads its MFMA fragments. `T` = number of 32-row MFMA blocks this wavefront multiplies.
 template <int R, int KIND, int T> struct Stream;
+
+__device__ const half8 g_zeros = {0, 0, 0, 0, 0, 0, 0, 0};   // what transfers past the end of K read
 
 template <int R, int T>
 struct Stream<R, 0, T> {  // K-contiguous: tile [R][64 k], chunk c of row r at slot c ^ swz16(r)
@@ -55,6 +57,12 @@ struct Stream<R, 0, T> {  // K-contiguous: tile [R][64 k], chunk c of row r at s
     template <int I>
     __device__ __forceinline__ void issue_one(const _Float16* base, int64_t, int k0, char* tile, int wave) const {
         lds_dma16(base + off[I] + k0, tile + (I * 4 + wave) * 1024);
+    }
+    // the same for a K step of which only `left` < 64 k exist: zeros behind them
+    template <int I>
+    __device__ __forceinline__ void issue_tail(const _Float16* base, int64_t, int k0, int left, char* tile, int wave, int lane) const {
+        const int kl = ((lane & 7) ^ swz16(wave * 8 + (lane >> 3))) * 8;
+        lds_dma16(kl < left ? base + off[I] + k0 : reinterpret_cast<const _Float16*>(&g_zeros), tile + (I * 4 + wave) * 1024);
     }
     template <int KK>
     __device__ __forceinline__ void frags(uint32_t stage_off, half8 (&f)[T]) const {
@@ -115,6 +123,12 @@ struct Stream<R, 1, T> {  // row-contiguous: tile [64 k][R], chunk c (8 rows) of
     __device__ __forceinline__ void issue_one(const _Float16* base, int64_t s_k, int k0, char* tile, int wave) const {
         lds_dma16(base + (int64_t)k0 * s_k + off[I], tile + (I * 4 + wave) * 1024);
     }
+    template <int I>
+    __device__ __forceinline__ void issue_tail(const _Float16* base, int64_t s_k, int k0, int left, char* tile, int wave, int lane) const {
+        const int kl = ((I * 4 + wave) * 1024 + lane * 16) / P;
+        lds_dma16(kl < left ? base + (int64_t)k0 * s_k + off[I] : reinterpret_cast<const _Float16*>(&g_zeros),
+                  tile + (I * 4 + wave) * 1024);
+    }
     template <int KK>
     __device__ __forceinline__ void frags(uint32_t stage_off, half8 (&f)[T]) const {
         static_for<0, T>([&](auto ic) {
@@ -145,12 +159,16 @@ struct Stream<R, 1, T> {  // row-contiguous: tile [64 k][R], chunk c (8 rows) of
 // bursts ahead of the MFMAs (during which the matrix pipe of this SIMD has nothing queued), every MFMA is followed by at
 // most a few fragment reads for the NEXT sub-step and, in the early sub-steps of a K step, by one transfer of the tile
 // that is being refilled: the wavefront's other instructions issue in the shadow of the MFMA before them.
+// RAGGED: the last K step is not a whole one (a weight gradient over a batch whose tokens are no multiple of 64). It is
+// transferred by a copy of the K step of its own, with zeros behind the last k, so the steady state is the same code.
+// 1024 x 1024 x 651, four products grouped with their row sums: 103 us one by one through staging registers, 14 us this way.
 template <int BM, int BN, int WM, int WN, int AKIND, int BKIND, int NSTAGE, int EPI, bool KSUM = false, bool ASUM = false,
-          bool ILV = false>
+          bool ILV = false, bool RAGGED = false>
 __global__ __launch_bounds__(kThreads) void gemm_f16_pipe_kernel(const _Float16* a_ptr, const _Float16* b_ptr, void* c_ptr,
                                                                  const void* bias_ptr, const void* res_ptr,
                                                                  void* pre_ptr, const GemmArgs g) {
     static_assert((BM / WM) * (BN / WN) == kThreads / kWave, "four wavefronts per workgroup");
+    static_assert(!RAGGED || (ILV && !KSUM), "a ragged K exists in the interleaved loop only");
     constexpr int TM = WM / 32, TN = WN / 32;
     constexpr int A_BYTES = BM * kRowBytes, B_BYTES = BN * kRowBytes, STAGE = A_BYTES + B_BYTES;
     constexpr int LPT = BM / 32 + BN / 32;  // DMA instructions per wavefront per tile
@@ -236,7 +254,7 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_pipe_kernel(const _Float16*
 
     // K steps: g.k / BK per operand pair; with ksum the pairs follow each other (the accumulators simply keep
     // running), and the fill cursor (fa, fb, fk) walks pair by pair.
-    const int nkg = g.k / BK;
+    const int nkg = RAGGED ? (g.k + BK - 1) / BK : g.k / BK;
     const int nk = KSUM ? nkg * g.groups : nkg;
     const _Float16* fa = A;
     const _Float16* fb = B;
@@ -257,7 +275,10 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_pipe_kernel(const _Float16*
     // prologue: tiles 0 .. NSTAGE-2 in flight
 #pragma unroll
     for (int s = 0; s < NSTAGE - 1; ++s) {
-        if (s < nk) {
+        if (RAGGED && s == nk - 1) {
+            static_for<0, BM / 32>([&](auto ic) { sa.template issue_tail<decltype(ic)::value>(A, g.sak, s * BK, g.k - s * BK, lds + s * STAGE, wave, lane); });
+            static_for<0, BN / 32>([&](auto ic) { sb.template issue_tail<decltype(ic)::value>(B, g.sbk, s * BK, g.k - s * BK, lds + s * STAGE + A_BYTES, wave, lane); });
+        } else if (s < nk) {
             sa.issue(KSUM ? fa : A, g.sak, (KSUM ? fk : s) * BK, lds + s * STAGE, wave);
             sb.issue(KSUM ? fb : B, g.sbk, (KSUM ? fk : s) * BK, lds + s * STAGE + A_BYTES, wave);
             if constexpr (KSUM) advance();
@@ -293,7 +314,8 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_pipe_kernel(const _Float16*
         // last sub-step. Three copies of the body (filling; draining; the very last step) and no per-slot branches in
         // any of them.
         int kt = 0;
-        auto step = [&](auto fill_c, auto more_c) {
+        auto step = [&](auto fill_c, auto more_c, auto tail_c) {
+            constexpr bool TAIL = decltype(tail_c)::value;   // the tile that is filled is the ragged one
             constexpr bool FILL = decltype(fill_c)::value;
             constexpr bool MORE = decltype(more_c)::value;
             static_assert(MORE || !FILL, "a step that refills the ring is never the last");
@@ -337,7 +359,11 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_pipe_kernel(const _Float16*
                     if constexpr (FILL && kk < DSUB) {
                         static_for<0, LPT>([&](auto dc) {
                             constexpr int d = decltype(dc)::value;
-                            if constexpr ((d * DSLOTS) / LPT == kk * NM + m) {
+                            if constexpr ((d * DSLOTS) / LPT == kk * NM + m && TAIL) {
+                                const int left = g.k - fill_k;
+                                if constexpr (d < NA) sa.template issue_tail<d>(fill_a, g.sak, fill_k, left, fill_tile, wave, lane);
+                                else sb.template issue_tail<d - NA>(fill_b, g.sbk, fill_k, left, fill_tile + A_BYTES, wave, lane);
+                            } else if constexpr ((d * DSLOTS) / LPT == kk * NM + m) {
                                 if constexpr (d < NA) sa.template issue_one<d>(fill_a, g.sak, fill_k, fill_tile, wave);
                                 else sb.template issue_one<d - NA>(fill_b, g.sbk, fill_k, fill_tile + A_BYTES, wave);
                             }
@@ -365,11 +391,17 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_pipe_kernel(const _Float16*
             });
             cur_stage = nxt_stage;
         };
-        for (; kt + NSTAGE - 1 < nk; ++kt) step(std::true_type{}, std::true_type{});
-        if constexpr (NSTAGE > 2) {
-            for (; kt + 1 < nk; ++kt) step(std::false_type{}, std::true_type{});
+        for (; kt + NSTAGE - 1 < nk - (RAGGED ? 1 : 0); ++kt) step(std::true_type{}, std::true_type{}, std::false_type{});
+        if constexpr (RAGGED) {
+            if (kt + NSTAGE - 1 < nk) {
+                step(std::true_type{}, std::true_type{}, std::true_type{});
+                ++kt;
+            }
         }
-        step(std::false_type{}, std::false_type{});  // kt == nk - 1 (the host passes k >= one K step)
+        if constexpr (NSTAGE > 2) {
+            for (; kt + 1 < nk; ++kt) step(std::false_type{}, std::true_type{}, std::false_type{});
+        }
+        step(std::false_type{}, std::false_type{}, std::false_type{});  // kt == nk - 1 (the host passes k >= one K step)
     } else {
         for (int kt = 0; kt < nk; ++kt) {
             const uint32_t cur_off = (uint32_t)cur_stage * STAGE;
@@ -500,7 +532,7 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_pipe_kernel(const _Float16*
     }
 }
 
-template <int BM, int BN, int WM, int WN, int NSTAGE, bool KSUM = false, bool ASUM = false, bool ILV = false>
+template <int BM, int BN, int WM, int WN, int NSTAGE, bool KSUM = false, bool ASUM = false, bool ILV = false, bool RAGGED = false>
 int launch_tile(GemmArgs& g, const _Float16* a, const _Float16* b, void* c, const void* bias, const void* res, void* pre,
                 int akind, int bkind, long long batch, hipStream_t st) {
     g.tiles_m = (g.m + BM - 1) / BM;
@@ -518,7 +550,7 @@ int launch_tile(GemmArgs& g, const _Float16* a, const _Float16* b, void* c, cons
     }
 #define DML_PIPE_CASE(AK, BKD, ACTV)                                                                          \
     if (akind == AK && bkind == BKD && ek == ACTV) {                                                          \
-        auto kern = gemm_f16_pipe_kernel<BM, BN, WM, WN, AK, BKD, NSTAGE, ACTV, KSUM, ASUM, ILV>;                  \
+        auto kern = gemm_f16_pipe_kernel<BM, BN, WM, WN, AK, BKD, NSTAGE, ACTV, KSUM, ASUM, ILV, RAGGED>;          \
         if (lds > 64 * 1024) {                                                                                \
             hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, \
                                                (int)lds);                                                     \
@@ -529,6 +561,11 @@ int launch_tile(GemmArgs& g, const _Float16* a, const _Float16* b, void* c, cons
         }                                                                                                     \
         hipLaunchKernelGGL(kern, (unsigned)total, kThreads, lds, st, a, b, c, bias, res, pre, g);             \
         return launch_status("gemm_f16(pipelined)");                                                          \
+    }
+    if constexpr (RAGGED) {
+        DML_PIPE_CASE(1, 1, EPI_PLAIN)
+        set_error("gemm_f16: a ragged K needs row-contiguous operands and a plain epilogue");
+        return DMLHIP_ERR_UNSUPPORTED;
     }
     DML_PIPE_CASE(0, 0, EPI_PLAIN) DML_PIPE_CASE(0, 1, EPI_PLAIN) DML_PIPE_CASE(1, 0, EPI_PLAIN) DML_PIPE_CASE(1, 1, EPI_PLAIN)
     if constexpr (ASUM) {

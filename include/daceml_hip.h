@@ -478,11 +478,11 @@ int dmlhip_batchnorm_backward_act_f32(const void* dy, const void* x, const void*
  * -1 / 0 / 1 respectively restores the default choice. The counter is process-wide and atomic. */
 /* Pin the tile configuration of the fp16 contraction kernels: 0 = 128x128 tile with a 4-stage ring, 1 = 256x128,
  * 2 = 256x256, 3 = 128x128 with a 2-stage ring; -1 = chosen per problem (default). 4, 5, 6, 7 = the tiles of 2, 0, 1, 3
- * with the interleaved K loop (fragment reads and global->LDS transfers issued one at a time between the MFMAs):
- * never chosen by the library, not yet measured or validated on hardware. 8 = 128x64 tile with a 3-stage ring (twice
- * the workgroups, two per compute unit, for products that give each compute unit a single 128x128 tile), 9 = the same
- * with the interleaved loop: likewise. Products with row sums or K-concatenated operand pairs exist on the 128x128 tile
- * only: 5 and 7 run them with the interleaved loop, 4, 6, 8 and 9 leave them on the plain one. */
+ * with the interleaved K loop (fragment reads and global->LDS transfers issued one at a time between the MFMAs).
+ * 8 = 128x64 tile with a 3-stage ring (twice the workgroups, two per compute unit, for products that give each compute
+ * unit a single 128x128 tile), 9 = the same with the interleaved loop. Products with row sums or K-concatenated operand pairs exist on the 128x128 tile
+ * only: 5 and 7 run them with the interleaved loop, 4, 6, 8 and 9 leave them on the plain one. 10 = 64x64, 12 = 32x32 tile
+ * with K split over the wavefronts (products with too few 128-wide tiles for the chip; any K, every form). */
 void dmlhip_debug_force_gemm_config(int cfg);
 /* Pin the tile of the fp32 contraction kernel: 0 = 128x128, 1 = 64x64, 2 = 32x32 with K split over the wavefronts;
  * -1 = chosen per problem (default). Operands that cannot be read 16 bytes at a time have no 128x128 form and run on 64x64.
@@ -496,7 +496,8 @@ void dmlhip_debug_gemm_direct_lds(int on);
  * LDS, end of the K loop, end of the epilogue) at buffer[4 * workgroup]; NULL (default) switches it off. The caller
  * sizes the buffer for the largest grid it launches. Per calling thread. */
 void dmlhip_debug_gemm_trace(void* buffer);
-/* Number of grouped / K-concatenated / row-sum contraction calls that went out as one launch so far. */
+/* Number of grouped / K-concatenated / row-sum contraction calls that went out as one launch so far, of those whose K is a
+ * multiple of 64. */
 long long dmlhip_debug_grouped_single_launches(void);
 /* Run dmlhip_conv2d_expand_depthwise_f32 on its strip kernel with this output-row strip height (used if it fits LDS);
  * 0 = default (the library's choice of kernel and geometry). */
