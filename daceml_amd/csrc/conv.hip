@@ -540,6 +540,9 @@ int conv_forward(const dmlhip_conv2d_desc* d, const void* x, const void* w, cons
 direct:
     if constexpr (sizeof(T) == 4) {
         // dense convolutions with enough work per output: implicit GEMM on the fp32 matrix pipe
+        bool done;
+        const int e = launch_conv_dense3_f32(g, (const float*)x, (const float*)w, (const float*)bias, (float*)y, st, &done);
+        if (done) return e;
         if (conv_implicit_applicable(g))
             return launch_conv_implicit_f32(g, (const float*)x, (const float*)w, (const float*)bias, (float*)y, st);
     }
@@ -548,6 +551,16 @@ direct:
     return launch_status("conv2d(direct)");
 }
 
+}  // namespace
+}  // namespace dml
+
+namespace dml {
+namespace {
+// per-workgroup-range results of the dense weight gradient: the 3 x 3 kernel's where it applies
+int64_t dense_weight_partials(const ConvGeom& g) {
+    const int64_t parts = conv_dense3_bwd_weight_partials(g);
+    return parts > 0 ? parts : dense_bwd_weight_partials(g.n, g.c, g.m, g.kh, g.kw, g.oh, g.ow, g.h, g.w);
+}
 }  // namespace
 }  // namespace dml
 
@@ -623,6 +636,9 @@ int dmlhip_conv2d_backward_data_f32(const dmlhip_conv2d_desc* d, const void* dy,
     if (is_depthwise_grad(g))
         return launch_depthwise_bwd_data((const float*)dy, (const float*)w, (float*)dx, g.n, g.c, g.h, g.w, g.oh, g.ow, g.kh,
                                          g.sh, st);
+    bool done;
+    const int e = launch_conv_dense3_bwd_data_f32(g, (const float*)dy, (const float*)w, (float*)dx, st, &done);
+    if (done) return e;
     if (conv_implicit_bwd_data_applicable(g))
         return launch_conv_implicit_bwd_data_f32(g, (const float*)dy, (const float*)w, (float*)dx, st);
     hipLaunchKernelGGL(conv_bwd_data_kernel, grid_for(total), 256, 0, st, (const float*)dy, (const float*)w, (float*)dx,
@@ -651,7 +667,7 @@ size_t dmlhip_conv2d_backward_weight_workspace_bytes(const dmlhip_conv2d_desc* d
         return (size_t)g.n * per * sizeof(float) + dmlhip_reduce_workspace_bytes(1, g.n, per);
     }
     if (g.group == 1) {
-        const int64_t parts = dense_bwd_weight_partials(g.n, g.c, g.m, g.kh, g.kw, g.oh, g.ow, g.h, g.w);
+        const int64_t parts = dense_weight_partials(g);
         const int64_t per = (int64_t)g.m * g.c * g.kh * g.kw;
         if (parts > 1) return (size_t)parts * per * sizeof(float) + dmlhip_reduce_workspace_bytes(1, parts, per);
     }
@@ -671,7 +687,7 @@ int dmlhip_conv2d_backward_weight_f32(const dmlhip_conv2d_desc* d, const void* x
     hipStream_t st = (hipStream_t)stream;
     const int64_t dense_parts =
         (!is_pointwise(g) && g.group == 1 && red > 0)
-            ? dense_bwd_weight_partials(g.n, g.c, g.m, g.kh, g.kw, g.oh, g.ow, g.h, g.w) : 0;
+            ? dense_weight_partials(g) : 0;
     if ((is_pointwise(g) || is_depthwise_grad(g) || dense_parts > 0) && red > 0) {
         const size_t need = dmlhip_conv2d_backward_weight_workspace_bytes(d);
         DML_REQUIRE(need == 0 || (workspace && workspace_bytes >= need), DMLHIP_ERR_WORKSPACE,
@@ -692,9 +708,18 @@ int dmlhip_conv2d_backward_weight_f32(const dmlhip_conv2d_desc* d, const void* x
     if (dense_parts > 0) {
         // implicit GEMM over ranges of the (image, pixel) space, then their sum in a fixed order
         float* part = dense_parts > 1 ? (float*)workspace : (float*)dw;
-        if (int e = launch_dense_bwd_weight((const float*)x, (const float*)dy, part, g.n, g.c, g.h, g.w, g.m, g.kh, g.kw,
-                                            g.sh, g.sw, g.ph, g.pw, g.dh, g.dw, g.oh, g.ow, st))
-            return e;
+        const int e = conv_dense3_bwd_weight_partials(g) > 0
+                          ? launch_conv_dense3_bwd_weight(g, (const float*)x, (const float*)dy, part, st)
+                          : launch_dense_bwd_weight((const float*)x, (const float*)dy, part, g.n, g.c, g.h, g.w, g.m, g.kh,
+                                                    g.kw, g.sh, g.sw, g.ph, g.pw, g.dh, g.dw, g.oh, g.ow, st);
+        if (e) return e;
+        if (dense_parts >= 32) {
+            // sixteen wavefronts share the ranges of 64 columns: one pass (128 x 36864: 6 us; the general reduction's two
+            // passes 10). With few ranges most of the sixteen would be idle (4 x 1.2 million: 45 us against 20)
+            hipLaunchKernelGGL((reduce_partials_kernel<OpSum, float>), (unsigned)ceil_div(total, (int64_t)kWave), 1024, 0, st,
+                               (const float*)part, (float*)dw, (int)dense_parts, total, total, 0.f, 1.f, (float*)nullptr, (int64_t)0);
+            return launch_status("conv2d_backward_weight(sum of ranges)");
+        }
         if (dense_parts == 1) return 0;
         const size_t part_bytes = (size_t)dense_parts * total * sizeof(float);
         return dmlhip_reduce_f32(DMLHIP_RSUM, part, dw, DMLHIP_F32, 1, dense_parts, total, (char*)workspace + part_bytes,

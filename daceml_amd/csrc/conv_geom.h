@@ -1,10 +1,37 @@
 // Geometry of a 2-D convolution after validation (all extents fit an int): shared by the convolution sources.
 #pragma once
 
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
 namespace dml {
 
 struct ConvGeom {
     int n, c, h, w, m, kh, kw, sh, sw, ph, pw, dh, dw, group, oh, ow, cg, mg, act;
 };
+
+// conv_dense3.hip: 3 x 3, group 1, with enough work. *applies = false: nothing launched, another kernel has to run
+int launch_conv_dense3_f32(const ConvGeom& g, const float* x, const float* w, const float* bias, float* y, hipStream_t st,
+                           bool* applies);
+int launch_conv_dense3_bwd_data_f32(const ConvGeom& g, const float* dy, const float* w, float* dx, hipStream_t st, bool* applies);
+// conv_dense3_weight.hip: per-range results (m * c * 9 floats each) its weight gradient writes; 0 = does not apply
+int64_t conv_dense3_bwd_weight_partials(const ConvGeom& g);
+int launch_conv_dense3_bwd_weight(const ConvGeom& g, const float* x, const float* dy, float* part, hipStream_t st);
+
+// The data gradient of a dense convolution as a convolution: dX = conv(dY with s - 1 zeros between its elements,
+// W with input / output channels exchanged and the taps reversed, stride 1, padding (k - 1) d - p).
+inline bool data_gradient_problem(const ConvGeom& f, ConvGeom* b) {
+    const int ph = (f.kh - 1) * f.dh - f.ph, pw = (f.kw - 1) * f.dw - f.pw;
+    if (f.group != 1 || ph < 0 || pw < 0) return false;
+    *b = f;
+    b->c = f.m; b->m = f.c;            // channels exchanged
+    b->h = f.oh; b->w = f.ow;          // the input is dY ...
+    b->oh = f.h; b->ow = f.w;          // ... the output dX
+    b->sh = b->sw = 1;
+    b->ph = ph; b->pw = pw;
+    b->cg = b->c; b->mg = b->m;
+    b->act = 0;
+    return true;
+}
 
 }  // namespace dml

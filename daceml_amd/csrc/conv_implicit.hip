@@ -238,22 +238,6 @@ bool plan_implicit(const ConvGeom& g, int ids_h, int ids_w, int wflip, ImplicitP
     return false;
 }
 
-// The data gradient of a dense convolution as a convolution: dX = conv(dY with s - 1 zeros between its elements,
-// W with input / output channels exchanged and the taps reversed, stride 1, padding (k - 1) d - p).
-bool data_gradient_problem(const ConvGeom& f, ConvGeom* b) {
-    const int ph = (f.kh - 1) * f.dh - f.ph, pw = (f.kw - 1) * f.dw - f.pw;
-    if (f.group != 1 || ph < 0 || pw < 0) return false;
-    *b = f;
-    b->c = f.m; b->m = f.c;            // channels exchanged
-    b->h = f.oh; b->w = f.ow;          // the input is dY ...
-    b->oh = f.h; b->ow = f.w;          // ... the output dX
-    b->sh = b->sw = 1;
-    b->ph = ph; b->pw = pw;
-    b->cg = b->c; b->mg = b->m;
-    b->act = DMLHIP_ACT_NONE;
-    return true;
-}
-
 int launch_planned(const ImplicitPlan& pl, const float* x, const float* w, const float* bias, float* y, hipStream_t st,
                    const char* what) {
 #define DML_IG(MT, PT)                                                                                                 \

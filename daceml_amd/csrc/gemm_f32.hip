@@ -67,13 +67,6 @@ __device__ __forceinline__ void lds_dma(const float* gptr, char* lds_dst) {
     else __builtin_amdgcn_global_load_lds(g, l, 4, 0, 0);
 }
 
-template <int OFFSET>
-[[nodiscard]] __device__ __forceinline__ float lds_read_b32(uint32_t addr) {
-    float v;
-    asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFFSET));
-    return v;
-}
-
 // One operand: R tile rows x 32 k per stage, transferred by NW wavefronts, T blocks of 32 rows multiplied per wavefront.
 // ROWS: 0 = LDS rows hold 32 k of one tile row, 1 = LDS rows hold R tile rows of one k. VEC: floats per lane and transfer.
 template <int R, int NW, int T, int ROWS, int VEC>

@@ -37,6 +37,13 @@ template <int OFFSET>
     return v;
 }
 
+template <int OFFSET>
+[[nodiscard]] __device__ __forceinline__ float lds_read_b32(uint32_t addr) {
+    float v;
+    asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFFSET));
+    return v;
+}
+
 // LDS transpose read: within each group of 16 lanes, lane s points at four consecutive 16-bit
 // elements of row s/4 (columns 4*(s%4)..+3 of the group's 16 columns); lane j receives column j of
 // the four rows. A lane thus gets four consecutive K values of "its" column, the MFMA operand layout.

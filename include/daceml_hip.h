@@ -488,6 +488,9 @@ void dmlhip_debug_force_gemm_config(int cfg);
  * -1 = chosen per problem (default). Operands that cannot be read 16 bytes at a time have no 128x128 form and run on 64x64.
  * Per calling thread. */
 void dmlhip_debug_force_gemm_f32_tile(int tile);
+/* Diagnostic: pin the tile of the calling thread's dense 3 x 3 fp32 convolutions and data gradients (0 = 32 channels x 128
+   pixels, 1 = 32 x 64, 2 = 32 x 32; -1 = the library chooses). */
+void dmlhip_debug_force_conv_dense3_tile(int tile);
 /* 0: the fp16 contractions stage their operands through registers instead of loading them straight into LDS;
  * 1 = default. */
 void dmlhip_debug_gemm_direct_lds(int on);

@@ -23,6 +23,13 @@ inline half8 lds_read_b128(uint32_t addr) {
     return v;
 }
 
+template <int OFFSET>
+inline float lds_read_b32(uint32_t addr) {
+    float v;
+    memcpy(&v, emu::g_lds + addr + OFFSET, 4);
+    return v;
+}
+
 // ds_read_b64_tr_b16: within each group of 16 lanes, lane s supplies the address of four consecutive 16-bit elements;
 // the 16 x 4 elements form rows s / 4 (four lanes side by side make one row of 16); lane j receives element j of each
 // of the four rows
