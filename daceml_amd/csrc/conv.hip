@@ -515,6 +515,10 @@ int conv_forward(const dmlhip_conv2d_desc* d, const void* x, const void* w, cons
         return sizeof(T) == 2 ? dmlhip_gemm_f16(&gd, w, x, y, bias, nullptr, nullptr, stream)
                               : dmlhip_gemm_f32(&gd, w, x, y, bias, nullptr, nullptr, stream);
     }
+    if constexpr (sizeof(T) == 4) {
+        if (depthwise_same_applicable(g))
+            return launch_depthwise_same(g, (const float*)x, (const float*)w, (const float*)bias, (float*)y, st);
+    }
     // depthwise with a small square-ish stencil
     if (g.group == g.c && g.m == g.c && ((g.kh == 3 && g.kw == 3) || (g.kh == 5 && g.kw == 5))) {
         if (g.pw > kDwLeft) goto direct;
@@ -633,6 +637,8 @@ int dmlhip_conv2d_backward_data_f32(const dmlhip_conv2d_desc* d, const void* dy,
         gd.alpha = 1.f; gd.out_dtype = DMLHIP_F32; gd.bias_dtype = DMLHIP_F32;
         return dmlhip_gemm_f32(&gd, w, dy, dx, nullptr, nullptr, nullptr, stream);
     }
+    if (depthwise_same_applicable(g))
+        return launch_depthwise_same_bwd_data(g, (const float*)dy, (const float*)w, (float*)dx, st);
     if (is_depthwise_grad(g))
         return launch_depthwise_bwd_data((const float*)dy, (const float*)w, (float*)dx, g.n, g.c, g.h, g.w, g.oh, g.ow, g.kh,
                                          g.sh, st);
@@ -697,9 +703,11 @@ int dmlhip_conv2d_backward_weight_f32(const dmlhip_conv2d_desc* d, const void* x
         // one result per (image, channel) plane, summed over the images in a fixed order
         const int64_t per = (int64_t)g.c * g.kh * g.kw;
         float* part = g.n > 1 ? (float*)workspace : (float*)dw;
-        if (int e = launch_depthwise_bwd_weight((const float*)x, (const float*)dy, part, g.n, g.c, g.h, g.w, g.oh, g.ow,
-                                                g.kh, g.sh, g.ph, st))
-            return e;
+        const int e = depthwise_same_applicable(g)
+                          ? launch_depthwise_same_bwd_weight(g, (const float*)x, (const float*)dy, part, st)
+                          : launch_depthwise_bwd_weight((const float*)x, (const float*)dy, part, g.n, g.c, g.h, g.w, g.oh, g.ow,
+                                                        g.kh, g.sh, g.ph, st);
+        if (e) return e;
         if (g.n == 1) return 0;
         const size_t part_bytes = (size_t)g.n * per * sizeof(float);
         return dmlhip_reduce_f32(DMLHIP_RSUM, part, dw, DMLHIP_F32, 1, g.n, per, (char*)workspace + part_bytes,

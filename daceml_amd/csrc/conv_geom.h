@@ -18,6 +18,12 @@ int launch_conv_dense3_bwd_data_f32(const ConvGeom& g, const float* dy, const fl
 int64_t conv_dense3_bwd_weight_partials(const ConvGeom& g);
 int launch_conv_dense3_bwd_weight(const ConvGeom& g, const float* x, const float* dy, float* part, hipStream_t st);
 
+// conv_depthwise.hip: depthwise 3 x 3 / 5 x 5, stride 1, output as large as the input
+bool depthwise_same_applicable(const ConvGeom& g);
+int launch_depthwise_same(const ConvGeom& g, const float* x, const float* w, const float* bias, float* y, hipStream_t st);
+int launch_depthwise_same_bwd_data(const ConvGeom& g, const float* dy, const float* w, float* dx, hipStream_t st);
+int launch_depthwise_same_bwd_weight(const ConvGeom& g, const float* x, const float* dy, float* part, hipStream_t st);
+
 // The data gradient of a dense convolution as a convolution: dX = conv(dY with s - 1 zeros between its elements,
 // W with input / output channels exchanged and the taps reversed, stride 1, padding (k - 1) d - p).
 inline bool data_gradient_problem(const ConvGeom& f, ConvGeom* b) {
