@@ -24,6 +24,11 @@ int launch_depthwise_same(const ConvGeom& g, const float* x, const float* w, con
 int launch_depthwise_same_bwd_data(const ConvGeom& g, const float* dy, const float* w, float* dx, hipStream_t st);
 int launch_depthwise_same_bwd_weight(const ConvGeom& g, const float* x, const float* dy, float* part, hipStream_t st);
 
+// conv_pointwise_few.hip: 1 x 1, few input channels, many output channels; w_transposed: w is [cin][cout]
+bool pointwise_few_applicable(int64_t n, int64_t cin, int64_t cout, int64_t hw);
+int launch_pointwise_few(const float* x, const float* w, const float* bias, float* y, int n, int cin, int cout, int64_t hw,
+                         int act, bool w_transposed, hipStream_t st);
+
 // The data gradient of a dense convolution as a convolution: dX = conv(dY with s - 1 zeros between its elements,
 // W with input / output channels exchanged and the taps reversed, stride 1, padding (k - 1) d - p).
 inline bool data_gradient_problem(const ConvGeom& f, ConvGeom* b) {
