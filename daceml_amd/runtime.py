@@ -126,8 +126,8 @@ class CompiledSDFG:
             expand_onnx_nodes(sdfg)
         self._keep = []                       # ctypes objects that must outlive the launches
         self._ptr: Dict[str, ctypes.c_void_p] = {}
-        self._derived = []                    # (c_void_p, base name, byte offset)
-        self._ptr_arrays = []                 # (ctypes array, [(slot, name)])
+        self._derived = []                    # (c_void_p, c_void_p of the base, byte offset)
+        self._ptr_arrays = []                 # (ctypes array, [(slot, c_void_p)])
         self._stream = ctypes.c_void_p(0)
         self._binding = 0                     # bumped whenever a pointer may have changed
         self.buffers: Dict[str, torch.Tensor] = {}
@@ -144,6 +144,8 @@ class CompiledSDFG:
         self._workspace = torch.empty(self._ws_bytes, dtype=torch.uint8, device=self.device)
         for state, node in self._order:
             self._bind_node(state, node)
+        # what a call has to pass, looked up once: a small program's step is bound by what the host does per call
+        self._arguments = [(name, self._ptr[name], d.dtype, d.shape, d.strides) for name, d in self.arglist().items()]
         self._refresh()
 
     # -- memory ------------------------------------------------------------
@@ -152,7 +154,7 @@ class CompiledSDFG:
             self._ptr[name] = ctypes.c_void_p(0)
         for name, desc in self.sdfg.arrays.items():
             if desc.view_of is not None:
-                self._derived.append((self._ptr[name], desc.view_of, desc.view_offset * _ITEM[desc.dtype]))
+                self._derived.append((self._ptr[name], self._ptr[desc.view_of], desc.view_offset * _ITEM[desc.dtype]))
             elif name in self.sdfg.constants:
                 t = self.sdfg.constants[name].to(device=self.device, dtype=desc.dtype).contiguous()
                 if tuple(t.shape) != desc.shape:
@@ -175,14 +177,13 @@ class CompiledSDFG:
         for name, t in self.buffers.items():
             self._ptr[name].value = t.data_ptr()
 
-    def _refresh(self, changed: bool = True):
-        if changed:
-            self._binding += 1
+    def _refresh(self):
+        self._binding += 1
         for obj, base, off in self._derived:
-            obj.value = (self._ptr[base].value or 0) + off
+            obj.value = (base.value or 0) + off
         for arr, slots in self._ptr_arrays:
-            for i, name in slots:
-                arr[i] = self._ptr[name].value
+            for i, ptr in slots:
+                arr[i] = ptr.value
 
     # -- binding -----------------------------------------------------------
     def _bind_node(self, state: SDFGState, node):
@@ -204,7 +205,7 @@ class CompiledSDFG:
                     name = conn_to_array[a.conn]
                     if a.offset:
                         obj = ctypes.c_void_p(0)
-                        self._derived.append((obj, name, a.offset * _ITEM[self.sdfg.arrays[name].dtype]))
+                        self._derived.append((obj, self._ptr[name], a.offset * _ITEM[self.sdfg.arrays[name].dtype]))
                         args.append(obj)
                     else:
                         args.append(self._ptr[name])
@@ -226,7 +227,7 @@ class CompiledSDFG:
                     args.append(arr)
                 elif isinstance(a, T.PtrArray):
                     arr = (ctypes.c_void_p * len(a.conns))()
-                    self._ptr_arrays.append((arr, [(i, conn_to_array[c]) for i, c in enumerate(a.conns)]))
+                    self._ptr_arrays.append((arr, [(i, self._ptr[conn_to_array[c]]) for i, c in enumerate(a.conns)]))
                     args.append(arr)
                 elif isinstance(a, T.Struct):
                     self._keep.append(a.value)
@@ -247,10 +248,8 @@ class CompiledSDFG:
 
     # -- execution -----------------------------------------------------------
     def _bind_arguments(self, kwargs: Dict[str, torch.Tensor], partial: bool = False):
-        changed = False
-        for name, desc in self.sdfg.arrays.items():
-            if desc.transient or name in self.sdfg.constants or desc.view_of is not None:
-                continue
+        found = []
+        for name, ptr, dtype, shape, strides in self._arguments:
             if name not in kwargs:
                 if partial:
                     continue
@@ -258,18 +257,21 @@ class CompiledSDFG:
             t = kwargs[name]
             if not isinstance(t, torch.Tensor) or t.device != self.device:
                 raise ValueError("argument %r must be a tensor on %s" % (name, self.device))
-            if t.dtype != desc.dtype or tuple(t.shape) != desc.shape:
-                raise ValueError("argument %r: expected %s %s, got %s %s" % (name, desc.dtype, desc.shape, t.dtype,
-                                                                             tuple(t.shape)))
-            if tuple(t.stride()) != desc.strides and t.numel() > 1:
-                raise ValueError("argument %r must have strides %s (pass a contiguous tensor)" % (name, desc.strides))
-            if self._ptr[name].value != t.data_ptr():
+            if t.dtype != dtype or t.shape != shape:
+                raise ValueError("argument %r: expected %s %s, got %s %s" % (name, dtype, shape, t.dtype, tuple(t.shape)))
+            if t.stride() != strides and t.numel() > 1:
+                raise ValueError("argument %r must have strides %s (pass a contiguous tensor)" % (name, strides))
+            found.append((ptr, t.data_ptr()))
+        for name in kwargs:
+            if name not in self.sdfg.arrays:
+                raise TypeError("unknown argument(s) %s" % sorted(set(kwargs) - set(self.sdfg.arrays)))
+        changed = False   # a refused call has changed nothing: the derived pointers are those of the last binding
+        for ptr, address in found:
+            if (ptr.value or 0) != address:   # a c_void_p that holds NULL reads as None
+                ptr.value = address
                 changed = True
-            self._ptr[name].value = t.data_ptr()
-        extra = set(kwargs) - set(self.sdfg.arrays)
-        if extra:
-            raise TypeError("unknown argument(s) %s" % sorted(extra))
-        self._refresh(changed)
+        if changed:
+            self._refresh()
 
     def arglist(self) -> Dict[str, Array]:
         return {k: v for k, v in self.sdfg.arrays.items()
@@ -299,10 +301,12 @@ class CompiledSDFG:
             if t.dtype != desc.dtype or tuple(t.shape) != desc.shape or not t.is_contiguous() or t.device != self.device:
                 raise ValueError("buffer for %r must be a dense %s %s tensor on %s" % (name, desc.dtype, desc.shape,
                                                                                         self.device))
+        for name, t in tensors.items():
             self._ptr[name].value = t.data_ptr()
             if release:
                 self.buffers[name] = t
-        self._refresh()
+        if tensors:
+            self._refresh()
 
     def launch(self, states: Optional[Sequence[str]] = None):
         """Enqueue every kernel (of the named states) on the current stream, with the pointers of the
