@@ -133,8 +133,9 @@ __global__ __launch_bounds__(kThreads) void conv_dense3_weight_kernel(const Weig
         const uint32_t x_row = so + (uint32_t)(g.a_bytes + l32 * g.plane * 4);
         const int pairs = (cur.px + 1) / 2;
         int sent = more ? 0 : mine;
-        // Pair i of pixels: 2 i in the lower lane half, 2 i + 1 in the upper. Reads run one pair ahead, the offsets two; every
-        // iteration waits for what it issued, so nothing is in flight when the loop ends.
+        // Pair i of pixels: 2 i in the lower lane half, 2 i + 1 in the upper. Reads run one pair ahead, the offsets two. Every
+        // pair waits for what it issued and keeps it up to there: behind the last pairs of a chunk nothing multiplies what
+        // was read ahead, and registers without a use would go to the transfers' addresses while the data is on its way.
         float a[2], b[2][kTaps];
         int off;
         auto read_b = [&](float (&v)[kTaps], int o) {
@@ -165,6 +166,10 @@ __global__ __launch_bounds__(kThreads) void conv_dense3_weight_kernel(const Weig
             }
             wait_lgkm<0>();
             __builtin_amdgcn_sched_barrier(0);
+            lds_keep(a_next);
+#pragma unroll
+            for (int t = 0; t < kTaps; ++t) lds_keep(b_next[t]);
+            lds_keep(off);
         };
         if (own > 0) {
             off = __builtin_bit_cast(int, lds_read_b32<0>(lds0 + pixel(kg)));

@@ -76,4 +76,11 @@ __device__ __forceinline__ void wait_vm_lgkm0() {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(VM) : "memory");
 }
 
+// The other way to consume a value: for the compiler it is used here, so its registers stay its own up to this point. For
+// reads that run ahead of a loop and are not multiplied when the loop ends; placed behind the wait that covers them.
+template <typename T>
+__device__ __forceinline__ void lds_keep(T v) {
+    asm volatile("" ::"v"(v));
+}
+
 }  // namespace dml

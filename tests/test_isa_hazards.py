@@ -69,6 +69,19 @@ def test_interleaved_gemm_loop(tmp_path):
     assert not found, _report(found)
 
 
+def _kernel_count(asm, name):
+    return sum(name in symbol and bool(body) for symbol, body in isa_hazards.kernels(asm))
+
+
+def test_dense_convolution_weight_gradient(tmp_path):
+    """The last pairs of pixels of a chunk read ahead for a pair that does not come, and transfers of the next chunk issue
+    before their wait."""
+    asm = _assembly(os.path.join(ROOT, "daceml_amd", "csrc", "conv_dense3_weight.hip"), tmp_path)
+    assert _kernel_count(asm, "conv_dense3_weight_kernel") == 8
+    found = isa_hazards.check_file(asm)[1]
+    assert not found, _report(found)
+
+
 def test_wide_stores_in_inline_assembly_carry_their_wait_states(tmp_path):
     """lds_ops.h stores GEMM results with an inline-assembly ``global_store_dwordx4 ... sc1``; the two wait states the
     compiler would have kept between such a store and the next write to its data registers are part of the statement."""
