@@ -65,6 +65,15 @@ __device__ __forceinline__ void lds_dma(const float* gptr, char* lds_dst) {
     else __builtin_amdgcn_global_load_lds(g, l, 4, 0, 0);
 }
 
+// Offset of the filter of a (channel, channel) pair. The product and the sum that follows are kept apart: as one 64-bit
+// multiply-add the sum's operand has a high half that nothing wrote, and the register it names may belong to an LDS read in
+// flight - harmless, its result is cut off, but the same to see as the hazard that lds_ops.h describes.
+__device__ __forceinline__ uint32_t taps_of(uint32_t pair) {
+    uint32_t at = pair * kTaps;
+    asm volatile("" : "+v"(at));
+    return at;
+}
+
 // The weights of a step in LDS. Forward: rows of one output channel, 9 CH floats and 4 of padding (16 rows 12 or 36 banks
 // apart start in 16 different groups of four banks). FLIP: as they lie in memory for one input channel, [CH][MB][9].
 template <int MB, int CH, bool FLIP, int VEC>
@@ -83,11 +92,11 @@ struct Weights {
         if constexpr (FLIP) {      // W is [input channel of this product][output channel][9]
             const int ch = f / (MB * kTaps), j = f % (MB * kTaps);
             ok = f < FLOATS && c0 + ch < g.c && j < (g.m - m0) * kTaps;
-            src = g.w + (uint32_t)(((c0 + ch) * g.m + m0) * kTaps + j);
+            src = g.w + (taps_of((uint32_t)((c0 + ch) * g.m + m0)) + (uint32_t)j);
         } else {
             const int row = f / PITCH, k = f % PITCH;
             ok = row < MB && m0 + row < g.m && k < min(CH, g.c - c0) * kTaps;
-            src = g.w + (uint32_t)(((m0 + row) * g.c + c0) * kTaps + k);
+            src = g.w + (taps_of((uint32_t)((m0 + row) * g.c + c0)) + (uint32_t)k);
         }
         if (!ok) src = reinterpret_cast<const float*>(&g_zeros);
         lds_dma<VEC * 4>(src, dst + (i * 4 + wave) * 64 * VEC * 4);

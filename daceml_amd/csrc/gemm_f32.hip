@@ -231,17 +231,7 @@ __global__ __launch_bounds__(kWave * WPG * KG) void gemm_f32_kernel(GemmArgs32 g
     typedef std::integral_constant<int, 0> i0;
     typedef std::integral_constant<int, 1> i1;
     typedef std::integral_constant<int, 2> i2;
-#pragma unroll
-    for (int s = 0; s < NSTAGE; ++s)
-        if (s < nk) issue(s, s, i0{}, i1{});
-    if (NSTAGE <= nk) wait_vm_lgkm0<(NSTAGE - 1) * LPT>();
-    else wait_vm_lgkm0<0>();
-    if constexpr (WPG > 1) __builtin_amdgcn_s_barrier();
     floatx4 af[2][T], bf[2][T];
-    if (nk > 0) {
-        sa.template frags<0>(0u, af[0]);
-        sb.template frags<0>(0u, bf[0]);
-    }
     int stage = 0;
     // One K step of four sub-steps. Reads of the next sub-step, the barrier and the refill of the ring all issue behind
     // MFMAs that are already queued. MORE: another step follows, whose first fragments are read under the last sub-step.
@@ -283,8 +273,20 @@ __global__ __launch_bounds__(kWave * WPG * KG) void gemm_f32_kernel(GemmArgs32 g
         });
         stage = nxt;
     };
-    for (int t = 0; t + 1 < nk; ++t) step(t, std::true_type{});
-    if (nk > 0) step(nk - 1, std::false_type{});
+    // one branch round all of it: a path on which the last step, which multiplies what was read ahead, is missing would leave
+    // those reads unused (lds_ops.h)
+    if (nk > 0) {
+#pragma unroll
+        for (int s = 0; s < NSTAGE; ++s)
+            if (s < nk) issue(s, s, i0{}, i1{});
+        if (NSTAGE <= nk) wait_vm_lgkm0<(NSTAGE - 1) * LPT>();
+        else wait_vm_lgkm0<0>();
+        if constexpr (WPG > 1) __builtin_amdgcn_s_barrier();
+        sa.template frags<0>(0u, af[0]);
+        sb.template frags<0>(0u, bf[0]);
+        for (int t = 0; t + 1 < nk; ++t) step(t, std::true_type{});
+        step(nk - 1, std::false_type{});
+    }
     wait_vm_lgkm0<0>();
 
     // element e of a block: row (e / 4) * 8 + (lane / 32) * 4 + e % 4, column lane % 32

@@ -1,4 +1,4 @@
-"""The kernels that place their own LDS reads and waits (fused attention, the interleaved GEMM loop) are compiled to
+"""The kernels that place their own LDS reads and waits (fused attention, contractions, dense convolutions) are compiled to
 assembly and checked: no instruction touches a register that an outstanding LDS read still has to write
 (tests/isa_hazards.py says why that can happen). Needs hipcc, no GPU."""
 import os
@@ -78,6 +78,19 @@ def test_dense_convolution_weight_gradient(tmp_path):
     before their wait."""
     asm = _assembly(os.path.join(ROOT, "daceml_amd", "csrc", "conv_dense3_weight.hip"), tmp_path)
     assert _kernel_count(asm, "conv_dense3_weight_kernel") == 8
+    found = isa_hazards.check_file(asm)[1]
+    assert not found, _report(found)
+
+
+@pytest.mark.parametrize("src,kernel,count", [
+    ("daceml_amd/csrc/gemm_f32.hip", "gemm_f32_kernel", 36),              # 4 + 16 + 16: tiles x operand layouts
+    ("daceml_amd/csrc/conv_dense3.hip", "conv_dense3_f32_kernel", 24),    # tiles x direction x transfers of W and X
+    ("daceml_amd/csrc/gemm_f16_split.hip", "gemm_f16_split_kernel", 44),
+    ("tests/isa/ragged_instances.hip", "gemm_f16_pipe_kernel", 6),        # the translation unit takes minutes to compile
+])
+def test_streamed_products_and_convolutions(src, kernel, count, tmp_path):
+    asm = _assembly(os.path.join(ROOT, *src.split("/")), tmp_path)
+    assert _kernel_count(asm, kernel) == count
     found = isa_hazards.check_file(asm)[1]
     assert not found, _report(found)
 
