@@ -410,7 +410,7 @@ void dmlhip_debug_force_gemm_config(int cfg) { g_force_cfg = cfg; }
 void dmlhip_debug_gemm_direct_lds(int on) { g_direct_lds = on; }
 void dmlhip_debug_gemm_trace(void* buffer) { g_trace = (unsigned long long*)buffer; }
 static std::atomic<long long> g_grouped_single_launches{0};
-// Number of grouped calls of whole K steps that went out as ONE launch (tests check that grouping really happens).
+// Number of grouped calls that went out as ONE launch (tests check that grouping really happens).
 long long dmlhip_debug_grouped_single_launches() { return g_grouped_single_launches.load(); }
 
 struct GemmGroup {
@@ -652,7 +652,7 @@ int dmlhip_gemm_f16_grouped(const dmlhip_gemm_desc* d, int groups, const void* c
         p.a_stride_batch[0] = p.b_stride_batch[0] = p.c_stride_batch[0] = 0;   // the outer batch index selects the group
         GemmGroup grp = {groups, a, b, c, bias, false};
         const int e = run_gemm_f16(&p, a[0], b[0], c[0], bias ? bias[0] : nullptr, nullptr, nullptr, stream, &grp);
-        if (e == 0 && d->k % BK == 0) ++g_grouped_single_launches;
+        if (e == 0) ++g_grouped_single_launches;
         if (e != DMLHIP_ERR_UNSUPPORTED) return e;
     }
     for (int i = 0; i < groups; ++i)
@@ -700,7 +700,7 @@ int dmlhip_gemm_f16_grouped_asum(const dmlhip_gemm_desc* d, int groups, const vo
         } else {
             e = run_gemm_f16(d, a[0], b[0], c[0], nullptr, nullptr, nullptr, stream, nullptr, asum, asum_dtype == DMLHIP_F32);
         }
-        if (e == 0 && d->k % BK == 0) ++g_grouped_single_launches;
+        if (e == 0) ++g_grouped_single_launches;
         if (e != DMLHIP_ERR_UNSUPPORTED) return e;
     }
     // products and column sums of the stored [k, m] matrices one after the other
@@ -728,7 +728,7 @@ int dmlhip_gemm_f16_ksum(const dmlhip_gemm_desc* d, int groups, const void* cons
     if (same) {
         GemmGroup grp = {groups, a, b, nullptr, nullptr, true};
         const int e = run_gemm_f16(d, a[0], b[0], c, bias, residual, nullptr, stream, &grp);
-        if (e == 0 && d->k % BK == 0) ++g_grouped_single_launches;
+        if (e == 0) ++g_grouped_single_launches;
         if (e != DMLHIP_ERR_UNSUPPORTED) return e;
     }
     // one product after the other, accumulating in C (rounded to C's type in between)

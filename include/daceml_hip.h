@@ -499,8 +499,7 @@ void dmlhip_debug_gemm_direct_lds(int on);
  * LDS, end of the K loop, end of the epilogue) at buffer[4 * workgroup]; NULL (default) switches it off. The caller
  * sizes the buffer for the largest grid it launches. Per calling thread. */
 void dmlhip_debug_gemm_trace(void* buffer);
-/* Number of grouped / K-concatenated / row-sum contraction calls that went out as one launch so far, of those whose K is a
- * multiple of 64. */
+/* Number of grouped / K-concatenated / row-sum contraction calls that went out as one launch so far. */
 long long dmlhip_debug_grouped_single_launches(void);
 /* Run dmlhip_conv2d_expand_depthwise_f32 on its strip kernel with this output-row strip height (used if it fits LDS);
  * 0 = default (the library's choice of kernel and geometry). */

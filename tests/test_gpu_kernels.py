@@ -798,7 +798,8 @@ def test_einsum_sum(eq, sa, sb, n, with_res, out_dtype, single):
     ((2, 256, 256), (2, 256, 128), 3, torch.float32, True),    # grouped; two tile rows
     ((4, 128, 384), (4, 128, 192), 4, torch.float16, True),    # three tile rows, two tile columns
     ((2, 256, 200), (2, 256, 72), 2, torch.float32, True),     # ragged m and n: clamped rows must not reach the sums
-    ((3, 50, 128), (3, 50, 64), 2, torch.float32, False),      # K = 150: separate products and column reductions
+    ((3, 50, 128), (3, 50, 64), 2, torch.float32, True),       # K = 150: the last K step is not a whole one
+    ((3, 50, 100), (3, 50, 64), 2, torch.float32, False),      # m % 8 != 0: separate products and column reductions
 ])
 def test_einsum_grouped_asum(sa, sb, n, sum_dtype, single):
     """dW_i = einsum("aij,aik->jk", dY_i, X_i) together with db_i = dY_i.sum((0, 1)) from the same launch."""
