@@ -31,6 +31,7 @@ constexpr int kTaps = 9;
 constexpr int kMaxPieces = 4;     // 256-float pieces of a channel's rectangle
 constexpr int kHalf = 2;          // channels per lane half of an MFMA and step
 constexpr int kCus = 256;
+constexpr int64_t kMaxBlocks = (1 << 24) - 1;   // of 256 threads: a grid has less than 2^32 threads
 
 __device__ const floatx4 g_zeros = {0.f, 0.f, 0.f, 0.f};   // what lanes outside an operand read
 
@@ -316,10 +317,13 @@ __global__ __launch_bounds__(256) void conv_dense3_f32_kernel(const Dense3Args g
 
 // Tile t: 128 >> t pixels, 1 << t wavefronts that split the input channels, 4 << t of them per step. The one with the least
 // estimated time is taken: a step of a workgroup that has its compute unit to itself, and of one among several, in us as
-// measured, and 3 us for first loads and stores per round of resident workgroups. What it decides (n x c x size -> m, us for
-// the three tiles): 32x64x56->64 87 / 87 / 130, 12x128x28->128 51 / 40 / 46, 1x256x14->256 77 / 52 / 41.
+// measured, and 3 us for first loads and stores per round of resident workgroups. X that moves 4 bytes per lane adds to a step
+// for every transfer: its instructions, and LDS that leaves no room for another workgroup. What it decides (n x c x size -> m,
+// us for the three tiles): 32x64x56->64 87 / 87 / 130, 12x128x28->128 51 / 40 / 46, 1x256x14->256 77 / 52 / 41; of odd sizes
+// 32x32x114->64 211 / 345 / 938, 12x128x29->128 62 / 50 / 76, 4x128x29->128 47 / 32 / 31.
 constexpr int kTiles = 3;
 constexpr double kStepAlone[kTiles] = {1.15, 1.5, 2.2}, kStepShared[kTiles] = {0.76, 0.8, 1.05};
+constexpr double kNarrowTransfer[kTiles] = {0.004, 0.004, 0.008};
 
 struct Dense3Plan {
     Dense3Args a;
@@ -364,8 +368,10 @@ int launch_form(const Dense3Plan& pl, hipStream_t st, const char* what) {
 }  // namespace
 
 // The geometry is the product's own: for a data gradient the stride-1 convolution of the (zero-dilated) dY. False where a
-// tile's rectangle is too large for LDS or an extent for 32-bit arithmetic.
-static bool plan_conv_dense3(const ConvGeom& g, int ids_h, int ids_w, bool flip, const void* x, const void* w, Dense3Plan* pl) {
+// tile's rectangle is too large for LDS, an extent for 32-bit arithmetic or the grid, or where the general kernel applies
+// (`general`) and is the faster one.
+static bool plan_conv_dense3(const ConvGeom& g, int ids_h, int ids_w, bool flip, bool general, const void* x, const void* w,
+                             Dense3Plan* pl) {
     if (g.kh != 3 || g.kw != 3 || g.group != 1 || g.n < 1 || g.c < 4 || g.m < 1 || g.oh < 1 || g.ow < 1) return false;
     const int64_t ohw = (int64_t)g.oh * g.ow, total = (int64_t)g.n * ohw;
     if ((double)total * g.m * g.c * kTaps < (double)(1 << 24)) return false;     // tiny: the direct kernel
@@ -383,6 +389,8 @@ static bool plan_conv_dense3(const ConvGeom& g, int ids_h, int ids_w, bool flip,
     a.img_rows = (int)img_rows; a.ids_h = ids_h; a.ids_w = ids_w; a.total_px = (int)total;
     pl->vec = aligned16(w) && (flip ? g.m : g.c) % 4 == 0 ? 4 : 1;
     double best = 0;
+    int64_t best_per_cu = 0;
+    bool widest = false;          // the tile of 128 pixels fits
     pl->tile = -1;
     for (int t = 0; t < kTiles; ++t) {
         if (g_force_tile >= 0 && t != g_force_tile) continue;
@@ -401,12 +409,15 @@ static bool plan_conv_dense3(const ConvGeom& g, int ids_h, int ids_w, bool flip,
         const size_t lds = 2 * ((size_t)x_bytes + weight_bytes(t, flip, pl->vec));
         if (lds > 160 * 1024) continue;
         const int64_t tiles_m = ceil_div(g.m, 32), blocks = tiles_m * ceil_div(total, (int64_t)px);
-        if (blocks > 2147483647LL) continue;
+        if (blocks > kMaxBlocks) continue;
+        if (t == 0) widest = true;
         const double steps = (double)ceil_div(g.c, ch);
-        const double per_cu = (double)ceil_div(blocks, (int64_t)kCus);
-        const double us = steps * fmax(kStepAlone[t], kStepShared[t] * per_cu) + 3.0 * ceil(per_cu / 3);
+        const int64_t per_cu = ceil_div(blocks, (int64_t)kCus);
+        const double narrow = pl->xvec == 1 ? kNarrowTransfer[t] * ch * (double)ceil_div(rect, (int64_t)64) : 0.0;
+        const double us = steps * fmax(kStepAlone[t] + narrow, (kStepShared[t] + narrow) * (double)per_cu) + 3.0 * ceil((double)per_cu / 3);
         if (pl->tile >= 0 && us >= best) continue;
         best = us;
+        best_per_cu = per_cu;
         pl->tile = t;
         pl->lds = lds;
         pl->blocks = (unsigned)blocks;
@@ -415,13 +426,21 @@ static bool plan_conv_dense3(const ConvGeom& g, int ids_h, int ids_w, bool flip,
         a.x_bytes = x_bytes;
         a.tiles_m = (int)tiles_m;
     }
-    return pl->tile >= 0;
+    if (pl->tile < 0) return false;
+    // With more than two workgroups per compute unit the general kernel is the faster one in two cases.
+    // X in 4-byte pieces whose rectangles under 128 pixels do not fit, stride 2 over wide rows (32x32x113->64 74 us against 155;
+    // up to two per unit 19 - 20 against 9 - 19). And one or two steps: 5 to 15 channels, unless X moves 16 bytes at a time for a
+    // single tile of output channels (32x8x129->64 92 against 104, 32x8x128->64 74 against 76; 32x8x128->8 38 against 36).
+    if (general && g_force_tile < 0 && best_per_cu > 2 &&
+        ((pl->xvec == 1 && !widest) || (g.c > 4 && g.c < 16 && (pl->xvec == 1 || g.m > 32))))
+        return false;
+    return true;
 }
 
-static int launch_planned(const ConvGeom& g, int ids_h, int ids_w, bool flip, const float* x, const float* w,
+static int launch_planned(const ConvGeom& g, int ids_h, int ids_w, bool flip, bool general, const float* x, const float* w,
                           const float* bias, float* y, hipStream_t st, const char* what, bool* applies) {
     Dense3Plan pl;
-    *applies = plan_conv_dense3(g, ids_h, ids_w, flip, x, w, &pl);
+    *applies = plan_conv_dense3(g, ids_h, ids_w, flip, general, x, w, &pl);
     if (!*applies) return 0;
     pl.a.x = x; pl.a.w = w; pl.a.bias = bias; pl.a.y = y;
 #define DML_D3(F, V, XV) \
@@ -434,14 +453,14 @@ static int launch_planned(const ConvGeom& g, int ids_h, int ids_w, bool flip, co
 
 int launch_conv_dense3_f32(const ConvGeom& g, const float* x, const float* w, const float* bias, float* y, hipStream_t st,
                            bool* applies) {
-    return launch_planned(g, 1, 1, false, x, w, bias, y, st, "conv2d(dense 3x3)", applies);
+    return launch_planned(g, 1, 1, false, conv_implicit_applicable(g), x, w, bias, y, st, "conv2d(dense 3x3)", applies);
 }
 
 int launch_conv_dense3_bwd_data_f32(const ConvGeom& g, const float* dy, const float* w, float* dx, hipStream_t st, bool* applies) {
     ConvGeom b;
     *applies = false;
     if (!data_gradient_problem(g, &b)) return 0;
-    return launch_planned(b, g.sh, g.sw, true, dy, w, nullptr, dx, st, "conv2d_backward_data(dense 3x3)", applies);
+    return launch_planned(b, g.sh, g.sw, true, conv_implicit_bwd_data_applicable(g), dy, w, nullptr, dx, st, "conv2d_backward_data(dense 3x3)", applies);
 }
 
 }  // namespace dml

@@ -10,6 +10,10 @@ struct ConvGeom {
     int n, c, h, w, m, kh, kw, sh, sw, ph, pw, dh, dw, group, oh, ow, cg, mg, act;
 };
 
+// conv_implicit.hip: does the general implicit-GEMM kernel take the convolution / its data gradient
+bool conv_implicit_applicable(const ConvGeom& g);
+bool conv_implicit_bwd_data_applicable(const ConvGeom& g);
+
 // conv_dense3.hip: 3 x 3, group 1, with enough work. *applies = false: nothing launched, another kernel has to run
 int launch_conv_dense3_f32(const ConvGeom& g, const float* x, const float* w, const float* bias, float* y, hipStream_t st,
                            bool* applies);
