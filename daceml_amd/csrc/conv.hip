@@ -28,9 +28,7 @@ int launch_pointwise_bwd_weight(const float* x, const float* dy, float* part, in
                                 hipStream_t st);
 
 // conv_implicit.hip
-bool conv_implicit_applicable(const ConvGeom& g);
 int launch_conv_implicit_f32(const ConvGeom& g, const float* x, const float* w, const float* bias, float* y, hipStream_t st);
-bool conv_implicit_bwd_data_applicable(const ConvGeom& g);
 int launch_conv_implicit_bwd_data_f32(const ConvGeom& g, const float* dy, const float* w, float* dx, hipStream_t st);
 
 namespace {
@@ -564,9 +562,12 @@ direct:
 
 namespace dml {
 namespace {
-// per-workgroup-range results of the dense weight gradient: the 3 x 3 kernel's where it applies
+// per-workgroup-range results of the dense weight gradient: of the 3 x 3 kernel where it runs, else of the general one
+int64_t dense3_weight_partials(const ConvGeom& g) {
+    return conv_dense3_bwd_weight_partials(g, dense_bwd_weight_partials(g.n, g.c, g.m, g.kh, g.kw, g.oh, g.ow, g.h, g.w) > 0);
+}
 int64_t dense_weight_partials(const ConvGeom& g) {
-    const int64_t parts = conv_dense3_bwd_weight_partials(g);
+    const int64_t parts = dense3_weight_partials(g);
     return parts > 0 ? parts : dense_bwd_weight_partials(g.n, g.c, g.m, g.kh, g.kw, g.oh, g.ow, g.h, g.w);
 }
 }  // namespace
@@ -723,7 +724,7 @@ int dmlhip_conv2d_backward_weight_f32(const dmlhip_conv2d_desc* d, const void* x
     if (dense_parts > 0) {
         // implicit GEMM over ranges of the (image, pixel) space, then their sum in a fixed order
         float* part = dense_parts > 1 ? (float*)workspace : (float*)dw;
-        const int e = conv_dense3_bwd_weight_partials(g) > 0
+        const int e = dense3_weight_partials(g) > 0
                           ? launch_conv_dense3_bwd_weight(g, (const float*)x, (const float*)dy, part, st)
                           : launch_dense_bwd_weight((const float*)x, (const float*)dy, part, g.n, g.c, g.h, g.w, g.m, g.kh,
                                                     g.kw, g.sh, g.sw, g.ph, g.pw, g.dh, g.dw, g.oh, g.ow, st);

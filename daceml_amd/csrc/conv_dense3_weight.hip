@@ -257,16 +257,27 @@ bool lay_out(const ConvGeom& g, int rows, int avec, int xvec, int mb, WeightPlan
     return pl->lds <= kLdsBytes;
 }
 
-// What does not depend on the operands' addresses: whether the kernel applies and into how many ranges of output rows the
-// work is cut (one workgroup per compute unit; at most 256 MiB of their results).
-int64_t plan_ranges(const ConvGeom& g) {
+// What does not depend on the operands' addresses: whether the kernel runs and into how many ranges of output rows the
+// work is cut (one workgroup per compute unit; at most 256 MiB of their results). general: another kernel takes the problem too.
+int64_t plan_ranges(const ConvGeom& g, bool general) {
     if (g.kh != 3 || g.kw != 3 || g.group != 1 || g.n < 1 || g.c < 1 || g.m < 1 || g.oh < 1 || g.ow < 1) return 0;
     const int64_t per = (int64_t)g.m * g.c * kTaps, rows = (int64_t)g.n * g.oh;
-    // First loads, the sums through LDS and the reduction take 18 us whatever the size: below 2^29 multiply-adds the general
-    // kernel is faster where it applies (1x64x56x56 -> 64 14 us against 20; 8x64x55x55 -> 64, 2^30, 44 against 44), from
-    // 2^24 on this one where that does not (fewer than 64 output pixels: 5x256x14x14 -> 512, stride 2, 1200 us against 35).
     const double macs = (double)rows * g.ow * per;
-    if (macs < (double)(1 << ((int64_t)g.oh * g.ow < 64 ? 24 : 29))) return 0;
+    // Where the general kernel does not apply (fewer than 64 output pixels: 5x256x14x14 -> 512, stride 2, 1200 us against 35)
+    // this one runs from 2^24 multiply-adds on. Where it does, the rules below hold what was measured against it, us there and
+    // here: first loads, the sums through LDS and the reduction take 18 us whatever the size (1x64x56x56 -> 64 14 and 20;
+    // 8x64x55x55 -> 64, 2^30, 44 and 44); channels are padded to 32, which the general kernel does over all c * 9 columns
+    // (16 of 112 x 112, 64 images -> 64 1.0 - 1.16 times its time, 24 of 33 x 33 0.76 - 1.01); rows of X that are no multiple
+    // of four floats cost a gather per float, too much with stride 2 (64x64x113x113 -> 64 301 and 355) and with long
+    // rows for a single tile of output channels (32x32x113x113 -> 32 155 and 185, -> 64 247 and 259, -> 128 525 and 492) or a
+    // last one that is half empty (32x96x57x57 -> 96 285 and 342).
+    if (macs < (double)(1 << (general ? 29 : 24))) return 0;
+    if (general) {
+        const bool narrow = g.w % 4 != 0;
+        if (2 * ceil_div(g.c, kCTile) * kCTile > 3 * g.c) return 0;
+        const int64_t mb = g.m > 32 ? 64 : 32;
+        if (narrow && (g.sw > 1 || (g.ow > 64 && g.m <= 64) || 4 * ceil_div(g.m, mb) * mb > 5 * g.m)) return 0;
+    }
     if (rows > (1LL << 30) || per > (1LL << 30) || (int64_t)g.oh * g.ow > (1LL << 28) || (int64_t)g.h * g.w > (1LL << 28)) return 0;
     WeightPlan pl;
     if (!lay_out(g, 1, 1, 1, g.m > 32 ? 64 : 32, &pl)) return 0;
@@ -293,7 +304,7 @@ int launch_weight(const WeightPlan& pl, unsigned blocks, hipStream_t st) {
 }
 
 bool plan_weight(const ConvGeom& g, const void* x, const void* dy, WeightPlan* pl, unsigned* blocks, int* avec, int* xvec) {
-    const int64_t ranges = plan_ranges(g);
+    const int64_t ranges = plan_ranges(g, false);
     if (ranges < 1) return false;
     const int mb = g.m > 32 ? 64 : 32;
     *avec = g.ow % 4 == 0 && aligned16(dy) ? 4 : 1;
@@ -318,8 +329,7 @@ bool plan_weight(const ConvGeom& g, const void* x, const void* dy, WeightPlan* p
 
 }  // namespace
 
-// number of per-range results (each m * c * 9 floats); 0 = not applicable
-int64_t conv_dense3_bwd_weight_partials(const ConvGeom& g) { return plan_ranges(g); }
+int64_t conv_dense3_bwd_weight_partials(const ConvGeom& g, bool general) { return plan_ranges(g, general); }
 
 int launch_conv_dense3_bwd_weight(const ConvGeom& g, const float* x, const float* dy, float* part, hipStream_t st) {
     WeightPlan pl;

@@ -18,8 +18,9 @@ bool conv_implicit_bwd_data_applicable(const ConvGeom& g);
 int launch_conv_dense3_f32(const ConvGeom& g, const float* x, const float* w, const float* bias, float* y, hipStream_t st,
                            bool* applies);
 int launch_conv_dense3_bwd_data_f32(const ConvGeom& g, const float* dy, const float* w, float* dx, hipStream_t st, bool* applies);
-// conv_dense3_weight.hip: per-range results (m * c * 9 floats each) its weight gradient writes; 0 = does not apply
-int64_t conv_dense3_bwd_weight_partials(const ConvGeom& g);
+// conv_dense3_weight.hip: per-range results (m * c * 9 floats each) its weight gradient writes; 0 = does not apply, or the
+// general kernel, where that applies (`general`), is the faster one
+int64_t conv_dense3_bwd_weight_partials(const ConvGeom& g, bool general);
 int launch_conv_dense3_bwd_weight(const ConvGeom& g, const float* x, const float* dy, float* part, hipStream_t st);
 
 // conv_depthwise.hip: depthwise 3 x 3 / 5 x 5, stride 1, output as large as the input
