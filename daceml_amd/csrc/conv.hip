@@ -729,9 +729,10 @@ int dmlhip_conv2d_backward_weight_f32(const dmlhip_conv2d_desc* d, const void* x
                           : launch_dense_bwd_weight((const float*)x, (const float*)dy, part, g.n, g.c, g.h, g.w, g.m, g.kh,
                                                     g.kw, g.sh, g.sw, g.ph, g.pw, g.dh, g.dw, g.oh, g.ow, st);
         if (e) return e;
-        if (dense_parts >= 32) {
+        if (dense_parts >= 32 && dense_parts <= 512) {
             // sixteen wavefronts share the ranges of 64 columns: one pass (128 x 36864: 6 us; the general reduction's two
-            // passes 10). With few ranges most of the sixteen would be idle (4 x 1.2 million: 45 us against 20)
+            // passes 10). With few ranges most of the sixteen would be idle (4 x 1.2 million: 45 us against 20), with many each
+            // of them walks a long chain (the whole gradient of 3 channels, 12x3x225x225 -> 8 with 1908 ranges: 43.6 against 37.6)
             hipLaunchKernelGGL((reduce_partials_kernel<OpSum, float>), (unsigned)ceil_div(total, (int64_t)kWave), 1024, 0, st,
                                (const float*)part, (float*)dw, (int)dense_parts, total, total, 0.f, 1.f, (float*)nullptr, (int64_t)0);
             return launch_status("conv2d_backward_weight(sum of ranges)");
