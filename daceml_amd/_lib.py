@@ -154,6 +154,8 @@ SIGNATURES = {
     "dmlhip_debug_force_conv_dense3_tile": (None, [c_int]),
     "dmlhip_debug_gemm_direct_lds": (None, [c_int]),
     "dmlhip_debug_grouped_single_launches": (ctypes.c_longlong, []),
+    "dmlhip_debug_force_conv_depthwise": (None, [c_int]),
+    "dmlhip_debug_conv_depthwise_strips": (c_int, [POINTER(Conv2dDesc), c_int]),
     "dmlhip_debug_force_fused_strip": (None, [c_int]),
     "dmlhip_debug_fused_rolling": (None, [c_int, c_int]),
     "dmlhip_debug_attention_trace": (None, [c_void_p]),

@@ -518,7 +518,7 @@ int conv_forward(const dmlhip_conv2d_desc* d, const void* x, const void* w, cons
                               : dmlhip_gemm_f32(&gd, w, x, y, bias, nullptr, nullptr, stream);
     }
     if constexpr (sizeof(T) == 4) {
-        if (depthwise_same_applicable(g))
+        if (depthwise_same_applicable(g) && depthwise_same_faster(g, x, y, false))
             return launch_depthwise_same(g, (const float*)x, (const float*)w, (const float*)bias, (float*)y, st);
     }
     // depthwise with a small square-ish stencil
@@ -607,6 +607,13 @@ int dmlhip_conv2d_gated_f32(const dmlhip_conv2d_desc* d, const void* x, const vo
                                 g.m, hw, g.act, (hipStream_t)stream);
 }
 
+int dmlhip_debug_conv_depthwise_strips(const dmlhip_conv2d_desc* d, int pass) {
+    ConvGeom g;
+    if (int e = make_geom(d, &g, "debug_conv_depthwise_strips")) return e;
+    if (!depthwise_same_applicable(g)) return 0;
+    return pass == 2 ? depthwise_same_weight_faster(g, nullptr, nullptr) : depthwise_same_faster(g, nullptr, nullptr, pass == 1);
+}
+
 int dmlhip_conv2d_f16(const dmlhip_conv2d_desc* d, const void* x, const void* w, const void* bias, void* y,
                       void* stream) {
     return conv_forward<_Float16>(d, x, w, bias, y, stream);
@@ -645,7 +652,7 @@ int dmlhip_conv2d_backward_data_f32(const dmlhip_conv2d_desc* d, const void* dy,
         gd.alpha = 1.f; gd.out_dtype = DMLHIP_F32; gd.bias_dtype = DMLHIP_F32;
         return dmlhip_gemm_f32(&gd, w, dy, dx, nullptr, nullptr, nullptr, stream);
     }
-    if (depthwise_same_applicable(g))
+    if (depthwise_same_applicable(g) && depthwise_same_faster(g, dy, dx, true))
         return launch_depthwise_same_bwd_data(g, (const float*)dy, (const float*)w, (float*)dx, st);
     if (is_depthwise_grad(g))
         return launch_depthwise_bwd_data((const float*)dy, (const float*)w, (float*)dx, g.n, g.c, g.h, g.w, g.oh, g.ow, g.kh,
@@ -711,7 +718,7 @@ int dmlhip_conv2d_backward_weight_f32(const dmlhip_conv2d_desc* d, const void* x
         // one result per (image, channel) plane, summed over the images in a fixed order
         const int64_t per = (int64_t)g.c * g.kh * g.kw;
         float* part = g.n > 1 ? (float*)workspace : (float*)dw;
-        const int e = depthwise_same_applicable(g)
+        const int e = depthwise_same_applicable(g) && depthwise_same_weight_faster(g, x, dy)
                           ? launch_depthwise_same_bwd_weight(g, (const float*)x, (const float*)dy, part, st)
                           : launch_depthwise_bwd_weight((const float*)x, (const float*)dy, part, g.n, g.c, g.h, g.w, g.oh, g.ow,
                                                         g.kh, g.sh, g.ph, st);

@@ -113,13 +113,15 @@ __global__ __launch_bounds__(256) void depthwise_same_weight_kernel(const PlaneA
     const int lane = (int)threadIdx.x % G;
     const bool live = plane < g.total;
     const size_t base = (size_t)(live ? plane : 0) * g.h * g.wd;
-    float acc[K * K];
+    // four rows' products per tap are summed on their own: one chain over all cells of a lane was 2.7 times as far from the
+    // exact sum as the general kernel's 256 shorter ones (8 planes of 448 x 448: 1.3e-7 of it)
+    float total[K * K];
 #pragma unroll
-    for (int i = 0; i < K * K; ++i) acc[i] = 0.f;
+    for (int i = 0; i < K * K; ++i) total[i] = 0.f;
     for (int cell = lane; live && cell < g.cells; cell += G) {
         const int strip = cell / g.cw, first = 4 * (cell - strip * g.cw), y0 = strip * R;
         const int c0 = min(first, g.wd - 4);
-        float v[R + K - 1][K + 3], d[R][4];
+        float v[R + K - 1][K + 3], d[R][4], acc[K * K];
         load_rows<K, R + K - 1, VEC>(g.x + base, g.h, g.wd, y0, c0, v);
 #pragma unroll
         for (int r = 0; r < R; ++r) {
@@ -132,7 +134,11 @@ __global__ __launch_bounds__(256) void depthwise_same_weight_kernel(const PlaneA
         // Products with a pixel outside either plane, or with a column that the thread before has added, are left out and not
         // multiplied by zero: the other factor may be infinite.
 #pragma unroll
-        for (int r = 0; r < R; ++r)
+        for (int r = 0; r < R; ++r) {
+            if (r % 4 == 0) {
+#pragma unroll
+                for (int i = 0; i < K * K; ++i) acc[i] = 0.f;
+            }
 #pragma unroll
             for (int hy = 0; hy < K; ++hy) {
                 const int iy = y0 + r + hy - P;
@@ -152,14 +158,19 @@ __global__ __launch_bounds__(256) void depthwise_same_weight_kernel(const PlaneA
                         }
                     }
             }
+            if (r % 4 == 3 || r == R - 1) {
+#pragma unroll
+                for (int i = 0; i < K * K; ++i) total[i] += acc[i];
+            }
+        }
     }
 #pragma unroll
     for (int i = 0; i < K * K; ++i)
 #pragma unroll
-        for (int s = 1; s < G; s *= 2) acc[i] += __shfl_xor(acc[i], s);
+        for (int s = 1; s < G; s *= 2) total[i] += __shfl_xor(total[i], s);
     if (live && lane == 0) {
 #pragma unroll
-        for (int i = 0; i < K * K; ++i) g.out[(size_t)plane * K * K + i] = acc[i];
+        for (int i = 0; i < K * K; ++i) g.out[(size_t)plane * K * K + i] = total[i];
     }
 }
 
@@ -198,10 +209,40 @@ int launch_same_weight(PlaneArgs a, int64_t planes, int h, int wd, hipStream_t s
     return launch_status("conv2d_backward_weight(depthwise)");
 }
 
+// Whether the kernels above are faster than those that cover the other depthwise convolutions too (a plane's tile in LDS; a
+// thread per four outputs; a workgroup per plane), from 1200 problems of 8 - 6144 planes of 4 x 4 to 448 x 448 timed on both,
+// us there / here. Few small planes are a matter of latency alone, and a strip's loads take longer than a tile's: forward
+// 256 planes of 4 x 4 2.8 / 5.2, of 12 x 12 3.4 / 4.7, of 28 x 28 4.6 / 4.6, of 33 x 33 6.7 / 4.6; data gradient 256 planes of
+// 28 x 28 3.2 / 3.8, of 40 x 40 4.8 / 3.9. The more planes, the smaller they may be (forward, 14 x 14: 512 4.5 / 4.7,
+// 1536 6.7 / 4.8). vec: rows in 16-byte pieces, which spread planes below 17 columns over a quarter of the lanes.
+bool same_faster(int64_t planes, int64_t hw, int k, bool vec, bool data) {
+    if (hw > 1024) return true;
+    if (hw >= 784) return planes >= 384;
+    const bool wide = k == 5 && !data;           // forward 5 x 5: a sixth more before a strip's loads are paid for
+    if (hw > 256) return planes >= (wide ? 768 : 512);
+    if (vec) return planes >= (hw > 64 ? 1408 : wide ? 3584 : 2816);
+    if (hw > 49) return planes >= 1024;
+    return planes >= (wide ? 1280 : 1024) || (data && k == 5);      // 256 planes of 5 x 5: 4.4 / 4.0
+}
+
+// The same for the weight gradient, where a plane has at most one wavefront here and four there: 3 x 3 on 96 planes of
+// 14 x 14 2.7 / 6.3, 768 of 56 x 56 13.0 / 11.9, 480 of 111 x 111 32.3 / 33.0, 4096 of 14 x 14 10.4 / 9.2; 5 x 5 on 512 planes of
+// 12 x 12 7.8 / 9.1, of 24 x 24 12.5 / 9.7, 96 of 112 x 112 116 / 56.
+bool same_weight_faster(int64_t planes, int64_t hw, int k, bool vec) {
+    if (hw <= 16) return planes >= (k == 3 ? 6144 : 3072);
+    if (k == 5) return hw >= (vec ? 576 : 784) || planes >= (vec ? 1536 : 2048) || (vec && hw >= 400 && planes >= 384);
+    if (!vec) return planes >= 4096 || (planes >= 2048 && hw >= 1024) || (planes >= 1024 && hw >= 8192);
+    return planes >= 3072 || planes * hw >= 2000000 || hw >= 40000 || (planes >= 768 && planes * hw >= 800000);
+}
+
+thread_local int g_force_same = -1;   // diagnostic: 0 = never, 1 = wherever they apply
+
 // every thread index and element offset fits 32 bits
 bool in_range(int64_t planes, int h, int wd) { return planes * h * wd < (1LL << 31) && planes * ((wd + 3) / 4) * ((h + 3) / 4) < (1LL << 31) && planes < (1LL << 25); }
 
 }  // namespace
+
+static bool vec_rows(const ConvGeom& g, const void* a, const void* b) { return g.w % 4 == 0 && aligned16(a) && aligned16(b); }
 
 // a group == c == m convolution of n images
 bool depthwise_same_applicable(const ConvGeom& g) {
@@ -209,10 +250,20 @@ bool depthwise_same_applicable(const ConvGeom& g) {
            same_size(g.kh, g.kw, g.sh, g.sw, g.ph, g.pw, g.dh, g.dw, g.h, g.w, g.oh, g.ow);
 }
 
+bool depthwise_same_faster(const ConvGeom& g, const void* in, const void* out, bool data) {
+    if (g_force_same >= 0) return g_force_same != 0;
+    return same_faster((int64_t)g.n * g.c, (int64_t)g.h * g.w, g.kh, vec_rows(g, in, out), data);
+}
+
+bool depthwise_same_weight_faster(const ConvGeom& g, const void* x, const void* dy) {
+    if (g_force_same >= 0) return g_force_same != 0;
+    return same_weight_faster((int64_t)g.n * g.c, (int64_t)g.h * g.w, g.kh, vec_rows(g, x, dy));
+}
+
 int launch_depthwise_same(const ConvGeom& g, const float* x, const float* w, const float* bias, float* y, hipStream_t st) {
     PlaneArgs a = {};
     a.x = x; a.w = w; a.bias = bias; a.out = y; a.c = g.c; a.act = g.act;
-    const bool vec = g.w % 4 == 0 && aligned16(x) && aligned16(y);
+    const bool vec = vec_rows(g, x, y);
     const int64_t planes = (int64_t)g.n * g.c;
     return g.kh == 3 ? launch_same<3, false>(a, planes, g.h, g.w, vec, st, "conv2d(depthwise)")
                      : launch_same<5, false>(a, planes, g.h, g.w, vec, st, "conv2d(depthwise)");
@@ -221,7 +272,7 @@ int launch_depthwise_same(const ConvGeom& g, const float* x, const float* w, con
 int launch_depthwise_same_bwd_data(const ConvGeom& g, const float* dy, const float* w, float* dx, hipStream_t st) {
     PlaneArgs a = {};
     a.x = dy; a.w = w; a.out = dx; a.c = g.c;
-    const bool vec = g.w % 4 == 0 && aligned16(dy) && aligned16(dx);
+    const bool vec = vec_rows(g, dy, dx);
     const int64_t planes = (int64_t)g.n * g.c;
     return g.kh == 3 ? launch_same<3, true>(a, planes, g.h, g.w, vec, st, "conv2d_backward_data(depthwise)")
                      : launch_same<5, true>(a, planes, g.h, g.w, vec, st, "conv2d_backward_data(depthwise)");
@@ -230,10 +281,12 @@ int launch_depthwise_same_bwd_data(const ConvGeom& g, const float* dy, const flo
 int launch_depthwise_same_bwd_weight(const ConvGeom& g, const float* x, const float* dy, float* part, hipStream_t st) {
     PlaneArgs a = {};
     a.x = x; a.dy = dy; a.out = part; a.c = g.c;
-    const bool vec = g.w % 4 == 0 && aligned16(x) && aligned16(dy);
+    const bool vec = vec_rows(g, x, dy);
     const int64_t planes = (int64_t)g.n * g.c;
     if (g.kh == 3) return vec ? launch_same_weight<3, true>(a, planes, g.h, g.w, st) : launch_same_weight<3, false>(a, planes, g.h, g.w, st);
     return vec ? launch_same_weight<5, true>(a, planes, g.h, g.w, st) : launch_same_weight<5, false>(a, planes, g.h, g.w, st);
 }
 
 }  // namespace dml
+
+extern "C" void dmlhip_debug_force_conv_depthwise(int strips) { dml::g_force_same = strips; }

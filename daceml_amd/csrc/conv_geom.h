@@ -25,6 +25,9 @@ int launch_conv_dense3_bwd_weight(const ConvGeom& g, const float* x, const float
 
 // conv_depthwise.hip: depthwise 3 x 3 / 5 x 5, stride 1, output as large as the input
 bool depthwise_same_applicable(const ConvGeom& g);
+// ... and are they the faster ones, where the general depthwise kernels take the problem too (data: the data gradient)
+bool depthwise_same_faster(const ConvGeom& g, const void* in, const void* out, bool data);
+bool depthwise_same_weight_faster(const ConvGeom& g, const void* x, const void* dy);
 int launch_depthwise_same(const ConvGeom& g, const float* x, const float* w, const float* bias, float* y, hipStream_t st);
 int launch_depthwise_same_bwd_data(const ConvGeom& g, const float* dy, const float* w, float* dx, hipStream_t st);
 int launch_depthwise_same_bwd_weight(const ConvGeom& g, const float* x, const float* dy, float* part, hipStream_t st);

@@ -498,6 +498,12 @@ void dmlhip_debug_gemm_direct_lds(int on);
  * the next launches set here, every workgroup stores four readings of the 100 MHz wall clock (start, first tile in
  * LDS, end of the K loop, end of the epilogue) at buffer[4 * workgroup]; NULL (default) switches it off. The caller
  * sizes the buffer for the largest grid it launches. Per calling thread. */
+/* Diagnostic: the calling thread's depthwise stride-1 fp32 convolutions and gradients whose output is as large as the input
+ * run on the strip kernels (1), on the general depthwise kernels (0), or on the faster of the two (-1, default). */
+void dmlhip_debug_force_conv_depthwise(int strips);
+/* Diagnostic: 1 if such a convolution (pass 0), its data gradient (1) or its weight gradient (2) runs on the strip kernel, given
+ * tensors aligned to 16 bytes; 0 if not. Launches nothing. */
+int dmlhip_debug_conv_depthwise_strips(const dmlhip_conv2d_desc* d, int pass);
 void dmlhip_debug_gemm_trace(void* buffer);
 /* Number of grouped / K-concatenated / row-sum contraction calls that went out as one launch so far. */
 long long dmlhip_debug_grouped_single_launches(void);
