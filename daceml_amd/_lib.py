@@ -150,12 +150,13 @@ SIGNATURES = {
     # diagnostics (switches for tests and measurements, declared at the end of the header)
     "dmlhip_conv2d_expand_depthwise_lds_bytes": (c_size_t, [c_int64, c_int64, c_int64]),
     "dmlhip_debug_force_gemm_config": (None, [c_int]),
+    "dmlhip_debug_last_gemm_config": (c_int, []),
     "dmlhip_debug_force_gemm_f32_tile": (None, [c_int]),
     "dmlhip_debug_force_conv_dense3_tile": (None, [c_int]),
-    "dmlhip_debug_gemm_direct_lds": (None, [c_int]),
-    "dmlhip_debug_grouped_single_launches": (ctypes.c_longlong, []),
     "dmlhip_debug_force_conv_depthwise": (None, [c_int]),
     "dmlhip_debug_conv_depthwise_strips": (c_int, [POINTER(Conv2dDesc), c_int]),
+    "dmlhip_debug_gemm_direct_lds": (None, [c_int]),
+    "dmlhip_debug_grouped_single_launches": (ctypes.c_longlong, []),
     "dmlhip_debug_force_fused_strip": (None, [c_int]),
     "dmlhip_debug_fused_rolling": (None, [c_int, c_int]),
     "dmlhip_debug_attention_trace": (None, [c_void_p]),

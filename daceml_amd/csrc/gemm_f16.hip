@@ -365,37 +365,41 @@ int operand_mode(const void* p, int64_t rows, int64_t k, int64_t s_row, int64_t 
     return 2;
 }
 
-// The configuration with the least estimated time for a product whose 128 x 128 tiles leave (much of) a round of compute
-// units idle. Estimate: fixed + (rounds of resident workgroups - 1) * round + tiles per compute unit * K steps * step, in us,
-// fitted to 330 products of encoder layers (24 - 2048 tokens, 512 - 1024 wide, every operand layout); its choice is within
-// 1 % of the fastest configuration in the mean, 19 % at worst. Decided by it (us, 128-wide tiles / 64 x 64 / 32 x 32):
-// 128 x 1024 x 4096 19 / 15 / 9; 651 x 1024 x 4096 24 / 17 / 23; 651 x 4096 x 1024 11 / 19 / 24; the K-concatenated
-// 651 x 1024 x 3 * 1024 26 / 14 / 22.
-int choose_small(const dmlhip_gemm_desc* d, long long batch, int pairs, bool narrow, bool pipe) {
+// Estimated time in us of the configuration (*cfg) that is the fastest for a product of few tiles: fixed + (rounds of
+// resident workgroups - 1) * round + tiles per compute unit * K steps * step, fitted to 330 products of encoder layers
+// (24 - 2048 tokens, 512 - 1024 wide, every operand layout); its choice is within 1 % of the fastest configuration in the
+// mean, 19 % at worst. Decided by it (us, 128-wide tiles / 64 x 64 / 32 x 32): 128 x 1024 x 4096 19 / 15 / 9; 651 x 1024 x 4096
+// 24 / 17 / 23; 651 x 4096 x 1024 11 / 19 / 24; the K-concatenated 651 x 1024 x 3 * 1024 26 / 14 / 22.
+// narrow: the 128 x 64 tile exists; pipe: the pipelined kernels do; general: so does the kernel that stages its operands in
+// registers (*cfg = -1), which is what a ragged K otherwise has. Its line is from 190 products of K = 8 - 1000, us there and
+// in the better of the two split ones: 1048 x 2432 x 48 6.5 / 12.3, 4960 x 1048 x 504 22 / 39, 3720 x 1536 x 1000 30 / 54,
+// 480 x 4096 x 520 15 / 11, 608 x 4096 x 1000 26 / 22, 72 x 256 x 520 13 / 5.
+double estimate_small(int64_t m, int64_t n, int64_t k, long long batch, int pairs, bool out_f32, bool narrow, bool pipe,
+                      bool general, int* cfg) {
     struct Est { int cfg, bm, bn, resident; double fixed, round, step; };
     constexpr Est kEst[] = {{5, 128, 128, 1, 5.59, 5.36, 0.353}, {7, 128, 128, 2, 5.26, 5.36, 0.484},
                             {9, 128, 64, 2, 3.22, 1.86, 0.326},  {10, 64, 64, 1, 4.51, 3.35, 0.182},
-                            {12, 32, 32, 2, 3.26, 1.81, 0.100}};
-    const double steps = (double)ceil_div(d->k, (int64_t)BK) * pairs;
-    int best = -1;
-    double best_us = 0;
+                            {12, 32, 32, 2, 3.26, 1.81, 0.100},  {-1, 128, 128, 2, 5.6, 0.0, 0.9}};
+    const double steps = (double)ceil_div(k, (int64_t)BK) * pairs;
+    double best_us = 1e30;
     for (const Est& e : kEst) {
-        if ((e.cfg == 9 && !narrow) || (e.cfg < 10 && !pipe)) continue;
+        if (e.cfg < 0 ? !general : (e.cfg == 9 && !narrow) || (e.cfg < 10 && !pipe)) continue;
         // an fp32 result is the same bits whatever the tile: one accumulation chain in K order, which a split K is not
-        if (e.cfg >= 10 && d->out_dtype == DMLHIP_F32 && pipe) continue;
-        const double n = (double)ceil_div(ceil_div(d->m, (int64_t)e.bm) * ceil_div(d->n, (int64_t)e.bn) * batch, (int64_t)kCus);
-        const double us = e.fixed + (ceil(n / e.resident) - 1) * e.round + n * steps * e.step;
-        if (best < 0 || us < best_us) {
-            best = e.cfg;
+        if (e.cfg >= 10 && out_f32 && pipe) continue;
+        const double t = (double)ceil_div(ceil_div(m, (int64_t)e.bm) * ceil_div(n, (int64_t)e.bn) * batch, (int64_t)kCus);
+        const double us = e.fixed + (ceil(t / e.resident) - 1) * e.round + t * steps * e.step;
+        if (us < best_us) {
+            *cfg = e.cfg;
             best_us = us;
         }
     }
-    return best;
+    return best_us;
 }
 
 // Diagnostic switches (declared in the public header). Per calling thread, so that one thread pinning a configuration
 // does not change what other threads launch.
 thread_local int g_force_cfg = -1;  // pin the tile configuration
+thread_local int g_last_cfg = -1;   // configuration of the last product, -1 = operands staged in registers
 thread_local int g_direct_lds = 1;  // 0 forces the register-staged loaders
 thread_local unsigned long long* g_trace = nullptr;  // per-workgroup clock readings of the pipelined kernel
 
@@ -409,6 +413,7 @@ extern "C" {
 void dmlhip_debug_force_gemm_config(int cfg) { g_force_cfg = cfg; }
 void dmlhip_debug_gemm_direct_lds(int on) { g_direct_lds = on; }
 void dmlhip_debug_gemm_trace(void* buffer) { g_trace = (unsigned long long*)buffer; }
+int dmlhip_debug_last_gemm_config() { return g_last_cfg; }
 static std::atomic<long long> g_grouped_single_launches{0};
 // Number of grouped calls that went out as ONE launch (tests check that grouping really happens).
 long long dmlhip_debug_grouped_single_launches() { return g_grouped_single_launches.load(); }
@@ -518,14 +523,17 @@ static int run_gemm_f16(const dmlhip_gemm_desc* d, const void* a, const void* b,
             // issuing MFMAs while transfers and fragment reads are in flight. Only when its tiles fill (nearly) every
             // round of compute units: 192 tiles on 256 units lose more than the tile gains.
             cfg = 4;
-        } else if (cfg < 0 && t128 < 2 * kCus && t128 * 10 < slots128 * 9) {
-            cfg = choose_small(d, batch, g.ksum ? g.groups : 1, !extra, pipe);
+        } else if (cfg < 0 && t128 < 2 * kCus && t128 * 10 < slots128 * 9 && (!pipe || d->k >= 512 || t128 <= kCus)) {
+            // rows of C that are not written in vectors hide what the general kernel's longer loop costs: one round only
+            const bool general = !pipe && !extra && (g.c_vec || t128 > kCus);
+            estimate_small(d->m, d->n, d->k, batch, g.ksum ? g.groups : 1, g.out_f32, !extra, pipe, general, &cfg);
         }
         if (cfg < 0) {
             if (d->k < 512) {
                 // a handful of K steps (the batched products of an unfused attention): bound by the epilogue, where two
-                // resident workgroups per compute unit overlap one's stores with the other's loads
-                cfg = t128 > kCus ? 3 : 0;
+                // resident workgroups per compute unit overlap one's stores with the other's loads. 361 tiles, K = 64 / 192, us on
+                // 3, 7 and the 128 x 64 tile: 5.5 / 7.2, 5.8 / 7.1, 7.0 / 7.8
+                cfg = t128 <= kCus ? 0 : d->k < 192 ? 3 : 7;
             } else if (d->k <= 1024 && t128 >= 2 * kCus) {
                 // several rounds of short K loops (the grouped q / k / v projections: 768 tiles of 16 steps): with two
                 // LDS stages instead of four, two workgroups share a compute unit and one's epilogue and first loads
@@ -543,6 +551,7 @@ static int run_gemm_f16(const dmlhip_gemm_desc* d, const void* a, const void* b,
             }
         }
         const _Float16 *pa = (const _Float16*)a, *pb = (const _Float16*)b;
+        g_last_cfg = cfg;
         if (cfg >= 10 && (!sums || amode == 1))
             return launch_split(g, pa, pb, c, bias, residual, pre_out, amode, bmode, cfg, batch, st);
         if (pipe && ragged) return launch_pipelined_ragged(g, pa, pb, c, bias, residual, pre_out, cfg, batch, st);
@@ -550,6 +559,7 @@ static int run_gemm_f16(const dmlhip_gemm_desc* d, const void* a, const void* b,
             return launch_pipelined(g, pa, pb, c, bias, residual, pre_out, amode == 1 ? 4 : 3, bmode == 1 ? 4 : 3, cfg, batch, st);
         if (g_force_cfg < 0) cfg = -1;
     }
+    g_last_cfg = -1;
     if (grp || asum) return DMLHIP_ERR_UNSUPPORTED;  // only the pipelined kernel takes pointer groups / makes row sums
     if (cfg < 0 || cfg > 2) {
         // Largest tile that still yields at least one workgroup per CU.

@@ -482,8 +482,12 @@ int dmlhip_batchnorm_backward_act_f32(const void* dy, const void* x, const void*
  * 8 = 128x64 tile with a 3-stage ring (twice the workgroups, two per compute unit, for products that give each compute
  * unit a single 128x128 tile), 9 = the same with the interleaved loop. Products with row sums or K-concatenated operand pairs exist on the 128x128 tile
  * only: 5 and 7 run them with the interleaved loop, 4, 6, 8 and 9 leave them on the plain one. 10 = 64x64, 12 = 32x32 tile
- * with K split over the wavefronts (products with too few 128-wide tiles for the chip; any K, every form). */
+ * with K split over the wavefronts (products with too few 128-wide tiles for the chip; any K; operands as for the others, no
+ * activation together with a residual, beta or a bias along m, row sums only of a row-contiguous A). */
 void dmlhip_debug_force_gemm_config(int cfg);
+/* Diagnostic: the configuration that the calling thread's last fp16 contraction launch ran on (of several launches, the
+ * last); -1 = the kernel that stages its operands through registers. */
+int dmlhip_debug_last_gemm_config(void);
 /* Pin the tile of the fp32 contraction kernel: 0 = 128x128, 1 = 64x64, 2 = 32x32 with K split over the wavefronts;
  * -1 = chosen per problem (default). Operands that cannot be read 16 bytes at a time have no 128x128 form and run on 64x64.
  * Per calling thread. */
@@ -491,6 +495,12 @@ void dmlhip_debug_force_gemm_f32_tile(int tile);
 /* Diagnostic: pin the tile of the calling thread's dense 3 x 3 fp32 convolutions and data gradients (0 = 32 channels x 128
    pixels, 1 = 32 x 64, 2 = 32 x 32; -1 = the library chooses). */
 void dmlhip_debug_force_conv_dense3_tile(int tile);
+/* Diagnostic: the calling thread's depthwise stride-1 fp32 convolutions and gradients whose output is as large as the input
+ * run on the strip kernels (1), on the general depthwise kernels (0), or on the faster of the two (-1, default). */
+void dmlhip_debug_force_conv_depthwise(int strips);
+/* Diagnostic: 1 if such a convolution (pass 0), its data gradient (1) or its weight gradient (2) runs on the strip kernel, given
+ * tensors aligned to 16 bytes; 0 if not. Launches nothing. */
+int dmlhip_debug_conv_depthwise_strips(const dmlhip_conv2d_desc* d, int pass);
 /* 0: the fp16 contractions stage their operands through registers instead of loading them straight into LDS;
  * 1 = default. */
 void dmlhip_debug_gemm_direct_lds(int on);
@@ -498,12 +508,6 @@ void dmlhip_debug_gemm_direct_lds(int on);
  * the next launches set here, every workgroup stores four readings of the 100 MHz wall clock (start, first tile in
  * LDS, end of the K loop, end of the epilogue) at buffer[4 * workgroup]; NULL (default) switches it off. The caller
  * sizes the buffer for the largest grid it launches. Per calling thread. */
-/* Diagnostic: the calling thread's depthwise stride-1 fp32 convolutions and gradients whose output is as large as the input
- * run on the strip kernels (1), on the general depthwise kernels (0), or on the faster of the two (-1, default). */
-void dmlhip_debug_force_conv_depthwise(int strips);
-/* Diagnostic: 1 if such a convolution (pass 0), its data gradient (1) or its weight gradient (2) runs on the strip kernel, given
- * tensors aligned to 16 bytes; 0 if not. Launches nothing. */
-int dmlhip_debug_conv_depthwise_strips(const dmlhip_conv2d_desc* d, int pass);
 void dmlhip_debug_gemm_trace(void* buffer);
 /* Number of grouped / K-concatenated / row-sum contraction calls that went out as one launch so far. */
 long long dmlhip_debug_grouped_single_launches(void);
