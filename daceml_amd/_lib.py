@@ -151,6 +151,7 @@ SIGNATURES = {
     "dmlhip_conv2d_expand_depthwise_lds_bytes": (c_size_t, [c_int64, c_int64, c_int64]),
     "dmlhip_debug_force_gemm_config": (None, [c_int]),
     "dmlhip_debug_last_gemm_config": (c_int, []),
+    "dmlhip_debug_gemm_f16_slices": (c_int, [POINTER(GemmDesc)]),
     "dmlhip_debug_force_gemm_f32_tile": (None, [c_int]),
     "dmlhip_debug_force_conv_dense3_tile": (None, [c_int]),
     "dmlhip_debug_force_conv_depthwise": (None, [c_int]),

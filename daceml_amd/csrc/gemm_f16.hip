@@ -579,29 +579,64 @@ static int run_gemm_f16(const dmlhip_gemm_desc* d, const void* a, const void* b,
     }
 }
 
-// Number of K splits worth taking for this problem (1 = none): only where even 64 x 64 tiles leave half of the compute units
-// idle and K is long enough to pay for the second launch (512 x 512 x 16384: 64 workgroups of 256 K steps otherwise).
-static int split_k_factor(const dmlhip_gemm_desc* d) {
-    if (!d || d->m <= 0 || d->n <= 0 || d->k < 2048 || d->batch[0] != 1) return 1;
-    const long long tiles = ceil_div(d->m, 64) * ceil_div(d->n, 64) * d->batch[1] * d->batch[2];
+// Whether both operands of a product are read 16 bytes at a time (then the slices of a split K run on the pipelined kernel).
+static bool vector_operands(const dmlhip_gemm_desc* d, const void* a, const void* b) {
+    return g_direct_lds && operand_mode(a, d->m, d->k, d->a_stride_m, d->a_stride_k, d->a_stride_batch, d->batch) != 2 &&
+           operand_mode(b, d->n, d->k, d->b_stride_n, d->b_stride_k, d->b_stride_batch, d->batch) != 2;
+}
+
+// Number of K slices of a plain product, in workgroups of their own with fp32 results that a second launch adds up (1 = none).
+static int split_k_factor(const dmlhip_gemm_desc* d, bool vec) {
+    if (!d || d->m <= 0 || d->n <= 0 || d->k < 1024 || d->batch[0] * d->batch[1] * d->batch[2] != 1) return 1;
     int s = 1;
-    while (tiles * s * 2 <= kCus && d->k / (s * 2) >= 1024 && d->k % (s * 2 * BK) == 0) s *= 2;
+    if (!vec) {
+        // The kernel that stages its operands in registers has 128 x 128 tiles and a long step: slices until they fill the
+        // chip (1024 x 30 x 1024, B of odd pitch: 144 us as one, 52 in four slices).
+        const long long tiles = ceil_div(d->m, 128) * ceil_div(d->n, 128);
+        while (tiles <= 128 && tiles * s * 2 <= kCus && d->k / (s * 2) >= 256 && d->k % (s * 2 * BK) == 0) s *= 2;
+        return s;
+    }
+    // The smallest estimate of both launches, at most 16 MiB of slices. The sum takes 3 us, 0.3 per slice and its reads and the
+    // slices' stores 2.4 TB/s, six times that for rows that are not stored in vectors. Unsplit, 64 x 64 and 32 x 32
+    // tiles fall behind their estimate when K is long, more so where an XCD's tiles cover many rows of A (2048 x 512 x 4096
+    // fp16 24 - 27 us, 512 x 2048 x 4096 16). Fitted to 840 products of 64 - 2048 rows and columns, K = 1024 - 65536,
+    // both result types, 1 - 32 slices each. Decided by it (us, one / 2 / 4 / 8 / 16 slices): 512 x 512 x 16384 fp32 79 / 43 / 26 / 20 /
+    // 22; 1024 x 1024 x 4096 fp32 24 / 20 / 22 / 27 / 37, fp16 18 in one launch; 256 x 256 x 4096 19 / 14 / 11 / 11 / 12.
+    int cfg;
+    const double steps = (double)d->k / 1024;
+    double best = estimate_small(d->m, d->n, d->k, 1, 1, d->out_dtype == DMLHIP_F32, true, true, false, &cfg) *
+                  (1.0 + (d->m >= 2 * d->n ? 0.2 : 0.1) * fmin(fmax(steps - 2.0, 0.0), 4.0));
+    for (int t = 2; d->k % (t * BK) == 0 && d->k / t >= 256; t *= 2) {
+        const double bytes = 4.0 * t * (double)d->m * (double)d->n;
+        if (bytes > 16.0 * 1048576) break;
+        const double us = estimate_small(d->m, d->n, d->k / t, t, 1, true, true, true, false, &cfg) + 3.0 + 0.3 * t +
+                          bytes * (d->n % 8 ? 6.0 : 1.0) / 2.4e6;
+        if (us >= 0.95 * best) continue;
+        best = us;
+        s = t;
+    }
     return s;
 }
 
+static size_t split_k_bytes(const dmlhip_gemm_desc* d, int s) {
+    return s > 1 ? (size_t)s * d->m * d->n * sizeof(float) : 0;
+}
+
+int dmlhip_debug_gemm_f16_slices(const dmlhip_gemm_desc* d) { return split_k_factor(d, d && vector_operands(d, nullptr, nullptr)); }
+
+// for the call with whatever addresses the operands have
 size_t dmlhip_gemm_f16_workspace_bytes(const dmlhip_gemm_desc* d) {
-    const int s = split_k_factor(d);
-    if (s <= 1) return 0;
-    return (size_t)s * d->batch[1] * d->batch[2] * d->m * d->n * sizeof(float);
+    const size_t any = split_k_bytes(d, split_k_factor(d, false));
+    const size_t vec = d && vector_operands(d, nullptr, nullptr) ? split_k_bytes(d, split_k_factor(d, true)) : 0;
+    return any > vec ? any : vec;
 }
 
 int dmlhip_gemm_f16_ws(const dmlhip_gemm_desc* d, const void* a, const void* b, void* c, const void* bias,
                        const void* residual, void* pre_out, void* workspace, size_t workspace_bytes, void* stream) {
-    const int s = split_k_factor(d);
-    const bool plain = d && !bias && !residual && !pre_out && d->beta == 0.f && d->act == DMLHIP_ACT_NONE;
-    if (s <= 1 || !plain || !workspace || workspace_bytes < dmlhip_gemm_f16_workspace_bytes(d) || !a || !b || !c ||
-        d->c_stride_m != d->n || (d->batch[1] * d->batch[2] > 1))
-        return run_gemm_f16(d, a, b, c, bias, residual, pre_out, stream);
+    const bool plain = d && !bias && !residual && !pre_out && d->beta == 0.f && d->act == DMLHIP_ACT_NONE && a && b && c &&
+                       workspace && d->c_stride_m == d->n;
+    const int s = plain ? split_k_factor(d, vector_operands(d, a, b)) : 1;
+    if (s <= 1 || workspace_bytes < split_k_bytes(d, s)) return run_gemm_f16(d, a, b, c, bias, residual, pre_out, stream);
     // stage 1: batch slot 0 enumerates the K slices; partial C tiles are dense fp32 [s][m][n]
     dmlhip_gemm_desc p = *d;
     p.k = d->k / s;

@@ -488,6 +488,9 @@ void dmlhip_debug_force_gemm_config(int cfg);
 /* Diagnostic: the configuration that the calling thread's last fp16 contraction launch ran on (of several launches, the
  * last); -1 = the kernel that stages its operands through registers. */
 int dmlhip_debug_last_gemm_config(void);
+/* Diagnostic: into how many slices of K, summed by a second launch, dmlhip_gemm_f16_ws cuts a plain product of operands
+ * aligned to 16 bytes. Launches nothing. */
+int dmlhip_debug_gemm_f16_slices(const dmlhip_gemm_desc* d);
 /* Pin the tile of the fp32 contraction kernel: 0 = 128x128, 1 = 64x64, 2 = 32x32 with K split over the wavefronts;
  * -1 = chosen per problem (default). Operands that cannot be read 16 bytes at a time have no 128x128 form and run on 64x64.
  * Per calling thread. */
