@@ -510,7 +510,7 @@ void dmlhip_debug_gemm_direct_lds(int on);
 /* Per-workgroup timing of the pipelined fp16 contraction kernel: with a device buffer of 4 x 8 bytes per workgroup of
  * the next launches set here, every workgroup stores four readings of the 100 MHz wall clock (start, first tile in
  * LDS, end of the K loop, end of the epilogue) at buffer[4 * workgroup]; NULL (default) switches it off. The caller
- * sizes the buffer for the largest grid it launches. Per calling thread. */
+ * sizes the buffer for the largest grid it launches. Products on configurations 10 and 12 store nothing. Per calling thread. */
 void dmlhip_debug_gemm_trace(void* buffer);
 /* Number of grouped / K-concatenated / row-sum contraction calls that went out as one launch so far. */
 long long dmlhip_debug_grouped_single_launches(void);
