@@ -50,10 +50,25 @@ inline half4v lds_read_tr16_b64(uint32_t addr) {
 
 inline void global_store_b128_through(void* p, half8 v) { *static_cast<half8*>(p) = v; }
 
+// Kernels whose wavefronts keep rings of their own have no barrier between a transfer and the read of another lane's piece,
+// nor between a read and the transfer that reuses its place: there the lanes' lockstep counts, and every wait is a point where
+// the lanes of a wavefront meet.
+#ifdef EMU_LOCKSTEP_WAITS
+inline void meet() { emu::wave_barrier(); }
+#else
+inline void meet() {}
+#endif
+
 template <int N>
-inline void wait_lgkm() {}
+inline void wait_lgkm() { meet(); }
 
 template <int VM>
-inline void wait_vm_lgkm0() { emu::dma_wait(VM); }
+inline void wait_vm_lgkm0() {
+    emu::dma_wait(VM);
+    meet();
+}
+
+template <typename T>
+inline void lds_keep(T) {}
 
 }  // namespace dml
