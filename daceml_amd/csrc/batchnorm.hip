@@ -11,9 +11,9 @@
 // last vector overlaps the one before and its leading elements are left out.
 // Measured, us: statistics, apply with Swish, backward sums, backward apply - before (chunks of 4096 elements per segment, one
 // load in flight, 4-byte loads where HW is no multiple of 8) and now: 32 x 144 x 56 x 56 fp32 12.5 / 20.1 / 21.5 / 27.8 and
-// 10.4 / 18.2 / 19.4 / 26.2 (57.8 MB a tensor, 4.4 to 6.6 TB/s), 55 x 55 18.1 / 25.0 / 24.4 / 32.3 and 10.6 / 18.0 / 20.1 / 26.6,
-// 32 x 480 x 14 x 14 11.9 / 13.0 / 13.3 / 13.0 and 4.1 / 5.9 / 5.5 / 7.3, 32 x 24 x 56 x 56 3.6 / 5.2 / 5.1 / 5.7 and
-// 4.1 / 5.3 / 5.9 / 6.3; fp16 32 x 144 x 56 x 56 8.9 / 11.5 / 15.0 / 15.9 and 6.9 / 10.9 / 13.6 / 15.5. Skipping the loads behind the
+// 9.8 / 18.1 / 18.3 / 26.9 (57.8 MB a tensor, 4.3 to 6.4 TB/s), 55 x 55 18.1 / 25.0 / 24.4 / 32.3 and 9.9 / 17.9 / 19.0 / 26.5,
+// 32 x 480 x 14 x 14 11.9 / 13.0 / 13.3 / 13.0 and 4.1 / 5.9 / 5.3 / 7.4, 32 x 24 x 56 x 56 3.6 / 5.2 / 5.1 / 5.7 and
+// 3.7 / 5.0 / 5.2 / 6.0; fp16 32 x 144 x 56 x 56 8.9 / 11.5 / 15.0 / 15.9 and 6.6 / 11.2 / 12.6 / 15.4. Skipping the loads behind the
 // end of a span by a branch each, instead of loading a vector again, cost more than the loads (12.3 instead of 10.4).
 // Pointers or extents that do not allow this (an fp16 segment that is no multiple of 16 bytes, HW below a vector) go
 // element by element: segments cut into chunks of at most kChunk, workgroup (c, s) takes the chunks s, s+S, ...
