@@ -602,7 +602,7 @@ static int split_k_factor(const dmlhip_gemm_desc* d, bool vec) {
     // tiles fall behind their estimate when K is long, more so where an XCD's tiles cover many rows of A (2048 x 512 x 4096
     // fp16 24 - 27 us, 512 x 2048 x 4096 16). Fitted to 840 products of 64 - 2048 rows and columns, K = 1024 - 65536,
     // both result types, 1 - 32 slices each. Decided by it (us, one / 2 / 4 / 8 / 16 slices): 512 x 512 x 16384 fp32 79 / 43 / 26 / 20 /
-    // 22; 1024 x 1024 x 4096 fp32 24 / 20 / 22 / 27 / 37, fp16 18 in one launch; 256 x 256 x 4096 19 / 14 / 11 / 11 / 12.
+    // 22; 1024 x 1024 x 4096 fp32 24 / 20 / 22 / 27 / 37, fp16 18 in one launch; 256 x 256 x 4096 fp32 19 / 14 / 11 / 11 / 12.
     int cfg;
     const double steps = (double)d->k / 1024;
     double best = estimate_small(d->m, d->n, d->k, 1, 1, d->out_dtype == DMLHIP_F32, true, true, false, &cfg) *

@@ -17,7 +17,7 @@ def _strides(rows, k, layout):
 # m, n, k, layouts of A and B (0 = K contiguous), result type, slices
 SLICES = [(512, 512, 16384, (1, 1), L.F32, 8), (1024, 1024, 4096, (0, 0), L.F32, 2), (1024, 1024, 4096, (0, 0), L.F16, 1),
           (768, 768, 16384, (1, 1), L.F32, 4), (2048, 512, 8192, (1, 1), L.F16, 4), (2048, 512, 4096, (1, 1), L.F16, 2),
-          (64, 64, 3072, (1, 1), L.F16, 4), (256, 256, 4096, (0, 0), L.F32, 8), (1024, 1024, 1024, (0, 0), L.F16, 1),
+          (64, 64, 3072, (1, 1), L.F16, 1), (64, 64, 8192, (1, 1), L.F16, 8), (256, 256, 4096, (0, 0), L.F32, 8), (1024, 1024, 1024, (0, 0), L.F16, 1),
           (1024, 30, 1024, (1, 1), L.F32, 4), (1024, 30, 8192, (1, 1), L.F16, 32), (512, 512, 4095, (0, 0), L.F16, 1),
           (4096, 4096, 4096, (0, 0), L.F16, 1), (1, 0, 4096, (0, 0), L.F16, 1)]
 
