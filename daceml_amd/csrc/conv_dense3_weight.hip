@@ -266,17 +266,27 @@ int64_t plan_ranges(const ConvGeom& g, bool general) {
     // Where the general kernel does not apply (fewer than 64 output pixels: 5x256x14x14 -> 512, stride 2, 1200 us against 35)
     // this one runs from 2^24 multiply-adds on. Where it does, the rules below hold what was measured against it, us there and
     // here: first loads, the sums through LDS and the reduction take 18 us whatever the size (1x64x56x56 -> 64 14 and 20;
-    // 8x64x55x55 -> 64, 2^30, 44 and 44); channels are padded to 32, which the general kernel does over all c * 9 columns
-    // (16 of 112 x 112, 64 images -> 64 1.0 - 1.16 times its time, 24 of 33 x 33 0.76 - 1.01); rows of X that are no multiple
-    // of four floats cost a gather per float, too much with stride 2 (64x64x113x113 -> 64 301 and 355) and with long
-    // rows for a single tile of output channels (32x32x113x113 -> 32 155 and 185, -> 64 247 and 259, -> 128 525 and 492) or a
+    // 8x64x55x55 -> 64, 2^30, 44 and 44); channels are padded to 32, which the general kernel does
+    // over all c * 9 columns (16 of 112 x 112, 64 images -> 64 1.0 - 1.16 times its time); rows of X that are no multiple of four
+    // floats cost a gather per float, too much with stride 2 (64x64x113x113 -> 64 301 and 355), with
+    // few multiply-adds (90 problems of 2^29 - 2^29.3: 14x64x35x35 -> 64 36 and 43, 3x64x57x57 -> 96 31 and 41, 7x32x33x33 -> 256 50 and 42; rows
+    // of whole vectors 0.64 - 0.95 of its time, 1.08 at worst), with long
+    // rows for a single tile of output channels (32x32x113x113 -> 32 155 and 185, -> 64 247 and 259, -> 128 525 and 492), for such a tile
+    // over padded channels (times its time at 2^29.1 / 2^30.2 / 2^31 / 2^31.8: 44 of 41 x 41 -> 64 1.29 / 1.20 / 1.16 / 1.00, 24 of 33 x 33 -> 64
+    // 1.17 / 1.10 / 1.07 / 1.03, 80 of 41 x 41 -> 32 1.10 / 1.11 / 1.05 / 0.88, 26 of 27 x 27 -> 32 1.06 / 0.90 / 0.83 / 0.81) or for a
     // last one that is half empty (32x96x57x57 -> 96 285 and 342).
     if (macs < (double)(1 << (general ? 29 : 24))) return 0;
     if (general) {
         const bool narrow = g.w % 4 != 0;
-        if (2 * ceil_div(g.c, kCTile) * kCTile > 3 * g.c) return 0;
+        const int64_t padded = ceil_div(g.c, kCTile) * kCTile;
+        if (2 * padded > 3 * g.c) return 0;
         const int64_t mb = g.m > 32 ? 64 : 32;
         if (narrow && (g.sw > 1 || (g.ow > 64 && g.m <= 64) || 4 * ceil_div(g.m, mb) * mb > 5 * g.m)) return 0;
+        if (narrow && g.m < 128 && macs < 7.0e8) return 0;
+        // columns here for one there
+        const double columns = (double)(padded * kTaps) / (double)(ceil_div((int64_t)g.c * kTaps, (int64_t)32) * 32);
+        const double least = columns > 1.35 ? 1e18 : columns > 1.2 ? (g.ow < 50 ? 3.0e9 : 1e18) : columns > 1.15 ? 2.2e9 : 1.1e9;
+        if (narrow && g.m <= 64 && columns > 1.0 && macs < least) return 0;
     }
     if (rows > (1LL << 30) || per > (1LL << 30) || (int64_t)g.oh * g.ow > (1LL << 28) || (int64_t)g.h * g.w > (1LL << 28)) return 0;
     WeightPlan pl;

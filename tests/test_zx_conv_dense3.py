@@ -28,7 +28,8 @@ def _check(what, got, exact, terms, k):
 # weight gradients that are large enough for the kernel, or too small in pixels for the general one
 WEIGHT_SHAPES = [(40, 33, 31, 33, 70, 1, 1, 1), (6, 64, 56, 56, 64, 1, 1, 1), (4, 96, 30, 64, 96, 1, 2, 2), (16, 32, 64, 64, 32, 1, 1, 1),
                  (40, 64, 57, 55, 64, 2, 1, 1), (20, 64, 14, 14, 64, 2, 1, 1), (6, 256, 7, 7, 65, 1, 1, 1), (1, 40, 300, 110, 70, 1, 0, 1),
-                 (40, 44, 31, 33, 60, 1, 1, 1), (20, 64, 13, 13, 64, 2, 1, 1), (1, 48, 300, 110, 120, 1, 0, 1)]
+                 (40, 44, 31, 33, 60, 1, 1, 1), (20, 64, 13, 13, 64, 2, 1, 1), (1, 48, 300, 110, 120, 1, 0, 1),
+                 (20, 44, 31, 33, 110, 1, 1, 1)]
 
 
 def _problem(shape):
