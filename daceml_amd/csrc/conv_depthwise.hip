@@ -215,8 +215,10 @@ int launch_same_weight(PlaneArgs a, int64_t planes, int h, int wd, hipStream_t s
 // 256 planes of 4 x 4 2.8 / 5.2, of 12 x 12 3.4 / 4.7, of 28 x 28 4.6 / 4.6, of 33 x 33 6.7 / 4.6; data gradient 256 planes of
 // 28 x 28 3.2 / 3.8, of 40 x 40 4.8 / 3.9. The more planes, the smaller they may be (forward, 14 x 14: 512 4.5 / 4.7,
 // 1536 6.7 / 4.8). vec: rows in 16-byte pieces, which spread planes below 17 columns over a quarter of the lanes.
-bool same_faster(int64_t planes, int64_t hw, int k, bool vec, bool data) {
-    if (hw > 1024) return true;
+// A single row fills a seventh of a strip: data gradient of 5120 planes of 1 x 1000 11.1 / 15.7, of 2 x 512 17.6 / 11.3.
+bool same_faster(int64_t planes, int h, int64_t hw, int k, bool vec, bool data) {
+    if (data && h == 1 && hw >= 512) return false;
+    if (hw > (data ? 1024 : 784)) return true;      // forward, 8 planes of 29 x 29 5.8 / 4.2
     if (hw >= 784) return planes >= 384;
     const bool wide = k == 5 && !data;           // forward 5 x 5: a sixth more before a strip's loads are paid for
     if (hw > 256) return planes >= (wide ? 768 : 512);
@@ -226,11 +228,22 @@ bool same_faster(int64_t planes, int64_t hw, int k, bool vec, bool data) {
 }
 
 // The same for the weight gradient, where a plane has at most one wavefront here and four there: 3 x 3 on 96 planes of
-// 14 x 14 2.7 / 6.3, 768 of 56 x 56 13.0 / 11.9, 480 of 111 x 111 32.3 / 33.0, 4096 of 14 x 14 10.4 / 9.2; 5 x 5 on 512 planes of
-// 12 x 12 7.8 / 9.1, of 24 x 24 12.5 / 9.7, 96 of 112 x 112 116 / 56.
-bool same_weight_faster(int64_t planes, int64_t hw, int k, bool vec) {
+// 14 x 14 2.7 / 6.3, 768 of 56 x 56 13.0 / 11.9, 480 of 111 x 111 32.3 / 33.0, 4096 of 14 x 14 10.4 / 9.2, 5120 of 3 x 301 23.8 / 26.6;
+// 5 x 5 on 512 planes of 12 x 12 7.8 / 9.1, of 24 x 24 12.5 / 9.7, 96 of 112 x 112 116 / 56. Few planes under 5 x 5 wait for every pass of
+// their wavefront, full or not: 29 x 29 is one full pass, 11.4 / 8.9, 60 x 33 three that are two thirds full, 21.0 / 28.9.
+template <int K> bool full_passes(int h, int wd, bool vec) {
+    const int64_t cells = (int64_t)((wd + 3) / 4) * ((h + strip_rows<K>() - 1) / strip_rows<K>());
+    const int64_t held = ceil_div(cells, (int64_t)64) * 64 * 4 * strip_rows<K>();
+    return (int64_t)h * wd * 100 >= held * (vec ? 45 : 75);
+}
+bool same_weight_faster(int64_t planes, int h, int wd, int k, bool vec) {
+    const int64_t hw = (int64_t)h * wd;
     if (hw <= 16) return planes >= (k == 3 ? 6144 : 3072);
-    if (k == 5) return hw >= (vec ? 576 : 784) || planes >= (vec ? 1536 : 2048) || (vec && hw >= 400 && planes >= 384);
+    if (k == 5) {
+        if (planes >= (vec ? 1536 : 2048)) return true;
+        return hw >= (vec ? (planes >= 384 ? 400 : 576) : 784) && (planes >= (vec ? 1024 : 512) || full_passes<5>(h, wd, vec));
+    }
+    if (hw >= 512 && h <= (vec ? 1 : 3)) return false;
     if (!vec) return planes >= 4096 || (planes >= 2048 && hw >= 1024) || (planes >= 1024 && hw >= 8192);
     return planes >= 3072 || planes * hw >= 2000000 || hw >= 40000 || (planes >= 768 && planes * hw >= 800000);
 }
@@ -252,12 +265,12 @@ bool depthwise_same_applicable(const ConvGeom& g) {
 
 bool depthwise_same_faster(const ConvGeom& g, const void* in, const void* out, bool data) {
     if (g_force_same >= 0) return g_force_same != 0;
-    return same_faster((int64_t)g.n * g.c, (int64_t)g.h * g.w, g.kh, vec_rows(g, in, out), data);
+    return same_faster((int64_t)g.n * g.c, g.h, (int64_t)g.h * g.w, g.kh, vec_rows(g, in, out), data);
 }
 
 bool depthwise_same_weight_faster(const ConvGeom& g, const void* x, const void* dy) {
     if (g_force_same >= 0) return g_force_same != 0;
-    return same_weight_faster((int64_t)g.n * g.c, (int64_t)g.h * g.w, g.kh, vec_rows(g, x, dy));
+    return same_weight_faster((int64_t)g.n * g.c, g.h, g.w, g.kh, vec_rows(g, x, dy));
 }
 
 int launch_depthwise_same(const ConvGeom& g, const float* x, const float* w, const float* bias, float* y, hipStream_t st) {
