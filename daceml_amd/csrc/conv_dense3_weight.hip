@@ -11,6 +11,8 @@
 // pixels. Rows of dY and the rows of X under them go global -> LDS without staging registers, a chunk of output rows of one
 // image at a time, one chunk ahead, issued between the MFMAs of the chunk before. The wavefronts' sums are added through LDS
 // and the ranges' results by the reduction kernel, all in a fixed order.
+// All sums are fp32. A wavefront adds 70 - 200 pixels in one chain where the general kernel's chains are shorter: 6.7e-8 - 1.3e-7 of the
+// gradient from the fp64 one (2-norm), 5.6e-8 - 7.0e-8 there; a second set of accumulators does not fit the registers.
 #include "common.h"
 #include "conv_geom.h"
 #include "lds_ops.h"
