@@ -28,6 +28,7 @@ SOURCES = [
     "gemm_f16_pipe_ragged.hip",
     "gemm_f16_split.hip",
     "gemm_f32.hip",
+    "gemm_f32_split.hip",
     "conv.hip",
     "conv_fused.hip", "conv_backward.hip", "conv_implicit.hip", "conv_dense3.hip", "conv_dense3_weight.hip", "conv_depthwise.hip",
     "conv_pointwise_few.hip",

@@ -1,6 +1,6 @@
-// fp32 strided batched GEMM on the matrix cores with true fp32 products
-// (v_mfma_f32_32x32x2_f32; no reduced-precision path), for the fp32 MatMul / Einsum / Gemm
-// nodes and the 1x1 convolutions.
+// fp32 strided batched GEMM on v_mfma_f32_32x32x2_f32, operands streamed through LDS, for the fp32 MatMul / Einsum / Gemm nodes
+// and the 1x1 convolutions: small and short products, and operands that cannot be read 16 bytes at a time (gemm_f32_split.hip has
+// the entry point, the rule and the kernel for the others).
 //
 // What bounds it: the fp32 matrix rate (256 operations per clock and compute unit). A 64 x 64 tile needs 16 bytes per
 // clock through L2 at that rate, a 32 x 32 tile 32 - both under the 64 that a compute unit takes in - so the tile is
@@ -375,8 +375,6 @@ int launch32(GemmArgs32& g, long long batch, hipStream_t st) {
     return launch_status("gemm_f32");
 }
 
-thread_local int g_force_tile = -1;   // diagnostic: 0 = 128 x 128, 1 = 64 x 64, 2 = 32 x 32
-
 template <int AROWS, int AVEC, int BROWS, int BVEC>
 int launch_operands(GemmArgs32& g, int tile, long long batch, hipStream_t st) {
     if constexpr (AVEC == 4 && BVEC == 4) {
@@ -403,52 +401,37 @@ int operand_mode32(const void* p, int64_t rows, int64_t k, int64_t s_row, int64_
 // MFMA: the smaller the tile, the more instructions beside each MFMA). What it decides, us for the three tiles:
 // 4096^3 1032 / 1124 / 1311; 1024 x 3072 x 768 (m x n x k) 62 / 51 / 63; 1024 x 768 x 3072 197 / 64 / 55;
 // 64 x 128 x 784 58 / 19 / 8.
-int choose_tile(const GemmArgs32& g, long long batch) {
+int choose_tile(int64_t m, int64_t n_cols, int64_t k, long long batch, double* estimate) {
     struct Tile { int size, resident; double round_us, step_us; };
     constexpr Tile kTiles[3] = {{128, 2, 8.0, 1.93}, {64, 3, 4.5, 0.56}, {32, 2, 4.5, 0.155}};
-    const double steps = (double)ceil_div(g.k, BK);
+    const double steps = (double)ceil_div(k, (int64_t)BK);
     int best = 0;
     double best_t = 0;
     for (int i = 0; i < 3; ++i) {
         const Tile& t = kTiles[i];
-        const double n = ceil((double)ceil_div(g.m, t.size) * ceil_div(g.n, t.size) * batch / kCus);
+        const double n = ceil((double)ceil_div(m, t.size) * ceil_div(n_cols, t.size) * batch / kCus);
         const double us = ceil(n / t.resident) * t.round_us + n * steps * t.step_us;
         if (i == 0 || us < best_t) {
             best = i;
             best_t = us;
         }
     }
+    if (estimate) *estimate = best_t;
     return best;
 }
 
 }  // namespace
-}  // namespace dml
 
-using namespace dml;
-extern "C" int dmlhip_gemm_f32(const dmlhip_gemm_desc* d, const void* a, const void* b, void* c, const void* bias,
-                               const void* residual, void* pre_out, void* stream) {
-    DML_REQUIRE(d, DMLHIP_ERR_NULL, "gemm_f32: NULL descriptor");
-    DML_REQUIRE(d->m >= 0 && d->n >= 0 && d->k >= 0, DMLHIP_ERR_SHAPE, "gemm_f32: negative extent");
-    DML_REQUIRE(d->m <= 2147483647 / 2 && d->n <= 2147483647 / 2 && d->k <= 2147483647 / 2, DMLHIP_ERR_SHAPE,
-                "gemm_f32: extent exceeds 2^30");
-    long long batch = 1;
-    for (int i = 0; i < 3; ++i) {
-        DML_REQUIRE(d->batch[i] >= 0 && d->batch[i] <= 2147483647, DMLHIP_ERR_SHAPE, "gemm_f32: bad batch extent");
-        batch *= d->batch[i];
-        DML_REQUIRE(batch <= 2147483647LL, DMLHIP_ERR_SHAPE, "gemm_f32: batch too large");
-    }
-    DML_REQUIRE(d->out_dtype == DMLHIP_F32, DMLHIP_ERR_ENUM, "gemm_f32: out_dtype must be DMLHIP_F32");
-    DML_REQUIRE(d->bias_dtype == DMLHIP_F16 || d->bias_dtype == DMLHIP_F32, DMLHIP_ERR_ENUM,
-                "gemm_f32: bad bias_dtype");
-    DML_REQUIRE(valid_act(d->act), DMLHIP_ERR_ENUM, "gemm_f32: bad act");
-    DML_REQUIRE(d->a_stride_m >= 0 && d->a_stride_k >= 0 && d->b_stride_k >= 0 && d->b_stride_n >= 0 &&
-                    d->c_stride_m >= 0,
-                DMLHIP_ERR_SHAPE, "gemm_f32: negative stride");
-    DML_REQUIRE(d->c_stride_m >= d->n || d->m <= 1, DMLHIP_ERR_SHAPE, "gemm_f32: rows of C overlap");
-    if (d->m == 0 || d->n == 0 || batch == 0) return 0;
-    DML_REQUIRE(c, DMLHIP_ERR_NULL, "gemm_f32: NULL output");
-    DML_REQUIRE(d->k == 0 || (a && b), DMLHIP_ERR_NULL, "gemm_f32: NULL operand");
+// What the chosen tile is estimated to take
+double gemm_f32_streamed_us(const dmlhip_gemm_desc* d, long long batch) {
+    double us;
+    choose_tile(d->m, d->n, d->k, batch, &us);
+    return us;
+}
 
+// The arguments are checked (gemm_f32_split.hip). tile: 0 = 128 x 128, 1 = 64 x 64, 2 = 32 x 32, -1: chosen here.
+int gemm_f32_streamed(const dmlhip_gemm_desc* d, const void* a, const void* b, void* c, const void* bias, const void* residual,
+                      void* pre_out, int tile, long long batch, hipStream_t st) {
     GemmArgs32 g;
     g.a = (const float*)a; g.b = (const float*)b; g.c = (float*)c;
     g.bias = bias; g.residual = (const float*)residual; g.pre = (float*)pre_out;
@@ -466,8 +449,7 @@ extern "C" int dmlhip_gemm_f32(const dmlhip_gemm_desc* d, const void* a, const v
         if (d->batch[i] > 1 && d->c_stride_batch[i] % 4 != 0) g.c_vec = 0;
     const int am = operand_mode32(a, d->m, d->k, d->a_stride_m, d->a_stride_k, d->a_stride_batch, d->batch);
     const int bm = operand_mode32(b, d->n, d->k, d->b_stride_n, d->b_stride_k, d->b_stride_batch, d->batch);
-    const int tile = g_force_tile >= 0 ? g_force_tile : choose_tile(g, batch);
-    hipStream_t st = (hipStream_t)stream;
+    if (tile < 0) tile = choose_tile(g.m, g.n, g.k, batch, nullptr);
 #define DML_G32(AM, BMD) \
     if (am == AM && bm == BMD) \
         return launch_operands<(AM) & 1, (AM) & 2 ? 1 : 4, (BMD) & 1, (BMD) & 2 ? 1 : 4>(g, tile, batch, st);
@@ -479,4 +461,4 @@ extern "C" int dmlhip_gemm_f32(const dmlhip_gemm_desc* d, const void* a, const v
     return DMLHIP_ERR_UNSUPPORTED;
 }
 
-extern "C" void dmlhip_debug_force_gemm_f32_tile(int tile) { g_force_tile = tile; }
+}  // namespace dml

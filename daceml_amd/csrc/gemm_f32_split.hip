@@ -1,0 +1,521 @@
+// fp32 strided batched GEMM on the bf16 matrix cores: the entry point of the fp32 products and the kernel behind most of them.
+//
+// An fp32 value is the sum of three bf16 values, exactly: x = h + m + l, each the rounding of what the ones before leave
+// (24 bits are 8 + 8 + 8; below 2^-110 the last ones fall under the smallest bf16). Of the nine products of two such sums six
+// matter: h h, h m, m h, m m, h l, l h (the others are below 2^-26 of the product, under the rounding of the sum). The bf16
+// matrix rate is 16 times the fp32 one, so six products take 0.375 of the time of the fp32 instruction.
+// Precision: 16 products per rounding of the fp32 accumulator, the small ones of a step first. Error against the fp64 product,
+// 2-norm over 2-norm, in one chain of K here / on v_mfma_f32_32x32x2_f32 (one product per rounding): N(0, 1) K = 64 1.1e-7 /
+// 1.4e-7, 768 4.2e-7 / 5.0e-7, 3072 8.5e-7 / 9.7e-7; uniform on [0, 1) 768 2.9e-7 / 4.2e-7; log-normal over twelve decades 768
+// 1.7e-7 / 2.4e-7; and K is cut into four or eight chains: 1024 x 768 x 768 1.5e-7 where the streamed tiles have 2.5e-7 - 5.0e-7.
+// Infinities and NaN have no such sum: an element that comes out not finite is computed again, as a chain of fp32 multiply-adds.
+//
+// What bounds it: vector issue beside the matrix pipe. A wavefront's 64 x 64 tile is 24 MFMAs per 16 k (0.36 us) and 176
+// instructions that split the operands; on a compute unit with eight wavefronts a step takes 0.57 us per wavefront and SIMD. So the
+// splitting of the next step is placed between the MFMAs of this one (all of it first, then the MFMAs: 0.8 us), and there is
+// one accumulator per block, not a second one for the small products (registers: 0.8 us again). Measured, us, the kernel of
+// gemm_f32.hip / here: 1024 x 768 x 768 20 / 14, 1024 x 3072 x 768 48 / 35, 3072 x 768 x 1024 (both operands row-contiguous) 59 / 39,
+// 4096^3 1016 / 715 - 760 = 181 - 192 TFLOP/s, where the fp32 instruction's own limit is 157.
+#include "common.h"
+#include "lds_ops.h"
+
+#include <float.h>
+
+#include <type_traits>
+
+namespace dml {
+
+int gemm_f32_streamed(const dmlhip_gemm_desc* d, const void* a, const void* b, void* c, const void* bias, const void* residual,
+                      void* pre_out, int tile, long long batch, hipStream_t st);
+double gemm_f32_streamed_us(const dmlhip_gemm_desc* d, long long batch);
+
+namespace {
+
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+
+constexpr int BK = 16;           // K per step of a wavefront
+constexpr int kXcds = 8;
+constexpr int kBlock = 64;       // rows and columns of a tile
+constexpr int kStages = 2;
+constexpr int kCus = 256;
+
+struct SplitArgs {
+    const float* a;
+    const float* b;
+    float* c;
+    const void* bias;
+    const float* residual;
+    float* pre;
+    int m, n, k;
+    int64_t sam, sak, sbn, sbk, scm;
+    int batch1, batch2;
+    int64_t sab[3], sbb[3], scb[3];
+    float alpha, beta;
+    int bias_f32, act, bias_m;
+    int tiles_m, tiles_n;
+    int c_vec;                   // C (and residual, pre) can be accessed four columns at a time
+    long long total_blocks;
+};
+
+struct Pieces {
+    bf16x8 h, m, l;
+};
+
+// Eleven vector instructions for two values. (What a rounding leaves is also a dot product of a packed pair with (-1, 0) or
+// (0, -1), seven instructions in all, but v_dot2c_f32_bf16 does not issue beside the matrix pipe: 16 MFMAs with 64 of them took
+// 6.0 us where with 64 subtractions they took 3.8.)
+struct Splitter {
+    static __device__ __forceinline__ floatx2 unpack(uint32_t v) {
+        return {__builtin_bit_cast(float, v << 16), __builtin_bit_cast(float, v & 0xffff0000u)};
+    }
+    static __device__ __forceinline__ void pair(floatx2 v, uint32_t& h, uint32_t& m, uint32_t& l) {
+        h = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+        const floatx2 uh = unpack(h);
+        floatx2 r = {v[0] - uh[0], v[1] - uh[1]};
+        m = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, bf16x2));
+        const floatx2 um = unpack(m);
+        r = floatx2{r[0] - um[0], r[1] - um[1]};
+        l = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, bf16x2));
+    }
+    static __device__ __forceinline__ Pieces eight(const float (&v)[8]) {
+        u32x4 h, m, l;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            uint32_t ph, pm, pl;
+            pair(floatx2{v[2 * i], v[2 * i + 1]}, ph, pm, pl);
+            h[i] = ph;
+            m[i] = pm;
+            l[i] = pl;
+        }
+        return {__builtin_bit_cast(bf16x8, h), __builtin_bit_cast(bf16x8, m), __builtin_bit_cast(bf16x8, l)};
+    }
+};
+
+template <int I, int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        static_for<I + 1, N>(f);
+    }
+}
+
+// what lanes outside the operand read
+__device__ const floatx4 g_zero_page = {0.f, 0.f, 0.f, 0.f};
+
+// One operand of a wavefront: 64 rows x 16 k per stage of its ring, 16 bytes per lane and transfer.
+// ROWS = 0: LDS rows of 16 k (64 bytes, 16-byte chunks XOR-swizzled), block b of 32 has rows 32 b + j.
+// ROWS = 1: LDS rows of one k, 64 tile rows each; block b has rows 2 j + b, so that one read fetches both blocks' values.
+// Lanes past the last row read it again (their results are not stored), lanes past the last k a page of zeros.
+template <int ROWS>
+struct Operand {
+    static constexpr int N = kBlock * BK / 256;      // transfers of a stage
+    uint32_t off[N];    // bytes
+    uint32_t faddr;
+    __device__ __forceinline__ void init(int64_t s_row, int64_t s_k, int rows_left, int lane, uint32_t ring) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            if constexpr (ROWS == 0) {
+                const int r = i * 16 + (lane >> 2);
+                off[i] = ((uint32_t)min(r, rows_left - 1) * (uint32_t)s_row + (uint32_t)k_of(i, lane)) * 4;
+            } else {
+                off[i] = ((uint32_t)k_of(i, lane) * (uint32_t)s_k + (uint32_t)min((lane & 15) * 4, rows_left - 4)) * 4;
+            }
+        }
+        const int j = lane & 31, half = lane >> 5;
+        if constexpr (ROWS == 0) faddr = ring + j * 64 + (((half * 2) ^ ((j >> 1) & 3)) << 4);
+        else faddr = ring + half * 8 * kBlock * 4 + j * 8;
+    }
+    // first k of the stage that this lane's transfer i holds
+    static __device__ __forceinline__ int k_of(int i, int lane) {
+        if constexpr (ROWS == 0) return ((lane & 3) ^ ((lane >> 3) & 3)) * 4;    // row i * 16 + lane / 4: (row / 2) % 4
+        return i * 4 + (lane >> 4);
+    }
+    __device__ __forceinline__ void issue(const float* p, char* stage) const {
+#pragma unroll
+        for (int i = 0; i < N; ++i) dma(reinterpret_cast<const char*>(p) + off[i], stage + i * 1024);
+    }
+    // the same for a stage that reaches past the end of K (`left` < 16)
+    __device__ __forceinline__ void issue_tail(const float* p, int left, char* stage, int lane) const {
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            dma(k_of(i, lane) < left ? reinterpret_cast<const char*>(p) + off[i] : reinterpret_cast<const char*>(&g_zero_page),
+                stage + i * 1024);
+    }
+    static __device__ __forceinline__ void dma(const char* p, char* lds_dst) {
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)p,
+                                         (__attribute__((address_space(3))) void*)lds_dst, 16, 0, 0);
+    }
+    // this lane's eight k (8 (lane / 32) on) of its row in either block
+    struct Raw {
+        floatx4 q[4];       // ROWS = 0: two of block 0, two of block 1
+        floatx2 p[8];       // ROWS = 1: k by k, both blocks
+    };
+    __device__ __forceinline__ void read(uint32_t stage, Raw& v) const {
+        if constexpr (ROWS == 0) {
+            const uint32_t a = faddr + stage;
+            v.q[0] = __builtin_bit_cast(floatx4, lds_read_b128<0>(a));
+            v.q[1] = __builtin_bit_cast(floatx4, lds_read_b128<0>(a ^ 16));
+            v.q[2] = __builtin_bit_cast(floatx4, lds_read_b128<32 * 64>(a));
+            v.q[3] = __builtin_bit_cast(floatx4, lds_read_b128<32 * 64>(a ^ 16));
+        } else {
+            static_for<0, 8>([&](auto ec) {
+                constexpr int e = decltype(ec)::value;
+                v.p[e] = lds_read_b64<e * kBlock * 4>(faddr + stage);
+            });
+        }
+    }
+    template <int B>
+    static __device__ __forceinline__ Pieces block(const Raw& v) {
+        float w[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) w[e] = ROWS == 0 ? v.q[2 * B + e / 4][e % 4] : v.p[e][B];
+        return Splitter::eight(w);
+    }
+};
+
+__device__ __forceinline__ float bias_at(const SplitArgs& g, int i) {
+    return g.bias_f32 ? reinterpret_cast<const float*>(g.bias)[i] : (float)reinterpret_cast<const _Float16*>(g.bias)[i];
+}
+
+// v = alpha * acc + bias, stored to pre; act(v) + residual + beta * C
+__device__ __forceinline__ float finish(const SplitArgs& g, float acc, float bias, int64_t off) {
+    float v = g.alpha * acc + bias;
+    if (g.pre) g.pre[off] = v;
+    v = apply_act(g.act, v);
+    if (g.residual) v += g.residual[off];
+    if (g.beta != 0.f) v += g.beta * g.c[off];
+    return v;
+}
+
+// The pieces exist from here on: they are not computed where they are used, behind the products that hide them.
+__device__ __forceinline__ void keep(Pieces (&p)[2]) {
+    asm volatile("" : "+v"(p[0].h), "+v"(p[0].m), "+v"(p[0].l), "+v"(p[1].h), "+v"(p[1].m), "+v"(p[1].l));
+}
+
+// A matrix instruction, then what the vector pipe can issue under it
+__device__ __forceinline__ void interleave() {
+#pragma unroll
+    for (int i = 0; i < 12; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x2, 8, 0);
+    }
+}
+
+// KG: wavefronts, each of which takes every KG-th step of K (16) of the same 64 x 64 tile, with a ring of its own: no barrier in
+// the loop. Their sums are added through LDS behind it.
+template <int KG, int AROWS, int BROWS>
+__global__ __launch_bounds__(kWave * KG, 2) void gemm_f32_split_kernel(const SplitArgs g) {
+    constexpr int TB = kBlock, THREADS = kWave * KG;
+    constexpr int A_BYTES = kBlock * BK * 4, STAGE = 2 * A_BYTES;
+    typedef Operand<AROWS> OA;
+    typedef Operand<BROWS> OB;
+    constexpr int LPT = OA::N + OB::N;                // transfers per step
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    uint32_t bid = blockIdx.x;
+    {
+        const uint32_t total = (uint32_t)g.total_blocks;
+        const uint32_t xcd = bid % kXcds, idx = bid / kXcds;
+        const uint32_t base = total / kXcds, rem = total % kXcds;
+        bid = xcd * base + (xcd < rem ? xcd : rem) + idx;
+    }
+    const uint32_t tiles = (uint32_t)(g.tiles_m * g.tiles_n);
+    const uint32_t batch = bid / tiles, tile = bid - batch * tiles;
+    // groups of eight tile rows, column by column: the tiles an XCD works on together share few rows and columns
+    constexpr uint32_t kGroupM = 8;
+    const uint32_t per_group = kGroupM * (uint32_t)g.tiles_n;
+    const uint32_t group = tile / per_group, in_group = tile - group * per_group;
+    const uint32_t rows_here = min((uint32_t)g.tiles_m - group * kGroupM, kGroupM);
+    const int tn = (int)(in_group / rows_here), tm = (int)(group * kGroupM + in_group % rows_here);
+    const int z2 = (int)(batch % (uint32_t)g.batch2);
+    const uint32_t q = batch / (uint32_t)g.batch2;
+    const int z1 = (int)(q % (uint32_t)g.batch1), z0 = (int)(q / (uint32_t)g.batch1);
+    const float* A = g.a + z0 * g.sab[0] + z1 * g.sab[1] + z2 * g.sab[2];
+    const float* B = g.b + z0 * g.sbb[0] + z1 * g.sbb[1] + z2 * g.sbb[2];
+    const int64_t coff = z0 * g.scb[0] + z1 * g.scb[1] + z2 * g.scb[2];
+
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int m0 = tm * TB, n0 = tn * TB;
+    char* const ring = lds + wave * kStages * STAGE;
+    const uint32_t ring0 = lds_addr(ring);
+
+    floatx16 acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+
+    OA oa;
+    OB ob;
+    oa.init(g.sam, g.sak, g.m - m0, lane, ring0);
+    ob.init(g.sbn, g.sbk, g.n - n0, lane, ring0 + A_BYTES);
+    const int steps = (g.k + BK - 1) / BK, mine = (steps - wave + KG - 1) / KG;
+    const float* pa = A + (int64_t)m0 * g.sam + (int64_t)wave * BK * g.sak;
+    const float* pb = B + (int64_t)n0 * g.sbn + (int64_t)wave * BK * g.sbk;
+    int left = g.k - wave * BK;                       // k from the next transfers' first one on
+    auto issue = [&](uint32_t stage) {                // this wavefront's next step
+        char* const at = ring + stage;
+        if (left >= BK) {
+            oa.issue(pa, at);
+            ob.issue(pb, at + A_BYTES);
+        } else {
+            oa.issue_tail(pa, left, at, lane);
+            ob.issue_tail(pb, left, at + A_BYTES, lane);
+        }
+        pa += KG * BK * g.sak;
+        pb += KG * BK * g.sbk;
+        left -= KG * BK;
+    };
+    if (mine > 0) {
+        typename OA::Raw va;
+        typename OB::Raw vb;
+        Pieces fa[2][2], fb[2][2];
+        // Step t, whose pieces are in set CUR, while the values of step t + 1 are split into the other set: A's, read half a step
+        // ago, then B's. Half way through every value of step t + 1 is in registers: its stage takes the transfers of step
+        // t + 3. LEFT: steps that follow (2 for more). Products in order of size, so that the large ones come last.
+        auto step = [&](int t, auto cur_c, auto left_c) {
+            constexpr int CUR = decltype(cur_c)::value, NXT = CUR ^ 1, LEFT = decltype(left_c)::value;
+            const uint32_t here = (uint32_t)((t & 1) * STAGE), other = STAGE - here;
+            const Pieces(&a)[2] = fa[CUR];
+            const Pieces(&b)[2] = fb[CUR];
+#define DML_PRODUCT(AP, BP)                                                                                               \
+    _Pragma("unroll") for (int i = 0; i < 2; ++i) _Pragma("unroll") for (int j = 0; j < 2; ++j)                           \
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i].AP, b[j].BP, acc[i][j], 0, 0, 0);
+            if constexpr (LEFT > 0) {
+                wait_lgkm<0>();
+                ob.read(other, vb);
+                __builtin_amdgcn_sched_barrier(0);
+                fa[NXT][0] = OA::template block<0>(va);
+                fa[NXT][1] = OA::template block<1>(va);
+            }
+            DML_PRODUCT(l, h)
+            DML_PRODUCT(h, l)
+            DML_PRODUCT(m, m)
+            if constexpr (LEFT > 0) {
+                interleave();
+                keep(fa[NXT]);
+                __builtin_amdgcn_sched_barrier(0);
+                wait_vm_lgkm0<0>();
+                if constexpr (LEFT > 1) {
+                    oa.read(here, va);
+                    if (t + 3 < mine) issue(other);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                fb[NXT][0] = OB::template block<0>(vb);
+                fb[NXT][1] = OB::template block<1>(vb);
+            }
+            DML_PRODUCT(m, h)
+            DML_PRODUCT(h, m)
+            DML_PRODUCT(h, h)
+            if constexpr (LEFT > 0) {
+                interleave();
+                keep(fb[NXT]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#undef DML_PRODUCT
+        };
+        typedef std::integral_constant<int, 0> c0;
+        typedef std::integral_constant<int, 1> c1;
+        typedef std::integral_constant<int, 2> c2;
+        issue(0);
+        if (mine > 1) {
+            issue(STAGE);
+            wait_vm_lgkm0<LPT>();
+        } else {
+            wait_vm_lgkm0<0>();
+        }
+        oa.read(0u, va);
+        ob.read(0u, vb);
+        wait_lgkm<0>();
+        __builtin_amdgcn_sched_barrier(0);
+        if (mine > 2) issue(0);
+        // the last step works from set 1, so the first one from set mine % 2
+        const bool odd = mine & 1;
+        if (odd) {
+            fa[1][0] = OA::template block<0>(va);
+            fa[1][1] = OA::template block<1>(va);
+            fb[1][0] = OB::template block<0>(vb);
+            fb[1][1] = OB::template block<1>(vb);
+        } else {
+            fa[0][0] = OA::template block<0>(va);
+            fa[0][1] = OA::template block<1>(va);
+            fb[0][0] = OB::template block<0>(vb);
+            fb[0][1] = OB::template block<1>(vb);
+        }
+        if (mine > 1) {
+            if (mine > 2) wait_vm_lgkm0<LPT>();
+            else wait_vm_lgkm0<0>();
+            oa.read(STAGE, va);
+            int t = 0;
+            if (odd) step(t++, c1{}, c2{});
+            for (; t + 2 < mine; t += 2) {
+                step(t, c0{}, c2{});
+                step(t + 1, c1{}, c2{});
+            }
+            step(t, c0{}, c1{});
+        }
+        step(mine - 1, c1{}, c0{});
+    }
+    __syncthreads();                     // the rings are done with
+
+    // The wavefronts' sums go through LDS: element e of a block is row (e / 4) * 8 + (lane / 32) * 4 + e % 4, column lane % 32.
+    constexpr int PITCH = kBlock + 4;                 // floats; rows stay 16-byte aligned
+    static_assert(KG * kBlock * PITCH * 4 <= 160 * 1024, "all partial tiles fit");
+    float* const part = reinterpret_cast<float*>(lds);
+    {
+        float* const own = part + wave * kBlock * PITCH;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int r = (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
+                float* const row = own + (AROWS ? 2 * r + i : 32 * i + r) * PITCH;
+                const float v0 = acc[i][0][e], v1 = acc[i][1][e];
+                if constexpr (BROWS) {
+                    *reinterpret_cast<floatx2*>(row + 2 * (lane & 31)) = floatx2{v0, v1};
+                } else {
+                    row[lane & 31] = v0;
+                    row[32 + (lane & 31)] = v1;
+                }
+            }
+    }
+    __syncthreads();
+    constexpr int CPR = kBlock / 4;                   // pieces of four columns per row
+    for (int i = threadIdx.x; i < kBlock * CPR; i += THREADS) {
+        const int r = i / CPR, c4 = (i % CPR) * 4;
+        const int m = m0 + r, n = n0 + c4;
+        if (m >= g.m || n >= g.n) continue;
+        floatx4 v = *reinterpret_cast<const floatx4*>(part + r * PITCH + c4);
+#pragma unroll
+        for (int s = 1; s < KG; ++s) v += *reinterpret_cast<const floatx4*>(part + (s * kBlock + r) * PITCH + c4);
+        const int cnt = min(4, g.n - n);
+        const float* ar = A + (int64_t)m * g.sam;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (e < cnt && !(fabsf(v[e]) <= FLT_MAX)) {
+                const float* bc = B + (int64_t)(n + e) * g.sbn;
+                float s = 0.f;
+                for (int k = 0; k < g.k; ++k) s = __builtin_fmaf(ar[k * g.sak], bc[k * g.sbk], s);
+                v[e] = s;
+            }
+        const int64_t off = coff + (int64_t)m * g.scm + n;
+        const float bm = g.bias && g.bias_m ? bias_at(g, m) : 0.f;
+        floatx4 out;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (e < cnt) out[e] = finish(g, v[e], g.bias && !g.bias_m ? bias_at(g, n + e) : bm, off + e);
+        if (g.c_vec && cnt == 4) {
+            *reinterpret_cast<floatx4*>(g.c + off) = out;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (e < cnt) g.c[off + e] = out[e];
+        }
+    }
+}
+
+template <int KG, int AROWS, int BROWS>
+int launch(SplitArgs& g, long long batch, hipStream_t st) {
+    constexpr int ring = KG * kStages * 2 * kBlock * BK * 4, sums = KG * kBlock * (kBlock + 4) * 4;
+    constexpr int lds = ring > sums ? ring : sums;
+    g.tiles_m = (g.m + kBlock - 1) / kBlock;
+    g.tiles_n = (g.n + kBlock - 1) / kBlock;
+    g.total_blocks = (long long)g.tiles_m * g.tiles_n * batch;
+    DML_REQUIRE(g.total_blocks <= 2147483647LL, DMLHIP_ERR_SHAPE, "gemm_f32: too many workgroups");
+    auto kern = gemm_f32_split_kernel<KG, AROWS, BROWS>;
+    const hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (e != hipSuccess) {
+        set_error("gemm_f32: cannot reserve %d bytes of LDS: %s", lds, hipGetErrorString(e));
+        return (int)e;
+    }
+    hipLaunchKernelGGL(kern, (unsigned)g.total_blocks, kWave * KG, lds, st, g);
+    return launch_status("gemm_f32");
+}
+
+template <int AROWS, int BROWS>
+int launch_form(SplitArgs& g, int form, long long batch, hipStream_t st) {
+    return form == 0 ? launch<8, AROWS, BROWS>(g, batch, st) : launch<4, AROWS, BROWS>(g, batch, st);
+}
+
+// ROWS of Operand, -1: 16 bytes at a time do not work. Offsets inside a tile and a step are 32 bits wide.
+int operand_rows(const void* p, int64_t rows, int64_t k, int64_t s_row, int64_t s_k, const int64_t* sb, const int64_t* batch) {
+    if (!aligned16(p) || 64.0 * s_row + 16.0 * s_k >= 1073741824.0) return -1;
+    for (int i = 0; i < 3; ++i)
+        if (batch[i] > 1 && sb[i] % 4 != 0) return -1;
+    if (s_k == 1 && s_row % 4 == 0 && k % 4 == 0) return 0;
+    return s_row == 1 && s_k % 4 == 0 && rows % 4 == 0 ? 1 : -1;
+}
+
+thread_local int g_force_tile = -1;   // diagnostic: 0 - 2 = the streamed kernel's tiles, 3 and 4 = the forms here
+
+// -1: the streamed kernel is the faster one. Measured: a step of eight wavefronts on a compute unit takes 1.14 us, whether
+// they share a tile or are two workgroups of four; first loads, the sum through LDS and stores 6.4 us per tile of eight, 7.1 us
+// per pair of tiles of four. So one tile per compute unit takes eight (1024 x 768 x 768: 14.3 us, four 15.1, streamed 20; 1024 x
+// 768 x 3072 34.8 / 36.0 / 51), more take four (1024 x 3072 x 768: 34.7, eight 39.8, streamed 48; 4096^3 761 / 768 / 1016). Few
+// tiles (512^3: 9.6, streamed 6.0) and short K (512 x 512 x 64, 24 times: 24, streamed 17) stay on the streamed kernel.
+int choose_form(const dmlhip_gemm_desc* d, long long batch) {
+    const double tiles = (double)ceil_div(d->m, kBlock) * ceil_div(d->n, kBlock) * batch, n = ceil(tiles / kCus);
+    const double eight = n * (6.4 + ceil_div(d->k, 8 * BK) * 1.14), four = ceil(n / 2) * 7.1 + 0.8 + n * ceil_div(d->k, 4 * BK) * 0.57;
+    if (gemm_f32_streamed_us(d, batch) <= fmin(eight, four)) return -1;
+    return eight <= four ? 0 : 1;
+}
+
+}  // namespace
+}  // namespace dml
+
+using namespace dml;
+extern "C" int dmlhip_gemm_f32(const dmlhip_gemm_desc* d, const void* a, const void* b, void* c, const void* bias,
+                               const void* residual, void* pre_out, void* stream) {
+    DML_REQUIRE(d, DMLHIP_ERR_NULL, "gemm_f32: NULL descriptor");
+    DML_REQUIRE(d->m >= 0 && d->n >= 0 && d->k >= 0, DMLHIP_ERR_SHAPE, "gemm_f32: negative extent");
+    DML_REQUIRE(d->m <= 2147483647 / 2 && d->n <= 2147483647 / 2 && d->k <= 2147483647 / 2, DMLHIP_ERR_SHAPE,
+                "gemm_f32: extent exceeds 2^30");
+    long long batch = 1;
+    for (int i = 0; i < 3; ++i) {
+        DML_REQUIRE(d->batch[i] >= 0 && d->batch[i] <= 2147483647, DMLHIP_ERR_SHAPE, "gemm_f32: bad batch extent");
+        batch *= d->batch[i];
+        DML_REQUIRE(batch <= 2147483647LL, DMLHIP_ERR_SHAPE, "gemm_f32: batch too large");
+    }
+    DML_REQUIRE(d->out_dtype == DMLHIP_F32, DMLHIP_ERR_ENUM, "gemm_f32: out_dtype must be DMLHIP_F32");
+    DML_REQUIRE(d->bias_dtype == DMLHIP_F16 || d->bias_dtype == DMLHIP_F32, DMLHIP_ERR_ENUM,
+                "gemm_f32: bad bias_dtype");
+    DML_REQUIRE(valid_act(d->act), DMLHIP_ERR_ENUM, "gemm_f32: bad act");
+    DML_REQUIRE(d->a_stride_m >= 0 && d->a_stride_k >= 0 && d->b_stride_k >= 0 && d->b_stride_n >= 0 &&
+                    d->c_stride_m >= 0,
+                DMLHIP_ERR_SHAPE, "gemm_f32: negative stride");
+    DML_REQUIRE(d->c_stride_m >= d->n || d->m <= 1, DMLHIP_ERR_SHAPE, "gemm_f32: rows of C overlap");
+    if (d->m == 0 || d->n == 0 || batch == 0) return 0;
+    DML_REQUIRE(c, DMLHIP_ERR_NULL, "gemm_f32: NULL output");
+    DML_REQUIRE(d->k == 0 || (a && b), DMLHIP_ERR_NULL, "gemm_f32: NULL operand");
+
+    if (g_force_tile >= 0 && g_force_tile < 3)
+        return gemm_f32_streamed(d, a, b, c, bias, residual, pre_out, g_force_tile, batch, (hipStream_t)stream);
+    SplitArgs g;
+    g.a = (const float*)a; g.b = (const float*)b; g.c = (float*)c;
+    g.bias = bias; g.residual = (const float*)residual; g.pre = (float*)pre_out;
+    g.m = (int)d->m; g.n = (int)d->n; g.k = (int)d->k;
+    g.sam = d->a_stride_m; g.sak = d->a_stride_k; g.sbn = d->b_stride_n; g.sbk = d->b_stride_k; g.scm = d->c_stride_m;
+    g.batch1 = (int)d->batch[1]; g.batch2 = (int)d->batch[2];
+    for (int i = 0; i < 3; ++i) {
+        g.sab[i] = d->a_stride_batch[i]; g.sbb[i] = d->b_stride_batch[i]; g.scb[i] = d->c_stride_batch[i];
+    }
+    g.alpha = d->alpha; g.beta = d->beta;
+    g.bias_f32 = d->bias_dtype == DMLHIP_F32; g.act = d->act;
+    g.bias_m = d->bias_along_m != 0;
+    g.c_vec = aligned16(c) && d->c_stride_m % 4 == 0;
+    for (int i = 0; i < 3; ++i)
+        if (d->batch[i] > 1 && d->c_stride_batch[i] % 4 != 0) g.c_vec = 0;
+    const int ar = operand_rows(a, d->m, d->k, d->a_stride_m, d->a_stride_k, d->a_stride_batch, d->batch);
+    const int br = operand_rows(b, d->n, d->k, d->b_stride_n, d->b_stride_k, d->b_stride_batch, d->batch);
+    const int form = ar < 0 || br < 0 ? -1 : g_force_tile >= 3 ? g_force_tile - 3 : choose_form(d, batch);
+    if (form < 0) return gemm_f32_streamed(d, a, b, c, bias, residual, pre_out, -1, batch, (hipStream_t)stream);
+    hipStream_t st = (hipStream_t)stream;
+    if (ar == 0) return br == 0 ? launch_form<0, 0>(g, form, batch, st) : launch_form<0, 1>(g, form, batch, st);
+    return br == 0 ? launch_form<1, 0>(g, form, batch, st) : launch_form<1, 1>(g, form, batch, st);
+}
+
+extern "C" void dmlhip_debug_force_gemm_f32_tile(int tile) { g_force_tile = tile; }

@@ -18,6 +18,7 @@
 namespace dml {
 
 typedef _Float16 half4v __attribute__((ext_vector_type(4)));
+typedef float float2v __attribute__((ext_vector_type(2)));
 
 // 16 bytes per lane, global -> LDS without staging registers. The LDS destination of lane l is
 // lds_dst + 16*l; lds_dst must be wavefront-uniform.
@@ -41,6 +42,13 @@ template <int OFFSET>
 [[nodiscard]] __device__ __forceinline__ float lds_read_b32(uint32_t addr) {
     float v;
     asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFFSET));
+    return v;
+}
+
+template <int OFFSET>
+[[nodiscard]] __device__ __forceinline__ float2v lds_read_b64(uint32_t addr) {
+    float2v v;
+    asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFFSET));
     return v;
 }
 

@@ -491,9 +491,10 @@ int dmlhip_debug_last_gemm_config(void);
 /* Diagnostic: into how many slices of K, summed by a second launch, dmlhip_gemm_f16_ws cuts a plain product of operands
  * aligned to 16 bytes. Launches nothing. */
 int dmlhip_debug_gemm_f16_slices(const dmlhip_gemm_desc* d);
-/* Pin the tile of the fp32 contraction kernel: 0 = 128x128, 1 = 64x64, 2 = 32x32 with K split over the wavefronts;
- * -1 = chosen per problem (default). Operands that cannot be read 16 bytes at a time have no 128x128 form and run on 64x64.
- * Per calling thread. */
+/* Pin the kernel and tile of fp32 contractions: fp32 matrix instructions, 0 = 128x128, 1 = 64x64, 2 = 32x32 with K split over the
+ * wavefronts; operands split into bf16 values, 64x64, 3 = K over eight wavefronts, 4 = over four; -1 = chosen per problem
+ * (default). Operands that cannot be read 16 bytes at a time have no 128x128 form and run on 64x64; 3 and 4 do not take them and
+ * choose among the first three. Per calling thread. */
 void dmlhip_debug_force_gemm_f32_tile(int tile);
 /* Diagnostic: pin the tile of the calling thread's dense 3 x 3 fp32 convolutions and data gradients (0 = 32 channels x 128
    pixels, 1 = 32 x 64, 2 = 32 x 32; -1 = the library chooses). */

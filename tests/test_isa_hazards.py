@@ -84,6 +84,7 @@ def test_dense_convolution_weight_gradient(tmp_path):
 
 @pytest.mark.parametrize("src,kernel,count", [
     ("daceml_amd/csrc/gemm_f32.hip", "gemm_f32_kernel", 36),              # 4 + 16 + 16: tiles x operand layouts
+    ("daceml_amd/csrc/gemm_f32_split.hip", "gemm_f32_split_kernel", 8),   # wavefronts x operand layouts
     ("daceml_amd/csrc/conv_dense3.hip", "conv_dense3_f32_kernel", 24),    # tiles x direction x transfers of W and X
     ("daceml_amd/csrc/gemm_f16_split.hip", "gemm_f16_split_kernel", 44),
     ("tests/isa/ragged_instances.hip", "gemm_f16_pipe_kernel", 6),        # the translation unit takes minutes to compile

@@ -1,0 +1,74 @@
+"""fp32 products on the bf16 matrix instructions, operands split into three bf16 values each: tiles, K steps and rings at their
+edges, K over four and eight wavefronts, both ways of reading an operand, batches, and values without such a split.
+
+Tolerance: the three values of an operand add up to it exactly, the products left out are below 3 * 2^-26 of |a| |b|, and a sum
+of k terms in any order is within k 2^-24 (sum of |a| |b|) of the exact one."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from tests.util import dev, host, rng
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [(4, 4, 4), (64, 64, 16), (68, 60, 64), (60, 132, 20), (128, 64, 128), (132, 68, 148), (64, 128, 260), (192, 64, 404)]
+
+
+def _product(lib, form, m, n, k, batch, a, b, strides_a, strides_b, c, bias=None, res=None, alpha=1.0):
+    from daceml_amd import _lib as L, kernels as K
+    d = L.GemmDesc()
+    d.m, d.n, d.k = m, n, k
+    (d.a_stride_m, d.a_stride_k), (d.b_stride_n, d.b_stride_k), d.c_stride_m = strides_a, strides_b, n
+    d.batch[0], d.batch[1], d.batch[2] = 1, 1, batch
+    d.a_stride_batch[2], d.b_stride_batch[2], d.c_stride_batch[2] = m * k, n * k, m * n
+    d.alpha, d.beta, d.out_dtype, d.bias_dtype, d.act = alpha, 0.0, L.F32, L.F32, L.ACT_NONE
+    p = lambda t: None if t is None else ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    lib.dmlhip_debug_force_gemm_f32_tile(form)
+    try:
+        L.check(lib.dmlhip_gemm_f32(ctypes.byref(d), p(a), p(b), p(c), p(bias), p(res), None, K._stream()))
+    finally:
+        lib.dmlhip_debug_force_gemm_f32_tile(-1)
+
+
+@pytest.mark.parametrize("form", [3, 4])
+@pytest.mark.parametrize("b_rows", ["k", "n"])
+@pytest.mark.parametrize("a_rows", ["k", "m"])
+def test_split_products(form, a_rows, b_rows, lib):
+    for m, n, k in SIZES:
+        r, batch = rng(m * 1000 + n * 10 + k), 1 if k % 16 else 3
+        a, b = r.standard_normal((batch, m, k)).astype(np.float32), r.standard_normal((batch, n, k)).astype(np.float32)
+        ta = dev(a if a_rows == "k" else np.ascontiguousarray(a.transpose(0, 2, 1)))
+        tb = dev(b if b_rows == "k" else np.ascontiguousarray(b.transpose(0, 2, 1)))
+        bias, res = r.standard_normal(n).astype(np.float32), r.standard_normal((batch, m, n)).astype(np.float32)
+        c = torch.full((batch, m, n), float("nan"), device="cuda")
+        _product(lib, form, m, n, k, batch, ta, tb, (k, 1) if a_rows == "k" else (1, m), (k, 1) if b_rows == "k" else (1, n), c,
+                 dev(bias), dev(res), 0.5)
+        exact = a.astype(np.float64) @ b.astype(np.float64).transpose(0, 2, 1)
+        terms = np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64).transpose(0, 2, 1)
+        bound = 0.5 * (k + 1) * 2.0 ** -24 * terms + 3 * 2.0 ** -24 * (np.abs(exact) + np.abs(bias) + np.abs(res))
+        err = np.abs(host(c).astype(np.float64) - (0.5 * exact + bias + res))
+        assert (err <= bound).all(), (form, a_rows, b_rows, m, n, k, float((err - bound).max()))
+
+
+@pytest.mark.parametrize("form", [3, 4])
+def test_values_without_a_split(form, lib):
+    """Infinities, NaN and finite values above the largest bf16: the results of an fp32 chain."""
+    r, (m, n, k) = rng(5), (72, 68, 100)
+    a, b = r.standard_normal((m, k)).astype(np.float32), r.standard_normal((n, k)).astype(np.float32)
+    a[3, 7], a[9, 0], a[9, 50], a[40, 99] = np.inf, np.inf, -np.inf, np.nan
+    b[5, 3], b[6, 7], b[66, 16] = -np.inf, 0.0, np.nan
+    a[20, :], b[20, :] = 0.0, 0.0
+    a[20, 30], b[20, 30], a[21, 4] = np.finfo(np.float32).max, 0.5, -np.finfo(np.float32).max
+    b[:, 4] = 0.25
+    c = torch.full((m, n), float("nan"), device="cuda")
+    _product(lib, form, m, n, k, 1, dev(a), dev(b), (k, 1), (k, 1), c)
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = (a.astype(np.float64) @ b.astype(np.float64).T).astype(np.float32)
+    got = host(c)
+    for same in (np.isnan, np.isposinf, np.isneginf):
+        np.testing.assert_array_equal(same(got), same(want))
+    finite = np.isfinite(want)
+    assert finite[20, 20] and finite[21, 0]
+    np.testing.assert_allclose(got[finite], want[finite], rtol=1e-5, atol=1e-4)
