@@ -547,7 +547,9 @@ direct:
     if constexpr (sizeof(T) == 4) {
         // dense convolutions with enough work per output: implicit GEMM on the fp32 matrix pipe
         bool done;
-        const int e = launch_conv_dense3_f32(g, (const float*)x, (const float*)w, (const float*)bias, (float*)y, st, &done);
+        int e = launch_conv_dense3_split_f32(g, (const float*)x, (const float*)w, (const float*)bias, (float*)y, st, &done);
+        if (done) return e;
+        e = launch_conv_dense3_f32(g, (const float*)x, (const float*)w, (const float*)bias, (float*)y, st, &done);
         if (done) return e;
         if (conv_implicit_applicable(g))
             return launch_conv_implicit_f32(g, (const float*)x, (const float*)w, (const float*)bias, (float*)y, st);
@@ -658,7 +660,9 @@ int dmlhip_conv2d_backward_data_f32(const dmlhip_conv2d_desc* d, const void* dy,
         return launch_depthwise_bwd_data((const float*)dy, (const float*)w, (float*)dx, g.n, g.c, g.h, g.w, g.oh, g.ow, g.kh,
                                          g.sh, st);
     bool done;
-    const int e = launch_conv_dense3_bwd_data_f32(g, (const float*)dy, (const float*)w, (float*)dx, st, &done);
+    int e = launch_conv_dense3_split_bwd_data_f32(g, (const float*)dy, (const float*)w, (float*)dx, st, &done);
+    if (done) return e;
+    e = launch_conv_dense3_bwd_data_f32(g, (const float*)dy, (const float*)w, (float*)dx, st, &done);
     if (done) return e;
     if (conv_implicit_bwd_data_applicable(g))
         return launch_conv_implicit_bwd_data_f32(g, (const float*)dy, (const float*)w, (float*)dx, st);

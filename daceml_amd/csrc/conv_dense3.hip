@@ -1,5 +1,6 @@
 // Dense (group 1) 3 x 3 convolution, fp32, as an implicit GEMM on v_mfma_f32_32x32x2_f32 that streams its operands
-// straight into LDS; the forward pass and, with the weights read transposed and reversed, the data gradient.
+// straight into LDS; the forward pass and, with the weights read transposed and reversed, the data gradient. For problems of fewer
+// tiles or channels than conv_dense3_split.hip takes, which is asked first.
 //   Y[n, m, p] = act(b[m] + sum_{c, hy, hx} W[m, c, hy, hx] * X[n, c, oy(p) s - pad + hy d, ox(p) s - pad + hx d])
 //
 // What bounds it: the fp32 matrix rate (256 operations per clock and compute unit), if the matrix pipes neither wait for
@@ -327,6 +328,7 @@ constexpr double kNarrowTransfer[kTiles] = {0.004, 0.004, 0.008};
 
 struct Dense3Plan {
     Dense3Args a;
+    double us;               // estimated
     int tile, vec, xvec;
     size_t lds;
     unsigned blocks;
@@ -418,6 +420,7 @@ static bool plan_conv_dense3(const ConvGeom& g, int ids_h, int ids_w, bool flip,
         if (pl->tile >= 0 && us >= best) continue;
         best = us;
         best_per_cu = per_cu;
+        pl->us = us;
         pl->tile = t;
         pl->lds = lds;
         pl->blocks = (unsigned)blocks;
@@ -451,6 +454,11 @@ static int launch_planned(const ConvGeom& g, int ids_h, int ids_w, bool flip, bo
     return DMLHIP_ERR_UNSUPPORTED;
 }
 
+double conv_dense3_us(const ConvGeom& g, int ids_h, int ids_w, bool flip, const void* x, const void* w) {
+    Dense3Plan pl;
+    return plan_conv_dense3(g, ids_h, ids_w, flip, false, x, w, &pl) ? pl.us : -1.0;
+}
+
 int launch_conv_dense3_f32(const ConvGeom& g, const float* x, const float* w, const float* bias, float* y, hipStream_t st,
                            bool* applies) {
     return launch_planned(g, 1, 1, false, conv_implicit_applicable(g), x, w, bias, y, st, "conv2d(dense 3x3)", applies);
@@ -463,6 +471,6 @@ int launch_conv_dense3_bwd_data_f32(const ConvGeom& g, const float* dy, const fl
     return launch_planned(b, g.sh, g.sw, true, conv_implicit_bwd_data_applicable(g), dy, w, nullptr, dx, st, "conv2d_backward_data(dense 3x3)", applies);
 }
 
-}  // namespace dml
+void conv_dense3_force_tile(int tile) { g_force_tile = tile; }
 
-extern "C" void dmlhip_debug_force_conv_dense3_tile(int tile) { dml::g_force_tile = tile; }
+}  // namespace dml

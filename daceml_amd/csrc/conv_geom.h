@@ -18,6 +18,12 @@ bool conv_implicit_bwd_data_applicable(const ConvGeom& g);
 int launch_conv_dense3_f32(const ConvGeom& g, const float* x, const float* w, const float* bias, float* y, hipStream_t st,
                            bool* applies);
 int launch_conv_dense3_bwd_data_f32(const ConvGeom& g, const float* dy, const float* w, float* dx, hipStream_t st, bool* applies);
+double conv_dense3_us(const ConvGeom& g, int ids_h, int ids_w, bool flip, const void* x, const void* w);   // its estimate; < 0: does not apply
+void conv_dense3_force_tile(int tile);     // diagnostic, this thread: -1 = chosen per problem
+// conv_dense3_split.hip: the same problems on the bf16 matrix instructions, where that is faster
+int launch_conv_dense3_split_f32(const ConvGeom& g, const float* x, const float* w, const float* bias, float* y, hipStream_t st,
+                                 bool* applies);
+int launch_conv_dense3_split_bwd_data_f32(const ConvGeom& g, const float* dy, const float* w, float* dx, hipStream_t st, bool* applies);
 // conv_dense3_weight.hip: per-range results (m * c * 9 floats each) its weight gradient writes; 0 = does not apply, or the
 // general kernel, where that applies (`general`), is the faster one
 int64_t conv_dense3_bwd_weight_partials(const ConvGeom& g, bool general);

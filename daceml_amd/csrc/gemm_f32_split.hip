@@ -1,14 +1,8 @@
 // fp32 strided batched GEMM on the bf16 matrix cores: the entry point of the fp32 products and the kernel behind most of them.
 //
-// An fp32 value is the sum of three bf16 values, exactly: x = h + m + l, each the rounding of what the ones before leave
-// (24 bits are 8 + 8 + 8; below 2^-110 the last ones fall under the smallest bf16). Of the nine products of two such sums six
-// matter: h h, h m, m h, m m, h l, l h (the others are below 2^-26 of the product, under the rounding of the sum). The bf16
-// matrix rate is 16 times the fp32 one, so six products take 0.375 of the time of the fp32 instruction.
-// Precision: 16 products per rounding of the fp32 accumulator, the small ones of a step first. Error against the fp64 product,
-// 2-norm over 2-norm, in one chain of K here / on v_mfma_f32_32x32x2_f32 (one product per rounding): N(0, 1) K = 64 1.1e-7 /
-// 1.4e-7, 768 4.2e-7 / 5.0e-7, 3072 8.5e-7 / 9.7e-7; uniform on [0, 1) 768 2.9e-7 / 4.2e-7; log-normal over twelve decades 768
-// 1.7e-7 / 2.4e-7; and K is cut into four or eight chains: 1024 x 768 x 768 1.5e-7 where the streamed tiles have 2.5e-7 - 5.0e-7.
-// Infinities and NaN have no such sum: an element that comes out not finite is computed again, as a chain of fp32 multiply-adds.
+// Operands are split into three bf16 values each (bf16_split.h has what that costs and keeps); K is cut into four or eight chains
+// on top: 1024 x 768 x 768 is 1.5e-7 from the fp64 product where the streamed tiles are 2.5e-7 - 5.0e-7. An element that comes
+// out not finite is computed again, as a chain of fp32 multiply-adds.
 //
 // What bounds it: vector issue beside the matrix pipe. A wavefront's 64 x 64 tile is 24 MFMAs per 16 k (0.36 us) and 176
 // instructions that split the operands; on a compute unit with eight wavefronts a step takes 0.57 us per wavefront and SIMD. So the
@@ -16,7 +10,7 @@
 // one accumulator per block, not a second one for the small products (registers: 0.8 us again). Measured, us, the kernel of
 // gemm_f32.hip / here: 1024 x 768 x 768 20 / 14, 1024 x 3072 x 768 48 / 35, 3072 x 768 x 1024 (both operands row-contiguous) 59 / 39,
 // 4096^3 1016 / 715 - 760 = 181 - 192 TFLOP/s, where the fp32 instruction's own limit is 157.
-#include "common.h"
+#include "bf16_split.h"
 #include "lds_ops.h"
 
 #include <float.h>
@@ -30,10 +24,6 @@ int gemm_f32_streamed(const dmlhip_gemm_desc* d, const void* a, const void* b, v
 double gemm_f32_streamed_us(const dmlhip_gemm_desc* d, long long batch);
 
 namespace {
-
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float floatx2 __attribute__((ext_vector_type(2)));
 
 constexpr int BK = 16;           // K per step of a wavefront
 constexpr int kXcds = 8;
@@ -57,40 +47,6 @@ struct SplitArgs {
     int tiles_m, tiles_n;
     int c_vec;                   // C (and residual, pre) can be accessed four columns at a time
     long long total_blocks;
-};
-
-struct Pieces {
-    bf16x8 h, m, l;
-};
-
-// Eleven vector instructions for two values. (What a rounding leaves is also a dot product of a packed pair with (-1, 0) or
-// (0, -1), seven instructions in all, but v_dot2c_f32_bf16 does not issue beside the matrix pipe: 16 MFMAs with 64 of them took
-// 6.0 us where with 64 subtractions they took 3.8.)
-struct Splitter {
-    static __device__ __forceinline__ floatx2 unpack(uint32_t v) {
-        return {__builtin_bit_cast(float, v << 16), __builtin_bit_cast(float, v & 0xffff0000u)};
-    }
-    static __device__ __forceinline__ void pair(floatx2 v, uint32_t& h, uint32_t& m, uint32_t& l) {
-        h = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
-        const floatx2 uh = unpack(h);
-        floatx2 r = {v[0] - uh[0], v[1] - uh[1]};
-        m = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, bf16x2));
-        const floatx2 um = unpack(m);
-        r = floatx2{r[0] - um[0], r[1] - um[1]};
-        l = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, bf16x2));
-    }
-    static __device__ __forceinline__ Pieces eight(const float (&v)[8]) {
-        u32x4 h, m, l;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            uint32_t ph, pm, pl;
-            pair(floatx2{v[2 * i], v[2 * i + 1]}, ph, pm, pl);
-            h[i] = ph;
-            m[i] = pm;
-            l[i] = pl;
-        }
-        return {__builtin_bit_cast(bf16x8, h), __builtin_bit_cast(bf16x8, m), __builtin_bit_cast(bf16x8, l)};
-    }
 };
 
 template <int I, int N, typename F>
@@ -171,7 +127,7 @@ struct Operand {
         float w[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) w[e] = ROWS == 0 ? v.q[2 * B + e / 4][e % 4] : v.p[e][B];
-        return Splitter::eight(w);
+        return split_eight(w);
     }
 };
 

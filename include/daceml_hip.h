@@ -496,8 +496,9 @@ int dmlhip_debug_gemm_f16_slices(const dmlhip_gemm_desc* d);
  * (default). Operands that cannot be read 16 bytes at a time have no 128x128 form and run on 64x64; 3 and 4 do not take them and
  * choose among the first three. Per calling thread. */
 void dmlhip_debug_force_gemm_f32_tile(int tile);
-/* Diagnostic: pin the tile of the calling thread's dense 3 x 3 fp32 convolutions and data gradients (0 = 32 channels x 128
-   pixels, 1 = 32 x 64, 2 = 32 x 32; -1 = the library chooses). */
+/* Diagnostic: pin the kernel and tile of the calling thread's dense 3 x 3 fp32 convolutions and data gradients (fp32 matrix
+   instructions, 0 = 32 channels x 128 pixels, 1 = 32 x 64, 2 = 32 x 32; operands split into bf16 values, 3 = 64 x 128, 4 = 64 x 256,
+   5 = 64 x 512; -1 = the library chooses). A problem that a kernel does not take runs on the next one. */
 void dmlhip_debug_force_conv_dense3_tile(int tile);
 /* Diagnostic: the calling thread's depthwise stride-1 fp32 convolutions and gradients whose output is as large as the input
  * run on the strip kernels (1), on the general depthwise kernels (0), or on the faster of the two (-1, default). */

@@ -1,0 +1,71 @@
+"""The dense 3 x 3 convolution and its data gradient on the bf16 matrix instructions (operands as three bf16 values each): tiles
+of 128, 256 and 512 pixels across rows and images, output channels that end inside a tile, a last step of eight channels, strides,
+dilation, wide padding, activations, values without a split.
+
+Tolerance: that of the fp32 kernels' test; the products left out are below 3 * 2^-26 of |a| |b|, one of its two spare terms."""
+import numpy as np
+import pytest
+import torch
+import torch.nn.functional as F
+
+from tests.test_zx_conv_dense3 import _check, _problem
+from tests.util import dev, host, rng
+
+pytestmark = pytest.mark.gpu
+
+# n, c, h, w, m, stride, pad, dilation
+SHAPES = [(3, 64, 56, 56, 64, 1, 1, 1), (5, 16, 31, 33, 72, 1, 1, 1), (9, 24, 14, 14, 136, 1, 1, 1), (4, 40, 27, 29, 64, 2, 1, 1),
+          (2, 16, 30, 64, 96, 1, 2, 2), (3, 24, 33, 20, 32, 1, 0, 1), (20, 64, 14, 14, 64, 2, 1, 1), (1, 32, 112, 112, 32, 1, 1, 1),
+          (6, 256, 7, 7, 64, 1, 1, 1), (50, 16, 3, 5, 16, 1, 1, 1)]
+
+
+def _forced(lib, tile, run):
+    lib.dmlhip_debug_force_conv_dense3_tile(tile)
+    try:
+        return run()
+    finally:
+        lib.dmlhip_debug_force_conv_dense3_tile(-1)
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_conv_dense3_split(shape, lib):
+    from daceml_amd import kernels as K
+    n, c, h, w, m, s, p, d = shape
+    x, wt, b, dy, exact, terms = _problem(shape)
+    for tile in (3, 4, 5):
+        y = _forced(lib, tile, lambda: K.conv2d(dev(x), dev(wt), dev(b), (s, s), (p, p), (d, d)))
+        dx, _ = _forced(lib, tile, lambda: K.conv2d_backward(dev(x), dev(wt), dev(dy), (s, s), (p, p), (d, d), need_dw=False))
+        _check((tile, "y"), y, exact[0], terms[0], 9 * c)
+        _check((tile, "dx"), dx, exact[1], terms[1], 9 * m)
+
+
+@pytest.mark.parametrize("act", ["RELU", "SWISH", "SIGMOID", "GELU"])
+def test_activations(act, lib):
+    from daceml_amd import _lib as L, kernels as K
+    r = rng(6)
+    x, wt, b = r.standard_normal((2, 16, 24, 24)).astype(np.float32), 0.1 * r.standard_normal((70, 16, 3, 3)).astype(np.float32), \
+        r.standard_normal(70).astype(np.float32)
+    y = _forced(lib, 4, lambda: K.conv2d(dev(x), dev(wt), dev(b), pads=(1, 1), act=getattr(L, "ACT_" + act)))
+    v = F.conv2d(*(torch.from_numpy(t).double() for t in (x, wt, b)), 1, 1)
+    want = {"RELU": torch.relu, "SWISH": F.silu, "SIGMOID": torch.sigmoid, "GELU": F.gelu}[act](v)
+    np.testing.assert_allclose(host(y), want.numpy(), rtol=2e-5, atol=2e-5)
+
+
+@pytest.mark.parametrize("tile", [3, 4, 5])
+def test_values_without_a_split(tile, lib):
+    """Infinities and NaN reach the pixels under them and no others; a finite value above the largest bf16 stays finite."""
+    from daceml_amd import kernels as K
+    r = rng(7)
+    x, wt = r.standard_normal((2, 16, 20, 22)).astype(np.float32), r.standard_normal((40, 16, 3, 3)).astype(np.float32)
+    x[0, 3, 5, 5], x[0, 4, 12, 0], x[1, 7, 19, 21] = np.inf, np.nan, -np.inf
+    x[1, :, 6:9, 6:9] = 0.0
+    x[1, 2, 7, 7] = np.finfo(np.float32).max
+    wt[:, 2, 1, 1] = 0.5
+    y = host(_forced(lib, tile, lambda: K.conv2d(dev(x), dev(wt), pads=(1, 1))))
+    with np.errstate(over="ignore"):
+        want = F.conv2d(torch.from_numpy(x).double(), torch.from_numpy(wt).double(), None, 1, 1).numpy().astype(np.float32)
+    for same in (np.isnan, np.isposinf, np.isneginf):
+        np.testing.assert_array_equal(same(y), same(want))
+    finite = np.isfinite(want)
+    assert finite[1, :, 7, 7].all()
+    np.testing.assert_allclose(y[finite], want[finite], rtol=1e-5, atol=1e-4)
