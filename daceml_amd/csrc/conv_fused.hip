@@ -11,6 +11,7 @@
 // zero rows outside the image — the depthwise convolution's padding. Phase 2 is the stencil: one wavefront per
 // (channel, output row), lanes along the output columns.
 #include "common.h"
+#include "conv_geom.h"
 
 namespace dml {
 namespace {
@@ -507,32 +508,15 @@ size_t dmlhip_conv2d_expand_depthwise_lds_bytes(int64_t w, int64_t cin, int64_t 
     return need <= 156 * 1024 ? need : 0;
 }
 
-int dmlhip_conv2d_expand_depthwise_f32(const dmlhip_conv2d_desc* pw, const dmlhip_conv2d_desc* dw, const void* x,
-                                       const void* w_pw, const void* b_pw, const void* w_dw, const void* b_dw, void* y,
-                                       void* stream) {
-    DML_REQUIRE(pw && dw, DMLHIP_ERR_NULL, "conv2d_expand_depthwise: NULL descriptor");
-    DML_REQUIRE(pw->n >= 0 && pw->c > 0 && pw->h > 0 && pw->w > 0 && pw->m > 0, DMLHIP_ERR_SHAPE,
-                "conv2d_expand_depthwise: extents must be positive");
-    DML_REQUIRE(valid_act(pw->act) && valid_act(dw->act) && pw->act != DMLHIP_ACT_GELU && dw->act != DMLHIP_ACT_GELU,
-                DMLHIP_ERR_ENUM, "conv2d_expand_depthwise: unsupported activation");
-    const bool pointwise = pw->kh == 1 && pw->kw == 1 && pw->stride_h == 1 && pw->stride_w == 1 && pw->pad_h == 0 &&
-                           pw->pad_w == 0 && pw->group == 1;
-    const bool depthwise = dw->kh == 3 && dw->kw == 3 && dw->pad_h == 1 && dw->pad_w == 1 && dw->dil_h == 1 &&
-                           dw->dil_w == 1 && dw->stride_h == dw->stride_w && (dw->stride_h == 1 || dw->stride_h == 2) &&
-                           dw->group == dw->c && dw->m == dw->c;
-    DML_REQUIRE(pointwise && depthwise, DMLHIP_ERR_UNSUPPORTED,
-                "conv2d_expand_depthwise: needs a 1x1 / stride 1 / unpadded convolution followed by a 3x3 depthwise "
-                "convolution with padding 1 and stride 1 or 2");
-    DML_REQUIRE(dw->n == pw->n && dw->c == pw->m && dw->h == pw->h && dw->w == pw->w, DMLHIP_ERR_SHAPE,
-                "conv2d_expand_depthwise: the depthwise input must be the pointwise output");
-    DML_REQUIRE(pw->c % 16 == 0 && pw->m % kCB == 0, DMLHIP_ERR_UNSUPPORTED,
-                "conv2d_expand_depthwise: needs input channels %% 16 == 0 and expanded channels %% 32 == 0");
-    DML_REQUIRE(pw->h * pw->w < (1LL << 30) && pw->w <= 4096 && pw->c * pw->h * pw->w < (1LL << 31), DMLHIP_ERR_UNSUPPORTED,
-                "conv2d_expand_depthwise: image too large");
-    if (pw->n == 0) return 0;
-    DML_REQUIRE(x && w_pw && w_dw && y, DMLHIP_ERR_NULL, "conv2d_expand_depthwise: NULL tensor pointer");
+}  // extern "C"
+
+namespace dml {
+
+bool expand_depthwise_pinned() { return g_rolling_rows != 0 || g_fused_toh > 0; }
+
+int launch_expand_depthwise_lds(const dmlhip_conv2d_desc* pw, const dmlhip_conv2d_desc* dw, const void* x, const void* w_pw,
+                                const void* b_pw, const void* w_dw, const void* b_dw, void* y, hipStream_t st) {
     const int stride = (int)dw->stride_h;
-    hipStream_t st = (hipStream_t)stream;
     RollArgs ra;
     // a pinned strip height asks for the strip kernel
     if (g_rolling_rows != -2 && g_fused_toh <= 0 && fill_rolling((int)pw->n, (int)pw->c, (int)pw->m, (int)pw->h, (int)pw->w, stride,
@@ -598,4 +582,4 @@ int dmlhip_conv2d_expand_depthwise_f32(const dmlhip_conv2d_desc* pw, const dmlhi
     return DMLHIP_ERR_UNSUPPORTED;
 }
 
-}  // extern "C"
+}  // namespace dml

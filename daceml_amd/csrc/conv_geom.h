@@ -43,6 +43,12 @@ bool pointwise_few_applicable(int64_t n, int64_t cin, int64_t cout, int64_t hw);
 int launch_pointwise_few(const float* x, const float* w, const float* bias, float* y, int n, int cin, int cout, int64_t hw,
                          int act, bool w_transposed, hipStream_t st);
 
+// conv_fused.hip: 1 x 1 expansion + 3 x 3 depthwise with the expanded rows in LDS (validated descriptors); is one of its
+// geometries asked for by this thread's diagnostic switches
+int launch_expand_depthwise_lds(const dmlhip_conv2d_desc* pw, const dmlhip_conv2d_desc* dw, const void* x, const void* w_pw,
+                                const void* b_pw, const void* w_dw, const void* b_dw, void* y, hipStream_t st);
+bool expand_depthwise_pinned();
+
 // The data gradient of a dense convolution as a convolution: dX = conv(dY with s - 1 zeros between its elements,
 // W with input / output channels exchanged and the taps reversed, stride 1, padding (k - 1) d - p).
 inline bool data_gradient_problem(const ConvGeom& f, ConvGeom* b) {

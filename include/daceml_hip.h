@@ -521,7 +521,8 @@ long long dmlhip_debug_grouped_single_launches(void);
 void dmlhip_debug_force_fused_strip(int toh);
 /* dmlhip_conv2d_expand_depthwise_f32 with a rolling window instead of strips: a workgroup walks down a segment of output
  * rows with the expanded rows in a ring in LDS, half of its wavefronts expanding the next rows while the other half runs
- * the stencil. This is what the library runs; the switch pins its geometry. rows: 0 = the library's choice (default: the
+ * the stencil. The switch pins its geometry. rows: 0 = the library's choice (default: wide images of few channels on the
+ * kernel that keeps expanded rows in registers, else the rolling window with the
  * most output rows per batch whose ring lets two workgroups share a compute unit's LDS, else the most that fit), -1 = as
  * many output rows per batch as fit LDS, > 0 = at most that many, -2 = the strip kernel; waves: 8 or 16 wavefronts per
  * workgroup. Shapes of which not one row fits LDS run on the strips. Per calling thread. */
