@@ -32,6 +32,7 @@ SOURCES = [
     "conv.hip",
     "conv_fused.hip", "conv_fused_columns.hip", "conv_backward.hip", "conv_implicit.hip", "conv_dense3.hip", "conv_dense3_split.hip", "conv_dense3_weight.hip", "conv_depthwise.hip",
     "conv_pointwise_few.hip",
+    "conv_pointwise_project.hip",
     "attention.hip",
     "batchnorm.hip",
 ]

@@ -489,8 +489,13 @@ int conv_forward(const dmlhip_conv2d_desc* d, const void* x, const void* w, cons
     if (g.kh == 1 && g.kw == 1 && g.sh == 1 && g.sw == 1 && g.ph == 0 && g.pw == 0 && g.group == 1 && g.c > 0) {
         const int64_t hw = (int64_t)g.h * g.w;
         if constexpr (sizeof(T) == 4) {
+            const bool streams = g.c % 32 == 0 && hw % 4 == 0 && hw >= 128 && g.n <= 65535 && aligned16(x) && aligned16(w) &&
+                                 !pointwise_splits_channels(g.n, g.c, g.m, hw);
+            if (pointwise_project_applicable(g.n, g.c, g.m, hw, false, streams))
+                return launch_pointwise_project((const float*)x, (const float*)w, (const float*)bias, nullptr, (float*)y, g.n, g.c,
+                                                g.m, hw, g.act, false, st);
             // many pixels, few channels: the streaming kernel (reads X once, writes Y in full rows)
-            if (g.c % 32 == 0 && hw % 4 == 0 && hw >= 128 && g.n <= 65535 && aligned16(x) && aligned16(w))
+            if (streams)
                 return launch_pointwise_f32((const float*)x, (const float*)w, (const float*)bias, nullptr, (float*)y, g.n,
                                             g.c, g.m, hw, g.act, st);
             // (behind it: 32 -> 192 channels of 56 x 56 take 32 us there and 38 here)
@@ -605,6 +610,9 @@ int dmlhip_conv2d_gated_f32(const dmlhip_conv2d_desc* d, const void* x, const vo
     if ((int64_t)g.n * g.m == 0) return 0;
     DML_REQUIRE(x && gate && w && y, DMLHIP_ERR_NULL, "conv2d_gated: NULL tensor pointer");
     DML_REQUIRE(aligned16(x) && aligned16(w), DMLHIP_ERR_ALIGN, "conv2d_gated: x and w must be 16-byte aligned");
+    if (pointwise_project_applicable(g.n, g.c, g.m, hw, false, true))
+        return launch_pointwise_project((const float*)x, (const float*)w, (const float*)bias, (const float*)gate, (float*)y, g.n,
+                                        g.c, g.m, hw, g.act, false, (hipStream_t)stream);
     return launch_pointwise_f32((const float*)x, (const float*)w, (const float*)bias, (const float*)gate, (float*)y, g.n, g.c,
                                 g.m, hw, g.act, (hipStream_t)stream);
 }
@@ -641,8 +649,13 @@ int dmlhip_conv2d_backward_data_f32(const dmlhip_conv2d_desc* d, const void* dy,
         if (pointwise_few_applicable(g.n, g.m, g.c, hw))
             return launch_pointwise_few((const float*)dy, (const float*)w, nullptr, (float*)dx, g.n, g.m, g.c, hw,
                                         DMLHIP_ACT_NONE, true, st);
+        const bool streams = hw % 4 == 0 && hw >= 128 && g.n <= 65535 && aligned16(dy) && aligned16(dx) &&
+                             !pointwise_splits_channels(g.n, g.m, g.c, hw);
+        if (pointwise_project_applicable(g.n, g.m, g.c, hw, true, streams))
+            return launch_pointwise_project((const float*)dy, (const float*)w, nullptr, nullptr, (float*)dx, g.n, g.m, g.c, hw,
+                                            DMLHIP_ACT_NONE, true, st);
         // many pixels: the streaming pointwise kernel with dY as its input and W read as [cin = M][cout = C]
-        if (hw % 4 == 0 && hw >= 128 && g.n <= 65535 && aligned16(dy) && aligned16(dx))
+        if (streams)
             return launch_pointwise_f32((const float*)dy, (const float*)w, nullptr, nullptr, (float*)dx, g.n, g.m, g.c, hw,
                                         DMLHIP_ACT_NONE, st, true);
         dmlhip_gemm_desc gd = {};

@@ -49,6 +49,12 @@ int launch_expand_depthwise_lds(const dmlhip_conv2d_desc* pw, const dmlhip_conv2
                                 const void* b_pw, const void* w_dw, const void* b_dw, void* y, hipStream_t st);
 bool expand_depthwise_pinned();
 
+// conv_pointwise_project.hip: 1 x 1, many input channels, few output channels; gate (optional): a factor per image and input channel
+bool pointwise_project_applicable(int64_t n, int64_t cin, int64_t cout, int64_t hw, bool w_transposed, bool streams);
+bool pointwise_splits_channels(int64_t n, int64_t cin, int64_t cout, int64_t hw);   // few pixels: the tiled GEMM is faster, without a gate
+int launch_pointwise_project(const float* x, const float* w, const float* bias, const float* gate, float* y, int n, int cin,
+                             int cout, int64_t hw, int act, bool w_transposed, hipStream_t st);
+
 // The data gradient of a dense convolution as a convolution: dX = conv(dY with s - 1 zeros between its elements,
 // W with input / output channels exchanged and the taps reversed, stride 1, padding (k - 1) d - p).
 inline bool data_gradient_problem(const ConvGeom& f, ConvGeom* b) {
