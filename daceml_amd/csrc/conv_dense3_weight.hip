@@ -1,19 +1,22 @@
-// Weight gradient of a dense (group 1) 3 x 3 convolution, fp32, on v_mfma_f32_32x32x2_f32:
+// Weight gradient of a dense (group 1) 3 x 3 convolution, fp32, on the bf16 matrix instructions with operands split into three
+// bf16 values each (stride and dilation 1; bf16_split.h), else on v_mfma_f32_32x32x2_f32:
 //   dW[m, c, hy, hx] = sum_{n, p} dY[n, m, p] * X[n, c, oy(p) s - pad + hy d, ox(p) s - pad + hx d]
 //
-// What bounds it: the fp32 matrix rate, once the nine taps share what is read. A wavefront keeps the nine 32 x 32 blocks
-// (channels of dY x channels of X, one per tap) in registers; a pair of pixels is one dY fragment and nine shifted reads of
-// the same rectangle of X for nine MFMAs. (The general kernel gathers X once per tap and 32 columns: 144 us for
-// 32 x 64 x 56 x 56 in 64 channels, reduction included; this one takes 95. At the matrix rate of a large product it would be
-// 48; addresses of transfers take 9 us, the ranges' sums and their results 7, the reduction 6, and the loop's own reads and
-// barriers most of the rest.) One workgroup of eight wavefronts per compute unit: 64 (32) channels of dY
-// x 32 channels of X over a range of output rows, the wavefronts of the same channels taking every fourth (eighth) pair of
+// What bounds it: the matrix rate, once the nine taps share what is read. A wavefront keeps the nine 32 x 32 blocks
+// (channels of dY x channels of X, one per tap) in registers; sixteen pixels (fp32: a pair) are one dY fragment and the shifted
+// reads of the same rectangle of X for 54 (nine) MFMAs. One workgroup of eight wavefronts per compute unit: 64 (32) channels of dY
+// x 32 channels of X over a range of output rows, the wavefronts of the same channels taking every fourth (eighth) set of
 // pixels. Rows of dY and the rows of X under them go global -> LDS without staging registers, a chunk of output rows of one
 // image at a time, one chunk ahead, issued between the MFMAs of the chunk before. The wavefronts' sums are added through LDS
 // and the ranges' results by the reduction kernel, all in a fixed order.
-// All sums are fp32. A wavefront adds 70 - 200 pixels in one chain where the general kernel's chains are shorter: 6.7e-8 - 1.3e-7 of the
-// gradient from the fp64 one (2-norm), 5.6e-8 - 7.0e-8 there; a second set of accumulators does not fit the registers.
-#include "common.h"
+// Measured, us with the reduction, fp32 instruction and split: 32x64x56x56 -> 64 92 and 67, -> 128 165 and 112, 32x128x28x28 -> 128 91
+// and 67, 32x96x40x40 -> 96 129 and 84, 32x256x14x14 -> 256 108 and 94 (rows of 14 are read as 16), 32x64x55x55 -> 64 115 and 93
+// (transfers of four bytes). Of the 67 the products are 20, and the split's 70 vector instructions for 18 MFMAs as much beside them; addresses
+// of transfers take 9, the ranges' sums and their results 7, the reduction 6.
+// All sums are fp32, errors against fp64, 2-norm, fp32 instruction and split: 32x64x56x56 -> 64 2.7e-7 and 2.4e-7, 32x32x112x112 -> 32 2.7e-7 and
+// 2.6e-7, 32x256x14x14 -> 256 2.5e-7 and 2.3e-7. The bf16 instruction loses the low bits of what it adds in one direction, which
+// 2048 partial sums add up to 6.2e-7 in the second of these: every other wavefront adds -dY X instead.
+#include "bf16_split.h"
 #include "conv_geom.h"
 #include "lds_ops.h"
 
@@ -49,13 +52,22 @@ __device__ __forceinline__ void lds_dma(const float* gptr, char* lds_dst) {
     else __builtin_amdgcn_global_load_lds(g, l, 4, 0, 0);
 }
 
+template <int I, int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        static_for<I + 1, N>(f);
+    }
+}
+
 struct Chunk {
     int img, oy, px;         // image, first output row, pixels
 };
 
-// WM: blocks of 32 channels of dY (1 or 2). AVEC, XVEC: floats per lane and transfer of dY and of X.
-template <int WM, int AVEC, int XVEC>
-__global__ __launch_bounds__(kThreads) void conv_dense3_weight_kernel(const WeightArgs g) {
+// WM: blocks of 32 channels of dY (1 or 2). AVEC, XVEC: floats per lane and transfer of dY and of X. SPLIT: stride and dilation
+// 1, on the bf16 matrix instructions.
+template <int WM, int AVEC, int XVEC, bool SPLIT>
+__device__ __forceinline__ void weight_gradient(const WeightArgs& g) {
     constexpr int MB = 32 * WM, KG = kWaves / WM;
     extern __shared__ __attribute__((aligned(16))) char lds[];
     char* const stages = lds + kMaxPixels * 4;        // behind the pixels' offsets
@@ -69,7 +81,7 @@ __global__ __launch_bounds__(kThreads) void conv_dense3_weight_kernel(const Weig
     const int m0 = tile % g.tiles_m * MB, c0 = tile / g.tiles_m * kCTile;
     const int total_rows = g.n * g.oh;
     int row = (int)((int64_t)total_rows * range / g.ranges);
-    const int row_end = (int)((int64_t)total_rows * (range + 1) / g.ranges);
+    const int first_row = row, row_end = (int)((int64_t)total_rows * (range + 1) / g.ranges);
     const int ohw = g.oh * g.ow, in_plane = g.h * g.w;
     const float inv_pitch = 1.0f / (float)g.pitch, inv_plane = 1.0f / (float)g.plane, inv_pwid = 1.0f / (float)g.pwid;
     const uint32_t lds0 = lds_addr(lds), stages0 = lds_addr(stages);
@@ -118,6 +130,9 @@ __global__ __launch_bounds__(kThreads) void conv_dense3_weight_kernel(const Weig
 #pragma unroll
     for (int t = 0; t < kTaps; ++t) toff[t] = (uint32_t)((t / 3 * g.dh * g.pwid + t % 3 * g.dw) * 4);
 
+    // see above: what the instruction loses in one direction cancels
+    const float sign = SPLIT && (kg & 1) ? -1.f : 1.f;
+
     Chunk cur = chunk_at(row);
     if (row < row_end)
         for (int i = 0; i < mine; ++i) issue(i, cur, stages);
@@ -133,62 +148,145 @@ __global__ __launch_bounds__(kThreads) void conv_dense3_weight_kernel(const Weig
         const uint32_t so = stages0 + (uint32_t)(stage * stage_bytes);
         const uint32_t a_row = so + (uint32_t)((wm * 32 + l32) * g.pitch * 4);
         const uint32_t x_row = so + (uint32_t)(g.a_bytes + l32 * g.plane * 4);
-        const int pairs = (cur.px + 1) / 2;
         int sent = more ? 0 : mine;
-        // Pair i of pixels: 2 i in the lower lane half, 2 i + 1 in the upper. Reads run one pair ahead, the offsets two. Every
-        // pair waits for what it issued and keeps it up to there: behind the last pairs of a chunk nothing multiplies what
-        // was read ahead, and registers without a use would go to the transfers' addresses while the data is on its way.
-        float a[2], b[2][kTaps];
-        int off;
-        auto read_b = [&](float (&v)[kTaps], int o) {
-#pragma unroll
-            for (int t = 0; t < kTaps; ++t) v[t] = lds_read_b32<0>(x_row + (uint32_t)o + toff[t]);
-        };
-        auto pixel = [&](int i) { return (uint32_t)(min(2 * i + half, cur.px - 1) * 4); };
-        const int own = (pairs - kg + KG - 1) / KG;      // kg, kg + KG, ...
-        auto pair = [&](int i, float& a_cur, float (&b_cur)[kTaps], float& a_next, float (&b_next)[kTaps]) {
-            if (2 * i + 1 >= cur.px) {          // the upper half is one pixel past the chunk
-                a_cur = half ? 0.f : a_cur;
-#pragma unroll
-                for (int t = 0; t < kTaps; ++t) b_cur[t] = half ? 0.f : b_cur[t];
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            acc[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a_cur, b_cur[0], acc[0], 0, 0, 0);
-            __builtin_amdgcn_sched_barrier(0);
-            a_next = lds_read_b32<0>(a_row + pixel(i + KG));
-            read_b(b_next, off);
-            off = __builtin_bit_cast(int, lds_read_b32<0>(lds0 + pixel(i + 2 * KG)));
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int t = 1; t < kTaps; ++t) {
-                acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(a_cur, b_cur[t], acc[t], 0, 0, 0);
+        if constexpr (SPLIT) {
+            // Sixteen pixels at a time: eight next to each other in a row for each lane half, a lane's fragment of dY. The ten
+            // values of X they meet in an image row serve three taps: as pairs of bf16 values tap 0 and tap 2 are the same
+            // registers one pair apart, tap 1 is shifted by half a register. Reads run one image row ahead and are waited for
+            // behind the products they run beside.
+            const int g8 = (g.ow + 7) / 8, groups = cur.px / g.ow * g8, steps = (groups + 1) / 2;
+            const float inv_g8 = 1.0f / (float)g8;
+            uint32_t aa, xa;
+            int nv;
+            auto locate = [&](int i) {
+                const int gi = 2 * i + half, gc = min(gi, groups - 1), r = fast_div(gc, g8, inv_g8), ox = 8 * (gc - r * g8);
+                aa = a_row + (uint32_t)((r * g.ow + ox) * 4);
+                xa = x_row + (uint32_t)((r * g.pwid + ox + g.col0) * 4);
+                nv = gi < groups ? min(8, g.ow - ox) : 0;
+            };
+            float ra[8], rb[10];
+            auto read_a = [&] {
+                static_for<0, 8>([&](auto e) { ra[e.value] = lds_read_b32<4 * e.value>(aa); });
+            };
+            auto read_x = [&](int hy) {
+                const uint32_t at = xa + (uint32_t)(hy * g.pwid * 4);
+                static_for<0, 10>([&](auto e) { rb[e.value] = lds_read_b32<4 * e.value>(at); });
+            };
+            auto settle = [&] {
                 __builtin_amdgcn_sched_barrier(0);
-                if ((t == 2 || t == 5) && sent < mine) issue(sent++, nxt, other);
+                wait_lgkm<0>();
                 __builtin_amdgcn_sched_barrier(0);
-            }
-            wait_lgkm<0>();
-            __builtin_amdgcn_sched_barrier(0);
-            lds_keep(a_next);
 #pragma unroll
-            for (int t = 0; t < kTaps; ++t) lds_keep(b_next[t]);
-            lds_keep(off);
-        };
-        if (own > 0) {
-            off = __builtin_bit_cast(int, lds_read_b32<0>(lds0 + pixel(kg)));
-            const int off1 = __builtin_bit_cast(int, lds_read_b32<0>(lds0 + pixel(kg + KG)));
-            a[0] = lds_read_b32<0>(a_row + pixel(kg));
-            wait_lgkm<0>();
-            __builtin_amdgcn_sched_barrier(0);
-            read_b(b[0], off);
-            wait_lgkm<0>();
-            __builtin_amdgcn_sched_barrier(0);
-            off = off1;
-            int k = 0, i = kg;
-            for (; k + 1 < own; k += 2, i += 2 * KG) {
-                pair(i, a[0], b[0], a[1], b[1]);
-                pair(i + KG, a[1], b[1], a[0], b[0]);
+                for (int e = 0; e < 8; ++e) lds_keep(ra[e]);
+#pragma unroll
+                for (int e = 0; e < 10; ++e) lds_keep(rb[e]);
+            };
+            if (kg < steps) {
+                locate(kg);
+                read_a();
+                read_x(0);
+                settle();
+                for (int i = kg; i < steps; i += KG) {
+                    const int valid = nv;
+                    const bool partial = __builtin_amdgcn_ballot_w64(valid < 8) != 0;
+                    if (partial)
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) ra[e] = e < valid ? ra[e] : 0.f;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) ra[e] *= sign;
+                    const Pieces pa = split_eight(ra);
+                    static_for<0, 3>([&](auto hyc) {
+                        constexpr int hy = hyc.value;
+                        if (partial)    // what lies behind the row: any bits
+#pragma unroll
+                            for (int e = 2; e < 10; ++e) rb[e] = e < valid + 2 ? rb[e] : 0.f;
+                        uint32_t ph[5], pm[5], pl[5];
+#pragma unroll
+                        for (int e = 0; e < 5; ++e) split_pair(floatx2{rb[2 * e], rb[2 * e + 1]}, ph[e], pm[e], pl[e]);
+                        __builtin_amdgcn_sched_barrier(0);
+                        if constexpr (hy == 2) {
+                            locate(min(i + KG, steps - 1));
+                            read_a();
+                            read_x(0);
+                        } else {
+                            read_x(hy + 1);
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                        Pieces pb[3];
+                        auto taps = [&](bf16x8 Pieces::*part, const uint32_t (&v)[5]) {
+                            u32x4 t1;
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) t1[e] = __builtin_amdgcn_alignbit(v[e + 1], v[e], 16);
+                            pb[0].*part = __builtin_bit_cast(bf16x8, u32x4{v[0], v[1], v[2], v[3]});
+                            pb[1].*part = __builtin_bit_cast(bf16x8, t1);
+                            pb[2].*part = __builtin_bit_cast(bf16x8, u32x4{v[1], v[2], v[3], v[4]});
+                        };
+                        taps(&Pieces::h, ph);
+                        taps(&Pieces::m, pm);
+                        taps(&Pieces::l, pl);
+                        mfma_split(pa, pb, acc + 3 * hy);
+                        if (sent < mine) issue(sent++, nxt, other);
+                        settle();
+                    });
+                }
             }
-            if (k < own) pair(i, a[0], b[0], a[1], b[1]);
+        } else {
+            const int pairs = (cur.px + 1) / 2;
+            // Pair i of pixels: 2 i in the lower lane half, 2 i + 1 in the upper. Reads run one pair ahead, the offsets two. Every
+            // pair waits for what it issued and keeps it up to there: behind the last pairs of a chunk nothing multiplies what
+            // was read ahead, and registers without a use would go to the transfers' addresses while the data is on its way.
+            float a[2], b[2][kTaps];
+            int off;
+            auto read_b = [&](float (&v)[kTaps], int o) {
+#pragma unroll
+                for (int t = 0; t < kTaps; ++t) v[t] = lds_read_b32<0>(x_row + (uint32_t)o + toff[t]);
+            };
+            auto pixel = [&](int i) { return (uint32_t)(min(2 * i + half, cur.px - 1) * 4); };
+            const int own = (pairs - kg + KG - 1) / KG;      // kg, kg + KG, ...
+            auto pair = [&](int i, float& a_cur, float (&b_cur)[kTaps], float& a_next, float (&b_next)[kTaps]) {
+                if (2 * i + 1 >= cur.px) {          // the upper half is one pixel past the chunk
+                    a_cur = half ? 0.f : a_cur;
+#pragma unroll
+                    for (int t = 0; t < kTaps; ++t) b_cur[t] = half ? 0.f : b_cur[t];
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                acc[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a_cur, b_cur[0], acc[0], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                a_next = lds_read_b32<0>(a_row + pixel(i + KG));
+                read_b(b_next, off);
+                off = __builtin_bit_cast(int, lds_read_b32<0>(lds0 + pixel(i + 2 * KG)));
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int t = 1; t < kTaps; ++t) {
+                    acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(a_cur, b_cur[t], acc[t], 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if ((t == 2 || t == 5) && sent < mine) issue(sent++, nxt, other);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                wait_lgkm<0>();
+                __builtin_amdgcn_sched_barrier(0);
+                lds_keep(a_next);
+#pragma unroll
+                for (int t = 0; t < kTaps; ++t) lds_keep(b_next[t]);
+                lds_keep(off);
+            };
+            if (own > 0) {
+                off = __builtin_bit_cast(int, lds_read_b32<0>(lds0 + pixel(kg)));
+                const int off1 = __builtin_bit_cast(int, lds_read_b32<0>(lds0 + pixel(kg + KG)));
+                a[0] = lds_read_b32<0>(a_row + pixel(kg));
+                wait_lgkm<0>();
+                __builtin_amdgcn_sched_barrier(0);
+                read_b(b[0], off);
+                wait_lgkm<0>();
+                __builtin_amdgcn_sched_barrier(0);
+                off = off1;
+                int k = 0, i = kg;
+                for (; k + 1 < own; k += 2, i += 2 * KG) {
+                    pair(i, a[0], b[0], a[1], b[1]);
+                    pair(i + KG, a[1], b[1], a[0], b[0]);
+                }
+                if (k < own) pair(i, a[0], b[0], a[1], b[1]);
+            }
         }
         for (; sent < mine; ++sent) issue(sent, nxt, other);
         row = next_row;
@@ -196,6 +294,43 @@ __global__ __launch_bounds__(kThreads) void conv_dense3_weight_kernel(const Weig
         stage ^= 1;
     }
     wait_vm_lgkm0<0>();
+
+    if constexpr (SPLIT) {
+        // A value without a split (infinite, NaN, above the largest bf16) makes a sum NaN: this wavefront's pixels once more, in fp32
+        float bad = 0.f;
+#pragma unroll
+        for (int t = 0; t < kTaps; ++t)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) bad = __builtin_fmaf(acc[t][e], 0.f, bad);
+        if (__builtin_amdgcn_ballot_w64(bad != 0.f) != 0) {
+#pragma unroll
+            for (int t = 0; t < kTaps; ++t)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) acc[t][e] = 0.f;
+            const bool has_m = m0 + wm * 32 + l32 < g.m, has_c = c0 + l32 < g.c;
+            const int g8 = (g.ow + 7) / 8;
+            for (int r0 = first_row; r0 < row_end;) {
+                const Chunk ch = chunk_at(r0);
+                const int groups = ch.px / g.ow * g8, steps = (groups + 1) / 2;
+                for (int i = kg; i < steps; i += KG) {
+                    const int gi = 2 * i + half, r = gi / g8, ox0 = 8 * (gi - r * g8);
+                    for (int e = 0; e < 8; ++e) {
+                        const int oy = ch.oy + r, ox = ox0 + e;
+                        const bool ok = gi < groups && ox < g.ow;
+                        const float av = ok && has_m ? g.dy[((int64_t)ch.img * g.m + m0 + wm * 32 + l32) * ohw + oy * g.ow + ox] : 0.f;
+#pragma unroll
+                        for (int t = 0; t < kTaps; ++t) {
+                            const int iy = oy - g.ph + t / 3, ix = ox - g.pw + t % 3;
+                            const bool in = ok && has_c && iy >= 0 && iy < g.h && ix >= 0 && ix < g.w;
+                            const float bv = in ? g.x[((int64_t)ch.img * g.c + c0 + l32) * in_plane + iy * g.w + ix] : 0.f;
+                            acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(av * sign, bv, acc[t], 0, 0, 0);
+                        }
+                    }
+                }
+                r0 += ch.px / g.ow;
+            }
+        }
+    }
 
     // Eight rows of every block at a time: element e of a block is row (e / 4) * 8 + (lane / 32) * 4 + e % 4, column
     // lane % 32. The wavefronts' sums of a row are added and its 288 values written next to each other, as dW has them.
@@ -209,7 +344,8 @@ __global__ __launch_bounds__(kThreads) void conv_dense3_weight_kernel(const Weig
 #pragma unroll
         for (int t = 0; t < kTaps; ++t)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) sums[(wave * 8 + half * 4 + e) * ROW + l32 * kTaps + t] = acc[t][eg * 4 + e];
+            for (int e = 0; e < 4; ++e)
+                sums[(wave * 8 + half * 4 + e) * ROW + l32 * kTaps + t] = SPLIT ? acc[t][eg * 4 + e] * sign : acc[t][eg * 4 + e];
         __syncthreads();
         // wavefront `wave` adds row `wave` of every block
         const int m = m0 + eg * 8 + wave;
@@ -231,11 +367,21 @@ __global__ __launch_bounds__(kThreads) void conv_dense3_weight_kernel(const Weig
     }
 }
 
+template <int WM, int AVEC, int XVEC>
+__global__ __launch_bounds__(kThreads) void conv_dense3_weight_kernel(const WeightArgs g) {
+    weight_gradient<WM, AVEC, XVEC, false>(g);
+}
+template <int WM, int AVEC, int XVEC>
+__global__ __launch_bounds__(kThreads) void conv_dense3_weight_split_kernel(const WeightArgs g) {
+    weight_gradient<WM, AVEC, XVEC, true>(g);
+}
+
 struct WeightPlan {
     WeightArgs a;
     size_t lds;
 };
 
+constexpr int kReadPast = 64;
 constexpr int kLdsBytes = 160 * 1024, kSumBytes = kWaves * 8 * (kCTile * kTaps + 4) * 4;
 
 // LDS layout of chunks of `rows` output rows; false if two of them do not fit
@@ -303,8 +449,8 @@ int64_t plan_ranges(const ConvGeom& g, bool general) {
 }
 
 template <int WM, int AVEC, int XVEC>
-int launch_weight(const WeightPlan& pl, unsigned blocks, hipStream_t st) {
-    auto kern = conv_dense3_weight_kernel<WM, AVEC, XVEC>;
+int launch_weight(const WeightPlan& pl, unsigned blocks, bool split, hipStream_t st) {
+    auto kern = split ? conv_dense3_weight_split_kernel<WM, AVEC, XVEC> : conv_dense3_weight_kernel<WM, AVEC, XVEC>;
     const size_t lds = pl.lds > (size_t)kSumBytes ? pl.lds : (size_t)kSumBytes;
     const hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) {
@@ -351,8 +497,11 @@ int launch_conv_dense3_bwd_weight(const ConvGeom& g, const float* x, const float
                 "conv2d_backward_weight: the 3x3 kernel does not apply");
     pl.a.x = x; pl.a.dy = dy; pl.a.part = part;
     const int wm = g.m > 32 ? 2 : 1;
+    // the last pixels of a row are read in eights, past the end of what is staged
+    const bool split = g.sh == 1 && g.sw == 1 && g.dh == 1 && g.dw == 1 && pl.lds + kReadPast <= (size_t)kLdsBytes;
+    if (split) pl.lds += kReadPast;
 #define DML_D3W(WM, AV, XV) \
-    if (wm == WM && avec == AV && xvec == XV) return launch_weight<WM, AV, XV>(pl, blocks, st);
+    if (wm == WM && avec == AV && xvec == XV) return launch_weight<WM, AV, XV>(pl, blocks, split, st);
     DML_D3W(1, 1, 1) DML_D3W(1, 1, 4) DML_D3W(1, 4, 1) DML_D3W(1, 4, 4)
     DML_D3W(2, 1, 1) DML_D3W(2, 1, 4) DML_D3W(2, 4, 1) DML_D3W(2, 4, 4)
 #undef DML_D3W

@@ -230,7 +230,7 @@ bool pointwise_project_applicable(int64_t n, int64_t cin, int64_t cout, int64_t 
 }
 
 // With few pixels a wavefront's chain over all input channels is what takes the time; the tiled GEMM cuts it into pieces. us, here and
-// there: 480 -> 80, one image of 14 x 14, 30 and 7, 96 images 42 and 38; 240 -> 40, 1 / 20 / 48 images of 28 x 28, 16 / 17 / 25 and 5 / 12 / 24; 144 -> 24, 3 / 9
+// there: 480 -> 80, one image of 14 x 14, 30 and 6, 96 images 42 and 27; 240 -> 40, 1 / 20 / 48 images of 28 x 28, 16 / 17 / 25 and 5 / 12 / 24; 144 -> 24, 3 / 9
 // images of 56 x 56, 8.9 / 10.7 and 6.5 / 13.0; 96 -> 16, one image of 112 x 112, 5.0 and 5.7.
 bool pointwise_splits_channels(int64_t n, int64_t cin, int64_t cout, int64_t hw) {
     return cin >= 96 && cin >= 2 * cout && cout <= kProjMaxOut && n * hw < 64 * cin;

@@ -1,0 +1,53 @@
+"""The weight gradient of the 3 x 3 convolution on the bf16 matrix instructions (stride and dilation 1): rows of whole eights of
+pixels, rows that end inside one, rows shorter than one, an odd number of eights, channels that end inside a tile, transfers of four and of
+sixteen bytes, wide and no padding, values without a split.
+
+Tolerance: that of the fp32 kernels' test; the products left out are below 3 * 2^-26 of |a| |b|, one of its two spare terms."""
+import numpy as np
+import pytest
+import torch
+
+from tests.test_zx_conv_dense3 import _check, _problem
+from tests.util import dev, host, rng
+
+pytestmark = pytest.mark.gpu
+
+# n, c, h, w, m, stride, pad, dilation
+SHAPES = [(6, 64, 56, 56, 64, 1, 1, 1), (40, 33, 31, 33, 70, 1, 1, 1), (24, 128, 28, 28, 64, 1, 1, 1), (150, 64, 7, 7, 64, 1, 1, 1),
+          (16, 32, 64, 64, 32, 1, 1, 1), (70, 48, 26, 30, 50, 1, 2, 1), (60, 64, 15, 60, 64, 1, 0, 1), (16, 64, 36, 57, 128, 1, 1, 1),
+          (50, 128, 14, 14, 256, 1, 1, 1), (300, 16, 5, 9, 40, 1, 1, 1), (3, 40, 200, 110, 70, 1, 1, 1), (30, 31, 40, 44, 64, 1, 4, 1)]
+
+
+def _weight_gradient(x, dy, shape):
+    from daceml_amd import kernels as K
+    n, c, h, w, m, s, p, d = shape
+    return K.conv2d_backward(dev(x), torch.empty((m, c, 3, 3), device="cuda"), dev(dy), (s, s), (p, p), (d, d), need_dx=False)[1]
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_weight_gradient(shape):
+    x, wt, b, dy, exact, terms = _problem(shape)
+    _check("dw", _weight_gradient(x, dy, shape), exact[2], terms[2], dy.shape[0] * dy.shape[2] * dy.shape[3])
+
+
+@pytest.mark.parametrize("shape", [SHAPES[0], SHAPES[7], SHAPES[3]])
+def test_values_without_a_split(shape):
+    """Infinities and NaN reach the channels they belong to and no others, a finite value above the largest bf16 stays finite."""
+    n, c, h, w, m, s, p, d = shape
+    r = rng(8)
+    x = r.standard_normal((n, c, h, w)).astype(np.float32)
+    dy = r.standard_normal((n, m, h + 2 * p - 2, w + 2 * p - 2)).astype(np.float32)
+    x[0, 3, h - 1, w - 1], x[n - 1, 4, 0, 0], dy[1, 5, 2, 3] = np.inf, np.nan, -np.inf
+    x[:, 9] = 0.0
+    x[0, 9, 2, 2] = np.finfo(np.float32).max
+    dy[:, 20] *= 1e-3
+    got = host(_weight_gradient(x, dy, shape))
+    want = torch.nn.grad.conv2d_weight(torch.from_numpy(x).double(), (m, c, 3, 3), torch.from_numpy(dy).double(), s, p).numpy()
+    with np.errstate(over="ignore"):
+        want32 = want.astype(np.float32)
+    for same in (np.isnan, np.isposinf, np.isneginf):
+        np.testing.assert_array_equal(same(got[:, [0, 3, 4, 8]]), same(want32[:, [0, 3, 4, 8]]))
+    assert np.isfinite(got[20, 9]).all()
+    np.testing.assert_allclose(got[20, 9], want32[20, 9], rtol=1e-5)
+    finite = np.isfinite(want32[:, 0])
+    np.testing.assert_allclose(got[:, 0][finite], want32[:, 0][finite], rtol=1e-4, atol=2e-3)
