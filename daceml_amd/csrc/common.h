@@ -120,9 +120,14 @@ __global__ __launch_bounds__(1024) void reduce_partials_kernel(const float* __re
     lds[wave][lane] = Op::f(Op::f(a0, a1), Op::f(a2, a3));
     __syncthreads();
     if (wave == 0 && c < cols) {
-        float a = lds[0][lane];
+        float v[16];
 #pragma unroll
-        for (int w = 1; w < 16; ++w) a = Op::f(a, lds[w][lane]);
+        for (int w = 0; w < 16; ++w) v[w] = lds[w][lane];
+#pragma unroll
+        for (int half = 8; half > 0; half /= 2)
+#pragma unroll
+            for (int w = 0; w < half; ++w) v[w] = Op::f(v[w], v[w + half]);
+        const float a = v[0];
         if (out1 && c >= cols0) out1[c - cols0] = from_f32<TOut>(a * scale);
         else out[c] = from_f32<TOut>(a * scale);
     }

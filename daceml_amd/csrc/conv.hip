@@ -476,6 +476,22 @@ inline unsigned grid_for(int64_t total) {
     return (unsigned)(gsz < 1 ? 1 : gsz);
 }
 
+// The results of `parts` ranges, `total` floats each at the front of the workspace, added in a fixed order.
+int sum_ranges(const float* part, float* dw, int64_t parts, int64_t total, void* workspace, size_t workspace_bytes, hipStream_t st) {
+    if (parts <= 1) return 0;
+    // Sixteen wavefronts share the ranges of 64 columns: one pass (128 x 36864: 6 us; the general reduction's two
+    // passes 10). With few ranges most of the sixteen would be idle (4 x 1.2 million: 45 us against 20), with many each
+    // of them walks a long chain (the whole gradient of 3 channels, 12x3x225x225 -> 8 with 1908 ranges: 43.6 against 37.6)
+    if (parts >= 32 && parts <= 512) {
+        hipLaunchKernelGGL((reduce_partials_kernel<OpSum, float>), (unsigned)ceil_div(total, (int64_t)kWave), 1024, 0, st, part, dw,
+                           (int)parts, total, total, 0.f, 1.f, (float*)nullptr, (int64_t)0);
+        return launch_status("conv2d_backward_weight(sum of ranges)");
+    }
+    const size_t part_bytes = (size_t)parts * total * sizeof(float);
+    return dmlhip_reduce_f32(DMLHIP_RSUM, part, dw, DMLHIP_F32, 1, parts, total, (char*)workspace + part_bytes,
+                             workspace_bytes - part_bytes, (void*)st);
+}
+
 template <typename T>
 int conv_forward(const dmlhip_conv2d_desc* d, const void* x, const void* w, const void* bias, void* y, void* stream) {
     ConvGeom g;
@@ -740,10 +756,7 @@ int dmlhip_conv2d_backward_weight_f32(const dmlhip_conv2d_desc* d, const void* x
                           : launch_depthwise_bwd_weight((const float*)x, (const float*)dy, part, g.n, g.c, g.h, g.w, g.oh, g.ow,
                                                         g.kh, g.sh, g.ph, st);
         if (e) return e;
-        if (g.n == 1) return 0;
-        const size_t part_bytes = (size_t)g.n * per * sizeof(float);
-        return dmlhip_reduce_f32(DMLHIP_RSUM, part, dw, DMLHIP_F32, 1, g.n, per, (char*)workspace + part_bytes,
-                                 workspace_bytes - part_bytes, stream);
+        return sum_ranges(part, (float*)dw, g.n, per, workspace, workspace_bytes, st);
     }
     if (dense_parts > 0) {
         // implicit GEMM over ranges of the (image, pixel) space, then their sum in a fixed order
@@ -753,18 +766,7 @@ int dmlhip_conv2d_backward_weight_f32(const dmlhip_conv2d_desc* d, const void* x
                           : launch_dense_bwd_weight((const float*)x, (const float*)dy, part, g.n, g.c, g.h, g.w, g.m, g.kh,
                                                     g.kw, g.sh, g.sw, g.ph, g.pw, g.dh, g.dw, g.oh, g.ow, st);
         if (e) return e;
-        if (dense_parts >= 32 && dense_parts <= 512) {
-            // sixteen wavefronts share the ranges of 64 columns: one pass (128 x 36864: 6 us; the general reduction's two
-            // passes 10). With few ranges most of the sixteen would be idle (4 x 1.2 million: 45 us against 20), with many each
-            // of them walks a long chain (the whole gradient of 3 channels, 12x3x225x225 -> 8 with 1908 ranges: 43.6 against 37.6)
-            hipLaunchKernelGGL((reduce_partials_kernel<OpSum, float>), (unsigned)ceil_div(total, (int64_t)kWave), 1024, 0, st,
-                               (const float*)part, (float*)dw, (int)dense_parts, total, total, 0.f, 1.f, (float*)nullptr, (int64_t)0);
-            return launch_status("conv2d_backward_weight(sum of ranges)");
-        }
-        if (dense_parts == 1) return 0;
-        const size_t part_bytes = (size_t)dense_parts * total * sizeof(float);
-        return dmlhip_reduce_f32(DMLHIP_RSUM, part, dw, DMLHIP_F32, 1, dense_parts, total, (char*)workspace + part_bytes,
-                                 workspace_bytes - part_bytes, stream);
+        return sum_ranges(part, (float*)dw, dense_parts, total, workspace, workspace_bytes, st);
     }
     if (is_pointwise(g) && red > 0 && (int64_t)g.h * g.w == 1 && total <= (1 << 22)) {
         hipLaunchKernelGGL(conv_1x1_spatial1_bwd_weight_kernel, (unsigned)ceil_div(total, 256), 256, 0, st,
@@ -779,10 +781,7 @@ int dmlhip_conv2d_backward_weight_f32(const dmlhip_conv2d_desc* d, const void* x
             const int64_t mc = (int64_t)g.m * g.c;
             float* part = parts > 1 ? (float*)workspace : (float*)dw;
             if (int e = launch_pointwise_bwd_weight((const float*)x, (const float*)dy, part, g.n, g.m, g.c, hw, st)) return e;
-            if (parts == 1) return 0;
-            const size_t part_bytes = (size_t)parts * mc * sizeof(float);
-            return dmlhip_reduce_f32(DMLHIP_RSUM, part, dw, DMLHIP_F32, 1, parts, mc, (char*)workspace + part_bytes,
-                                     workspace_bytes - part_bytes, stream);
+            return sum_ranges(part, (float*)dw, parts, mc, workspace, workspace_bytes, st);
         }
         // per image: P[b] (M x C) = dY[b] (M x HW) . X[b]^T (HW x C); then dW = sum_b P[b]
         dmlhip_gemm_desc gd = {};
