@@ -152,6 +152,7 @@ __global__ __launch_bounds__(256) void depthwise_bwd_weight_kernel(const float* 
 
 // ---------------------------------------------------------------- pointwise, weight gradient
 constexpr int kSlab = 64;        // pixels per LDS slab
+constexpr int kPwGradBlocks = 3; // blocks of 32 accumulator rows per workgroup, at most
 constexpr int kPitch = kSlab + 2;  // rows land two banks apart: the two k halves of a wavefront read disjoint banks
 
 struct PwGradArgs {
@@ -166,7 +167,12 @@ struct PwGradArgs {
     int64_t out_elems;
 };
 
-template <int TA>
+// Bound by reading both operands once, for few channels, and by the matrix pipe for many. Up to three blocks of rows per workgroup: with
+// eight the registers spilled and one workgroup per compute unit was all there was. Measured, us, with the sum of the results,
+// up to eight blocks and 1024 workgroups, and three and 512: 24 -> 144 channels, 32 x 56 x 56, 29.7 and 26.0 (67 MB), 16 -> 96, 32 x 112 x 112, 53
+// and 43 (180 MB, 4.2 TB/s), 40 -> 240, 2 / 32 x 28 x 28, 31 / 53 and 9.4 / 19.7, 128 -> 256, 32 x 28 x 28, 69 and 33.
+// SETS: sets of accumulators; two of them, for every other pair of pixels, halve the chains of sums
+template <int TA, int SETS>
 __global__ __launch_bounds__(256, 2) void pointwise_bwd_weight_kernel(const PwGradArgs g) {
     extern __shared__ __attribute__((aligned(16))) float pg_lds[];
     constexpr int ROWS = (TA + 1) * 32;              // TA blocks of a, then one block of b
@@ -181,11 +187,13 @@ __global__ __launch_bounds__(256, 2) void pointwise_bwd_weight_kernel(const PwGr
     const float* an = g.a + (int64_t)img * g.ra * g.hw;
     const float* bn = g.b + (int64_t)img * g.rb * g.hw;
 
-    floatx16 acc[TA];
+    floatx16 acc[SETS][TA];
 #pragma unroll
-    for (int t = 0; t < TA; ++t)
+    for (int i = 0; i < SETS; ++i)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) acc[t][e] = 0.f;
+        for (int t = 0; t < TA; ++t)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][t][e] = 0.f;
 
     // row / column of the slab this thread moves, per load
     floatx4 pre[NV];
@@ -223,7 +231,7 @@ __global__ __launch_bounds__(256, 2) void pointwise_bwd_weight_kernel(const PwGr
             const float bv = bl[2 * ks];
 #pragma unroll
             for (int t = 0; t < TA; ++t)
-                acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(al[t * 32 * kPitch + 2 * ks], bv, acc[t], 0, 0, 0);
+                acc[ks % SETS][t] = __builtin_amdgcn_mfma_f32_32x32x2f32(al[t * 32 * kPitch + 2 * ks], bv, acc[ks % SETS][t], 0, 0, 0);
         }
     }
     // sum the four wavefronts' blocks through LDS and write the workgroup's result
@@ -232,7 +240,7 @@ __global__ __launch_bounds__(256, 2) void pointwise_bwd_weight_kernel(const PwGr
     for (int t = 0; t < TA; ++t) {
         __syncthreads();
 #pragma unroll
-        for (int e = 0; e < 16; ++e) pg_lds[wave * 1024 + e * 64 + lane] = acc[t][e];
+        for (int e = 0; e < 16; ++e) pg_lds[wave * 1024 + e * 64 + lane] = SETS == 2 ? acc[0][t][e] + acc[SETS - 1][t][e] : acc[0][t][e];
         __syncthreads();
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -399,16 +407,16 @@ bool plan_dense_bwd_weight(int n, int c, int m, int kk, int oh, int ow, int h, i
 
 struct PwGradPlan {
     bool swap;            // a = X (rows = input channels) instead of a = dY
-    int ta, a_groups, b_tiles, chunk_px, chunks_per_img;
+    int ta, a_groups, b_tiles, chunk_px, chunks_per_img, sets;
     int64_t blocks_x;
 };
 
-bool plan_pointwise_bwd_weight(int n, int m, int c, int64_t hw, PwGradPlan* pl) {
-    if (n < 1 || m < 1 || c < 1 || hw < 256 || hw % 4 != 0) return false;
+// Orientation, groups of up to `most` blocks of rows, and chunks of an image's pixels for about `wgs` workgroups. Returns the traffic of
+// the orientation in units of one pixel of one channel: the operand on the accumulators' columns is re-read once per group of a, the other
+// once per 32 rows of b.
+double lay_out_pointwise(int n, int m, int c, int64_t hw, int most, int64_t wgs, int64_t most_px, PwGradPlan* pl) {
     const int tm = (int)ceil_div(m, 32), tc = (int)ceil_div(c, 32);
-    // traffic of the two orientations in units of one pixel of one channel: the operand on the accumulators' columns
-    // is re-read once per group of a, the other once per 32 rows of b
-    auto groups = [](int tiles) { return (tiles + 7) / 8; };
+    auto groups = [=](int tiles) { return (tiles + most - 1) / most; };
     const double cost_dy_rows = (double)m * tc + (double)c * groups(tm);
     const double cost_x_rows = (double)c * tm + (double)m * groups(tc);
     pl->swap = cost_x_rows < cost_dy_rows;
@@ -416,18 +424,31 @@ bool plan_pointwise_bwd_weight(int n, int m, int c, int64_t hw, PwGradPlan* pl) 
     pl->b_tiles = pl->swap ? tm : tc;
     pl->a_groups = groups(ta_tiles);
     pl->ta = (ta_tiles + pl->a_groups - 1) / pl->a_groups;
-    if ((pl->swap ? cost_x_rows : cost_dy_rows) > 4.0 * (m + c)) return false;   // a tiled GEMM re-reads less
-    const int64_t ygroups = (int64_t)pl->a_groups * pl->b_tiles;
-    int64_t per_img = ceil_div((int64_t)1024, (int64_t)n * ygroups);
+    int64_t per_img = ceil_div(wgs, (int64_t)n * pl->a_groups * pl->b_tiles);
+    if (per_img < ceil_div(hw, most_px)) per_img = ceil_div(hw, most_px);
     const int64_t max_per_img = ceil_div(hw, (int64_t)256);
     if (per_img > max_per_img) per_img = max_per_img;
-    if (per_img < 1) per_img = 1;
-    int64_t px = ceil_div(ceil_div(hw, per_img), (int64_t)kSlab) * kSlab;
-    if (px > (1 << 30)) return false;
-    pl->chunk_px = (int)px;
+    const int64_t px = ceil_div(ceil_div(hw, per_img), (int64_t)kSlab) * kSlab;
+    pl->chunk_px = px > (1 << 30) ? 0 : (int)px;
     pl->chunks_per_img = (int)ceil_div(hw, px);
     pl->blocks_x = (int64_t)n * pl->chunks_per_img;
-    return pl->blocks_x <= 2147483647LL && ygroups <= 65535;
+    pl->sets = 1;
+    return pl->swap ? cost_x_rows : cost_dy_rows;
+}
+
+bool plan_pointwise_bwd_weight(int n, int m, int c, int64_t hw, PwGradPlan* pl) {
+    if (n < 1 || m < 1 || c < 1 || hw < 256 || hw % 4 != 0) return false;
+    if (lay_out_pointwise(n, m, c, hw, 8, 1024, hw, pl) > 4.0 * (m + c)) return false;   // a tiled GEMM re-reads less
+    if (pl->chunk_px == 0) return false;
+    // More than three blocks of rows, or three that make all of the rows: groups of three, two workgroups for each of 256 compute units
+    // and two sets of accumulators, for chunks up to twice as long. Three blocks against several of columns stay with more
+    // workgroups: 96 -> 96, 32 x 56 x 56, 43 us and 49.
+    if (pl->ta > kPwGradBlocks || pl->a_groups > 1 || (pl->ta == kPwGradBlocks && pl->b_tiles == 1)) {
+        const int px = pl->chunk_px;
+        lay_out_pointwise(n, m, c, hw, kPwGradBlocks, 512, 2 * (int64_t)px, pl);
+        pl->sets = 2;
+    }
+    return pl->blocks_x <= 2147483647LL && (int64_t)pl->a_groups * pl->b_tiles <= 65535;
 }
 
 }  // namespace
@@ -545,27 +566,15 @@ int launch_pointwise_bwd_weight(const float* x, const float* dy, float* part, in
     g.out_elems = (int64_t)m * c;
     const dim3 grid((unsigned)pl.blocks_x, (unsigned)(pl.a_groups * pl.b_tiles));
     const size_t lds = (size_t)(pl.ta + 1) * 32 * kPitch * sizeof(float);
-#define DML_PWG(TA)                                                                                                    \
-    case TA: {                                                                                                         \
-        auto kern = pointwise_bwd_weight_kernel<TA>;                                                                   \
-        if (lds > 64 * 1024) {                                                                                         \
-            hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
-            if (e != hipSuccess) {                                                                                     \
-                set_error("conv2d_backward_weight: cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e));  \
-                return (int)e;                                                                                         \
-            }                                                                                                          \
-        }                                                                                                              \
-        hipLaunchKernelGGL(kern, grid, 256, lds, st, g);                                                               \
-        break;                                                                                                         \
+#define DML_PWG(TA, SETS)                                                        \
+    if (pl.ta == TA && pl.sets == SETS) {                                        \
+        hipLaunchKernelGGL((pointwise_bwd_weight_kernel<TA, SETS>), grid, 256, lds, st, g); \
+        return launch_status("conv2d_backward_weight(pointwise)");               \
     }
-    switch (pl.ta) {
-        DML_PWG(1) DML_PWG(2) DML_PWG(3) DML_PWG(4) DML_PWG(5) DML_PWG(6) DML_PWG(7) DML_PWG(8)
-        default:
-            set_error("conv2d_backward_weight: bad block count %d", pl.ta);
-            return DMLHIP_ERR_UNSUPPORTED;
-    }
+    DML_PWG(1, 1) DML_PWG(2, 1) DML_PWG(3, 1) DML_PWG(2, 2) DML_PWG(3, 2)
 #undef DML_PWG
-    return launch_status("conv2d_backward_weight(pointwise)");
+    set_error("conv2d_backward_weight: bad block count %d", pl.ta);
+    return DMLHIP_ERR_UNSUPPORTED;
 }
 
 }  // namespace dml

@@ -81,3 +81,18 @@ def test_infinities_and_nan_stay_in_their_pixel(hw):
     want = F.conv2d(*(torch.from_numpy(t).double() for t in (x, wt, b))).numpy()
     for same in (np.isnan, np.isposinf, np.isneginf):
         np.testing.assert_array_equal(same(got), same(want))
+
+
+# n, cin, cout, h, w: one to five groups of three blocks of rows, one and two results per image, both orientations
+@pytest.mark.parametrize("shape", [(2, 24, 144, 56, 56), (1, 40, 240, 28, 28), (33, 480, 72, 16, 16), (3, 33, 97, 20, 54), (40, 64, 128, 44, 44)])
+def test_weight_gradient(shape):
+    from daceml_amd import kernels as K
+    n, cin, cout, h, w = shape
+    r = np.random.default_rng(4)
+    x, dy = (torch.from_numpy(r.standard_normal((n, c, h, w)).astype(np.float32)).cuda() for c in (cin, cout))
+    _, dw = K.conv2d_backward(x, torch.empty((cout, cin, 1, 1), device="cuda"), dy, need_dx=False)
+    flat = lambda t: t.double().transpose(0, 1).reshape(t.shape[1], -1)  # noqa: E731
+    exact, size = (torch.mm(flat(f(dy)), flat(f(x)).t().contiguous()) for f in (lambda t: t, torch.abs))
+    k = n * h * w
+    assert ((dw.double().view(cout, cin) - exact).abs() <= k * 2.0 ** -24 * size).all()
+    assert ((dw.double().view(cout, cin) - exact).norm() / exact.norm()).item() < 1e-6
