@@ -454,9 +454,11 @@ static int launch_planned(const ConvGeom& g, int ids_h, int ids_w, bool flip, bo
     return DMLHIP_ERR_UNSUPPORTED;
 }
 
-double conv_dense3_us(const ConvGeom& g, int ids_h, int ids_w, bool flip, const void* x, const void* w) {
+double conv_dense3_us(const ConvGeom& g, int ids_h, int ids_w, bool flip, const void* x, const void* w, int* chains) {
     Dense3Plan pl;
-    return plan_conv_dense3(g, ids_h, ids_w, flip, false, x, w, &pl) ? pl.us : -1.0;
+    if (!plan_conv_dense3(g, ids_h, ids_w, flip, false, x, w, &pl)) return -1.0;
+    *chains = 1 << pl.tile;
+    return pl.us;
 }
 
 int launch_conv_dense3_f32(const ConvGeom& g, const float* x, const float* w, const float* bias, float* y, hipStream_t st,

@@ -12,8 +12,8 @@
 // the loads of the chunks beside them (1 us per step: 8 loads of 4 bytes per lane for a chunk; with the loads left out P = 4 takes
 // 7.3 us, P = 1 2.5 of 3.2), 0.5 us for the stores to LDS and the barriers, and per tile 5 us of first loads and 3 - 9 us of
 // results, which one workgroup per compute unit does not hide. Measured, us forward / data gradient, the kernel of
-// conv_dense3.hip and here: 32x64x56x56 -> 64 92 / 86 and 56 / 55, 32x64x56x56 -> 128 160 / 154 and 112 / 97, 32x128x28x28 -> 128
-// 92 / 88 and 54 / 52, 32x256x14x14 -> 256 110 / 106 and 61 / 58. What the products waited for until it was changed: 64 copies of the
+// conv_dense3.hip and here: 32x64x56x56 -> 64 92 / 86 and 56 / 55, 32x64x56x56 -> 128 148 / 153 and 105 / 91, 32x128x28x28 -> 128
+// 85 / 84 and 66 / 64 (54 / 52 with P = 4, see the rule at the launch), 32x256x14x14 -> 256 107 / 104 and 59 / 56. What the products waited for until it was changed: 64 copies of the
 // activation in the epilogue (12 us per tile), loads behind branches (their addresses in 64 registers, 2 us per step), MFMAs
 // of one block in a row (0.4 us).
 #include "bf16_split.h"
@@ -338,7 +338,7 @@ thread_local int g_force_p = 0;     // diagnostic: blocks of 32 pixels per wavef
 }  // namespace
 
 // The geometry is the product's own: for a data gradient the stride-1 convolution of the (zero-dilated) dY. *us: estimated time.
-static bool plan_split(const ConvGeom& g, int ids_h, int ids_w, SplitPlan3* pl, double* us) {
+static bool plan_split(const ConvGeom& g, int ids_h, int ids_w, int most_p, SplitPlan3* pl, double* us) {
     if (g_force_p < 0 || g.kh != 3 || g.kw != 3 || g.group != 1 || g.n < 1 || g.c < 16 || g.c % 8 || g.m < 1 || g.oh < 1 || g.ow < 1) return false;
     const int64_t ohw = (int64_t)g.oh * g.ow, total = (int64_t)g.n * ohw;
     const int64_t img_rows = (int64_t)(g.oh - 1) * g.sh + 2LL * g.dh + 1, pwid = (int64_t)(g.ow - 1) * g.sw + 2LL * g.dw + 1;
@@ -346,7 +346,7 @@ static bool plan_split(const ConvGeom& g, int ids_h, int ids_w, SplitPlan3* pl, 
         return false;                                                                        // fast_div's range
     if (pwid > 1024 || g.dh > 1024 || (int64_t)g.m * g.c * kTaps > (1LL << 28)) return false;
     pl->p = 0;
-    for (int p = 1; p <= 4; p *= 2) {
+    for (int p = 1; p <= most_p; p *= 2) {
         if (g_force_p > 0 && p != g_force_p) continue;
         const int64_t px = 128LL * p;
         // rows of the stacked images that PX consecutive pixels reach; every image boundary among them adds the rows between
@@ -381,8 +381,18 @@ static int launch_split(const ConvGeom& g, int ids_h, int ids_w, bool flip, cons
                         hipStream_t st, const char* what, bool* applies) {
     SplitPlan3 pl;
     double us;
-    *applies = plan_split(g, ids_h, ids_w, &pl, &us);
-    if (*applies && g_force_p == 0) *applies = us < conv_dense3_us(g, ids_h, ids_w, flip, x, w);
+    // The error of a sum grows with the root of its roundings: 54 for 16 channels in one sum (P = 2, 4), 27 in two (P = 1), on the fp32
+    // instruction 72, 36 or 18 in one, two or four. Where that kernel would take two, only P = 1 is as exact (2.5e-7 where it has 3.0e-7,
+    // 64 channels; 3.6e-7 with P = 4), where four, none.
+    int chains = 1;
+    double other = 0;
+    if (g_force_p == 0) {
+        other = conv_dense3_us(g, ids_h, ids_w, flip, x, w, &chains);
+        *applies = other > 0 && chains <= 2;
+        if (!*applies) return 0;
+    }
+    *applies = plan_split(g, ids_h, ids_w, chains == 2 ? 1 : 4, &pl, &us);
+    if (*applies && g_force_p == 0) *applies = us < other;
     if (!*applies) return 0;
     pl.a.x = x; pl.a.w = w; pl.a.bias = bias; pl.a.y = y;
     return flip ? launch_form<true>(pl, st, what) : launch_form<false>(pl, st, what);
