@@ -30,7 +30,7 @@ SOURCES = [
     "gemm_f32.hip",
     "gemm_f32_split.hip",
     "conv.hip",
-    "conv_fused.hip", "conv_fused_columns.hip", "conv_backward.hip", "conv_implicit.hip", "conv_dense3.hip", "conv_dense3_split.hip", "conv_dense3_weight.hip", "conv_depthwise.hip",
+    "conv_fused.hip", "conv_fused_columns.hip", "conv_backward.hip", "conv_implicit.hip", "conv_dense3.hip", "conv_dense3_split.hip", "conv_dense3_weight_split.hip", "conv_depthwise.hip",
     "conv_pointwise_few.hip",
     "conv_pointwise_project.hip",
     "attention.hip",

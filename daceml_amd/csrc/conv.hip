@@ -762,7 +762,7 @@ int dmlhip_conv2d_backward_weight_f32(const dmlhip_conv2d_desc* d, const void* x
         // implicit GEMM over ranges of the (image, pixel) space, then their sum in a fixed order
         float* part = dense_parts > 1 ? (float*)workspace : (float*)dw;
         const int e = dense3_weight_partials(g) > 0
-                          ? launch_conv_dense3_bwd_weight(g, (const float*)x, (const float*)dy, part, st)
+                          ? launch_conv_dense3_weight(g, (const float*)x, (const float*)dy, part, st)
                           : launch_dense_bwd_weight((const float*)x, (const float*)dy, part, g.n, g.c, g.h, g.w, g.m, g.kh,
                                                     g.kw, g.sh, g.sw, g.ph, g.pw, g.dh, g.dw, g.oh, g.ow, st);
         if (e) return e;

@@ -1,22 +1,15 @@
-// Weight gradient of a dense (group 1) 3 x 3 convolution, fp32, on the bf16 matrix instructions with operands split into three
-// bf16 values each (stride and dilation 1; bf16_split.h), else on v_mfma_f32_32x32x2_f32:
+// Weight gradient of a dense (group 1) 3 x 3 convolution, fp32, on v_mfma_f32_32x32x2_f32 (strides and dilations; the others on
+// the bf16 matrix instructions, conv_dense3_weight_split.hip, which includes this file for the frame that both share):
 //   dW[m, c, hy, hx] = sum_{n, p} dY[n, m, p] * X[n, c, oy(p) s - pad + hy d, ox(p) s - pad + hx d]
 //
 // What bounds it: the matrix rate, once the nine taps share what is read. A wavefront keeps the nine 32 x 32 blocks
-// (channels of dY x channels of X, one per tap) in registers; sixteen pixels (fp32: a pair) are one dY fragment and the shifted
-// reads of the same rectangle of X for 54 (nine) MFMAs. One workgroup of eight wavefronts per compute unit: 64 (32) channels of dY
+// (channels of dY x channels of X, one per tap) in registers; a pair of pixels (split: sixteen) is one dY fragment and the shifted
+// reads of the same rectangle of X for nine MFMAs (54). One workgroup of eight wavefronts per compute unit: 64 (32) channels of dY
 // x 32 channels of X over a range of output rows, the wavefronts of the same channels taking every fourth (eighth) set of
 // pixels. Rows of dY and the rows of X under them go global -> LDS without staging registers, a chunk of output rows of one
 // image at a time, one chunk ahead, issued between the MFMAs of the chunk before. The wavefronts' sums are added through LDS
-// and the ranges' results by the reduction kernel, all in a fixed order.
-// Measured, us with the reduction, fp32 instruction and split: 32x64x56x56 -> 64 92 and 67, -> 128 165 and 112, 32x128x28x28 -> 128 91
-// and 67, 32x96x40x40 -> 96 129 and 84, 32x256x14x14 -> 256 108 and 94 (rows of 14 are read as 16), 32x64x55x55 -> 64 115 and 93
-// (transfers of four bytes). Of the 67 the products are 20, and the split's 70 vector instructions for 18 MFMAs as much beside them; addresses
-// of transfers take 9, the ranges' sums and their results 7, the reduction 6.
-// All sums are fp32, errors against fp64, 2-norm, fp32 instruction and split: 32x64x56x56 -> 64 2.7e-7 and 2.4e-7, 32x32x112x112 -> 32 2.7e-7 and
-// 2.6e-7, 32x256x14x14 -> 256 2.5e-7 and 2.3e-7. The bf16 instruction loses the low bits of what it adds in one direction, which
-// 2048 partial sums add up to 6.2e-7 in the second of these: every other wavefront adds -dY X instead.
-#include "bf16_split.h"
+// and the ranges' results by the reduction kernel, all in a fixed order. All sums are fp32.
+#include "common.h"
 #include "conv_geom.h"
 #include "lds_ops.h"
 
@@ -52,21 +45,17 @@ __device__ __forceinline__ void lds_dma(const float* gptr, char* lds_dst) {
     else __builtin_amdgcn_global_load_lds(g, l, 4, 0, 0);
 }
 
-template <int I, int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        static_for<I + 1, N>(f);
-    }
-}
+struct NoSplit {
+    static constexpr bool on = false;
+};
 
 struct Chunk {
     int img, oy, px;         // image, first output row, pixels
 };
 
-// WM: blocks of 32 channels of dY (1 or 2). AVEC, XVEC: floats per lane and transfer of dY and of X. SPLIT: stride and dilation
-// 1, on the bf16 matrix instructions.
-template <int WM, int AVEC, int XVEC, bool SPLIT>
+// WM: blocks of 32 channels of dY (1 or 2). AVEC, XVEC: floats per lane and transfer of dY and of X. SPLIT: the products on the
+// bf16 matrix instructions (conv_dense3_weight_split.hip), NoSplit for the fp32 one.
+template <int WM, int AVEC, int XVEC, typename SPLIT>
 __device__ __forceinline__ void weight_gradient(const WeightArgs& g) {
     constexpr int MB = 32 * WM, KG = kWaves / WM;
     extern __shared__ __attribute__((aligned(16))) char lds[];
@@ -130,8 +119,8 @@ __device__ __forceinline__ void weight_gradient(const WeightArgs& g) {
 #pragma unroll
     for (int t = 0; t < kTaps; ++t) toff[t] = (uint32_t)((t / 3 * g.dh * g.pwid + t % 3 * g.dw) * 4);
 
-    // see above: what the instruction loses in one direction cancels
-    const float sign = SPLIT && (kg & 1) ? -1.f : 1.f;
+    // the bf16 instruction loses low bits in one direction: with every other wavefront adding -dY X what is lost cancels
+    const float sign = SPLIT::on && (kg & 1) ? -1.f : 1.f;
 
     Chunk cur = chunk_at(row);
     if (row < row_end)
@@ -149,87 +138,10 @@ __device__ __forceinline__ void weight_gradient(const WeightArgs& g) {
         const uint32_t a_row = so + (uint32_t)((wm * 32 + l32) * g.pitch * 4);
         const uint32_t x_row = so + (uint32_t)(g.a_bytes + l32 * g.plane * 4);
         int sent = more ? 0 : mine;
-        if constexpr (SPLIT) {
-            // Sixteen pixels at a time: eight next to each other in a row for each lane half, a lane's fragment of dY. The ten
-            // values of X they meet in an image row serve three taps: as pairs of bf16 values tap 0 and tap 2 are the same
-            // registers one pair apart, tap 1 is shifted by half a register. Reads run one image row ahead and are waited for
-            // behind the products they run beside.
-            const int g8 = (g.ow + 7) / 8, groups = cur.px / g.ow * g8, steps = (groups + 1) / 2;
-            const float inv_g8 = 1.0f / (float)g8;
-            uint32_t aa, xa;
-            int nv;
-            auto locate = [&](int i) {
-                const int gi = 2 * i + half, gc = min(gi, groups - 1), r = fast_div(gc, g8, inv_g8), ox = 8 * (gc - r * g8);
-                aa = a_row + (uint32_t)((r * g.ow + ox) * 4);
-                xa = x_row + (uint32_t)((r * g.pwid + ox + g.col0) * 4);
-                nv = gi < groups ? min(8, g.ow - ox) : 0;
-            };
-            float ra[8], rb[10];
-            auto read_a = [&] {
-                static_for<0, 8>([&](auto e) { ra[e.value] = lds_read_b32<4 * e.value>(aa); });
-            };
-            auto read_x = [&](int hy) {
-                const uint32_t at = xa + (uint32_t)(hy * g.pwid * 4);
-                static_for<0, 10>([&](auto e) { rb[e.value] = lds_read_b32<4 * e.value>(at); });
-            };
-            auto settle = [&] {
-                __builtin_amdgcn_sched_barrier(0);
-                wait_lgkm<0>();
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int e = 0; e < 8; ++e) lds_keep(ra[e]);
-#pragma unroll
-                for (int e = 0; e < 10; ++e) lds_keep(rb[e]);
-            };
-            if (kg < steps) {
-                locate(kg);
-                read_a();
-                read_x(0);
-                settle();
-                for (int i = kg; i < steps; i += KG) {
-                    const int valid = nv;
-                    const bool partial = __builtin_amdgcn_ballot_w64(valid < 8) != 0;
-                    if (partial)
-#pragma unroll
-                        for (int e = 0; e < 8; ++e) ra[e] = e < valid ? ra[e] : 0.f;
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) ra[e] *= sign;
-                    const Pieces pa = split_eight(ra);
-                    static_for<0, 3>([&](auto hyc) {
-                        constexpr int hy = hyc.value;
-                        if (partial)    // what lies behind the row: any bits
-#pragma unroll
-                            for (int e = 2; e < 10; ++e) rb[e] = e < valid + 2 ? rb[e] : 0.f;
-                        uint32_t ph[5], pm[5], pl[5];
-#pragma unroll
-                        for (int e = 0; e < 5; ++e) split_pair(floatx2{rb[2 * e], rb[2 * e + 1]}, ph[e], pm[e], pl[e]);
-                        __builtin_amdgcn_sched_barrier(0);
-                        if constexpr (hy == 2) {
-                            locate(min(i + KG, steps - 1));
-                            read_a();
-                            read_x(0);
-                        } else {
-                            read_x(hy + 1);
-                        }
-                        __builtin_amdgcn_sched_barrier(0);
-                        Pieces pb[3];
-                        auto taps = [&](bf16x8 Pieces::*part, const uint32_t (&v)[5]) {
-                            u32x4 t1;
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) t1[e] = __builtin_amdgcn_alignbit(v[e + 1], v[e], 16);
-                            pb[0].*part = __builtin_bit_cast(bf16x8, u32x4{v[0], v[1], v[2], v[3]});
-                            pb[1].*part = __builtin_bit_cast(bf16x8, t1);
-                            pb[2].*part = __builtin_bit_cast(bf16x8, u32x4{v[1], v[2], v[3], v[4]});
-                        };
-                        taps(&Pieces::h, ph);
-                        taps(&Pieces::m, pm);
-                        taps(&Pieces::l, pl);
-                        mfma_split(pa, pb, acc + 3 * hy);
-                        if (sent < mine) issue(sent++, nxt, other);
-                        settle();
-                    });
-                }
-            }
+        if constexpr (SPLIT::on) {
+            SPLIT::template chunk<KG>(g, acc, a_row, x_row, cur.px, kg, half, sign, [&] {
+                if (sent < mine) issue(sent++, nxt, other);
+            });
         } else {
             const int pairs = (cur.px + 1) / 2;
             // Pair i of pixels: 2 i in the lower lane half, 2 i + 1 in the upper. Reads run one pair ahead, the offsets two. Every
@@ -295,42 +207,7 @@ __device__ __forceinline__ void weight_gradient(const WeightArgs& g) {
     }
     wait_vm_lgkm0<0>();
 
-    if constexpr (SPLIT) {
-        // A value without a split (infinite, NaN, above the largest bf16) makes a sum NaN: this wavefront's pixels once more, in fp32
-        float bad = 0.f;
-#pragma unroll
-        for (int t = 0; t < kTaps; ++t)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) bad = __builtin_fmaf(acc[t][e], 0.f, bad);
-        if (__builtin_amdgcn_ballot_w64(bad != 0.f) != 0) {
-#pragma unroll
-            for (int t = 0; t < kTaps; ++t)
-#pragma unroll
-                for (int e = 0; e < 16; ++e) acc[t][e] = 0.f;
-            const bool has_m = m0 + wm * 32 + l32 < g.m, has_c = c0 + l32 < g.c;
-            const int g8 = (g.ow + 7) / 8;
-            for (int r0 = first_row; r0 < row_end;) {
-                const Chunk ch = chunk_at(r0);
-                const int groups = ch.px / g.ow * g8, steps = (groups + 1) / 2;
-                for (int i = kg; i < steps; i += KG) {
-                    const int gi = 2 * i + half, r = gi / g8, ox0 = 8 * (gi - r * g8);
-                    for (int e = 0; e < 8; ++e) {
-                        const int oy = ch.oy + r, ox = ox0 + e;
-                        const bool ok = gi < groups && ox < g.ow;
-                        const float av = ok && has_m ? g.dy[((int64_t)ch.img * g.m + m0 + wm * 32 + l32) * ohw + oy * g.ow + ox] : 0.f;
-#pragma unroll
-                        for (int t = 0; t < kTaps; ++t) {
-                            const int iy = oy - g.ph + t / 3, ix = ox - g.pw + t % 3;
-                            const bool in = ok && has_c && iy >= 0 && iy < g.h && ix >= 0 && ix < g.w;
-                            const float bv = in ? g.x[((int64_t)ch.img * g.c + c0 + l32) * in_plane + iy * g.w + ix] : 0.f;
-                            acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(av * sign, bv, acc[t], 0, 0, 0);
-                        }
-                    }
-                }
-                r0 += ch.px / g.ow;
-            }
-        }
-    }
+    if constexpr (SPLIT::on) SPLIT::template repair<KG>(g, acc, chunk_at, first_row, row_end, m0 + wm * 32 + l32, c0 + l32, kg, half, sign);
 
     // Eight rows of every block at a time: element e of a block is row (e / 4) * 8 + (lane / 32) * 4 + e % 4, column
     // lane % 32. The wavefronts' sums of a row are added and its 288 values written next to each other, as dW has them.
@@ -345,7 +222,7 @@ __device__ __forceinline__ void weight_gradient(const WeightArgs& g) {
         for (int t = 0; t < kTaps; ++t)
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                sums[(wave * 8 + half * 4 + e) * ROW + l32 * kTaps + t] = SPLIT ? acc[t][eg * 4 + e] * sign : acc[t][eg * 4 + e];
+                sums[(wave * 8 + half * 4 + e) * ROW + l32 * kTaps + t] = SPLIT::on ? acc[t][eg * 4 + e] * sign : acc[t][eg * 4 + e];
         __syncthreads();
         // wavefront `wave` adds row `wave` of every block
         const int m = m0 + eg * 8 + wave;
@@ -369,11 +246,7 @@ __device__ __forceinline__ void weight_gradient(const WeightArgs& g) {
 
 template <int WM, int AVEC, int XVEC>
 __global__ __launch_bounds__(kThreads) void conv_dense3_weight_kernel(const WeightArgs g) {
-    weight_gradient<WM, AVEC, XVEC, false>(g);
-}
-template <int WM, int AVEC, int XVEC>
-__global__ __launch_bounds__(kThreads) void conv_dense3_weight_split_kernel(const WeightArgs g) {
-    weight_gradient<WM, AVEC, XVEC, true>(g);
+    weight_gradient<WM, AVEC, XVEC, NoSplit>(g);
 }
 
 struct WeightPlan {
@@ -381,7 +254,6 @@ struct WeightPlan {
     size_t lds;
 };
 
-constexpr int kReadPast = 64;
 constexpr int kLdsBytes = 160 * 1024, kSumBytes = kWaves * 8 * (kCTile * kTaps + 4) * 4;
 
 // LDS layout of chunks of `rows` output rows; false if two of them do not fit
@@ -448,9 +320,7 @@ int64_t plan_ranges(const ConvGeom& g, bool general) {
     return ranges * tiles <= 2147483647LL ? ranges : 0;
 }
 
-template <int WM, int AVEC, int XVEC>
-int launch_weight(const WeightPlan& pl, unsigned blocks, bool split, hipStream_t st) {
-    auto kern = split ? conv_dense3_weight_split_kernel<WM, AVEC, XVEC> : conv_dense3_weight_kernel<WM, AVEC, XVEC>;
+int launch_weight(void (*kern)(const WeightArgs), const WeightPlan& pl, unsigned blocks, hipStream_t st) {
     const size_t lds = pl.lds > (size_t)kSumBytes ? pl.lds : (size_t)kSumBytes;
     const hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) {
@@ -497,11 +367,8 @@ int launch_conv_dense3_bwd_weight(const ConvGeom& g, const float* x, const float
                 "conv2d_backward_weight: the 3x3 kernel does not apply");
     pl.a.x = x; pl.a.dy = dy; pl.a.part = part;
     const int wm = g.m > 32 ? 2 : 1;
-    // the last pixels of a row are read in eights, past the end of what is staged
-    const bool split = g.sh == 1 && g.sw == 1 && g.dh == 1 && g.dw == 1 && pl.lds + kReadPast <= (size_t)kLdsBytes;
-    if (split) pl.lds += kReadPast;
 #define DML_D3W(WM, AV, XV) \
-    if (wm == WM && avec == AV && xvec == XV) return launch_weight<WM, AV, XV>(pl, blocks, split, st);
+    if (wm == WM && avec == AV && xvec == XV) return launch_weight(conv_dense3_weight_kernel<WM, AV, XV>, pl, blocks, st);
     DML_D3W(1, 1, 1) DML_D3W(1, 1, 4) DML_D3W(1, 4, 1) DML_D3W(1, 4, 4)
     DML_D3W(2, 1, 1) DML_D3W(2, 1, 4) DML_D3W(2, 4, 1) DML_D3W(2, 4, 4)
 #undef DML_D3W

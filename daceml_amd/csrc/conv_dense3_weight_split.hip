@@ -1,0 +1,182 @@
+// Weight gradient of a dense (group 1) 3 x 3 convolution, stride and dilation 1, fp32, on the bf16 matrix instructions: operands
+// split into three bf16 values each (bf16_split.h), in the frame of conv_dense3_weight.hip.
+//
+// Measured, us with the reduction, fp32 instruction and split: 32x64x56x56 -> 64 92 and 67, -> 128 165 and 112, 32x128x28x28 -> 128 91
+// and 67, 32x96x40x40 -> 96 129 and 84, 32x256x14x14 -> 256 108 and 94 (rows of 14 are read as 16), 32x64x55x55 -> 64 115 and 93
+// (transfers of four bytes). Of the 67 the products are 20, and the split's 70 vector instructions for 18 MFMAs as much beside them; addresses
+// of transfers take 9, the ranges' sums and their results 7, the reduction 6.
+// Errors against fp64, 2-norm, fp32 instruction and split: 32x64x56x56 -> 64 2.7e-7 and 2.4e-7, 32x32x112x112 -> 32 2.7e-7 and
+// 2.6e-7, 32x256x14x14 -> 256 2.5e-7 and 2.3e-7. The bf16 instruction loses the low bits of what it adds in one direction, which
+// 2048 partial sums add up to 6.2e-7 in the second of these: every other wavefront adds -dY X instead.
+#include "bf16_split.h"
+#include "conv_dense3_weight.hip"
+
+namespace dml {
+namespace {
+
+template <int I, int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        static_for<I + 1, N>(f);
+    }
+}
+
+struct Split {
+    static constexpr bool on = true;
+
+    // The products of a chunk: this wavefront's share of its pixels. a_row, x_row: LDS addresses of the lane's rows of dY and X.
+    template <int KG, typename Issue>
+    static __device__ __forceinline__ void chunk(const WeightArgs& g, floatx16 (&acc)[kTaps], uint32_t a_row, uint32_t x_row, int px, int kg,
+                                                 int half, float sign, Issue&& issue_next) {
+        // Sixteen pixels at a time: eight next to each other in a row for each lane half, a lane's fragment of dY. The ten
+        // values of X they meet in an image row serve three taps: as pairs of bf16 values tap 0 and tap 2 are the same
+        // registers one pair apart, tap 1 is shifted by half a register. Reads run one image row ahead and are waited for
+        // behind the products they run beside.
+        const int g8 = (g.ow + 7) / 8, groups = px / g.ow * g8, steps = (groups + 1) / 2;
+        const float inv_g8 = 1.0f / (float)g8;
+        uint32_t aa, xa;
+        int nv;
+        auto locate = [&](int i) {
+            const int gi = 2 * i + half, gc = min(gi, groups - 1), r = fast_div(gc, g8, inv_g8), ox = 8 * (gc - r * g8);
+            aa = a_row + (uint32_t)((r * g.ow + ox) * 4);
+            xa = x_row + (uint32_t)((r * g.pwid + ox + g.col0) * 4);
+            nv = gi < groups ? min(8, g.ow - ox) : 0;
+        };
+        float ra[8], rb[10];
+        auto read_a = [&] {
+            static_for<0, 8>([&](auto e) { ra[e.value] = lds_read_b32<4 * e.value>(aa); });
+        };
+        auto read_x = [&](int hy) {
+            const uint32_t at = xa + (uint32_t)(hy * g.pwid * 4);
+            static_for<0, 10>([&](auto e) { rb[e.value] = lds_read_b32<4 * e.value>(at); });
+        };
+        auto settle = [&] {
+            __builtin_amdgcn_sched_barrier(0);
+            wait_lgkm<0>();
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) lds_keep(ra[e]);
+#pragma unroll
+            for (int e = 0; e < 10; ++e) lds_keep(rb[e]);
+        };
+        if (kg < steps) {
+            locate(kg);
+            read_a();
+            read_x(0);
+            settle();
+            for (int i = kg; i < steps; i += KG) {
+                const int valid = nv;
+                const bool partial = __builtin_amdgcn_ballot_w64(valid < 8) != 0;
+                if (partial)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) ra[e] = e < valid ? ra[e] : 0.f;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) ra[e] *= sign;
+                const Pieces pa = split_eight(ra);
+                static_for<0, 3>([&](auto hyc) {
+                    constexpr int hy = hyc.value;
+                    if (partial)    // what lies behind the row: any bits
+#pragma unroll
+                        for (int e = 2; e < 10; ++e) rb[e] = e < valid + 2 ? rb[e] : 0.f;
+                    uint32_t ph[5], pm[5], pl[5];
+#pragma unroll
+                    for (int e = 0; e < 5; ++e) split_pair(floatx2{rb[2 * e], rb[2 * e + 1]}, ph[e], pm[e], pl[e]);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if constexpr (hy == 2) {
+                        locate(min(i + KG, steps - 1));
+                        read_a();
+                        read_x(0);
+                    } else {
+                        read_x(hy + 1);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    Pieces pb[3];
+                    auto taps = [&](bf16x8 Pieces::*part, const uint32_t (&v)[5]) {
+                        u32x4 t1;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) t1[e] = __builtin_amdgcn_alignbit(v[e + 1], v[e], 16);
+                        pb[0].*part = __builtin_bit_cast(bf16x8, u32x4{v[0], v[1], v[2], v[3]});
+                        pb[1].*part = __builtin_bit_cast(bf16x8, t1);
+                        pb[2].*part = __builtin_bit_cast(bf16x8, u32x4{v[1], v[2], v[3], v[4]});
+                    };
+                    taps(&Pieces::h, ph);
+                    taps(&Pieces::m, pm);
+                    taps(&Pieces::l, pl);
+                    mfma_split(pa, pb, acc + 3 * hy);
+                    issue_next();
+                    settle();
+                });
+            }
+        }
+    }
+
+    // The sums once more where they are not finite. m, c: the lane's rows of dY and X.
+    template <int KG, typename ChunkAt>
+    static __device__ __forceinline__ void repair(const WeightArgs& g, floatx16 (&acc)[kTaps], ChunkAt&& chunk_at, int first_row, int row_end,
+                                                  int m, int c, int kg, int half, float sign) {
+        // A value without a split (infinite, NaN, above the largest bf16) makes a sum NaN: this wavefront's pixels once more, in fp32
+        float bad = 0.f;
+#pragma unroll
+        for (int t = 0; t < kTaps; ++t)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) bad = __builtin_fmaf(acc[t][e], 0.f, bad);
+        if (__builtin_amdgcn_ballot_w64(bad != 0.f) != 0) {
+#pragma unroll
+            for (int t = 0; t < kTaps; ++t)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) acc[t][e] = 0.f;
+            const bool has_m = m < g.m, has_c = c < g.c;
+            const int ohw = g.oh * g.ow, in_plane = g.h * g.w;
+            const int g8 = (g.ow + 7) / 8;
+            for (int r0 = first_row; r0 < row_end;) {
+                const Chunk ch = chunk_at(r0);
+                const int groups = ch.px / g.ow * g8, steps = (groups + 1) / 2;
+                for (int i = kg; i < steps; i += KG) {
+                    const int gi = 2 * i + half, r = gi / g8, ox0 = 8 * (gi - r * g8);
+                    for (int e = 0; e < 8; ++e) {
+                        const int oy = ch.oy + r, ox = ox0 + e;
+                        const bool ok = gi < groups && ox < g.ow;
+                        const float av = ok && has_m ? g.dy[((int64_t)ch.img * g.m + m) * ohw + oy * g.ow + ox] : 0.f;
+#pragma unroll
+                        for (int t = 0; t < kTaps; ++t) {
+                            const int iy = oy - g.ph + t / 3, ix = ox - g.pw + t % 3;
+                            const bool in = ok && has_c && iy >= 0 && iy < g.h && ix >= 0 && ix < g.w;
+                            const float bv = in ? g.x[((int64_t)ch.img * g.c + c) * in_plane + iy * g.w + ix] : 0.f;
+                            acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(av * sign, bv, acc[t], 0, 0, 0);
+                        }
+                    }
+                }
+                r0 += ch.px / g.ow;
+            }
+        }
+    }
+};
+
+template <int WM, int AVEC, int XVEC>
+__global__ __launch_bounds__(kThreads) void conv_dense3_weight_split_kernel(const WeightArgs g) {
+    weight_gradient<WM, AVEC, XVEC, Split>(g);
+}
+
+}  // namespace
+
+int launch_conv_dense3_weight(const ConvGeom& g, const float* x, const float* dy, float* part, hipStream_t st) {
+    constexpr size_t kReadPast = 64;      // the last pixels of a row are read in eights, past the end of what is staged
+    WeightPlan pl;
+    unsigned blocks;
+    int avec, xvec;
+    const bool split = g.sh == 1 && g.sw == 1 && g.dh == 1 && g.dw == 1 && plan_weight(g, x, dy, &pl, &blocks, &avec, &xvec) &&
+                       pl.lds + kReadPast <= (size_t)kLdsBytes;
+    if (!split) return launch_conv_dense3_bwd_weight(g, x, dy, part, st);
+    pl.lds += kReadPast;
+    pl.a.x = x; pl.a.dy = dy; pl.a.part = part;
+    const int wm = g.m > 32 ? 2 : 1;
+#define DML_D3W(WM, AV, XV) \
+    if (wm == WM && avec == AV && xvec == XV) return launch_weight(conv_dense3_weight_split_kernel<WM, AV, XV>, pl, blocks, st);
+    DML_D3W(1, 1, 1) DML_D3W(1, 1, 4) DML_D3W(1, 4, 1) DML_D3W(1, 4, 4)
+    DML_D3W(2, 1, 1) DML_D3W(2, 1, 4) DML_D3W(2, 4, 1) DML_D3W(2, 4, 4)
+#undef DML_D3W
+    return DMLHIP_ERR_UNSUPPORTED;
+}
+
+}  // namespace dml

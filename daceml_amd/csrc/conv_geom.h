@@ -28,6 +28,8 @@ int launch_conv_dense3_split_bwd_data_f32(const ConvGeom& g, const float* dy, co
 // conv_dense3_weight.hip: per-range results (m * c * 9 floats each) its weight gradient writes; 0 = does not apply, or the
 // general kernel, where that applies (`general`), is the faster one
 int64_t conv_dense3_bwd_weight_partials(const ConvGeom& g, bool general);
+// ... on the bf16 matrix instructions (conv_dense3_weight_split.hip) or the fp32 one
+int launch_conv_dense3_weight(const ConvGeom& g, const float* x, const float* dy, float* part, hipStream_t st);
 int launch_conv_dense3_bwd_weight(const ConvGeom& g, const float* x, const float* dy, float* part, hipStream_t st);
 
 // conv_depthwise.hip: depthwise 3 x 3 / 5 x 5, stride 1, output as large as the input
