@@ -257,7 +257,7 @@ __global__ __launch_bounds__(kThreads, 2) void conv_dense3_split_kernel(const Sp
     }
     // The activation in the loop is none or ReLU. The others are applied behind it to what was stored, in a loop that is not
     // unrolled: 16 P copies of them do not fit the instruction cache (P = 4: 12 us per tile for the stores alone).
-    const float least = g.act == DMLHIP_ACT_RELU ? 0.f : -__builtin_inff();
+    const bool relu = g.act == DMLHIP_ACT_RELU;
     float zero = 0.f;        // stays one if every sum is finite
 #pragma unroll
     for (int j = 0; j < P; ++j) {
@@ -270,7 +270,8 @@ __global__ __launch_bounds__(kThreads, 2) void conv_dense3_split_kernel(const Sp
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
             const int r = (e >> 2) * 8 + (e & 3);
-            if (mw + r < g.m) out[(int64_t)r * ohw] = fmaxf(acc[j][e] + b[e], least);
+            const float v = acc[j][e] + b[e];       // NaN of a bias stays NaN but under ReLU
+            if (mw + r < g.m) out[(int64_t)r * ohw] = relu ? fmaxf(v, 0.f) : v;
         }
     }
     if (g.act != DMLHIP_ACT_NONE && g.act != DMLHIP_ACT_RELU) {

@@ -69,3 +69,20 @@ def test_values_without_a_split(tile, lib):
     finite = np.isfinite(want)
     assert finite[1, :, 7, 7].all()
     np.testing.assert_allclose(y[finite], want[finite], rtol=1e-5, atol=1e-4)
+
+
+@pytest.mark.parametrize("tile", [3, 4, 5])
+@pytest.mark.parametrize("act", ["NONE", "RELU", "SWISH", "SIGMOID", "GELU"])
+def test_biases_that_are_not_finite(act, tile, lib):
+    """NaN and both infinities give what the kernel on the fp32 instruction gives."""
+    from daceml_amd import _lib as L, kernels as K
+    r = rng(9)
+    x, wt = r.standard_normal((2, 16, 18, 20)).astype(np.float32), r.standard_normal((70, 16, 3, 3)).astype(np.float32)
+    b = r.standard_normal(70).astype(np.float32)
+    b[0], b[33], b[34], b[69], b[7] = np.nan, np.inf, -np.inf, np.nan, np.finfo(np.float32).max
+    y, want = (host(_forced(lib, t, lambda: K.conv2d(dev(x), dev(wt), dev(b), pads=(1, 1), act=getattr(L, "ACT_" + act)))) for t in (tile, 0))
+    for same in (np.isnan, np.isposinf, np.isneginf):
+        np.testing.assert_array_equal(same(y), same(want))
+    assert np.isnan(want[:, 0]).all() or act == "RELU"
+    finite = np.isfinite(want)
+    np.testing.assert_allclose(y[finite], want[finite], rtol=2e-5, atol=2e-5)
