@@ -19,8 +19,6 @@
 #include "bf16_split.h"
 #include "conv_geom.h"
 
-#include <float.h>
-
 #include <type_traits>
 
 namespace dml {
@@ -104,6 +102,19 @@ __global__ __launch_bounds__(kThreads, 2) void conv_dense3_split_kernel(const Sp
     // the rectangle. Buffer loads: byte offset of the chunk from channel 0 of the weights or of image n_first, kZeros (past the
     // end of either) where there is nothing to read. `late`: chunks of the upper eight channels of a step.
     const int in_plane = g.h * g.w_in;
+    // row and column of the padded image n_first + n, channel c
+    auto x_offset = [&](int n, int row, int col, int c) -> uint32_t {
+        int iy = row - g.ph, ix = col - g.pw;
+        bool ok = iy >= 0 && ix >= 0;
+        if (g.ids_h > 1 || g.ids_w > 1) {
+            const int qy = max(iy, 0) / g.ids_h, qx = max(ix, 0) / g.ids_w;
+            ok = ok && qy * g.ids_h == iy && qx * g.ids_w == ix;
+            iy = qy;
+            ix = qx;
+        }
+        ok = ok && iy < g.h && ix < g.w_in;
+        return ok ? (uint32_t)((n * g.c + c) * in_plane + iy * g.w_in + ix) * 4 : kZeros;
+    };
     const int wstep = (FLIP ? g.m : 1) * kTaps;        // elements from one channel to the next
     uint32_t off[TASKS], late = 0;
 #pragma unroll
@@ -118,18 +129,8 @@ __global__ __launch_bounds__(kThreads, 2) void conv_dense3_split_kernel(const Sp
             const int task = first + lane - kWTasks;
             kh = fast_div(task, g.rect, inv_rect);
             const int pos = task - kh * g.rect, row = fast_div(pos, g.pwid, inv_pwid);
-            int ix = pos - row * g.pwid - g.pw;
             const int n = fast_div(r_first + row, g.img_rows, inv_rows);
-            int iy = r_first + row - n * g.img_rows - g.ph;
-            bool ok = kh < 2 && n_first + n < g.n && iy >= 0 && ix >= 0;
-            if (g.ids_h > 1 || g.ids_w > 1) {
-                const int qy = max(iy, 0) / g.ids_h, qx = max(ix, 0) / g.ids_w;
-                ok = ok && qy * g.ids_h == iy && qx * g.ids_w == ix;
-                iy = qy;
-                ix = qx;
-            }
-            ok = ok && iy < g.h && ix < g.w_in;
-            off[u] = ok ? (uint32_t)((n * g.c + 8 * kh) * in_plane + iy * g.w_in + ix) * 4 : kZeros;
+            off[u] = kh < 2 && n_first + n < g.n ? x_offset(n, r_first + row - n * g.img_rows, pos - row * g.pwid, 8 * kh) : kZeros;
         }
         late |= kh == 1 ? 1u << u : 0u;
     }
@@ -247,8 +248,58 @@ __global__ __launch_bounds__(kThreads, 2) void conv_dense3_split_kernel(const Sp
     step(0, std::false_type{});
     if constexpr (P == 1) acc[0] += low;
 
+    // What follows finds its pixels again: addresses kept from the start would be registers that the loop does not have.
+    int tid = threadIdx.x, pixels = ohw;
+    asm volatile("" : "+v"(tid), "+s"(pixels));
+    const int row32 = tid & 31, upper = tid >> 5 & 1;
+    const float inv_pixels = 1.0f / (float)pixels;
+    const int first = p0 + wp * P * 32 + row32;         // this lane's pixel of block 0
+
+    // A value without a split (infinite, NaN, above the largest bf16) makes a sum that is not finite: this wavefront's sums once more,
+    // on the fp32 instruction (32x64x56x56 -> 64 with NaN in one pixel / everywhere: one such product 12.0 / 10.5 ms when every lane did
+    // its sums one after the other).
+    float bad = 0.f;
+#pragma unroll
+    for (int j = 0; j < P; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) bad = __builtin_fmaf(acc[j][e], 0.f, bad);
+    if (__builtin_amdgcn_ballot_w64(bad != 0.f) != 0) {
+#pragma unroll
+        for (int j = 0; j < P; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[j][e] = 0.f;
+        const int m = m0 + wm * 32 + row32;
+#pragma unroll 1
+        for (int tap = 0; tap < kTaps; ++tap) {
+            // of channel `upper`: the instruction takes two, one per lane half
+            const uint32_t woff = m < g.m ? (uint32_t)(weight_at<FLIP>(g, m, upper, tap) * 4) : kZeros;
+            uint32_t xoff[P];
+#pragma unroll
+            for (int j = 0; j < P; ++j) {
+                const int q0 = min(first + j * 32, g.total_px - 1) - n_first * pixels;
+                const int n = fast_div(q0, pixels, inv_pixels), q = q0 - n * pixels, oy = q / g.ow;
+                xoff[j] = x_offset(n, oy * g.sh + tap / 3 * g.dh, (q - oy * g.ow) * g.sw + tap % 3 * g.dw, upper);
+            }
+#pragma unroll 1
+            for (int c = 0; c < g.c; c += 8) {      // channels come in eights
+                float a[4], b[4][P];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    a[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(wbuf, woff, (c + 2 * i) * wstep * 4, 0));
+#pragma unroll
+                    for (int j = 0; j < P; ++j)
+                        b[i][j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xbuf, xoff[j], (c + 2 * i) * in_plane * 4, 0));
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int j = 0; j < P; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[i][j], acc[j], 0, 0, 0);
+            }
+        }
+    }
+
     // element e of a block: row (e / 4) * 8 + (lane / 32) * 4 + e % 4, column lane % 32
-    const int mw = m0 + wm * 32 + half * 4;
+    const int mw = m0 + wm * 32 + upper * 4;
     float b[16];
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
@@ -258,53 +309,30 @@ __global__ __launch_bounds__(kThreads, 2) void conv_dense3_split_kernel(const Sp
     // The activation in the loop is none or ReLU. The others are applied behind it to what was stored, in a loop that is not
     // unrolled: 16 P copies of them do not fit the instruction cache (P = 4: 12 us per tile for the stores alone).
     const bool relu = g.act == DMLHIP_ACT_RELU;
-    float zero = 0.f;        // stays one if every sum is finite
 #pragma unroll
     for (int j = 0; j < P; ++j) {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) zero += acc[j][e] * 0.f;
-        const int p = p0 + (wp * P + j) * 32 + l32;
+        const int p = first + j * 32;
         if (p >= g.total_px) continue;
-        const int n = fast_div(p - n_first * ohw, ohw, inv_ohw), q = p - (n_first + n) * ohw;
-        float* const out = g.y + ((int64_t)(n_first + n) * g.m + mw) * ohw + q;
+        const int n = fast_div(p - n_first * pixels, pixels, inv_pixels), q = p - (n_first + n) * pixels;
+        float* const out = g.y + ((int64_t)(n_first + n) * g.m + mw) * pixels + q;
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
             const int r = (e >> 2) * 8 + (e & 3);
             const float v = acc[j][e] + b[e];       // NaN of a bias stays NaN but under ReLU
-            if (mw + r < g.m) out[(int64_t)r * ohw] = relu ? fmaxf(v, 0.f) : v;
+            if (mw + r < g.m) out[(int64_t)r * pixels] = relu ? fmaxf(v, 0.f) : v;
         }
     }
     if (g.act != DMLHIP_ACT_NONE && g.act != DMLHIP_ACT_RELU) {
         for (int j = 0; j < P; ++j) {
-            const int p = p0 + (wp * P + j) * 32 + l32;
+            const int p = first + j * 32;
             if (p >= g.total_px) continue;
-            const int n = p / ohw, q = p - n * ohw;
-            float* const out = g.y + ((int64_t)n * g.m + mw) * ohw + q;
+            const int n = p / pixels, q = p - n * pixels;
+            float* const out = g.y + ((int64_t)n * g.m + mw) * pixels + q;
 #pragma unroll 1
             for (int e = 0; e < 16; ++e) {
                 const int r = (e >> 2) * 8 + (e & 3);
-                if (mw + r < g.m) out[(int64_t)r * ohw] = apply_act(g.act, out[(int64_t)r * ohw]);
+                if (mw + r < g.m) out[(int64_t)r * pixels] = apply_act(g.act, out[(int64_t)r * pixels]);
             }
-        }
-    }
-    if (zero == 0.f) return;
-    // This lane has a sum that is not finite: its pixels again, from the fp32 values.
-    for (int j = 0; j < P; ++j) {
-        const int p = p0 + (wp * P + j) * 32 + l32;
-        if (p >= g.total_px) continue;
-        const int n = p / ohw, q = p - n * ohw, oy = q / g.ow, ox = q - oy * g.ow;
-        for (int e = 0; e < 16; ++e) {
-            const int m = mw + (e >> 2) * 8 + (e & 3);
-            if (m >= g.m) continue;
-            float s = 0.f;
-            for (int c = 0; c < g.c; ++c)
-                for (int tap = 0; tap < kTaps; ++tap) {
-                    const int iy = oy * g.sh - g.ph + tap / 3 * g.dh, ix = ox * g.sw - g.pw + tap % 3 * g.dw;
-                    const bool in = iy >= 0 && ix >= 0 && iy % g.ids_h == 0 && ix % g.ids_w == 0 && iy / g.ids_h < g.h && ix / g.ids_w < g.w_in;
-                    const float v = in ? g.x[((int64_t)n * g.c + c) * in_plane + (int64_t)(iy / g.ids_h) * g.w_in + ix / g.ids_w] : 0.f;
-                    s = __builtin_fmaf(g.w[weight_at<FLIP>(g, m, c, tap)], v, s);     // the padding's zeros too
-                }
-            g.y[((int64_t)n * g.m + m) * ohw + q] = apply_act(g.act, s + (g.bias ? g.bias[m] : 0.f));
         }
     }
 }

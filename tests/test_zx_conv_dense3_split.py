@@ -9,7 +9,7 @@ import torch
 import torch.nn.functional as F
 
 from tests.test_zx_conv_dense3 import _check, _problem
-from tests.util import dev, host, rng
+from tests.util import dev, host, launch_us, rng
 
 pytestmark = pytest.mark.gpu
 
@@ -86,3 +86,36 @@ def test_biases_that_are_not_finite(act, tile, lib):
     assert np.isnan(want[:, 0]).all() or act == "RELU"
     finite = np.isfinite(want)
     np.testing.assert_allclose(y[finite], want[finite], rtol=2e-5, atol=2e-5)
+
+
+@pytest.mark.parametrize("shape", [SHAPES[2], SHAPES[3], SHAPES[4], SHAPES[6], SHAPES[8]])
+def test_values_without_a_split_in_every_geometry(shape, lib):
+    """Strides, dilation, padding, both directions: NaN and infinities where the kernel on the fp32 instruction has them. The infinities
+    are one of a kind, since the two kernels add in different orders."""
+    from daceml_amd import kernels as K
+    n, c, h, w, m, s, p, d = shape
+    x, wt, b, dy, _, _ = _problem(shape)
+    for t in (x, dy):
+        t[0, 3, 1, 1], t[-1, 4, -1, -1] = np.inf, np.nan
+    wt[1, 5, 0, 2] = -np.inf
+    def run(tile):
+        y = _forced(lib, tile, lambda: K.conv2d(dev(x), dev(wt), dev(b), (s, s), (p, p), (d, d)))
+        return y, _forced(lib, tile, lambda: K.conv2d_backward(dev(x), dev(wt), dev(dy), (s, s), (p, p), (d, d), need_dw=False)[0])
+    want = [host(t) for t in run(0)]
+    for tile in (3, 4, 5):
+        for got, ref, k in zip(map(host, run(tile)), want, (9 * c, 9 * m)):
+            for same in (np.isnan, np.isposinf, np.isneginf):
+                np.testing.assert_array_equal(same(got), same(ref))
+            finite = np.isfinite(ref)
+            # two sums of k terms of order one, k roundings of at most 2^-24 of partial sums of about sqrt(k) each
+            np.testing.assert_allclose(got[finite], ref[finite], rtol=1e-5, atol=2 * k * 2.0 ** -24 * k ** 0.5)
+
+
+@pytest.mark.parametrize("everywhere", [False, True])
+def test_time_with_nan(everywhere):
+    """2.8 times what finite operands take at most (it was 200); the bound leaves room for a busy machine."""
+    from daceml_amd import kernels as K
+    x, wt = torch.randn(16, 64, 56, 56, device="cuda"), torch.randn(64, 64, 3, 3, device="cuda")
+    finite = launch_us(lambda: K.conv2d(x, wt, pads=(1, 1)))
+    x[(slice(None) if everywhere else 0), 5, 9, 9] = float("nan")
+    assert launch_us(lambda: K.conv2d(x, wt, pads=(1, 1))) < 10 * finite

@@ -41,3 +41,17 @@ def assert_close(got, want, dtype, what="", rtol=None, atol=None):
         a_here = float(np.broadcast_to(np.asarray(atol, dtype=np.float64), err.shape)[i])   # atol may be per element
         raise AssertionError("%s: %d / %d elements out of tolerance (rtol=%g atol=%g); worst at %s: got %r want %r"
                              % (what, bad.sum(), bad.size, rtol, a_here, i, got[i], want[i]))
+
+
+def launch_us(run, launches=20):
+    """Time of one of several calls in a row, the best of three rows."""
+    best = float("inf")
+    for _ in range(4):
+        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        start.record()
+        for _ in range(launches):
+            run()
+        end.record()
+        end.synchronize()
+        best = min(best, start.elapsed_time(end) / launches * 1e3)
+    return best
