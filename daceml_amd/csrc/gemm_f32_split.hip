@@ -1,8 +1,8 @@
 // fp32 strided batched GEMM on the bf16 matrix cores: the entry point of the fp32 products and the kernel behind most of them.
 //
 // Operands are split into three bf16 values each (bf16_split.h has what that costs and keeps); K is cut into four or eight chains
-// on top: 1024 x 768 x 768 is 1.5e-7 from the fp64 product where the streamed tiles are 2.5e-7 - 5.0e-7. An element that comes
-// out not finite is computed again, as a chain of fp32 multiply-adds.
+// on top: 1024 x 768 x 768 is 1.5e-7 from the fp64 product where the streamed tiles are 2.5e-7 - 5.0e-7. A wavefront whose sums
+// come out not finite computes them again on the fp32 instruction.
 //
 // What bounds it: vector issue beside the matrix pipe. A wavefront's 64 x 64 tile is 24 MFMAs per 16 k (0.36 us) and 176
 // instructions that split the operands; on a compute unit with eight wavefronts a step takes 0.57 us per wavefront and SIMD. So the
@@ -12,8 +12,6 @@
 // 4096^3 1016 / 715 - 760 = 181 - 192 TFLOP/s, where the fp32 instruction's own limit is 157.
 #include "bf16_split.h"
 #include "lds_ops.h"
-
-#include <float.h>
 
 #include <type_traits>
 
@@ -88,6 +86,8 @@ struct Operand {
         if constexpr (ROWS == 0) return ((lane & 3) ^ ((lane >> 3) & 3)) * 4;    // row i * 16 + lane / 4: (row / 2) % 4
         return i * 4 + (lane >> 4);
     }
+    // tile row of row j of block b
+    static __device__ __forceinline__ int row_of(int b, int j) { return ROWS == 0 ? 32 * b + j : 2 * j + b; }
     __device__ __forceinline__ void issue(const float* p, char* stage) const {
 #pragma unroll
         for (int i = 0; i < N; ++i) dma(reinterpret_cast<const char*>(p) + off[i], stage + i * 1024);
@@ -120,6 +120,28 @@ struct Operand {
                 constexpr int e = decltype(ec)::value;
                 v.p[e] = lds_read_b64<e * kBlock * 4>(faddr + stage);
             });
+        }
+    }
+    // the same from global memory, 16 or 8 bytes at a time; k0: first k of the step, zeros from k on
+    static __device__ __forceinline__ void values(const float* p, int64_t s_row, int64_t s_k, int rows_left, int k0, int k, int lane,
+                                                  float (&v)[2][8]) {
+        const int j = lane & 31, first = k0 + 8 * (lane >> 5);
+        if constexpr (ROWS == 0) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int at = first + i % 2 * 4, row = min(32 * (i / 2) + j, rows_left - 1);
+                const floatx4 q = *reinterpret_cast<const floatx4*>(p + row * s_row + min(at, k - 4));
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[i / 2][i % 2 * 4 + e] = at < k ? q[e] : 0.f;
+            }
+        } else {
+            p += min(2 * j, rows_left - 2);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const floatx2 q = *reinterpret_cast<const floatx2*>(p + min(first + e, k - 1) * s_k);
+#pragma unroll
+                for (int i = 0; i < 2; ++i) v[i][e] = first + e < k ? q[i] : 0.f;
+            }
         }
     }
     template <int B>
@@ -315,6 +337,36 @@ __global__ __launch_bounds__(kWave * KG, 2) void gemm_f32_split_kernel(const Spl
             step(t, c0{}, c1{});
         }
         step(mine - 1, c1{}, c0{});
+
+        // A value without a split (infinite, NaN, above the largest bf16) makes a sum that is not finite: this wavefront's steps once
+        // more, on the fp32 instruction, operands from global memory.
+        float bad = 0.f;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) bad = __builtin_fmaf(acc[i][j][e], 0.f, bad);
+        if (__builtin_amdgcn_ballot_w64(bad != 0.f) != 0) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+#pragma unroll 1
+            for (int s = wave; s < steps; s += KG) {
+                float va[2][8], vb[2][8];
+                OA::values(A + (int64_t)m0 * g.sam, g.sam, g.sak, g.m - m0, s * BK, g.k, lane, va);
+                OB::values(B + (int64_t)n0 * g.sbn, g.sbn, g.sbk, g.n - n0, s * BK, g.k, lane, vb);
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+#pragma unroll
+                        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(va[i][e], vb[j][e], acc[i][j], 0, 0, 0);
+            }
+        }
     }
     __syncthreads();                     // the rings are done with
 
@@ -329,7 +381,7 @@ __global__ __launch_bounds__(kWave * KG, 2) void gemm_f32_split_kernel(const Spl
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
                 const int r = (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
-                float* const row = own + (AROWS ? 2 * r + i : 32 * i + r) * PITCH;
+                float* const row = own + OA::row_of(i, r) * PITCH;
                 const float v0 = acc[i][0][e], v1 = acc[i][1][e];
                 if constexpr (BROWS) {
                     *reinterpret_cast<floatx2*>(row + 2 * (lane & 31)) = floatx2{v0, v1};
@@ -349,15 +401,6 @@ __global__ __launch_bounds__(kWave * KG, 2) void gemm_f32_split_kernel(const Spl
 #pragma unroll
         for (int s = 1; s < KG; ++s) v += *reinterpret_cast<const floatx4*>(part + (s * kBlock + r) * PITCH + c4);
         const int cnt = min(4, g.n - n);
-        const float* ar = A + (int64_t)m * g.sam;
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-            if (e < cnt && !(fabsf(v[e]) <= FLT_MAX)) {
-                const float* bc = B + (int64_t)(n + e) * g.sbn;
-                float s = 0.f;
-                for (int k = 0; k < g.k; ++k) s = __builtin_fmaf(ar[k * g.sak], bc[k * g.sbk], s);
-                v[e] = s;
-            }
         const int64_t off = coff + (int64_t)m * g.scm + n;
         const float bm = g.bias && g.bias_m ? bias_at(g, m) : 0.f;
         floatx4 out;

@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 import torch
 
-from tests.util import dev, host, rng
+from tests.util import dev, host, launch_us, rng
 
 pytestmark = pytest.mark.gpu
 
@@ -72,3 +72,37 @@ def test_values_without_a_split(form, lib):
     finite = np.isfinite(want)
     assert finite[20, 20] and finite[21, 0]
     np.testing.assert_allclose(got[finite], want[finite], rtol=1e-5, atol=1e-4)
+
+
+@pytest.mark.parametrize("form", [3, 4])
+@pytest.mark.parametrize("b_rows", ["k", "n"])
+@pytest.mark.parametrize("a_rows", ["k", "m"])
+def test_values_without_a_split_in_every_layout(form, a_rows, b_rows, lib):
+    """Rows that end inside a tile and a K that ends inside a step, both ways of reading an operand."""
+    r, (m, n, k) = rng(6), (76, 132, 148)
+    a, b = r.standard_normal((m, k)).astype(np.float32), r.standard_normal((n, k)).astype(np.float32)
+    a[3, 7], a[75, 147], a[40, 99], b[131, 16], b[64, 145] = np.inf, np.inf, np.nan, np.nan, -np.inf
+    a[20, :] = 0.0
+    a[20, 130], b[:, 130] = np.finfo(np.float32).max, 0.25
+    c = torch.full((m, n), float("nan"), device="cuda")
+    ta, tb = (dev(t if rows == "k" else np.ascontiguousarray(t.T)) for t, rows in ((a, a_rows), (b, b_rows)))
+    _product(lib, form, m, n, k, 1, ta, tb, (k, 1) if a_rows == "k" else (1, m), (k, 1) if b_rows == "k" else (1, n), c)
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = (a.astype(np.float64) @ b.astype(np.float64).T).astype(np.float32)
+    got = host(c)
+    for same in (np.isnan, np.isposinf, np.isneginf):
+        np.testing.assert_array_equal(same(got), same(want))
+    finite = np.isfinite(want)
+    assert finite[20, 0]
+    np.testing.assert_allclose(got[finite], want[finite], rtol=1e-5, atol=1e-4)
+
+
+@pytest.mark.parametrize("everywhere", [False, True])
+def test_time_with_nan(everywhere, lib):
+    """2.5 times what finite operands take at most (it was 137); the bound leaves room for a busy machine."""
+    m, n, k = 1024, 768, 3072
+    a, b, c = torch.randn(m, k, device="cuda"), torch.randn(n, k, device="cuda"), torch.empty((m, n), device="cuda")
+    run = lambda: _product(lib, 3, m, n, k, 1, a, b, (k, 1), (k, 1), c)  # noqa: E731
+    finite = launch_us(run)
+    a[slice(None) if everywhere else 5, 5] = float("nan")
+    assert launch_us(run) < 10 * finite
