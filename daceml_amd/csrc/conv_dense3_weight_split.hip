@@ -129,23 +129,32 @@ struct Split {
             const bool has_m = m < g.m, has_c = c < g.c;
             const int ohw = g.oh * g.ow, in_plane = g.h * g.w;
             const int g8 = (g.ow + 7) / 8;
+            auto at = [](bool there, const float* p) { return *(there ? p : reinterpret_cast<const float*>(&g_zeros)); };   // no branches
             for (int r0 = first_row; r0 < row_end;) {
                 const Chunk ch = chunk_at(r0);
                 const int groups = ch.px / g.ow * g8, steps = (groups + 1) / 2;
                 for (int i = kg; i < steps; i += KG) {
                     const int gi = 2 * i + half, r = gi / g8, ox0 = 8 * (gi - r * g8);
-                    for (int e = 0; e < 8; ++e) {
-                        const int oy = ch.oy + r, ox = ox0 + e;
-                        const bool ok = gi < groups && ox < g.ow;
-                        const float av = ok && has_m ? g.dy[((int64_t)ch.img * g.m + m) * ohw + oy * g.ow + ox] : 0.f;
+                    const int oy = ch.oy + r;
+                    float av[8], xv[3][10];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        av[e] = at(gi < groups && ox0 + e < g.ow && has_m, g.dy + ((int64_t)ch.img * g.m + m) * ohw + oy * g.ow + ox0 + e) * sign;
+#pragma unroll
+                    for (int hy = 0; hy < 3; ++hy)
+#pragma unroll
+                        for (int e = 0; e < 10; ++e) {
+                            const int iy = oy - g.ph + hy, ix = ox0 - g.pw + e;
+                            const bool in = gi < groups && ox0 + e < g.ow + 2 && has_c && iy >= 0 && iy < g.h && ix >= 0 && ix < g.w;
+                            xv[hy][e] = at(in, g.x + ((int64_t)ch.img * g.c + c) * in_plane + iy * g.w + ix);
+                        }
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
 #pragma unroll
                         for (int t = 0; t < kTaps; ++t) {
-                            const int iy = oy - g.ph + t / 3, ix = ox - g.pw + t % 3;
-                            const bool in = ok && has_c && iy >= 0 && iy < g.h && ix >= 0 && ix < g.w;
-                            const float bv = in ? g.x[((int64_t)ch.img * g.c + c) * in_plane + iy * g.w + ix] : 0.f;
-                            acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(av * sign, bv, acc[t], 0, 0, 0);
+                            const float bv = ox0 + e < g.ow ? xv[t / 3][e + t % 3] : 0.f;
+                            acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[e], bv, acc[t], 0, 0, 0);
                         }
-                    }
                 }
                 r0 += ch.px / g.ow;
             }
