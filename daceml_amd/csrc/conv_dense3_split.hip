@@ -255,7 +255,7 @@ __global__ __launch_bounds__(kThreads, 2) void conv_dense3_split_kernel(const Sp
     const float inv_pixels = 1.0f / (float)pixels;
     const int first = p0 + wp * P * 32 + row32;         // this lane's pixel of block 0
 
-    // A value without a split (infinite, NaN, above the largest bf16) makes a sum that is not finite: this wavefront's sums once more,
+    // A value without a split (infinite, NaN, from 2^112 on) makes a sum that is not finite: this wavefront's sums once more,
     // on the fp32 instruction (32x64x56x56 -> 64 with NaN in one pixel / everywhere: one such product 12.0 / 10.5 ms when every lane did
     // its sums one after the other).
     float bad = 0.f;
@@ -296,6 +296,11 @@ __global__ __launch_bounds__(kThreads, 2) void conv_dense3_split_kernel(const Sp
                     for (int j = 0; j < P; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[i][j], acc[j], 0, 0, 0);
             }
         }
+    } else {
+#pragma unroll
+        for (int j = 0; j < P; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[j][e] *= kSplitBack;
     }
 
     // element e of a block: row (e / 4) * 8 + (lane / 32) * 4 + e % 4, column lane % 32

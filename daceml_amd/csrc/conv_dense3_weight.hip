@@ -207,7 +207,9 @@ __device__ __forceinline__ void weight_gradient(const WeightArgs& g) {
     }
     wait_vm_lgkm0<0>();
 
-    if constexpr (SPLIT::on) SPLIT::template repair<KG>(g, acc, chunk_at, first_row, row_end, m0 + wm * 32 + l32, c0 + l32, kg, half, sign);
+    float back = 1.f;
+    if constexpr (SPLIT::on)
+        back = SPLIT::template repair<KG>(g, acc, chunk_at, first_row, row_end, m0 + wm * 32 + l32, c0 + l32, kg, half, sign);
 
     // Eight rows of every block at a time: element e of a block is row (e / 4) * 8 + (lane / 32) * 4 + e % 4, column
     // lane % 32. The wavefronts' sums of a row are added and its 288 values written next to each other, as dW has them.
@@ -222,7 +224,7 @@ __device__ __forceinline__ void weight_gradient(const WeightArgs& g) {
         for (int t = 0; t < kTaps; ++t)
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                sums[(wave * 8 + half * 4 + e) * ROW + l32 * kTaps + t] = SPLIT::on ? acc[t][eg * 4 + e] * sign : acc[t][eg * 4 + e];
+                sums[(wave * 8 + half * 4 + e) * ROW + l32 * kTaps + t] = SPLIT::on ? acc[t][eg * 4 + e] * back : acc[t][eg * 4 + e];
         __syncthreads();
         // wavefront `wave` adds row `wave` of every block
         const int m = m0 + eg * 8 + wave;

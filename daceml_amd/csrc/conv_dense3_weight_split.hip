@@ -3,7 +3,7 @@
 //
 // Measured, us with the reduction, fp32 instruction and split: 32x64x56x56 -> 64 92 and 67, -> 128 165 and 112, 32x128x28x28 -> 128 91
 // and 67, 32x96x40x40 -> 96 129 and 84, 32x256x14x14 -> 256 108 and 94 (rows of 14 are read as 16), 32x64x55x55 -> 64 115 and 93
-// (transfers of four bytes). Of the 67 the products are 20, and the split's 70 vector instructions for 18 MFMAs as much beside them; addresses
+// (transfers of four bytes). Of the 67 the products are 20, and the split's 80 vector instructions for 18 MFMAs as much beside them; addresses
 // of transfers take 9, the ranges' sums and their results 7, the reduction 6.
 // Errors against fp64, 2-norm, fp32 instruction and split: 32x64x56x56 -> 64 2.7e-7 and 2.4e-7, 32x32x112x112 -> 32 2.7e-7 and
 // 2.6e-7, 32x256x14x14 -> 256 2.5e-7 and 2.3e-7. The bf16 instruction loses the low bits of what it adds in one direction, which
@@ -71,9 +71,7 @@ struct Split {
                 if (partial)
 #pragma unroll
                     for (int e = 0; e < 8; ++e) ra[e] = e < valid ? ra[e] : 0.f;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) ra[e] *= sign;
-                const Pieces pa = split_eight(ra);
+                const Pieces pa = split_eight(ra, kSplitScale * sign);
                 static_for<0, 3>([&](auto hyc) {
                     constexpr int hy = hyc.value;
                     if (partial)    // what lies behind the row: any bits
@@ -81,7 +79,7 @@ struct Split {
                         for (int e = 2; e < 10; ++e) rb[e] = e < valid + 2 ? rb[e] : 0.f;
                     uint32_t ph[5], pm[5], pl[5];
 #pragma unroll
-                    for (int e = 0; e < 5; ++e) split_pair(floatx2{rb[2 * e], rb[2 * e + 1]}, ph[e], pm[e], pl[e]);
+                    for (int e = 0; e < 5; ++e) split_pair(floatx2{rb[2 * e], rb[2 * e + 1]}, kSplitScale, ph[e], pm[e], pl[e]);
                     __builtin_amdgcn_sched_barrier(0);
                     if constexpr (hy == 2) {
                         locate(min(i + KG, steps - 1));
@@ -111,17 +109,18 @@ struct Split {
         }
     }
 
-    // The sums once more where they are not finite. m, c: the lane's rows of dY and X.
+    // The sums once more where they are not finite. m, c: the lane's rows of dY and X. Returns what gives the sums their size and sign.
     template <int KG, typename ChunkAt>
-    static __device__ __forceinline__ void repair(const WeightArgs& g, floatx16 (&acc)[kTaps], ChunkAt&& chunk_at, int first_row, int row_end,
+    static __device__ __forceinline__ float repair(const WeightArgs& g, floatx16 (&acc)[kTaps], ChunkAt&& chunk_at, int first_row, int row_end,
                                                   int m, int c, int kg, int half, float sign) {
-        // A value without a split (infinite, NaN, above the largest bf16) makes a sum NaN: this wavefront's pixels once more, in fp32
+        // A value without a split (infinite, NaN, from 2^112 on) makes a sum that is not finite: this wavefront's pixels once more, in fp32
         float bad = 0.f;
 #pragma unroll
         for (int t = 0; t < kTaps; ++t)
 #pragma unroll
             for (int e = 0; e < 16; ++e) bad = __builtin_fmaf(acc[t][e], 0.f, bad);
-        if (__builtin_amdgcn_ballot_w64(bad != 0.f) != 0) {
+        const bool again = __builtin_amdgcn_ballot_w64(bad != 0.f) != 0;
+        if (again) {
 #pragma unroll
             for (int t = 0; t < kTaps; ++t)
 #pragma unroll
@@ -159,6 +158,7 @@ struct Split {
                 r0 += ch.px / g.ow;
             }
         }
+        return again ? sign : sign * kSplitBack;
     }
 };
 

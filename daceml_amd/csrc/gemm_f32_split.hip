@@ -177,7 +177,7 @@ __device__ __forceinline__ void interleave() {
 #pragma unroll
     for (int i = 0; i < 12; ++i) {
         __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x2, 8, 0);
+        __builtin_amdgcn_sched_group_barrier(0x2, 9, 0);
     }
 }
 
@@ -338,7 +338,7 @@ __global__ __launch_bounds__(kWave * KG, 2) void gemm_f32_split_kernel(const Spl
         }
         step(mine - 1, c1{}, c0{});
 
-        // A value without a split (infinite, NaN, above the largest bf16) makes a sum that is not finite: this wavefront's steps once
+        // A value without a split (infinite, NaN, from 2^112 on) makes a sum that is not finite: this wavefront's steps once
         // more, on the fp32 instruction, operands from global memory.
         float bad = 0.f;
 #pragma unroll
@@ -366,6 +366,13 @@ __global__ __launch_bounds__(kWave * KG, 2) void gemm_f32_split_kernel(const Spl
 #pragma unroll
                         for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(va[i][e], vb[j][e], acc[i][j], 0, 0, 0);
             }
+        } else {
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) acc[i][j][e] *= kSplitBack;
         }
     }
     __syncthreads();                     // the rings are done with

@@ -119,3 +119,17 @@ def test_time_with_nan(everywhere):
     finite = launch_us(lambda: K.conv2d(x, wt, pads=(1, 1)))
     x[(slice(None) if everywhere else 0), 5, 9, 9] = float("nan")
     assert launch_us(lambda: K.conv2d(x, wt, pads=(1, 1))) < 10 * finite
+
+
+@pytest.mark.parametrize("tile", [3, 4, 5])
+@pytest.mark.parametrize("exponent", [-112, -120, -128, -140])
+def test_operands_of_every_size(exponent, tile, lib):
+    """Operands around and below the smallest normal value keep all of their bits: relative 2-norm error as for any others."""
+    from daceml_amd import kernels as K
+    r = rng(11)
+    for small in (0, 1):
+        x, wt = r.standard_normal((2, 16, 24, 20)), r.standard_normal((64, 16, 3, 3))
+        x, wt = ((t * 2.0 ** (exponent if i == small else 100)).astype(np.float32) for i, t in enumerate((x, wt)))
+        y = _forced(lib, tile, lambda: K.conv2d(dev(x), dev(wt), pads=(1, 1)))
+        exact = F.conv2d(torch.from_numpy(x).double(), torch.from_numpy(wt).double(), None, 1, 1).numpy()
+        assert np.linalg.norm(host(y) - exact) < 3e-7 * np.linalg.norm(exact)

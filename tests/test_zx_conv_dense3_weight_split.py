@@ -51,3 +51,16 @@ def test_values_without_a_split(shape):
     np.testing.assert_allclose(got[20, 9], want32[20, 9], rtol=1e-5)
     finite = np.isfinite(want32[:, 0])
     np.testing.assert_allclose(got[:, 0][finite], want32[:, 0][finite], rtol=1e-4, atol=2e-3)
+
+
+@pytest.mark.parametrize("exponent", [-112, -120, -128, -140])
+def test_operands_of_every_size(exponent):
+    """Operands around and below the smallest normal value keep all of their bits: relative 2-norm error as for any others."""
+    r, shape = rng(11), SHAPES[9]
+    n, c, h, w, m, s, p, d = shape
+    for small in (0, 1):
+        x, dy = r.standard_normal((n, c, h, w)), r.standard_normal((n, m, h, w))
+        x, dy = ((t * 2.0 ** (exponent if i == small else 100)).astype(np.float32) for i, t in enumerate((x, dy)))
+        got = host(_weight_gradient(x, dy, shape))
+        exact = torch.nn.grad.conv2d_weight(torch.from_numpy(x).double(), (m, c, 3, 3), torch.from_numpy(dy).double(), s, p).numpy()
+        assert np.linalg.norm(got - exact) < 3e-7 * np.linalg.norm(exact)
