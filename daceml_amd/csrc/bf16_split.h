@@ -5,10 +5,13 @@
 // the factor operands below 2^-110 lose their last bits: a product of operands around 2^-120 was 3.5e-5 from the exact one.) Sums are of
 // 2^32 times their size. Of the nine products of two such sums six matter: h h, h m, m h, m m, h l, l h (the others are below
 // 2^-26 of the product, under the rounding of the sum). The bf16 matrix rate is 16 times the fp32 one, so six products take 0.375
-// of the time of the fp32 instruction, and 8 products share a rounding of the fp32 accumulator where that instruction rounds
-// every one. Error against the fp64 product, 2-norm over 2-norm, in one chain of K here / there: N(0, 1) K = 64 1.1e-7 / 1.4e-7,
-// 768 4.2e-7 / 5.0e-7, 3072 8.5e-7 / 9.7e-7; uniform on [0, 1) 768 2.9e-7 / 4.2e-7; log-normal over twelve decades 768 1.7e-7 /
-// 2.4e-7. Infinities, NaN and values from 2^112 on have no such sum: a result that comes out not finite (or above 2^96) has to be
+// of the time of the fp32 instruction, and 8 products share a rounding of the fp32 accumulator where that instruction rounds every
+// two. That makes 12 roundings for sixteen products, more than it has where operands are zero, unless the five small products have a sum
+// of their own (mfma_small): 2, and the small sum's are 2^-8 of their size. Error against fp64, 2-norm over 2-norm, one such pair of sums here
+// / one sum on the fp32 instruction: 576 products of N(0, 1) 1.4e-7 / 4.3e-7, one operand behind a ReLU 1.0e-7 / 3.0e-7, uniform on [0, 1)
+// 1.3e-7 / 3.6e-7; 9216 products 5.9e-7 / 1.7e-6, 5.1e-7 / 1.2e-6, 5.0e-7 / 1.4e-6. (All six products in one sum: behind a ReLU 3.4e-7 and
+// 1.4e-6.)
+// Infinities, NaN and values from 2^112 on have no such sum: a result that comes out not finite (or above 2^96) has to be
 // computed again from the fp32 values.
 #pragma once
 
@@ -69,14 +72,16 @@ __device__ __forceinline__ void mfma_split(const Pieces& a, const Pieces (&b)[N]
     DML_PRODUCT(h, h)
 #undef DML_PRODUCT
 }
-// One block: two sums, the second one for half of the small products
-__device__ __forceinline__ void mfma_split2(const Pieces& a, const Pieces& b, floatx16& acc, floatx16& low) {
+// Five of the six products, each at most 2^-8 of the sixth, and the sixth
+__device__ __forceinline__ floatx16 mfma_small(const Pieces& a, const Pieces& b, floatx16 low) {
     low = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.l, b.h, low, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.m, b.h, acc, 0, 0, 0);
     low = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.h, b.l, low, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.h, b.m, acc, 0, 0, 0);
     low = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.m, b.m, low, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.h, b.h, acc, 0, 0, 0);
+    low = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.m, b.h, low, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.h, b.m, low, 0, 0, 0);
+}
+__device__ __forceinline__ floatx16 mfma_large(const Pieces& a, const Pieces& b, floatx16 acc) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.h, b.h, acc, 0, 0, 0);
 }
 
 }  // namespace dml

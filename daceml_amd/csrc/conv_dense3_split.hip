@@ -12,10 +12,15 @@
 // the loads of the chunks beside them (1 us per step: 8 loads of 4 bytes per lane for a chunk; with the loads left out P = 4 takes
 // 7.3 us, P = 1 2.5 of 3.2), 0.5 us for the stores to LDS and the barriers, and per tile 5 us of first loads and 3 - 9 us of
 // results, which one workgroup per compute unit does not hide. Measured, us forward / data gradient, the kernel of
-// conv_dense3.hip and here: 32x64x56x56 -> 64 92 / 86 and 56 / 55, 32x64x56x56 -> 128 148 / 153 and 105 / 91, 32x128x28x28 -> 128
-// 85 / 84 and 66 / 64 (54 / 52 with P = 4, see the rule at the launch), 32x256x14x14 -> 256 107 / 104 and 59 / 56. What the products waited for until it was changed: 64 copies of the
-// activation in the epilogue (12 us per tile), loads behind branches (their addresses in 64 registers, 2 us per step), MFMAs
-// of one block in a row (0.4 us).
+// conv_dense3.hip and here: 32x64x56x56 -> 64 82 / 80 and 58 / 57, 32x64x56x56 -> 128 144 / 150 and 112 / 100, 32x128x28x28 -> 128
+// 84 / 83 and 65 / 63, 32x256x14x14 -> 256 107 / 105 and 58 / 56. What the products waited for until it was changed: 64 copies of the
+// activation in the epilogue (12 us per tile), loads behind branches (their addresses in 64 registers, 2 us per step).
+//
+// The large product h h has a sum of its own (P = 1: two), so that the roundings of the five small ones are not roundings of the
+// result: 2 of these for sixteen products instead of 12. Error against fp64 as a share of that of the fp32 instruction (one sum for P = 2 and
+// 4, two for P = 1; 16 - 2048 channels; with all six products in one sum in brackets): normal operands 0.31 - 0.41 (0.83 - 0.87), X
+// behind a ReLU 0.34 - 0.52 (1.08 - 1.20), nothing negative 0.27 - 0.62 (0.9 - 1.7). P = 4 has registers for the small products of one tap only
+// and adds them tap by tap: 51 -> 57 us at 32x64x56x56 -> 64, P = 1 and 2 take the same time as before.
 #include "bf16_split.h"
 #include "conv_geom.h"
 
@@ -169,9 +174,16 @@ __global__ __launch_bounds__(kThreads, 2) void conv_dense3_split_kernel(const Sp
     for (int j = 0; j < P; ++j)
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[j][e] = 0.f;
-    floatx16 low;                                              // P = 1: the second sum of the only block
+    floatx16 odd;                                              // P = 1: a second sum, of the odd taps
 #pragma unroll
-    for (int e = 0; e < 16; ++e) low[e] = 0.f;
+    for (int e = 0; e < 16; ++e) odd[e] = 0.f;
+    // Sums of the small products: P = 1 and 2 keep them to the end, P = 4 has registers for those of one tap and adds them to acc.
+    constexpr int LOW = P < 4 ? P : 1;
+    floatx16 low[LOW];
+#pragma unroll
+    for (int j = 0; j < LOW; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) low[j][e] = 0.f;
 
     auto weights_at = [&](int tap) -> Pieces {
         const char* const p = lds + waddr + tap * 16;
@@ -183,38 +195,36 @@ __global__ __launch_bounds__(kThreads, 2) void conv_dense3_split_kernel(const Sp
         return {*reinterpret_cast<const bf16x8*>(p), *reinterpret_cast<const bf16x8*>(p + xplane),
                 *reinterpret_cast<const bf16x8*>(p + 2 * xplane)};
     };
-    // The products of a step. Fragments are read one group of blocks ahead; SPLIT: the chunks of the next step are split under the
-    // products. With few products per step their values are loaded a step ahead, as soon as the registers are free (at the start
-    // of the step that splits them, 1 us of it was a wait); with many, when the step begins, and are split under the last taps.
-    constexpr bool AHEAD = P < 4;
+    // The products of a step. Fragments are read one block ahead; SPLIT: the chunks of the next step are split under the
+    // products. Where registers allow, their values are loaded a step ahead, as soon as the registers are free (at the start
+    // of the step that splits them, 1 us of it was a wait); elsewhere when the step begins, and are split under the last taps.
+    constexpr bool AHEAD = P < 4 && TASKS < 7;
     constexpr int FIRST = kTaps - TASKS;
     auto step = [&](int next, auto split_c) {                  // next: first channel of the chunks that are loaded
         constexpr bool SPLIT = decltype(split_c)::value;
-        constexpr int G = P == 1 ? 1 : 2, GROUPS = P / G;      // blocks multiplied in turns
-        Pieces a[2], b[2][G];
-        auto group_at = [&](int i, Pieces(&f)[G]) {            // group i of the step
-#pragma unroll
-            for (int j = 0; j < G; ++j) f[j] = pixels_at(i % GROUPS * G + j, i / GROUPS);
-        };
+        Pieces a[2], b[2];
         a[0] = weights_at(0);
-        group_at(0, b[0]);
+        b[0] = pixels_at(0, 0);
         static_for<0, kTaps>([&](auto tc) {
             constexpr int tap = decltype(tc)::value, u = tap - FIRST;
             __builtin_amdgcn_sched_barrier(0);
-            static_for<0, GROUPS>([&](auto jc) {
-                constexpr int j = decltype(jc)::value, i = tap * GROUPS + j;
-                if constexpr (i + 1 < kTaps * GROUPS) {
-                    if constexpr (j + 1 == GROUPS) a[(tap + 1) & 1] = weights_at(tap + 1);
-                    group_at(i + 1, b[(i + 1) & 1]);
+            static_for<0, P>([&](auto jc) {
+                constexpr int j = decltype(jc)::value, i = tap * P + j;
+                if constexpr (i + 1 < kTaps * P) {
+                    if constexpr (j + 1 == P) a[(tap + 1) & 1] = weights_at(tap + 1);
+                    b[(i + 1) & 1] = pixels_at((i + 1) % P, (i + 1) / P);
                 }
-                if constexpr (P == 1) mfma_split2(a[tap & 1], b[i & 1][0], acc[0], low);
-                else mfma_split(a[tap & 1], b[i & 1], acc + j * G);
+                if constexpr (P == 1 && tap % 2) odd = mfma_large(a[tap & 1], b[i & 1], odd);
+                else acc[j] = mfma_large(a[tap & 1], b[i & 1], acc[j]);
+                if constexpr (P < 4) low[j] = mfma_small(a[tap & 1], b[i & 1], low[j]);
+                else acc[j] += mfma_small(a[tap & 1], b[i & 1], floatx16{});
+                if constexpr (P == 4) asm volatile("" : "+v"(acc[j]));
             });
             if constexpr (SPLIT && u >= 0) pieces[u] = split_eight(raw[u]);
 #pragma unroll
             for (int i = 0; i < 6 * P; ++i) {       // a matrix instruction, then what can issue under it
                 __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x2, P == 4 ? 2 : 9 / P, 0);
+                __builtin_amdgcn_sched_group_barrier(0x2, P == 4 ? 5 : 9 / P, 0);
             }
             if constexpr (SPLIT && u >= 0) {
                 asm volatile("" : "+v"(pieces[u].h), "+v"(pieces[u].m), "+v"(pieces[u].l));   // computed here, not at the stores
@@ -246,7 +256,11 @@ __global__ __launch_bounds__(kThreads, 2) void conv_dense3_split_kernel(const Sp
         __syncthreads();
     }
     step(0, std::false_type{});
-    if constexpr (P == 1) acc[0] += low;
+    if constexpr (P == 1) acc[0] += odd;
+    if constexpr (P < 4) {
+#pragma unroll
+        for (int j = 0; j < P; ++j) acc[j] += low[j];
+    }
 
     // What follows finds its pixels again: addresses kept from the start would be registers that the loop does not have.
     int tid = threadIdx.x, pixels = ohw;
@@ -394,9 +408,9 @@ static bool plan_split(const ConvGeom& g, int ids_h, int ids_w, int most_p, Spli
         if (blocks > (1LL << 22)) continue;
         const double steps = (double)ceil_div(g.c, (int64_t)kCh), rounds = (double)ceil_div(blocks, (int64_t)kCus);
         // us of a tile: first loads and results, and per step; whole rounds of one tile per compute unit. Rounds decide: 32x64x56x56 ->
-        // 64 is one round of 196 tiles of 512 pixels (51 us), two of 392 (58) or four (95), 32x256x14x14 -> 256 one of 196 tiles of 128
-        // (61; of 256 83, of 512 150).
-        const double t = rounds * (p == 1 ? 7.0 + 3.4 * steps : p == 2 ? 9.0 + 4.9 * steps : 11.0 + 9.0 * steps);
+        // 64 is one round of 196 tiles of 512 pixels (57 us), two of 392 (58) or four (92), 32x256x14x14 -> 256 one of 196 tiles of 128
+        // (58; of 256 81, of 512 178), 32x96x40x40 -> 96 one of 200 tiles of 512 (77) or two of 400 (74).
+        const double t = rounds * (p == 1 ? 7.0 + 3.4 * steps : p == 2 ? 9.0 + 4.9 * steps : 15.0 + 10.3 * steps);
         if (pl->p > 0 && t >= *us) continue;
         *us = t;
         pl->p = p;
@@ -415,9 +429,8 @@ static int launch_split(const ConvGeom& g, int ids_h, int ids_w, bool flip, cons
                         hipStream_t st, const char* what, bool* applies) {
     SplitPlan3 pl;
     double us;
-    // The error of a sum grows with the root of its roundings: 54 for 16 channels in one sum (P = 2, 4), 27 in two (P = 1), on the fp32
-    // instruction 72, 36 or 18 in one, two or four. Where that kernel would take two, only P = 1 is as exact (2.5e-7 where it has 3.0e-7,
-    // 64 channels; 3.6e-7 with P = 4), where four, none.
+    // No larger errors than the kernel on the fp32 instruction would have, whatever the operands. P = 2 and 4 have 0.37 - 0.62 of those of its
+    // one sum, up to 1.01 and 1.23 of those of two (nothing negative), P = 1 0.27 - 0.53 of those of two; of four none is as exact everywhere.
     int chains = 1;
     double other = 0;
     if (g_force_p == 0) {
