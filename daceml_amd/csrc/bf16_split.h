@@ -58,20 +58,6 @@ __device__ __forceinline__ Pieces split_eight(const float (&v)[8], float scale =
     return {__builtin_bit_cast(bf16x8, h), __builtin_bit_cast(bf16x8, m), __builtin_bit_cast(bf16x8, l)};
 }
 
-// The six products of one set of pieces with N others, in order of size so that the large ones round the sums last. The N sums
-// take turns: an MFMA that waits for the one before it holds up the vector instructions behind it too.
-template <int N>
-__device__ __forceinline__ void mfma_split(const Pieces& a, const Pieces (&b)[N], floatx16* acc) {
-#define DML_PRODUCT(AP, BP) \
-    _Pragma("unroll") for (int i = 0; i < N; ++i) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.AP, b[i].BP, acc[i], 0, 0, 0);
-    DML_PRODUCT(l, h)
-    DML_PRODUCT(h, l)
-    DML_PRODUCT(m, m)
-    DML_PRODUCT(m, h)
-    DML_PRODUCT(h, m)
-    DML_PRODUCT(h, h)
-#undef DML_PRODUCT
-}
 // Five of the six products, each at most 2^-8 of the sixth, and the sixth
 __device__ __forceinline__ floatx16 mfma_small(const Pieces& a, const Pieces& b, floatx16 low) {
     low = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.l, b.h, low, 0, 0, 0);

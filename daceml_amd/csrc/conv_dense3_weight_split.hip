@@ -1,13 +1,16 @@
 // Weight gradient of a dense (group 1) 3 x 3 convolution, stride and dilation 1, fp32, on the bf16 matrix instructions: operands
 // split into three bf16 values each (bf16_split.h), in the frame of conv_dense3_weight.hip.
 //
-// Measured, us with the reduction, fp32 instruction and split: 32x64x56x56 -> 64 92 and 67, -> 128 165 and 112, 32x128x28x28 -> 128 91
-// and 67, 32x96x40x40 -> 96 129 and 84, 32x256x14x14 -> 256 108 and 94 (rows of 14 are read as 16), 32x64x55x55 -> 64 115 and 93
-// (transfers of four bytes). Of the 67 the products are 20, and the split's 80 vector instructions for 18 MFMAs as much beside them; addresses
-// of transfers take 9, the ranges' sums and their results 7, the reduction 6.
-// Errors against fp64, 2-norm, fp32 instruction and split: 32x64x56x56 -> 64 2.7e-7 and 2.4e-7, 32x32x112x112 -> 32 2.7e-7 and
-// 2.6e-7, 32x256x14x14 -> 256 2.5e-7 and 2.3e-7. The bf16 instruction loses the low bits of what it adds in one direction, which
-// 2048 partial sums add up to 6.2e-7 in the second of these: every other wavefront adds -dY X instead.
+// Measured, us with the reduction, fp32 instruction and split: 32x64x56x56 -> 64 86 and 71, -> 128 156 and 125, 32x128x28x28 -> 128 86
+// and 72, 32x96x40x40 -> 96 125 and 91, 32x256x14x14 -> 256 107 and 104 (rows of 14 are read as 16), 32x64x55x55 -> 64 110 and 99
+// (transfers of four bytes). Of the 71 the products are 20, and the split's 80 vector instructions for 18 MFMAs as much beside them; the 48 that
+// add the small products take 5, addresses of transfers 9, the ranges' sums and their results 7, the reduction 6.
+// The five small products of a tap and sixteen pixels have a sum of their own, which is added to the tap's: 3 roundings of that instead of 12.
+// Errors against fp64, 2-norm, fp32 instruction and split (all products in one sum in brackets): 32x64x56x56 -> 64, normal operands, 2.7e-7 and
+// 1.3e-7 (2.3e-7), X behind a ReLU 2.1e-7 and 1.3e-7 (2.3e-7), both 5.6e-8 and 2.9e-8 (3.0e-8); 32x128x28x28 -> 256 3.5e-7 and 1.6e-7 (3.2e-7),
+// 2.5e-7 and 1.4e-7 (3.0e-7), 4.0e-8 and 3.9e-8 (4.5e-8); 32x256x14x14 -> 256 2.5e-7 and 1.2e-7, 1.8e-7 and 1.1e-7, 4.2e-8 and 4.0e-8. The bf16
+// instruction loses the low bits of what it adds in one direction, which 2048 partial sums add up to twice the error: every other
+// wavefront adds -dY X instead.
 #include "bf16_split.h"
 #include "conv_dense3_weight.hip"
 
@@ -89,19 +92,22 @@ struct Split {
                         read_x(hy + 1);
                     }
                     __builtin_amdgcn_sched_barrier(0);
-                    Pieces pb[3];
-                    auto taps = [&](bf16x8 Pieces::*part, const uint32_t (&v)[5]) {
-                        u32x4 t1;
+                    // tap 0 and 2 are the same registers, one pair apart; tap 1 lies half a register further on
+                    auto fragment = [&](auto tc, const uint32_t (&v)[5]) {
+                        constexpr int t = tc.value;
+                        u32x4 f;
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) t1[e] = __builtin_amdgcn_alignbit(v[e + 1], v[e], 16);
-                        pb[0].*part = __builtin_bit_cast(bf16x8, u32x4{v[0], v[1], v[2], v[3]});
-                        pb[1].*part = __builtin_bit_cast(bf16x8, t1);
-                        pb[2].*part = __builtin_bit_cast(bf16x8, u32x4{v[1], v[2], v[3], v[4]});
+                        for (int e = 0; e < 4; ++e) f[e] = t == 1 ? __builtin_amdgcn_alignbit(v[e + 1], v[e], 16) : v[e + t / 2];
+                        return __builtin_bit_cast(bf16x8, f);
                     };
-                    taps(&Pieces::h, ph);
-                    taps(&Pieces::m, pm);
-                    taps(&Pieces::l, pl);
-                    mfma_split(pa, pb, acc + 3 * hy);
+                    static_for<0, 3>([&](auto tc) {
+                        constexpr int tap = 3 * hy + tc.value;
+                        const Pieces pb = {fragment(tc, ph), fragment(tc, pm), fragment(tc, pl)};
+                        acc[tap] = mfma_large(pa, pb, acc[tap]);
+                        acc[tap] += mfma_small(pa, pb, floatx16{});
+                        asm volatile("" : "+v"(acc[tap]));      // added here, not where the next eights' sums are
+                        __builtin_amdgcn_sched_barrier(0);
+                    });
                     issue_next();
                     settle();
                 });
