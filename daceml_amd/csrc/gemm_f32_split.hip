@@ -1,15 +1,18 @@
 // fp32 strided batched GEMM on the bf16 matrix cores: the entry point of the fp32 products and the kernel behind most of them.
 //
 // Operands are split into three bf16 values each (bf16_split.h has what that costs and keeps); K is cut into four or eight chains
-// on top: 1024 x 768 x 768 is 1.5e-7 from the fp64 product where the streamed tiles are 2.5e-7 - 5.0e-7. A wavefront whose sums
-// come out not finite computes them again on the fp32 instruction.
+// on top: 1024 x 768 x 768 is 0.8e-7 from the fp64 product where the streamed tiles are 2.5e-7 - 5.0e-7. Behind a ReLU and where nothing is
+// negative errors are 0.08 - 0.67 of theirs, K of 256 - 65536. A wavefront whose sums come out not finite computes them again on the
+// fp32 instruction.
 //
-// What bounds it: vector issue beside the matrix pipe. A wavefront's 64 x 64 tile is 24 MFMAs per 16 k (0.36 us) and 176
+// What bounds it: vector issue beside the matrix pipe. A wavefront's 64 x 64 tile is 24 MFMAs per 16 k (0.36 us) and 208
 // instructions that split the operands; on a compute unit with eight wavefronts a step takes 0.57 us per wavefront and SIMD. So the
-// splitting of the next step is placed between the MFMAs of this one (all of it first, then the MFMAs: 0.8 us), and there is
-// one accumulator per block, not a second one for the small products (registers: 0.8 us again). Measured, us, the kernel of
-// gemm_f32.hip / here: 1024 x 768 x 768 20 / 14, 1024 x 3072 x 768 48 / 35, 3072 x 768 x 1024 (both operands row-contiguous) 59 / 39,
-// 4096^3 1016 / 715 - 760 = 181 - 192 TFLOP/s, where the fp32 instruction's own limit is 157.
+// splitting of the next step is placed between the MFMAs of this one (all of it first, then the MFMAs: 0.8 us). The sums of the large and
+// the small products, two sets of pieces and the values read ahead are 240 of 256 registers: transfers share one or two offsets per
+// operand, and the lane's number is found again where it is needed (four registers of offsets kept in scratch memory: 1024 x 768 x 3072 42.9 us
+// instead of 39.7). Measured, us, the kernel of gemm_f32.hip / here: 1024 x 768 x 768 20 / 16, 1024 x 3072 x 768 51 / 39, 1024 x 768 x 3072 52 / 40,
+// 3072 x 768 x 1024 (both operands row-contiguous) 59 / 43, 768 x 768 x 16384 (same) 244 / 148, 2048^3 136 / 115, 4096^3 1016 / 850. With all
+// products in one sum, 1.0 - 1.6 times the error of the fp32 instruction where operands are half zero, these take 1 - 7 % less (15, 38, 38, 42, 146, 112).
 #include "bf16_split.h"
 #include "lds_ops.h"
 
@@ -55,6 +58,13 @@ __device__ __forceinline__ void static_for(F&& f) {
     }
 }
 
+// The lane's number found again: a register less that the loop has to keep
+__device__ __forceinline__ int lane_again() {
+    uint32_t all = ~0u;
+    asm volatile("" : "+s"(all));
+    return (int)__builtin_amdgcn_mbcnt_hi(all, __builtin_amdgcn_mbcnt_lo(all, 0));
+}
+
 // what lanes outside the operand read
 __device__ const floatx4 g_zero_page = {0.f, 0.f, 0.f, 0.f};
 
@@ -65,17 +75,23 @@ __device__ const floatx4 g_zero_page = {0.f, 0.f, 0.f, 0.f};
 template <int ROWS>
 struct Operand {
     static constexpr int N = kBlock * BK / 256;      // transfers of a stage
-    uint32_t off[N];    // bytes
+    // bytes, the same for every transfer, `next` elements apart; ROWS = 0: sixteen rows each, off[1] from transfer `full` on, which has rows
+    // past the last one
+    uint32_t off[ROWS ? 1 : 2];
     uint32_t faddr;
+    int64_t next;
+    int full, last;
     __device__ __forceinline__ void init(int64_t s_row, int64_t s_k, int rows_left, int lane, uint32_t ring) {
+        if constexpr (ROWS == 0) {
+            next = 16 * s_row;
+            full = rows_left / 16;
+            last = (rows_left - 1) / 16;
 #pragma unroll
-        for (int i = 0; i < N; ++i) {
-            if constexpr (ROWS == 0) {
-                const int r = i * 16 + (lane >> 2);
-                off[i] = ((uint32_t)min(r, rows_left - 1) * (uint32_t)s_row + (uint32_t)k_of(i, lane)) * 4;
-            } else {
-                off[i] = ((uint32_t)k_of(i, lane) * (uint32_t)s_k + (uint32_t)min((lane & 15) * 4, rows_left - 4)) * 4;
-            }
+            for (int i = 0; i < 2; ++i)
+                off[i] = ((uint32_t)(i ? min(lane >> 2, (rows_left - 1) % 16) : lane >> 2) * (uint32_t)s_row + (uint32_t)k_of(0, lane)) * 4;
+        } else {
+            next = 4 * s_k;
+            off[0] = ((uint32_t)k_of(0, lane) * (uint32_t)s_k + (uint32_t)min((lane & 15) * 4, rows_left - 4)) * 4;
         }
         const int j = lane & 31, half = lane >> 5;
         if constexpr (ROWS == 0) faddr = ring + j * 64 + (((half * 2) ^ ((j >> 1) & 3)) << 4);
@@ -88,16 +104,20 @@ struct Operand {
     }
     // tile row of row j of block b
     static __device__ __forceinline__ int row_of(int b, int j) { return ROWS == 0 ? 32 * b + j : 2 * j + b; }
+    __device__ __forceinline__ const char* source(const float* p, int i) const {
+        if constexpr (ROWS == 0) return reinterpret_cast<const char*>(p + min(i, last) * next) + (i < full ? off[0] : off[1]);
+        else return reinterpret_cast<const char*>(p + i * next) + off[0];
+    }
     __device__ __forceinline__ void issue(const float* p, char* stage) const {
 #pragma unroll
-        for (int i = 0; i < N; ++i) dma(reinterpret_cast<const char*>(p) + off[i], stage + i * 1024);
+        for (int i = 0; i < N; ++i) dma(source(p, i), stage + i * 1024);
     }
     // the same for a stage that reaches past the end of K (`left` < 16)
-    __device__ __forceinline__ void issue_tail(const float* p, int left, char* stage, int lane) const {
+    __device__ __forceinline__ void issue_tail(const float* p, int left, char* stage) const {
+        const int lane = lane_again();
 #pragma unroll
         for (int i = 0; i < N; ++i)
-            dma(k_of(i, lane) < left ? reinterpret_cast<const char*>(p) + off[i] : reinterpret_cast<const char*>(&g_zero_page),
-                stage + i * 1024);
+            dma(k_of(i, lane) < left ? source(p, i) : reinterpret_cast<const char*>(&g_zero_page), stage + i * 1024);
     }
     static __device__ __forceinline__ void dma(const char* p, char* lds_dst) {
         __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)p,
@@ -144,12 +164,22 @@ struct Operand {
             }
         }
     }
-    template <int B>
-    static __device__ __forceinline__ Pieces block(const Raw& v) {
-        float w[8];
+    // both blocks' pieces, pair by pair: registers of values that are split are free
+    static __device__ __forceinline__ void split(const Raw& v, Pieces (&f)[2]) {
+        u32x4 h[2], m[2], l[2];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) w[e] = ROWS == 0 ? v.q[2 * B + e / 4][e % 4] : v.p[e][B];
-        return split_eight(w);
+        for (int i = 0; i < 8; ++i) {
+            const int blk = ROWS == 0 ? i / 4 : i % 2, e = ROWS == 0 ? i % 4 : i / 2;
+            const floatx2 w = ROWS == 0 ? floatx2{v.q[i / 2][2 * (i % 2)], v.q[i / 2][2 * (i % 2) + 1]} : floatx2{v.p[2 * e][blk], v.p[2 * e + 1][blk]};
+            uint32_t ph, pm, pl;
+            split_pair(w, kSplitScale, ph, pm, pl);
+            h[blk][e] = ph;
+            m[blk][e] = pm;
+            l[blk][e] = pl;
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            f[i] = {__builtin_bit_cast(bf16x8, h[i]), __builtin_bit_cast(bf16x8, m[i]), __builtin_bit_cast(bf16x8, l[i])};
     }
 };
 
@@ -241,8 +271,8 @@ __global__ __launch_bounds__(kWave * KG, 2) void gemm_f32_split_kernel(const Spl
             oa.issue(pa, at);
             ob.issue(pb, at + A_BYTES);
         } else {
-            oa.issue_tail(pa, left, at, lane);
-            ob.issue_tail(pb, left, at + A_BYTES, lane);
+            oa.issue_tail(pa, left, at);
+            ob.issue_tail(pb, left, at + A_BYTES);
         }
         pa += KG * BK * g.sak;
         pb += KG * BK * g.sbk;
@@ -252,27 +282,39 @@ __global__ __launch_bounds__(kWave * KG, 2) void gemm_f32_split_kernel(const Spl
         typename OA::Raw va;
         typename OB::Raw vb;
         Pieces fa[2][2], fb[2][2];
+        typedef std::integral_constant<int, 0> c0;
+        typedef std::integral_constant<int, 1> c1;
+        typedef std::integral_constant<int, 2> c2;
+        floatx16 low[2][2];              // sums of the small products
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) low[i][j][e] = 0.f;
         // Step t, whose pieces are in set CUR, while the values of step t + 1 are split into the other set: A's, read half a step
         // ago, then B's. Half way through every value of step t + 1 is in registers: its stage takes the transfers of step
-        // t + 3. LEFT: steps that follow (2 for more). Products in order of size, so that the large ones come last.
+        // t + 3. LEFT: steps that follow (2 for more).
         auto step = [&](int t, auto cur_c, auto left_c) {
             constexpr int CUR = decltype(cur_c)::value, NXT = CUR ^ 1, LEFT = decltype(left_c)::value;
             const uint32_t here = (uint32_t)((t & 1) * STAGE), other = STAGE - here;
             const Pieces(&a)[2] = fa[CUR];
             const Pieces(&b)[2] = fb[CUR];
-#define DML_PRODUCT(AP, BP)                                                                                               \
-    _Pragma("unroll") for (int i = 0; i < 2; ++i) _Pragma("unroll") for (int j = 0; j < 2; ++j)                           \
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i].AP, b[j].BP, acc[i][j], 0, 0, 0);
+            auto products = [&](auto ic) {            // of the two blocks in row I
+                constexpr int I = decltype(ic)::value;
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    low[I][j] = mfma_small(a[I], b[j], low[I][j]);
+                    acc[I][j] = mfma_large(a[I], b[j], acc[I][j]);
+                }
+            };
             if constexpr (LEFT > 0) {
                 wait_lgkm<0>();
                 ob.read(other, vb);
                 __builtin_amdgcn_sched_barrier(0);
-                fa[NXT][0] = OA::template block<0>(va);
-                fa[NXT][1] = OA::template block<1>(va);
+                OA::split(va, fa[NXT]);
             }
-            DML_PRODUCT(l, h)
-            DML_PRODUCT(h, l)
-            DML_PRODUCT(m, m)
+            products(c0{});
             if constexpr (LEFT > 0) {
                 interleave();
                 keep(fa[NXT]);
@@ -283,22 +325,15 @@ __global__ __launch_bounds__(kWave * KG, 2) void gemm_f32_split_kernel(const Spl
                     if (t + 3 < mine) issue(other);
                 }
                 __builtin_amdgcn_sched_barrier(0);
-                fb[NXT][0] = OB::template block<0>(vb);
-                fb[NXT][1] = OB::template block<1>(vb);
+                OB::split(vb, fb[NXT]);
             }
-            DML_PRODUCT(m, h)
-            DML_PRODUCT(h, m)
-            DML_PRODUCT(h, h)
+            products(c1{});
             if constexpr (LEFT > 0) {
                 interleave();
                 keep(fb[NXT]);
                 __builtin_amdgcn_sched_barrier(0);
             }
-#undef DML_PRODUCT
         };
-        typedef std::integral_constant<int, 0> c0;
-        typedef std::integral_constant<int, 1> c1;
-        typedef std::integral_constant<int, 2> c2;
         issue(0);
         if (mine > 1) {
             issue(STAGE);
@@ -314,15 +349,11 @@ __global__ __launch_bounds__(kWave * KG, 2) void gemm_f32_split_kernel(const Spl
         // the last step works from set 1, so the first one from set mine % 2
         const bool odd = mine & 1;
         if (odd) {
-            fa[1][0] = OA::template block<0>(va);
-            fa[1][1] = OA::template block<1>(va);
-            fb[1][0] = OB::template block<0>(vb);
-            fb[1][1] = OB::template block<1>(vb);
+            OA::split(va, fa[1]);
+            OB::split(vb, fb[1]);
         } else {
-            fa[0][0] = OA::template block<0>(va);
-            fa[0][1] = OA::template block<1>(va);
-            fb[0][0] = OB::template block<0>(vb);
-            fb[0][1] = OB::template block<1>(vb);
+            OA::split(va, fa[0]);
+            OB::split(vb, fb[0]);
         }
         if (mine > 1) {
             if (mine > 2) wait_vm_lgkm0<LPT>();
@@ -337,6 +368,10 @@ __global__ __launch_bounds__(kWave * KG, 2) void gemm_f32_split_kernel(const Spl
             step(t, c0{}, c1{});
         }
         step(mine - 1, c1{}, c0{});
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[i][j] += low[i][j];
 
         // A value without a split (infinite, NaN, from 2^112 on) makes a sum that is not finite: this wavefront's steps once
         // more, on the fp32 instruction, operands from global memory.
@@ -357,8 +392,8 @@ __global__ __launch_bounds__(kWave * KG, 2) void gemm_f32_split_kernel(const Spl
 #pragma unroll 1
             for (int s = wave; s < steps; s += KG) {
                 float va[2][8], vb[2][8];
-                OA::values(A + (int64_t)m0 * g.sam, g.sam, g.sak, g.m - m0, s * BK, g.k, lane, va);
-                OB::values(B + (int64_t)n0 * g.sbn, g.sbn, g.sbk, g.n - n0, s * BK, g.k, lane, vb);
+                OA::values(A + (int64_t)m0 * g.sam, g.sam, g.sak, g.m - m0, s * BK, g.k, lane_again(), va);
+                OB::values(B + (int64_t)n0 * g.sbn, g.sbn, g.sbk, g.n - n0, s * BK, g.k, lane_again(), vb);
 #pragma unroll
                 for (int e = 0; e < 8; ++e)
 #pragma unroll
@@ -376,6 +411,7 @@ __global__ __launch_bounds__(kWave * KG, 2) void gemm_f32_split_kernel(const Spl
         }
     }
     __syncthreads();                     // the rings are done with
+    const int at = lane_again();
 
     // The wavefronts' sums go through LDS: element e of a block is row (e / 4) * 8 + (lane / 32) * 4 + e % 4, column lane % 32.
     constexpr int PITCH = kBlock + 4;                 // floats; rows stay 16-byte aligned
@@ -387,20 +423,20 @@ __global__ __launch_bounds__(kWave * KG, 2) void gemm_f32_split_kernel(const Spl
         for (int i = 0; i < 2; ++i)
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
-                const int r = (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
+                const int r = (e >> 2) * 8 + (at >> 5) * 4 + (e & 3);
                 float* const row = own + OA::row_of(i, r) * PITCH;
                 const float v0 = acc[i][0][e], v1 = acc[i][1][e];
                 if constexpr (BROWS) {
-                    *reinterpret_cast<floatx2*>(row + 2 * (lane & 31)) = floatx2{v0, v1};
+                    *reinterpret_cast<floatx2*>(row + 2 * (at & 31)) = floatx2{v0, v1};
                 } else {
-                    row[lane & 31] = v0;
-                    row[32 + (lane & 31)] = v1;
+                    row[at & 31] = v0;
+                    row[32 + (at & 31)] = v1;
                 }
             }
     }
     __syncthreads();
     constexpr int CPR = kBlock / 4;                   // pieces of four columns per row
-    for (int i = threadIdx.x; i < kBlock * CPR; i += THREADS) {
+    for (int i = wave * kWave + at; i < kBlock * CPR; i += THREADS) {
         const int r = i / CPR, c4 = (i % CPR) * 4;
         const int m = m0 + r, n = n0 + c4;
         if (m >= g.m || n >= g.n) continue;

@@ -121,3 +121,29 @@ def test_operands_of_every_size(exponent, form, lib):
         _product(lib, form, m, n, k, 1, dev(a), dev(b), (k, 1), (k, 1), c)
         exact = a.astype(np.float64) @ b.astype(np.float64).T
         assert np.linalg.norm(host(c) - exact) < 3e-7 * np.linalg.norm(exact)
+
+
+@pytest.mark.parametrize("rows", ["k", "mn"])
+@pytest.mark.parametrize("k", [512, 4096, 16384])
+@pytest.mark.parametrize("kind", ["normal", "relu and masked", "both relu"])
+def test_no_less_exact_than_the_fp32_instruction(kind, k, rows, lib):
+    """Relative 2-norm error against fp64 beside that of the kernel on the fp32 instruction that cuts K into four sums, the most exact of them:
+    0.24 - 0.67 of it measured (0.84 at K = 512, where the result's own rounding is most of either), 1.06 - 1.5 with all products of the split in
+    one sum, half of either operand zero and a K of thousands."""
+    g = torch.Generator(device="cuda").manual_seed(k)
+    m, n = 128, 192
+    a, b = torch.randn(m, k, device="cuda", generator=g), torch.randn(n, k, device="cuda", generator=g)
+    if kind != "normal":
+        a = a.relu()
+        b = b.relu() if kind == "both relu" else b * (torch.rand(n, k, device="cuda", generator=g) < 0.5)
+    exact = a.double() @ b.double().T
+    if rows == "mn":
+        a, b = a.T.contiguous(), b.T.contiguous()
+
+    def error(form):
+        c = torch.full((m, n), float("nan"), device="cuda")
+        _product(lib, form, m, n, k, 1, a, b, (k, 1) if rows == "k" else (1, m), (k, 1) if rows == "k" else (1, n), c)
+        return ((c.double() - exact).norm() / exact.norm()).item()
+    other = error(2)
+    for form in (3, 4):
+        assert error(form) < 0.9 * other, (form, error(form), other)
