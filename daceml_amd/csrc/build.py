@@ -5,6 +5,7 @@ the sources so that it travels with the source tree; nothing is installed.
 """
 import concurrent.futures
 import os
+import re
 import shutil
 import subprocess
 import sys
@@ -65,14 +66,24 @@ def _compile(src: str) -> str:
     return obj
 
 
+def _includes(src: str) -> set:
+    """`src` and every file of this folder or of include/ that it includes, directly or not."""
+    found, todo = set(), [os.path.join(HERE, src)]
+    while todo:
+        path = os.path.normpath(todo.pop())
+        if path in found or not os.path.exists(path):
+            continue
+        found.add(path)
+        with open(path) as f:
+            for name in re.findall(r'^\s*#\s*include\s*"([^"]+)"', f.read(), re.M):
+                todo.append(os.path.join(os.path.dirname(path), name))
+    return found
+
+
 def _stale(src: str) -> bool:
-    """Is the object file of `src` older than the source or any header?"""
+    """Is the object file of `src` older than the source or anything it includes?"""
     obj = os.path.join(OBJ_DIR, os.path.splitext(src)[0] + ".o")
-    if not os.path.exists(obj):
-        return True
-    deps = [os.path.join(HERE, src)] + [os.path.join(HERE, f) for f in os.listdir(HERE) if f.endswith(".h")]
-    deps.append(os.path.join(HERE, "..", "..", "include", "daceml_hip.h"))
-    return os.path.getmtime(obj) < max(os.path.getmtime(d) for d in deps)
+    return not os.path.exists(obj) or os.path.getmtime(obj) < max(os.path.getmtime(d) for d in _includes(src))
 
 
 def build(force: bool = True, jobs: int = 8) -> str:
