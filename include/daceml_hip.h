@@ -281,7 +281,6 @@ size_t dmlhip_gemm_f16_workspace_bytes(const dmlhip_gemm_desc* desc);
 int dmlhip_gemm_f16_ws(const dmlhip_gemm_desc* desc, const void* a, const void* b, void* c,
                        const void* bias, const void* residual, void* pre_out, void* workspace,
                        size_t workspace_bytes, void* stream);
-/* inputs fp32, true fp32 MFMA (no reduced-precision path); out_dtype must be DMLHIP_F32 */
 /* Several products of identical shape, strides and epilogue (alpha, column bias) on different tensors in one
  * launch: groups <= DMLHIP_GROUP_MAX, tensor i uses a[i], b[i], c[i], bias[i] (bias may be NULL: none). This is
  * HorizontalEinsumFusion's purpose (daceml/transformation/einsum_fusion.py:102-151: the three Q/K/V projections of
@@ -311,6 +310,12 @@ int dmlhip_gemm_f16_grouped_asum(const dmlhip_gemm_desc* d, int groups, const vo
  * calls of dmlhip_gemm_f16 when one launch is not possible. */
 int dmlhip_gemm_f16_ksum(const dmlhip_gemm_desc* d, int groups, const void* const* a, const void* const* b,
                          void* c, const void* bias, const void* residual, void* stream);
+/* Inputs fp32, out_dtype must be DMLHIP_F32. Multiplies and adds at fp32 precision, on the fp32 matrix instruction or, where that is
+ * faster and the operands can be read 16 bytes at a time, on the bf16 one: every operand as the exact sum of three bf16 values, six of the
+ * nine products of their pairs (the others are below 2^-26 of the product), fp32 sums. The second is no further from the
+ * fp64 product than the first (2-norm; normal operands, operands of one sign, half of either or both zero). Infinities, NaN,
+ * the largest and subnormal values give on both what an fp32 sum gives. Dense 3x3 fp32 convolutions and their gradients (below)
+ * choose in the same way. */
 int dmlhip_gemm_f32(const dmlhip_gemm_desc* desc, const void* a, const void* b, void* c,
                     const void* bias, const void* residual, void* pre_out, void* stream);
 
