@@ -154,6 +154,7 @@ SIGNATURES = {
     "dmlhip_debug_gemm_f16_slices": (c_int, [POINTER(GemmDesc)]),
     "dmlhip_debug_force_gemm_f32_tile": (None, [c_int]),
     "dmlhip_debug_force_conv_dense3_tile": (None, [c_int]),
+    "dmlhip_debug_last_conv_form": (c_int, []),
     "dmlhip_debug_force_conv_depthwise": (None, [c_int]),
     "dmlhip_debug_conv_depthwise_strips": (c_int, [POINTER(Conv2dDesc), c_int]),
     "dmlhip_debug_gemm_direct_lds": (None, [c_int]),

@@ -445,6 +445,7 @@ static int launch_planned(const ConvGeom& g, int ids_h, int ids_w, bool flip, bo
     Dense3Plan pl;
     *applies = plan_conv_dense3(g, ids_h, ids_w, flip, general, x, w, &pl);
     if (!*applies) return 0;
+    note_conv_form(pl.tile);
     pl.a.x = x; pl.a.w = w; pl.a.bias = bias; pl.a.y = y;
 #define DML_D3(F, V, XV) \
     if (flip == F && pl.vec == V && pl.xvec == XV) return launch_form<F, V, XV>(pl, st, what);

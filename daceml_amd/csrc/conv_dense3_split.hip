@@ -370,6 +370,7 @@ int launch(const SplitPlan3& pl, hipStream_t st, const char* what) {
         set_error("%s: cannot reserve %zu bytes of LDS: %s", what, pl.lds, hipGetErrorString(e));
         return (int)e;
     }
+    note_conv_form((P == 1 ? 3 : P == 2 ? 4 : 5) + (TASKS == 7 ? 8 : 0));
     hipLaunchKernelGGL(kern, pl.a.blocks, kThreads, pl.lds, st, pl.a);
     return launch_status(what);
 }
@@ -381,6 +382,7 @@ int launch_form(const SplitPlan3& pl, hipStream_t st, const char* what) {
     return pl.tasks <= 6 ? launch<4, 6, FLIP>(pl, st, what) : launch<4, 7, FLIP>(pl, st, what);
 }
 
+thread_local int g_last_form = -1;   // diagnostic
 thread_local int g_force_p = 0;     // diagnostic: blocks of 32 pixels per wavefront (0 = chosen here); -1: not this kernel
 
 }  // namespace
@@ -457,7 +459,15 @@ int launch_conv_dense3_split_bwd_data_f32(const ConvGeom& g, const float* dy, co
     return launch_split(b, g.sh, g.sw, true, dy, w, nullptr, dx, st, "conv2d_backward_data(dense 3x3)", applies);
 }
 
+void note_conv_form(int form) { g_last_form = form; }
+
 }  // namespace dml
+
+extern "C" int dmlhip_debug_last_conv_form(void) {
+    const int form = dml::g_last_form;
+    dml::g_last_form = -1;
+    return form;
+}
 
 extern "C" void dmlhip_debug_force_conv_dense3_tile(int tile) {
     dml::g_force_p = tile < 0 ? 0 : tile < 3 ? -1 : 1 << (tile - 3);

@@ -217,6 +217,7 @@ int launch_columns(const ColArgs& a, int stride, const float* x, const float* we
     const bool swish = a.act1 == DMLHIP_ACT_SWISH && a.act2 == DMLHIP_ACT_SWISH;
     const auto kern = stride == 1 ? (swish ? expand_depthwise_columns_kernel<CHUNKS, 1, true> : expand_depthwise_columns_kernel<CHUNKS, 1, false>)
                                   : (swish ? expand_depthwise_columns_kernel<CHUNKS, 2, true> : expand_depthwise_columns_kernel<CHUNKS, 2, false>);
+    note_conv_form(16);
     hipLaunchKernelGGL(kern, a.blocks, kColWaves * 64, 0, st, x, we, be, wd, bd, y, a);
     return launch_status("conv2d_expand_depthwise");
 }

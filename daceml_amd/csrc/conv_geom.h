@@ -20,6 +20,7 @@ int launch_conv_dense3_f32(const ConvGeom& g, const float* x, const float* w, co
 int launch_conv_dense3_bwd_data_f32(const ConvGeom& g, const float* dy, const float* w, float* dx, hipStream_t st, bool* applies);
 // its estimate, < 0: does not apply; *chains: sums that it cuts the input channels into
 double conv_dense3_us(const ConvGeom& g, int ids_h, int ids_w, bool flip, const void* x, const void* w, int* chains);
+void note_conv_form(int form);             // diagnostic, this thread: what dmlhip_debug_last_conv_form returns
 void conv_dense3_force_tile(int tile);     // diagnostic, this thread: -1 = chosen per problem
 // conv_dense3_split.hip: the same problems on the bf16 matrix instructions, where that is faster
 int launch_conv_dense3_split_f32(const ConvGeom& g, const float* x, const float* w, const float* bias, float* y, hipStream_t st,

@@ -1,6 +1,6 @@
 """The dense 3 x 3 convolution and its data gradient on the bf16 matrix instructions (operands as three bf16 values each): tiles
-of 128, 256 and 512 pixels across rows and images, output channels that end inside a tile, a last step of eight channels, strides,
-dilation, wide padding, activations, values without a split.
+of 128, 256 and 512 pixels across rows and images, output channels that end inside a tile, a last step of eight channels, strides
+(forward with 128 pixels, larger rectangles do not fit), dilation, wide padding, activations, values without a split.
 
 Tolerance: that of the fp32 kernels' test; the products left out are below 3 * 2^-26 of |a| |b|, one of its two spare terms."""
 import numpy as np
@@ -16,25 +16,47 @@ pytestmark = pytest.mark.gpu
 # n, c, h, w, m, stride, pad, dilation
 SHAPES = [(3, 64, 56, 56, 64, 1, 1, 1), (5, 16, 31, 33, 72, 1, 1, 1), (9, 24, 14, 14, 136, 1, 1, 1), (4, 40, 27, 29, 64, 2, 1, 1),
           (2, 16, 30, 64, 96, 1, 2, 2), (3, 24, 33, 20, 32, 1, 0, 1), (20, 64, 14, 14, 64, 2, 1, 1), (1, 32, 112, 112, 32, 1, 1, 1),
-          (6, 256, 7, 7, 64, 1, 1, 1), (50, 16, 3, 5, 16, 1, 1, 1)]
+          (6, 256, 7, 7, 64, 1, 1, 1), (50, 16, 3, 5, 16, 1, 1, 1),
+          # large rectangles: 80 and 144 columns, dilation
+          (1, 16, 32, 80, 40, 1, 1, 1), (1, 24, 32, 80, 16, 1, 2, 2), (2, 16, 32, 16, 24, 1, 2, 2), (1, 16, 16, 144, 16, 1, 2, 2)]
+
+# What runs with each of the tiles 3, 4 and 5 asked for, forward and data gradient: 11 - 13 are their forms for large rectangles; where a
+# rectangle does not fit LDS the kernel on the fp32 instruction (0 - 2) or the general one (-1) takes the problem.
+FORMS = [((11, 4, 5), (11, 4, 5)), ((3, 4, 5), (3, 4, 5)), ((3, 4, 5), (3, 4, 5)), ((11, 2, 2), (3, 4, 5)), ((11, 12, 2), (11, 12, 2)),
+         ((3, 4, 5), (3, 4, 5)), ((11, 2, 2), (3, 4, 5)), ((11, 4, 2), (11, 4, 2)), ((3, 4, 5), (3, 4, 5)), ((3, 4, -1), (3, 4, -1)),
+         ((3, 4, 5), (3, 4, 5)), ((11, 12, 13), (11, 12, 13)), ((3, 4, 5), (3, 4, 5)), ((11, 12, -1), (11, 12, -1))]
 
 
-def _forced(lib, tile, run):
+def test_every_form_has_a_shape():
+    for direction in (0, 1):
+        assert {f for forms in FORMS for f in forms[direction]} >= {3, 4, 5, 11, 12, 13}
+    assert len(FORMS) == len(SHAPES)
+
+
+def _forced(lib, tile, run, takes=True):
+    """takes: the tile is known to take the problem."""
+    lib.dmlhip_debug_last_conv_form()
     lib.dmlhip_debug_force_conv_dense3_tile(tile)
     try:
-        return run()
+        result = run()
     finally:
         lib.dmlhip_debug_force_conv_dense3_tile(-1)
+    if takes:
+        assert lib.dmlhip_debug_last_conv_form() % 8 == tile
+    return result
 
 
-@pytest.mark.parametrize("shape", SHAPES)
-def test_conv_dense3_split(shape, lib):
+@pytest.mark.parametrize("shape,forms", zip(SHAPES, FORMS))
+def test_conv_dense3_split(shape, forms, lib):
     from daceml_amd import kernels as K
     n, c, h, w, m, s, p, d = shape
     x, wt, b, dy, exact, terms = _problem(shape)
     for tile in (3, 4, 5):
-        y = _forced(lib, tile, lambda: K.conv2d(dev(x), dev(wt), dev(b), (s, s), (p, p), (d, d)))
-        dx, _ = _forced(lib, tile, lambda: K.conv2d_backward(dev(x), dev(wt), dev(dy), (s, s), (p, p), (d, d), need_dw=False))
+        y = _forced(lib, tile, lambda: K.conv2d(dev(x), dev(wt), dev(b), (s, s), (p, p), (d, d)), False)
+        ran = [lib.dmlhip_debug_last_conv_form()]
+        dx, _ = _forced(lib, tile, lambda: K.conv2d_backward(dev(x), dev(wt), dev(dy), (s, s), (p, p), (d, d), need_dw=False), False)
+        ran.append(lib.dmlhip_debug_last_conv_form())
+        assert ran == [f[tile - 3] for f in forms]
         _check((tile, "y"), y, exact[0], terms[0], 9 * c)
         _check((tile, "dx"), dx, exact[1], terms[1], 9 * m)
 
@@ -80,7 +102,8 @@ def test_biases_that_are_not_finite(act, tile, lib):
     x, wt = r.standard_normal((2, 16, 18, 20)).astype(np.float32), r.standard_normal((70, 16, 3, 3)).astype(np.float32)
     b = r.standard_normal(70).astype(np.float32)
     b[0], b[33], b[34], b[69], b[7] = np.nan, np.inf, -np.inf, np.nan, np.finfo(np.float32).max
-    y, want = (host(_forced(lib, t, lambda: K.conv2d(dev(x), dev(wt), dev(b), pads=(1, 1), act=getattr(L, "ACT_" + act)))) for t in (tile, 0))
+    y, want = (host(_forced(lib, t, lambda: K.conv2d(dev(x), dev(wt), dev(b), pads=(1, 1), act=getattr(L, "ACT_" + act)), t == tile))
+               for t in (tile, 0))
     for same in (np.isnan, np.isposinf, np.isneginf):
         np.testing.assert_array_equal(same(y), same(want))
     assert np.isnan(want[:, 0]).all() or act == "RELU"
@@ -99,8 +122,8 @@ def test_values_without_a_split_in_every_geometry(shape, lib):
         t[0, 3, 1, 1], t[-1, 4, -1, -1] = np.inf, np.nan
     wt[1, 5, 0, 2] = -np.inf
     def run(tile):
-        y = _forced(lib, tile, lambda: K.conv2d(dev(x), dev(wt), dev(b), (s, s), (p, p), (d, d)))
-        return y, _forced(lib, tile, lambda: K.conv2d_backward(dev(x), dev(wt), dev(dy), (s, s), (p, p), (d, d), need_dw=False)[0])
+        y = _forced(lib, tile, lambda: K.conv2d(dev(x), dev(wt), dev(b), (s, s), (p, p), (d, d)), False)
+        return y, _forced(lib, tile, lambda: K.conv2d_backward(dev(x), dev(wt), dev(dy), (s, s), (p, p), (d, d), need_dw=False)[0], False)
     want = [host(t) for t in run(0)]
     for tile in (3, 4, 5):
         for got, ref, k in zip(map(host, run(tile)), want, (9 * c, 9 * m)):

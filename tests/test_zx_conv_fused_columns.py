@@ -28,7 +28,7 @@ def _run(rows, x, w1, b1, w2, b2, stride, acts):
 
 @pytest.mark.parametrize("stride", [1, 2])
 @pytest.mark.parametrize("shape", SHAPES)
-def test_same_bits_as_the_strips(shape, stride):
+def test_same_bits_as_the_strips(shape, stride, lib):
     from daceml_amd import _lib as L
     n, cin, cmid, h, w = shape
     g = torch.Generator().manual_seed(h * w)
@@ -37,7 +37,10 @@ def test_same_bits_as_the_strips(shape, stride):
     for acts, biases in (((L.ACT_SWISH, L.ACT_SWISH), (b1, b2)), ((L.ACT_RELU, L.ACT_NONE), (b1, None)),
                          ((L.ACT_NONE, L.ACT_RELU), (None, b2))):
         want = _run(-2, x, w1, biases[0], w2, biases[1], stride, acts)
-        assert np.array_equal(_run(0, x, w1, biases[0], w2, biases[1], stride, acts), want), acts
+        lib.dmlhip_debug_last_conv_form()
+        got = _run(0, x, w1, biases[0], w2, biases[1], stride, acts)
+        assert lib.dmlhip_debug_last_conv_form() == 16       # the kernel that this file is about
+        assert np.array_equal(got, want), acts
 
 
 @pytest.mark.parametrize("stride", [1, 2])
