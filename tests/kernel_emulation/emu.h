@@ -66,6 +66,23 @@ inline f16v mfma_32x32x16_f16(h8 a, h8 b, f16v c) {
     return d;
 }
 
+// The same in bf16
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+inline f16v mfma_32x32x16_bf16(b8 a, b8 b, f16v c) {
+    struct Ops { b8 a, b; } mine = {a, b};
+    const Ops* all = static_cast<const Ops*>(wave_exchange(&mine, sizeof(mine)));
+    const int lane = thread_idx().x & 63, col = lane & 31;
+    f16v d = c;
+    for (int e = 0; e < 16; ++e) {
+        const int row = 8 * (e / 4) + 4 * (lane / 32) + e % 4;
+        double acc = c[e];
+        for (int k = 0; k < 16; ++k)
+            acc += (double)(float)all[row + 32 * (k / 8)].a[k % 8] * (double)(float)all[col + 32 * (k / 8)].b[k % 8];
+        d[e] = (float)acc;
+    }
+    return d;
+}
+
 // D = C + A B, 32 x 32 x 2 in fp32: lane l holds A[l % 32][l / 32] and B[l / 32][l % 32]; C / D as above.
 inline f16v mfma_32x32x2_f32(float a, float b, f16v c) {
     struct Ops { float a, b; } mine = {a, b};
@@ -123,6 +140,11 @@ typedef emu_dim3 dim3;
 #define __builtin_amdgcn_sched_barrier(x) ((void)0)
 #define __builtin_amdgcn_readfirstlane(x) (x)
 #define __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, x, y, z) emu::mfma_32x32x16_f16(a, b, c)
+#define __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, x, y, z) emu::mfma_32x32x16_bf16(a, b, c)
+#define __builtin_amdgcn_sched_group_barrier(mask, size, id) ((void)0)
+#define __builtin_amdgcn_alignbit(hi, lo, shift) ((uint32_t)((((uint64_t)(hi) << 32) | (uint32_t)(lo)) >> (shift)))
+#define __builtin_amdgcn_mbcnt_lo(mask, add) (0u)           /* of a full mask, with the other half: the lane's number */
+#define __builtin_amdgcn_mbcnt_hi(mask, add) ((add) + (threadIdx.x & 63))
 #define __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, x, y, z) emu::mfma_32x32x2_f32(a, b, c)
 #define __builtin_amdgcn_ds_bpermute(i, v) emu::ds_bpermute(i, v)
 #define __builtin_amdgcn_ballot_w64(p) emu::ballot(p)

@@ -30,6 +30,14 @@ inline float lds_read_b32(uint32_t addr) {
     return v;
 }
 
+typedef float float2v __attribute__((ext_vector_type(2)));
+template <int OFFSET>
+inline float2v lds_read_b64(uint32_t addr) {
+    float2v v;
+    memcpy(&v, emu::g_lds + addr + OFFSET, 8);
+    return v;
+}
+
 // ds_read_b64_tr_b16: within each group of 16 lanes, lane s supplies the address of four consecutive 16-bit elements;
 // the 16 x 4 elements form rows s / 4 (four lanes side by side make one row of 16); lane j receives element j of each
 // of the four rows

@@ -12,8 +12,12 @@ namespace dml { namespace gemm16 { namespace { alignas(16) char lds[160 * 1024];
 namespace dml { namespace { alignas(16) char lds[160 * 1024]; } }
 #if defined(EMU_F32)
 #include "gemm_f32_emu.h"
+#elif defined(EMU_F32SPLIT)
+#include "gemm_f32_split_emu.h"
 #elif defined(EMU_DENSE3)
 #include "conv_dense3_emu.h"
+#elif defined(EMU_DENSE3WS)
+#include "conv_dense3_weight_split_emu.h"
 #else
 #include "conv_dense3_weight_emu.h"
 #endif
@@ -28,7 +32,12 @@ void set_error(const char* fmt, ...) {
     fputc('\n', stderr);
 }
 int launch_status(const char*) { return 0; }
+#if defined(EMU_F32SPLIT)
+int gemm_f32_streamed(const dmlhip_gemm_desc*, const void*, const void*, void*, const void*, const void*, void*, int, long long, hipStream_t) { return 0; }
+double gemm_f32_streamed_us(const dmlhip_gemm_desc*, long long) { return 0.0; }
+#endif
 #if defined(EMU_DENSE3)
+void note_conv_form(int) {}
 // asked by the launch functions only, which are not called here
 bool conv_implicit_applicable(const ConvGeom&) { return false; }
 bool conv_implicit_bwd_data_applicable(const ConvGeom&) { return false; }
@@ -133,6 +142,37 @@ extern "C" int emu_gemm_f32(int tile, int ak, int bk, int m, int n, int k, const
     return emu::run_grid(fn, &g, (unsigned)g.total_blocks, 256, seed, late, lds);
 }
 
+#elif defined(EMU_F32SPLIT)
+using namespace dml;
+
+namespace {
+template <int KG, int AR, int BR> void entry(void* p) { gemm_f32_split_kernel<KG, AR, BR>(*static_cast<const SplitArgs*>(p)); }
+template <int KG> emu::kernel_fn pick(int ar, int br) {
+    if (ar) return br ? entry<KG, 1, 1> : entry<KG, 1, 0>;
+    return br ? entry<KG, 0, 1> : entry<KG, 0, 0>;
+}
+}  // namespace
+
+// K over kg (8 or 4) wavefronts; kinds 0 = K contiguous, 1 = rows contiguous
+extern "C" int emu_gemm_f32_split(int kg, int ak, int bk, int m, int n, int k, const float* a, const float* b, float* c, unsigned seed,
+                                  int late) {
+    SplitArgs g = {};
+    g.a = a; g.b = b; g.c = c;
+    g.m = m; g.n = n; g.k = k;
+    g.sam = ak ? 1 : k; g.sak = ak ? m : 1;
+    g.sbn = bk ? 1 : k; g.sbk = bk ? n : 1;
+    g.scm = n;
+    g.batch1 = g.batch2 = 1;
+    g.alpha = 1.f;
+    g.c_vec = n % 4 == 0;
+    const int64_t one[3] = {1, 1, 1}, zero[3] = {0, 0, 0};
+    if (operand_rows(a, m, k, g.sam, g.sak, zero, one) != ak || operand_rows(b, n, k, g.sbn, g.sbk, zero, one) != bk) return 3;
+    g.tiles_m = (m + kBlock - 1) / kBlock;
+    g.tiles_n = (n + kBlock - 1) / kBlock;
+    g.total_blocks = (long long)g.tiles_m * g.tiles_n;
+    return emu::run_grid(kg == 8 ? pick<8>(ak, bk) : pick<4>(ak, bk), &g, (unsigned)g.total_blocks, 64 * kg, seed, late, lds);
+}
+
 #else
 using namespace dml;
 
@@ -177,7 +217,11 @@ extern "C" int emu_dense3(int tile, int data, int n, int c, int h, int w, int m,
 
 #else
 namespace {
+#if defined(EMU_DENSE3WS)
+template <int WM, int AV, int XV> void entry(void* p) { conv_dense3_weight_split_kernel<WM, AV, XV>(*static_cast<const WeightArgs*>(p)); }
+#else
 template <int WM, int AV, int XV> void entry(void* p) { conv_dense3_weight_kernel<WM, AV, XV>(*static_cast<const WeightArgs*>(p)); }
+#endif
 template <int WM> emu::kernel_fn pick(int av, int xv) {
     if (av == 4) return xv == 4 ? entry<WM, 4, 4> : entry<WM, 4, 1>;
     return xv == 4 ? entry<WM, 1, 4> : entry<WM, 1, 1>;

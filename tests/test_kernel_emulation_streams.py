@@ -1,7 +1,8 @@
 """The kernels that stream their operands into LDS with waits and barriers of their own - fp16 products with K split over the
-wavefronts, fp32 products, dense 3 x 3 convolutions and their weight gradient - run on the CPU, lane by lane, from their own source
+wavefronts, fp32 products, dense 3 x 3 convolutions and their weight gradient, on the fp32 and on the bf16 matrix instructions - run on the CPU, lane by lane, from their own source
 (tests/test_kernel_emulation.py says how, and what transfers that land early and late expose). No GPU."""
 import ctypes
+import re
 
 import numpy as np
 import pytest
@@ -9,8 +10,18 @@ import pytest
 from tests.test_kernel_emulation import _build, _fails
 
 FILES = {"SPLIT": ["common.h", "gemm_f16_common.h", "gemm_f16_split.hip"], "F32": ["common.h", "gemm_f32.hip"],
+         "F32SPLIT": ["common.h", "bf16_split.h", "gemm_f32_split.hip"],
+         "DENSE3WS": ["common.h", "conv_geom.h", "bf16_split.h", "conv_dense3_weight.hip", "conv_dense3_weight_split.hip"],
          "DENSE3": ["common.h", "conv_geom.h", "conv_dense3.hip"], "DENSE3W": ["common.h", "conv_geom.h", "conv_dense3_weight.hip"]}
 P = ctypes.c_void_p
+
+
+def _split_source(text):
+    """Without assembly statements that have no instructions and tell the compiler where a value has to exist, and without the second
+    computation of sums that are not finite: LDS that nobody wrote holds NaN, and a read of it has to show."""
+    text, repairs = re.subn(r"__builtin_amdgcn_ballot_w64\(bad != 0.f\) != 0", "false", text)
+    assert repairs == 1
+    return re.sub(r'asm volatile\("" : [^;]*;', "", text)
 
 
 def _stage(tmp, kernel, change=None):
@@ -19,6 +30,11 @@ def _stage(tmp, kernel, change=None):
         edits["conv_dense3_emu.h"] = lambda t: t.replace('asm volatile("" : "+v"(at));', "").replace("(double)(1 << 24)", "(double)(1 << 10)")
     elif kernel == "DENSE3W":
         edits["conv_dense3_weight_emu.h"] = lambda t: t.replace("(1 << (general ? 29 : 24))", "(1 << (general ? 29 : 10))")
+    elif kernel == "DENSE3WS":
+        edits["conv_dense3_weight_emu.h"] = lambda t: t.replace("(1 << (general ? 29 : 24))", "(1 << (general ? 29 : 10))")
+        edits["conv_dense3_weight_split_emu.h"] = lambda t: _split_source(t.replace("conv_dense3_weight.hip\"", "conv_dense3_weight_emu.h\""))
+    elif kernel == "F32SPLIT":
+        edits["gemm_f32_split_emu.h"] = _split_source
     if change:
         name = FILES[kernel][-1][:-4] + "_emu.h"
         before = edits.get(name, lambda t: t)
@@ -98,6 +114,25 @@ def test_fp32_products(library, tile, late):
             _f32(lib, tile, ak, bk, m, n, k, offset, late)
 
 
+def _f32_split(lib, kg, ak, bk, m, n, k, late):
+    r = np.random.default_rng(m + n + k)
+    a, b = (r.standard_normal((rows, k)).astype(np.float32) for rows in (m, n))
+    sa, sb = (_place(np.ascontiguousarray(v.T) if kind else v) for v, kind in ((a, ak), (b, bk)))
+    c = np.full((m, n), np.nan, np.float32)
+    _ran(lib.emu_gemm_f32_split(kg, ak, bk, m, n, k, _p(sa), _p(sb), _p(c), 2 + k, late))
+    np.testing.assert_allclose(c, a.astype(np.float64) @ b.astype(np.float64).T, rtol=1e-5, atol=2e-6 * k ** 0.5)
+
+
+@pytest.mark.parametrize("late", [0, 1])
+@pytest.mark.parametrize("kg", [4, 8])
+def test_fp32_products_of_split_operands(library, kg, late):
+    """No step, one, two, an odd and an even number of them per wavefront, the last one short; rows that end inside a transfer."""
+    lib = library("F32SPLIT")
+    for ak, bk in ((0, 0), (0, 1), (1, 0), (1, 1)):
+        for m, n, k in ((68, 32, 16), (20, 68, 16 * kg * 2), (44, 36, 16 * kg * 4 + 20), (64, 56, 16 * kg * 5 - 4)):
+            _f32_split(lib, kg, ak, bk, m, n, k, late)
+
+
 def _conv(x, w, s, p, d):
     n, c, h, wd = x.shape
     oh, ow = (h + 2 * p - 2 * d - 1) // s + 1, (wd + 2 * p - 2 * d - 1) // s + 1
@@ -160,6 +195,24 @@ def _dense3_weight(lib, shape, ranges, rows, offset, late):
 def test_dense_weight_gradient(library, shape, ranges, rows, offset, late):
     """Odd and even numbers of pixel pairs per wavefront, chunks that end inside an image, several chunks per range."""
     _dense3_weight(library("DENSE3W"), shape, ranges, rows, offset, late)
+
+
+@pytest.mark.parametrize("late", [0, 1])
+@pytest.mark.parametrize("shape,ranges,rows,offset", [(CONVOLUTIONS[0], 3, 5, 0), (CONVOLUTIONS[0], 2, 3, 1), (CONVOLUTIONS[1], 4, 2, 0),
+                                                      ((7, 40, 13, 13, 24, 1, 1, 1), 5, 1, 0), ((2, 33, 12, 7, 34, 1, 0, 1), 2, 4, 0)])
+def test_dense_weight_gradient_of_split_operands(library, shape, ranges, rows, offset, late):
+    """Rows of whole eights, rows that end inside one and rows shorter than one; several chunks per range."""
+    _dense3_weight(library("DENSE3WS"), shape, ranges, rows, offset, late)
+
+
+def test_a_ring_of_split_operands_read_or_refilled_too_early_is_detected(tmp_path):
+    first = _stage(tmp_path / "first", "F32SPLIT", lambda t: t.replace("wait_vm_lgkm0<LPT>();\n        } else {", "wait_vm_lgkm0<2 * LPT>();\n        } else {"))
+    assert _fails(lambda: _f32_split(first, 4, 0, 0, 20, 36, 16 * 4 * 3, 1))
+    inside = _stage(tmp_path / "inside", "F32SPLIT", lambda t: t.replace("wait_vm_lgkm0<0>();\n                if constexpr (LEFT > 1)",
+                                                                         "wait_lgkm<0>();\n                if constexpr (LEFT > 1)"))
+    assert _fails(lambda: _f32_split(inside, 4, 0, 0, 20, 36, 16 * 4 * 6, 1))
+    refilled = _stage(tmp_path / "refilled", "F32SPLIT", lambda t: t.replace("if (t + 3 < mine) issue(other);", "if (t + 3 < mine) issue(here);"))
+    assert _fails(lambda: _f32_split(refilled, 4, 0, 0, 20, 36, 16 * 4 * 6, 0))
 
 
 def test_a_chunk_read_before_it_has_landed_is_detected(tmp_path):
