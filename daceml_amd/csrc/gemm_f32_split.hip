@@ -495,14 +495,27 @@ int operand_rows(const void* p, int64_t rows, int64_t k, int64_t s_row, int64_t 
 thread_local int g_force_tile = -1;   // diagnostic: 0 - 2 = the streamed kernel's tiles, 3 and 4 = the forms here
 
 // -1: the streamed kernel is the faster one. Measured: a step of eight wavefronts on a compute unit takes 1.14 us, whether
-// they share a tile or are two workgroups of four; first loads, the sum through LDS and stores 6.4 us per tile of eight, 7.1 us
-// per pair of tiles of four. So one tile per compute unit takes eight (1024 x 768 x 768: 14.3 us, four 15.1, streamed 20; 1024 x
-// 768 x 3072 34.8 / 36.0 / 51), more take four (1024 x 3072 x 768: 34.7, eight 39.8, streamed 48; 4096^3 761 / 768 / 1016). Few
+// they share a tile or are two workgroups of four (0.61 alone); first loads, the sum through LDS and stores 6.4 us per tile of eight, 7.1 us
+// per pair of tiles of four. So one tile per compute unit takes eight (1024 x 768 x 768: 15.9 us, four 16.5, streamed 20; 1024 x
+// 768 x 3072 38.6 / 40.1 / 52), more take four (1024 x 3072 x 768: 38.5, eight 45, streamed 51; 4096^3 850 / 880 / 1016). Few
 // tiles (512^3: 9.6, streamed 6.0) and short K (512 x 512 x 64, 24 times: 24, streamed 17) stay on the streamed kernel.
-int choose_form(const dmlhip_gemm_desc* d, long long batch) {
+// Rows of K that do not start at a multiple of 64 bytes make two requests of each of a step's: 1.4 - 1.55 us for eight wavefronts
+// (640 x 472 x 20284, streamed / eight / four, 211 / 253 / 209). Operands of more than the 256 MB of the last-level cache: 1.5 - 2.2 us and
+// the streamed kernel a fifth more than it estimates (768 x 36 x 51788, 8 times, 585 / 909 / 806). 680 products of 32 - 4096 rows, K of 16 - 65536:
+// none takes more than 1.03 of the streamed kernel's time, 0.91 on average; without these two 1.55, ten more than 1.1.
+int choose_form(const dmlhip_gemm_desc* d, long long batch, const void* a, const void* b, int a_rows, int b_rows) {
     const double tiles = (double)ceil_div(d->m, kBlock) * ceil_div(d->n, kBlock) * batch, n = ceil(tiles / kCus);
-    const double eight = n * (6.4 + ceil_div(d->k, 8 * BK) * 1.14), four = ceil(n / 2) * 7.1 + 0.8 + n * ceil_div(d->k, 4 * BK) * 0.57;
-    if (gemm_f32_streamed_us(d, batch) <= fmin(eight, four)) return -1;
+    auto unaligned = [](const void* p, int rows, int64_t s_row) { return rows == 0 && (s_row % 16 != 0 || reinterpret_cast<uintptr_t>(p) % 64 != 0); };
+    double a_bytes = 4.0 * d->m * d->k, b_bytes = 4.0 * d->n * d->k;
+    for (int i = 0; i < 3; ++i) {
+        if (d->a_stride_batch[i] != 0) a_bytes *= d->batch[i];
+        if (d->b_stride_batch[i] != 0) b_bytes *= d->batch[i];
+    }
+    const bool twice = unaligned(a, a_rows, d->a_stride_m) || unaligned(b, b_rows, d->b_stride_n), memory = a_bytes + b_bytes > 256e6;
+    const double step8 = (twice ? 1.5 : 1.14) * (memory ? 1.4 : 1.0);
+    const double step4 = twice ? 0.66 * (memory ? 1.5 : 1.0) : 0.61 * (memory ? 1.25 : 1.0);
+    const double eight = n * (6.4 + ceil_div(d->k, 8 * BK) * step8), four = ceil(n / 2) * 7.1 + 0.8 + n * ceil_div(d->k, 4 * BK) * step4;
+    if (gemm_f32_streamed_us(d, batch) * (memory ? 1.2 : 1.0) <= fmin(eight, four)) return -1;
     return eight <= four ? 0 : 1;
 }
 
@@ -553,7 +566,7 @@ extern "C" int dmlhip_gemm_f32(const dmlhip_gemm_desc* d, const void* a, const v
         if (d->batch[i] > 1 && d->c_stride_batch[i] % 4 != 0) g.c_vec = 0;
     const int ar = operand_rows(a, d->m, d->k, d->a_stride_m, d->a_stride_k, d->a_stride_batch, d->batch);
     const int br = operand_rows(b, d->n, d->k, d->b_stride_n, d->b_stride_k, d->b_stride_batch, d->batch);
-    const int form = ar < 0 || br < 0 ? -1 : g_force_tile >= 3 ? g_force_tile - 3 : choose_form(d, batch);
+    const int form = ar < 0 || br < 0 ? -1 : g_force_tile >= 3 ? g_force_tile - 3 : choose_form(d, batch, a, b, ar, br);
     if (form < 0) return gemm_f32_streamed(d, a, b, c, bias, residual, pre_out, -1, batch, (hipStream_t)stream);
     hipStream_t st = (hipStream_t)stream;
     if (ar == 0) return br == 0 ? launch_form<0, 0>(g, form, batch, st) : launch_form<0, 1>(g, form, batch, st);

@@ -147,3 +147,19 @@ def test_no_less_exact_than_the_fp32_instruction(kind, k, rows, lib):
     other = error(2)
     for form in (3, 4):
         assert error(form) < 0.9 * other, (form, error(form), other)
+
+
+@pytest.mark.parametrize("m,n,k,batch,chosen", [(640, 472, 20284, 1, 2), (640, 472, 20288, 1, 3), (64, 256, 24000, 24, 2), (256, 512, 1024, 8, 3),
+                                                (1088, 336, 2548, 1, 2), (1024, 768, 768, 1, 3), (1024, 3072, 768, 1, 4)])
+def test_the_kernel_that_is_chosen(m, n, k, batch, chosen, lib):
+    """Rows of K that do not start at multiples of 64 bytes and operands that do not fit the last-level cache stay on the fp32 instruction's
+    kernel where that is the faster one. The kernels add in different orders: equal bits are the same kernel."""
+    g = torch.Generator(device="cuda").manual_seed(k)
+    a, b = torch.randn(batch, m, k, device="cuda", generator=g), torch.randn(batch, n, k, device="cuda", generator=g)
+
+    def run(form):
+        c = torch.full((batch, m, n), float("nan"), device="cuda")
+        _product(lib, form, m, n, k, batch, a, b, (k, 1), (k, 1), c)
+        return c
+    got = run(-1)
+    assert [form for form in (2, 3, 4) if torch.equal(run(form), got)] == [chosen]
