@@ -370,14 +370,15 @@ int launch(const SplitPlan3& pl, hipStream_t st, const char* what) {
         set_error("%s: cannot reserve %zu bytes of LDS: %s", what, pl.lds, hipGetErrorString(e));
         return (int)e;
     }
-    note_conv_form((P == 1 ? 3 : P == 2 ? 4 : 5) + (TASKS == 7 ? 8 : 0));
+    note_conv_form(P == 1 ? (TASKS == 4 ? 3 : TASKS == 6 ? 11 : 19) : P == 2 ? (TASKS == 5 ? 4 : 12) : TASKS == 6 ? 5 : 13);
     hipLaunchKernelGGL(kern, pl.a.blocks, kThreads, pl.lds, st, pl.a);
     return launch_status(what);
 }
 
 template <bool FLIP>
 int launch_form(const SplitPlan3& pl, hipStream_t st, const char* what) {
-    if (pl.p == 1) return pl.tasks <= 4 ? launch<1, 4, FLIP>(pl, st, what) : launch<1, 7, FLIP>(pl, st, what);
+    if (pl.p == 1 && pl.tasks > 4) return pl.tasks <= 6 ? launch<1, 6, FLIP>(pl, st, what) : launch<1, 7, FLIP>(pl, st, what);
+    if (pl.p == 1) return launch<1, 4, FLIP>(pl, st, what);
     if (pl.p == 2) return pl.tasks <= 5 ? launch<2, 5, FLIP>(pl, st, what) : launch<2, 7, FLIP>(pl, st, what);
     return pl.tasks <= 6 ? launch<4, 6, FLIP>(pl, st, what) : launch<4, 7, FLIP>(pl, st, what);
 }
@@ -412,11 +413,14 @@ static bool plan_split(const ConvGeom& g, int ids_h, int ids_w, int most_p, Spli
         // us of a tile: first loads and results, and per step; whole rounds of one tile per compute unit. Rounds decide: 32x64x56x56 ->
         // 64 is one round of 196 tiles of 512 pixels (57 us), two of 392 (58) or four (92), 32x256x14x14 -> 256 one of 196 tiles of 128
         // (58; of 256 81, of 512 178), 32x96x40x40 -> 96 one of 200 tiles of 512 (77) or two of 400 (74).
-        const double t = rounds * (p == 1 ? 7.0 + 3.4 * steps : p == 2 ? 9.0 + 4.9 * steps : 15.0 + 10.3 * steps);
+        // More chunks per thread, larger rectangles, take longer (18 shapes, strides, dilation, 28 - 112 pixels wide).
+        const int tasks = (int)ceil_div(kWTasks + 2 * rect, (int64_t)kThreads);
+        const double step = p == 1 ? (tasks <= 4 ? 3.4 : tasks <= 6 ? 4.1 : 4.9) : p == 2 ? (tasks <= 5 ? 4.9 : 6.0) : tasks <= 6 ? 10.3 : 11.0;
+        const double t = rounds * ((p == 1 ? 7.0 : p == 2 ? 9.0 : steps > 1 ? 15.0 : 10.0) + step * steps);
         if (pl->p > 0 && t >= *us) continue;
         *us = t;
         pl->p = p;
-        pl->tasks = (int)ceil_div(kWTasks + 2 * rect, (int64_t)kThreads);
+        pl->tasks = tasks;
         pl->lds = (size_t)(kWBytes + rect * 96);
         SplitArgs3& a = pl->a;
         a.n = g.n; a.c = g.c; a.h = g.h; a.w_in = g.w; a.m = g.m; a.sh = g.sh; a.sw = g.sw; a.ph = g.ph; a.pw = g.pw;

@@ -505,8 +505,9 @@ void dmlhip_debug_force_gemm_f32_tile(int tile);
    instructions, 0 = 32 channels x 128 pixels, 1 = 32 x 64, 2 = 32 x 32; operands split into bf16 values, 3 = 64 x 128, 4 = 64 x 256,
    5 = 64 x 512; -1 = the library chooses). A problem that a kernel does not take runs on the next one. */
 void dmlhip_debug_force_conv_dense3_tile(int tile);
-/* Diagnostic: what the calling thread launched last for a convolution since it last asked: 0 - 5 as above, 11 - 13 for 3 - 5 in the form
- * with seven transfers of X and W per thread (large rectangles), 16 for the expansion + depthwise kernel with its rows in registers; -1: none of these. */
+/* Diagnostic: what the calling thread launched last for a convolution since it last asked: 0 - 5 as above, 11 - 13 for 3 - 5 in their form
+ * for large rectangles of X and 19 for 3 in the one for still larger ones, 16 for the expansion + depthwise kernel with its rows in
+ * registers; -1: none of these. */
 int dmlhip_debug_last_conv_form(void);
 /* Diagnostic: the calling thread's depthwise stride-1 fp32 convolutions and gradients whose output is as large as the input
  * run on the strip kernels (1), on the general depthwise kernels (0), or on the faster of the two (-1, default). */

@@ -17,19 +17,21 @@ pytestmark = pytest.mark.gpu
 SHAPES = [(3, 64, 56, 56, 64, 1, 1, 1), (5, 16, 31, 33, 72, 1, 1, 1), (9, 24, 14, 14, 136, 1, 1, 1), (4, 40, 27, 29, 64, 2, 1, 1),
           (2, 16, 30, 64, 96, 1, 2, 2), (3, 24, 33, 20, 32, 1, 0, 1), (20, 64, 14, 14, 64, 2, 1, 1), (1, 32, 112, 112, 32, 1, 1, 1),
           (6, 256, 7, 7, 64, 1, 1, 1), (50, 16, 3, 5, 16, 1, 1, 1),
-          # large rectangles: 80 and 144 columns, dilation
-          (1, 16, 32, 80, 40, 1, 1, 1), (1, 24, 32, 80, 16, 1, 2, 2), (2, 16, 32, 16, 24, 1, 2, 2), (1, 16, 16, 144, 16, 1, 2, 2)]
+          # large rectangles: 80, 144 and 160 columns, dilation
+          (1, 16, 32, 80, 40, 1, 1, 1), (1, 24, 32, 80, 16, 1, 2, 2), (2, 16, 32, 16, 24, 1, 2, 2), (1, 16, 16, 144, 16, 1, 2, 2),
+          (1, 16, 8, 160, 16, 1, 2, 2)]
 
-# What runs with each of the tiles 3, 4 and 5 asked for, forward and data gradient: 11 - 13 are their forms for large rectangles; where a
+# What runs with each of the tiles 3, 4 and 5 asked for, forward and data gradient: 11 - 13 and 19 are their forms for large rectangles; where a
 # rectangle does not fit LDS the kernel on the fp32 instruction (0 - 2) or the general one (-1) takes the problem.
 FORMS = [((11, 4, 5), (11, 4, 5)), ((3, 4, 5), (3, 4, 5)), ((3, 4, 5), (3, 4, 5)), ((11, 2, 2), (3, 4, 5)), ((11, 12, 2), (11, 12, 2)),
          ((3, 4, 5), (3, 4, 5)), ((11, 2, 2), (3, 4, 5)), ((11, 4, 2), (11, 4, 2)), ((3, 4, 5), (3, 4, 5)), ((3, 4, -1), (3, 4, -1)),
-         ((3, 4, 5), (3, 4, 5)), ((11, 12, 13), (11, 12, 13)), ((3, 4, 5), (3, 4, 5)), ((11, 12, -1), (11, 12, -1))]
+         ((3, 4, 5), (3, 4, 5)), ((11, 12, 13), (11, 12, 13)), ((3, 4, 5), (3, 4, 5)), ((11, 12, -1), (11, 12, -1)),
+         ((19, -1, -1), (19, -1, -1))]
 
 
 def test_every_form_has_a_shape():
     for direction in (0, 1):
-        assert {f for forms in FORMS for f in forms[direction]} >= {3, 4, 5, 11, 12, 13}
+        assert {f for forms in FORMS for f in forms[direction]} >= {3, 4, 5, 11, 12, 13, 19}
     assert len(FORMS) == len(SHAPES)
 
 
