@@ -180,10 +180,15 @@ int launch_conv_dense3_weight(const ConvGeom& g, const float* x, const float* dy
     WeightPlan pl;
     unsigned blocks;
     int avec, xvec;
-    const bool split = g.sh == 1 && g.sw == 1 && g.dh == 1 && g.dw == 1 && plan_weight(g, x, dy, &pl, &blocks, &avec, &xvec) &&
+    // Rows are read as whole eights of pixels: not where that is more than 1.42 times as many. Times those of the fp32 instruction, 5 - 65 columns,
+    // 64 - 192 channels: 5, 6, 9, 10, 11 columns 1.18 - 1.29, 1.07 - 1.18, 0.97 - 1.08, 0.98 - 1.03, 0.98 - 1.03; 7 columns 0.94 - 1.07; 8 and
+    // 12 - 65 0.73 - 1.01 (17 to 19 columns 0.97 - 1.01, whole eights 0.73 - 1.00).
+    const bool eights = g.ow >= 8 && 100 * ceil_div(g.ow, 8) * 8 <= 142 * g.ow;
+    const bool split = eights && g.sh == 1 && g.sw == 1 && g.dh == 1 && g.dw == 1 && plan_weight(g, x, dy, &pl, &blocks, &avec, &xvec) &&
                        pl.lds + kReadPast <= (size_t)kLdsBytes;
     if (!split) return launch_conv_dense3_bwd_weight(g, x, dy, part, st);
     pl.lds += kReadPast;
+    note_conv_form(20);
     pl.a.x = x; pl.a.dy = dy; pl.a.part = part;
     const int wm = g.m > 32 ? 2 : 1;
 #define DML_D3W(WM, AV, XV) \

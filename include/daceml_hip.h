@@ -507,7 +507,7 @@ void dmlhip_debug_force_gemm_f32_tile(int tile);
 void dmlhip_debug_force_conv_dense3_tile(int tile);
 /* Diagnostic: what the calling thread launched last for a convolution since it last asked: 0 - 5 as above, 11 - 13 for 3 - 5 in their form
  * for large rectangles of X and 19 for 3 in the one for still larger ones, 16 for the expansion + depthwise kernel with its rows in
- * registers; -1: none of these. */
+ * registers, 20 for the 3 x 3 weight gradient of operands split into bf16 values; -1: none of these. */
 int dmlhip_debug_last_conv_form(void);
 /* Diagnostic: the calling thread's depthwise stride-1 fp32 convolutions and gradients whose output is as large as the input
  * run on the strip kernels (1), on the general depthwise kernels (0), or on the faster of the two (-1, default). */

@@ -36,8 +36,10 @@ int launch_status(const char*) { return 0; }
 int gemm_f32_streamed(const dmlhip_gemm_desc*, const void*, const void*, void*, const void*, const void*, void*, int, long long, hipStream_t) { return 0; }
 double gemm_f32_streamed_us(const dmlhip_gemm_desc*, long long) { return 0.0; }
 #endif
-#if defined(EMU_DENSE3)
+#if defined(EMU_DENSE3) || defined(EMU_DENSE3WS)
 void note_conv_form(int) {}
+#endif
+#if defined(EMU_DENSE3)
 // asked by the launch functions only, which are not called here
 bool conv_implicit_applicable(const ConvGeom&) { return false; }
 bool conv_implicit_bwd_data_applicable(const ConvGeom&) { return false; }

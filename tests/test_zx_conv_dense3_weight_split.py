@@ -1,5 +1,5 @@
 """The weight gradient of the 3 x 3 convolution on the bf16 matrix instructions (stride and dilation 1): rows of whole eights of
-pixels, rows that end inside one, rows shorter than one, an odd number of eights, channels that end inside a tile, transfers of four and of
+pixels, rows that end inside one, an odd number of eights, channels that end inside a tile, transfers of four and of
 sixteen bytes, wide and no padding, values without a split.
 
 Tolerance: that of the fp32 kernels' test; the products left out are below 3 * 2^-26 of |a| |b|, one of its two spare terms."""
@@ -15,7 +15,10 @@ pytestmark = pytest.mark.gpu
 # n, c, h, w, m, stride, pad, dilation
 SHAPES = [(6, 64, 56, 56, 64, 1, 1, 1), (40, 33, 31, 33, 70, 1, 1, 1), (24, 128, 28, 28, 64, 1, 1, 1), (150, 64, 7, 7, 64, 1, 1, 1),
           (16, 32, 64, 64, 32, 1, 1, 1), (70, 48, 26, 30, 50, 1, 2, 1), (60, 64, 15, 60, 64, 1, 0, 1), (16, 64, 36, 57, 128, 1, 1, 1),
-          (50, 128, 14, 14, 256, 1, 1, 1), (300, 16, 5, 9, 40, 1, 1, 1), (3, 40, 200, 110, 70, 1, 1, 1), (30, 31, 40, 44, 64, 1, 4, 1)]
+          (50, 128, 14, 14, 256, 1, 1, 1), (300, 16, 5, 9, 40, 1, 1, 1), (3, 40, 200, 110, 70, 1, 1, 1), (30, 31, 40, 44, 64, 1, 4, 1),
+          (24, 60, 40, 40, 70, 1, 1, 1), (16, 45, 43, 44, 100, 1, 1, 1), (8, 50, 61, 66, 180, 1, 0, 1), (30, 64, 26, 30, 128, 1, 2, 1)]
+# on the fp32 instruction: rows that are much longer as whole eights, and channels or rows with which that kernel or the general one is faster
+OTHERS = [SHAPES[i] for i in (1, 3, 5, 9, 10)]
 
 
 def _weight_gradient(x, dy, shape):
@@ -25,12 +28,14 @@ def _weight_gradient(x, dy, shape):
 
 
 @pytest.mark.parametrize("shape", SHAPES)
-def test_weight_gradient(shape):
+def test_weight_gradient(shape, lib):
     x, wt, b, dy, exact, terms = _problem(shape)
+    lib.dmlhip_debug_last_conv_form()
     _check("dw", _weight_gradient(x, dy, shape), exact[2], terms[2], dy.shape[0] * dy.shape[2] * dy.shape[3])
+    assert lib.dmlhip_debug_last_conv_form() == (-1 if shape in OTHERS else 20)
 
 
-@pytest.mark.parametrize("shape", [SHAPES[0], SHAPES[7], SHAPES[3]])
+@pytest.mark.parametrize("shape", [SHAPES[0], SHAPES[7], SHAPES[3], SHAPES[8]])
 def test_values_without_a_split(shape):
     """Infinities and NaN reach the channels they belong to and no others, a finite value above the largest bf16 stays finite."""
     n, c, h, w, m, s, p, d = shape
@@ -56,7 +61,7 @@ def test_values_without_a_split(shape):
 @pytest.mark.parametrize("exponent", [-112, -120, -128, -140])
 def test_operands_of_every_size(exponent):
     """Operands around and below the smallest normal value keep all of their bits: relative 2-norm error as for any others."""
-    r, shape = rng(11), SHAPES[9]
+    r, shape = rng(11), SHAPES[2]
     n, c, h, w, m, s, p, d = shape
     for small in (0, 1):
         x, dy = r.standard_normal((n, c, h, w)), r.standard_normal((n, m, h, w))
