@@ -12,15 +12,15 @@
 // the loads of the chunks beside them (1 us per step: 8 loads of 4 bytes per lane for a chunk; with the loads left out P = 4 takes
 // 7.3 us, P = 1 2.5 of 3.2), 0.5 us for the stores to LDS and the barriers, and per tile 5 us of first loads and 3 - 9 us of
 // results, which one workgroup per compute unit does not hide. Measured, us forward / data gradient, the kernel of
-// conv_dense3.hip and here: 32x64x56x56 -> 64 82 / 80 and 58 / 57, 32x64x56x56 -> 128 144 / 150 and 112 / 100, 32x128x28x28 -> 128
+// conv_dense3.hip and here: 32x64x56x56 -> 64 82 / 80 and 54 / 54, 32x64x56x56 -> 128 144 / 150 and 104 / 90, 32x128x28x28 -> 128
 // 84 / 83 and 65 / 63, 32x256x14x14 -> 256 107 / 105 and 58 / 56. What the products waited for until it was changed: 64 copies of the
 // activation in the epilogue (12 us per tile), loads behind branches (their addresses in 64 registers, 2 us per step).
 //
 // The large product h h has a sum of its own (P = 1: two), so that the roundings of the five small ones are not roundings of the
 // result: 2 of these for sixteen products instead of 12. Error against fp64 as a share of that of the fp32 instruction (one sum for P = 2 and
 // 4, two for P = 1; 16 - 2048 channels; with all six products in one sum in brackets): normal operands 0.31 - 0.41 (0.83 - 0.87), X
-// behind a ReLU 0.34 - 0.52 (1.08 - 1.20), nothing negative 0.27 - 0.62 (0.9 - 1.7). P = 4 has registers for the small products of one tap only
-// and adds them tap by tap: 51 -> 57 us at 32x64x56x56 -> 64, P = 1 and 2 take the same time as before.
+// behind a ReLU 0.34 - 0.52 (1.08 - 1.20), nothing negative 0.27 - 0.62 (0.9 - 1.7). None takes more than 1 - 2 % longer for it. (P = 4
+// has registers for two such sums. Added after every tap, and not once per step and pair of blocks, they took 5 us of 32x64x56x56 -> 64.)
 #include "bf16_split.h"
 #include "conv_geom.h"
 
@@ -177,11 +177,12 @@ __global__ __launch_bounds__(kThreads, 2) void conv_dense3_split_kernel(const Sp
     floatx16 odd;                                              // P = 1: a second sum, of the odd taps
 #pragma unroll
     for (int e = 0; e < 16; ++e) odd[e] = 0.f;
-    // Sums of the small products: P = 1 and 2 keep them to the end, P = 4 has registers for those of one tap and adds them to acc.
-    constexpr int LOW = P < 4 ? P : 1;
-    floatx16 low[LOW];
+    // Sums of the small products. P = 1 and 2 keep them to the end; P = 4 has registers for two and takes its blocks in two passes over the
+    // taps of a step, which add them to acc.
+    constexpr int PASSES = P == 4 ? 2 : 1, B = P / PASSES;
+    floatx16 low[B];
 #pragma unroll
-    for (int j = 0; j < LOW; ++j)
+    for (int j = 0; j < B; ++j)
 #pragma unroll
         for (int e = 0; e < 16; ++e) low[j][e] = 0.f;
 
@@ -199,32 +200,33 @@ __global__ __launch_bounds__(kThreads, 2) void conv_dense3_split_kernel(const Sp
     // products. Where registers allow, their values are loaded a step ahead, as soon as the registers are free (at the start
     // of the step that splits them, 1 us of it was a wait); elsewhere when the step begins, and are split under the last taps.
     constexpr bool AHEAD = P < 4 && TASKS < 7;
-    constexpr int FIRST = kTaps - TASKS;
     auto step = [&](int next, auto split_c) {                  // next: first channel of the chunks that are loaded
         constexpr bool SPLIT = decltype(split_c)::value;
         Pieces a[2], b[2];
         a[0] = weights_at(0);
         b[0] = pixels_at(0, 0);
-        static_for<0, kTaps>([&](auto tc) {
-            constexpr int tap = decltype(tc)::value, u = tap - FIRST;
+        static_for<0, kTaps * PASSES>([&](auto tc) {
+            constexpr int at = decltype(tc)::value, tap = at % kTaps, pass = at / kTaps, u = at - (kTaps * PASSES - TASKS);
             __builtin_amdgcn_sched_barrier(0);
-            static_for<0, P>([&](auto jc) {
-                constexpr int j = decltype(jc)::value, i = tap * P + j;
-                if constexpr (i + 1 < kTaps * P) {
-                    if constexpr (j + 1 == P) a[(tap + 1) & 1] = weights_at(tap + 1);
-                    b[(i + 1) & 1] = pixels_at((i + 1) % P, (i + 1) / P);
+            static_for<0, B>([&](auto jc) {
+                constexpr int j = decltype(jc)::value, i = at * B + j, n = i + 1;
+                if constexpr (n < kTaps * P) {
+                    if constexpr (j + 1 == B) a[(at + 1) & 1] = weights_at((at + 1) % kTaps);
+                    b[n & 1] = pixels_at(n / B / kTaps * B + n % B, n / B % kTaps);
                 }
-                if constexpr (P == 1 && tap % 2) odd = mfma_large(a[tap & 1], b[i & 1], odd);
-                else acc[j] = mfma_large(a[tap & 1], b[i & 1], acc[j]);
-                if constexpr (P < 4) low[j] = mfma_small(a[tap & 1], b[i & 1], low[j]);
-                else acc[j] += mfma_small(a[tap & 1], b[i & 1], floatx16{});
-                if constexpr (P == 4) asm volatile("" : "+v"(acc[j]));
+                floatx16& large = P == 1 && tap % 2 ? odd : acc[pass * B + j];
+                large = mfma_large(a[at & 1], b[i & 1], large);
+                low[j] = mfma_small(a[at & 1], b[i & 1], P == 4 && tap == 0 ? floatx16{} : low[j]);
+                if constexpr (P == 4 && tap + 1 == kTaps) {
+                    acc[pass * B + j] += low[j];
+                    asm volatile("" : "+v"(acc[pass * B + j]));
+                }
             });
             if constexpr (SPLIT && u >= 0) pieces[u] = split_eight(raw[u]);
 #pragma unroll
-            for (int i = 0; i < 6 * P; ++i) {       // a matrix instruction, then what can issue under it
+            for (int i = 0; i < 6 * B; ++i) {       // a matrix instruction, then what can issue under it
                 __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x2, P == 4 ? 5 : 9 / P, 0);
+                __builtin_amdgcn_sched_group_barrier(0x2, P == 1 ? 9 : P == 2 ? 4 : 5, 0);
             }
             if constexpr (SPLIT && u >= 0) {
                 asm volatile("" : "+v"(pieces[u].h), "+v"(pieces[u].m), "+v"(pieces[u].l));   // computed here, not at the stores
@@ -411,12 +413,12 @@ static bool plan_split(const ConvGeom& g, int ids_h, int ids_w, int most_p, Spli
         if (blocks > (1LL << 22)) continue;
         const double steps = (double)ceil_div(g.c, (int64_t)kCh), rounds = (double)ceil_div(blocks, (int64_t)kCus);
         // us of a tile: first loads and results, and per step; whole rounds of one tile per compute unit. Rounds decide: 32x64x56x56 ->
-        // 64 is one round of 196 tiles of 512 pixels (57 us), two of 392 (58) or four (92), 32x256x14x14 -> 256 one of 196 tiles of 128
-        // (58; of 256 81, of 512 178), 32x96x40x40 -> 96 one of 200 tiles of 512 (77) or two of 400 (74).
+        // 64 is one round of 196 tiles of 512 pixels (54 us), two of 392 (58) or four (92), 32x256x14x14 -> 256 one of 196 tiles of 128
+        // (58; of 256 81, of 512 154).
         // More chunks per thread, larger rectangles, take longer (18 shapes, strides, dilation, 28 - 112 pixels wide).
         const int tasks = (int)ceil_div(kWTasks + 2 * rect, (int64_t)kThreads);
-        const double step = p == 1 ? (tasks <= 4 ? 3.4 : tasks <= 6 ? 4.1 : 4.9) : p == 2 ? (tasks <= 5 ? 4.9 : 6.0) : tasks <= 6 ? 10.3 : 11.0;
-        const double t = rounds * ((p == 1 ? 7.0 : p == 2 ? 9.0 : steps > 1 ? 15.0 : 10.0) + step * steps);
+        const double step = p == 1 ? (tasks <= 4 ? 3.4 : tasks <= 6 ? 4.1 : 4.9) : p == 2 ? (tasks <= 5 ? 4.9 : 6.0) : tasks <= 6 ? 8.9 : 10.2;
+        const double t = rounds * ((p == 1 ? 7.0 : p == 2 ? 9.0 : steps > 1 ? 15.0 : 12.0) + step * steps);
         if (pl->p > 0 && t >= *us) continue;
         *us = t;
         pl->p = p;
