@@ -28,6 +28,7 @@ SOURCES = [
     "gemm_f16_pipe_ilv.hip",
     "gemm_f16_pipe_ragged.hip",
     "gemm_f16_split.hip",
+    "gemm_f16_wide.hip",
     "gemm_f32.hip",
     "gemm_f32_split.hip",
     "conv.hip",

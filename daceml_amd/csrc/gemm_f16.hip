@@ -396,6 +396,18 @@ double estimate_small(int64_t m, int64_t n, int64_t k, long long batch, int pair
     return best_us;
 }
 
+// Whether the workgroups that stay for several 256 x 256 tiles (gemm_f16_wide.h) beat the 128 x 128 tile, as times in us of
+// fixed + tiles per compute unit * (steps * step + what writing a tile takes); a residual is read while nothing is multiplied.
+// Over 120 products of encoder layers (1536 - 16384 tokens, 512 - 1024 wide, every operand layout, groups and operand pairs)
+// the faster of the two is missed by at most 4 % and by 0.1 % in the sum. Decided by it (us, 128-wide tiles or the 256 x 256
+// tile of gemm_f16_pipe.h / here): 4096 x 4096 x 1024 37.5 / 33.4, three of 4096 x 1024 x 1024 36.4 / 34.2, 16384 x 1024 x 4096
+// with residual 120 / 104, three pairs of 16384 x 1024 x 1024 113 / 83, 8192 x 1024 x 4096 77 / 88, 651 x 4096 x 1024 15 / 27.
+bool wide_is_faster(long long t256, long long t128, int64_t k, int pairs, bool residual) {
+    const double steps = (double)(k / BK) * pairs;
+    const double t = (double)ceil_div(t256, (long long)kCus), s = (double)ceil_div(t128, (long long)kCus);
+    return 5.5 + t * (1.33 * steps + (residual ? 12.5 : 6.5)) < 4.0 + s * (0.55 * steps + (residual ? 3.5 : 2.0));
+}
+
 // Diagnostic switches (declared in the public header). Per calling thread, so that one thread pinning a configuration
 // does not change what other threads launch.
 thread_local int g_force_cfg = -1;  // pin the tile configuration
@@ -513,15 +525,19 @@ static int run_gemm_f16(const dmlhip_gemm_desc* d, const void* a, const void* b,
     if (vec) {
         auto blocks = [&](int bm, int bn) { return (long long)ceil_div(d->m, bm) * ceil_div(d->n, bn) * batch; };
         const bool sums = g.asum || (grp && g.gasum[0]);
+        // what the kernel of 256 x 256 tiles in gemm_f16_wide.h takes
+        const bool wide = pipe && !ragged && !sums && g.beta == 0.f && g.act == DMLHIP_ACT_NONE && !pre_out && g.c_vec && d->n % 8 == 0 && d->k * (g.ksum ? g.groups : 1) >= 3 * BK &&
+                          (!bias || g.bias_m || aligned16(bias));
         const bool extra = grp || asum;   // operand pairs / row sums: the 128 x 128 tile only
         const long long t256 = blocks(256, 256), t128 = blocks(128, 128);
         const long long slots256 = ceil_div(t256, (long long)kCus) * kCus, slots128 = ceil_div(t128, (long long)kCus) * kCus;
-        if (cfg < 0 && d->k >= 512 && !extra && t256 * 10 >= slots256 * 9) {
-            // Measured on MI355X, alone and inside the BERT layer (4096 x 4096 x 1024: 39 us against 45 - 54 us for
-            // every 128-wide tile; 8192^3: 1176 TFLOP/s): the 256 x 256 tile halves the bytes each compute unit
-            // pulls through L2 and LDS per MFMA, and the interleaved loop keeps its single wavefront per SIMD
-            // issuing MFMAs while transfers and fragment reads are in flight. Only when its tiles fill (nearly) every
-            // round of compute units: 192 tiles on 256 units lose more than the tile gains.
+        const bool full256 = !extra && t256 * 10 >= slots256 * 9;
+        if (cfg < 0 && d->k >= 512 && wide && (full256 || wide_is_faster(t256, t128, d->k, g.ksum ? g.groups : 1, residual))) {
+            cfg = 13;
+        } else if (cfg < 0 && d->k >= 512 && full256) {
+            // What the kernel above does not take (activations, beta, rows that are not stored in vectors, a ragged K). The
+            // 256 x 256 tile halves the bytes each compute unit pulls through L2 and LDS per MFMA (4096 x 4096 x 1024: 39 us
+            // against 45 - 54 us for every 128-wide tile), as long as its tiles fill (nearly) every round of compute units.
             cfg = 4;
         } else if (cfg < 0 && t128 < 2 * kCus && t128 * 10 < slots128 * 9 && (!pipe || d->k >= 512 || t128 <= kCus)) {
             // rows of C that are not written in vectors hide what the general kernel's longer loop costs: one round only
@@ -553,6 +569,10 @@ static int run_gemm_f16(const dmlhip_gemm_desc* d, const void* a, const void* b,
         }
         const _Float16 *pa = (const _Float16*)a, *pb = (const _Float16*)b;
         g_last_cfg = cfg;
+        if (cfg == 13) {
+            if (wide) return launch_wide(g, pa, pb, c, bias, residual, amode, bmode, batch, st);
+            g_last_cfg = cfg = 4;
+        }
         if (cfg >= 10 && (!sums || amode == 1))
             return launch_split(g, pa, pb, c, bias, residual, pre_out, amode, bmode, cfg, batch, st);
         if (pipe && ragged) return launch_pipelined_ragged(g, pa, pb, c, bias, residual, pre_out, cfg, batch, st);

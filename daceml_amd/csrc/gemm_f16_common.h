@@ -259,6 +259,9 @@ int launch_pipelined_ilv(GemmArgs& g, const _Float16* a, const _Float16* b, void
 // Configurations 4, 5, 7 and 9 with any K, both operands row-contiguous, plain epilogue (row sums on 5 and 7).
 int launch_pipelined_ragged(GemmArgs& g, const _Float16* a, const _Float16* b, void* c, const void* bias, const void* residual,
                             void* pre, int cfg, long long batch, hipStream_t st);
+// Configuration 13 (gemm_f16_wide.h): 256 x 256 tiles, no activation.
+int launch_wide(GemmArgs& g, const _Float16* a, const _Float16* b, void* c, const void* bias, const void* residual, int ak,
+                int bk, long long batch, hipStream_t st);
 // Configurations 10 (64 x 64 tile) and 12 (32 x 32): K split over the wavefronts (gemm_f16_split.hip); any K, every epilogue
 // but EPI_GENERAL_ACT.
 int launch_split(GemmArgs& g, const _Float16* a, const _Float16* b, void* c, const void* bias, const void* residual, void* pre,
