@@ -728,11 +728,44 @@ int dmlhip_gemm_f16_grouped(const dmlhip_gemm_desc* d, int groups, const void* c
     return 0;
 }
 
+// Number of workgroups that share the K steps of a weight gradient's 256 x 256 tile (gemm_f16_wide.h); 0 = other kernels.
+// The fewest us of: both launches 9.5, a step 1.4, 0.3 per MB of partial results (written, read and summed) - against the
+// 128 x 128 tiles' 4 + rounds * (2 + steps * (0.42 + 0.14 where all compute units have one)). Fitted to 96 weight gradients with
+// row sums (1024 - 16384 tokens, 512 - 1024 wide, one product or three or four). us on those / here: 4096 x 1024 over 4096 /
+// 8192 / 16384 tokens 42 / 51, 79 / 75, 153 / 122; 512 x 2048 over 4096 / 16384 34 / 31, 122 / 54; three of 1024 x 1024 over 16384
+// 143 / 100.
+static int weight_gradient_slices(const dmlhip_gemm_desc* d, int groups) {
+    if (d->m <= 0 || d->n <= 0 || d->k <= 0 || d->k % BK || d->m % 8 || d->n % 8 || d->c_stride_m != d->n || !g_direct_lds) return 0;
+    if (d->m > 65536 || d->n > 65536 || (g_force_cfg >= 0 && g_force_cfg != 13)) return 0;
+    const long long t256 = ceil_div(d->m, (int64_t)kWideTile) * ceil_div(d->n, (int64_t)kWideTile) * groups;
+    const long long t128 = ceil_div(d->m, (int64_t)128) * ceil_div(d->n, (int64_t)128) * groups;
+    const long long steps = d->k / BK, most = steps / 3 < kCus / t256 ? steps / 3 : kCus / t256;   // three steps each at least
+    if (most < 2) return 0;
+    if (g_force_cfg == 13) return (int)most;
+    const double mb = 4e-6 * groups * (double)d->m * (double)d->n;
+    double best = 0.93 * (4.0 + (double)ceil_div(t128, (long long)kCus) * (2.0 + steps * (0.42 + 0.14 * fmin(1.0, t128 / (double)kCus))));
+    int slices = 0;
+    for (int s = 2; s <= most; ++s) {
+        const double us = 9.5 + 1.4 * (double)ceil_div(steps, (long long)s) + 0.3 * mb * s;
+        if (us < best) {
+            best = us;
+            slices = s;
+        }
+    }
+    return slices;
+}
+
 size_t dmlhip_gemm_f16_grouped_asum_workspace_bytes(const dmlhip_gemm_desc* d) {
     if (!d) return 0;
     const size_t g = dmlhip_gemm_f16_workspace_bytes(d);
     const size_t r = dmlhip_reduce_workspace_bytes(1, d->k, d->m);
-    return g > r ? g : r;
+    size_t most = g > r ? g : r, row_offset;
+    for (int groups = 1; groups <= DMLHIP_GROUP_MAX; ++groups)
+        if (const int s = weight_gradient_slices(d, groups)) {
+            const size_t w = wide_sliced_bytes(d->m, d->n, groups, s, &row_offset);
+            if (w > most) most = w;
+        }
+    return most;
 }
 
 int dmlhip_gemm_f16_grouped_asum(const dmlhip_gemm_desc* d, int groups, const void* const* a, const void* const* b,
@@ -756,6 +789,30 @@ int dmlhip_gemm_f16_grouped_asum(const dmlhip_gemm_desc* d, int groups, const vo
     bool same = d->k > 0;
     for (int i = 0; i < groups && same; ++i)
         same = aligned16(a[i]) && aligned16(b[i]) && reinterpret_cast<uintptr_t>(c[i]) % 32 == 0;
+    const int slices = same ? weight_gradient_slices(d, groups) : 0;
+    if (slices) {
+        const int64_t one[3] = {1, 1, 1};
+        size_t row_offset;
+        const int amode = operand_mode(a[0], d->m, d->k, d->a_stride_m, d->a_stride_k, d->a_stride_batch, one);
+        const int bmode = operand_mode(b[0], d->n, d->k, d->b_stride_n, d->b_stride_k, d->b_stride_batch, one);
+        if (amode == 1 && bmode != 2 && workspace && aligned16(workspace) &&
+            workspace_bytes >= wide_sliced_bytes(d->m, d->n, groups, slices, &row_offset)) {
+            GemmArgs g{};
+            g.m = (int)d->m; g.n = (int)d->n; g.k = (int)d->k;
+            g.sam = d->a_stride_m; g.sak = d->a_stride_k; g.sbn = d->b_stride_n; g.sbk = d->b_stride_k;
+            g.alpha = d->alpha;
+            g.out_f32 = d->out_dtype == DMLHIP_F32;
+            g.c_vec = 1;
+            g_last_cfg = 13;
+            const _Float16 *ga[DMLHIP_GROUP_MAX], *gb[DMLHIP_GROUP_MAX];
+            for (int i = 0; i < groups; ++i) {
+                ga[i] = (const _Float16*)a[i];
+                gb[i] = (const _Float16*)b[i];
+            }
+            return launch_wide_sliced(g, groups, slices, ga, gb, c, asum, asum_dtype == DMLHIP_F32, bmode, workspace,
+                                      (hipStream_t)stream);
+        }
+    }
     if (same) {
         int e;
         if (groups > 1) {

@@ -259,9 +259,16 @@ int launch_pipelined_ilv(GemmArgs& g, const _Float16* a, const _Float16* b, void
 // Configurations 4, 5, 7 and 9 with any K, both operands row-contiguous, plain epilogue (row sums on 5 and 7).
 int launch_pipelined_ragged(GemmArgs& g, const _Float16* a, const _Float16* b, void* c, const void* bias, const void* residual,
                             void* pre, int cfg, long long batch, hipStream_t st);
+constexpr int kWideTile = 256;   // rows and columns of a tile of gemm_f16_wide.h
 // Configuration 13 (gemm_f16_wide.h): 256 x 256 tiles, no activation.
 int launch_wide(GemmArgs& g, const _Float16* a, const _Float16* b, void* c, const void* bias, const void* residual, int ak,
                 int bk, long long batch, hipStream_t st);
+// Products of few 256 x 256 tiles with A row-contiguous: `slices` workgroups share the K steps of a tile (three each at least),
+// their fp32 results are summed by a second launch, as are the row sums of A where asked for. Dense results, n % 8 == 0.
+// wide_sliced_bytes: what lies in the workspace; the partial row sums begin at *row_offset.
+size_t wide_sliced_bytes(int64_t m, int64_t n, int groups, int slices, size_t* row_offset);
+int launch_wide_sliced(GemmArgs& g, int groups, int slices, const _Float16* const* a, const _Float16* const* b, void* const* c,
+                       void* const* asum, int asum_f32, int bk, void* workspace, hipStream_t st);
 // Configurations 10 (64 x 64 tile) and 12 (32 x 32): K split over the wavefronts (gemm_f16_split.hip); any K, every epilogue
 // but EPI_GENERAL_ACT.
 int launch_split(GemmArgs& g, const _Float16* a, const _Float16* b, void* c, const void* bias, const void* residual, void* pre,

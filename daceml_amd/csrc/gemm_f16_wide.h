@@ -23,6 +23,10 @@
 // RC (rows contiguous): [64 k][256 rows], chunk c (8 rows) of K row k at slot c ^ ((k & 3) << 2) ^ ((k >> 3 & 1) << 1): the
 // transpose read of 16 lanes touches four K rows, 32 bytes of each, the two groups that are read together are eight K rows
 // apart. Neither has bank conflicts.
+//  * SLICED (weight gradients: few tiles, a long K): the workgroups of a tile share its K steps and write fp32 partial results
+//    that wide_sum_kernel adds up, four times over for 64 tiles: 64 MB written and read, about 30 us whatever K is. The row
+//    sums of A (the bias gradient) are taken from the fragments: the workgroups of tile column c add those of every step that
+//    leaves c modulo the number of columns, so that none of them falls behind the others.
 // Requirements (checked by the host): K % 64 == 0 and at least three steps, no activation, beta == 0, n % 8 == 0, 16-byte aligned operands, column
 // bias and result rows, 32-bit element offsets, rows % 8 == 0 for RC operands.
 #pragma once
@@ -33,7 +37,6 @@ namespace dml {
 namespace gemm16 {
 namespace {
 
-constexpr int kWideTile = 256;
 constexpr int kWideOperand = kWideTile * kRowBytes;   // bytes of one operand's tile: 32 KB
 constexpr int kWideLds = 5 * kWideOperand;            // two of A, three of B
 
@@ -144,7 +147,7 @@ __device__ __forceinline__ void* uniform(const void* p) {
 
 // Where a tile is and what its operands' transfers read: all of it uniform.
 struct WideTile {
-    int m0, n0, z0;
+    int m0, n0, z0, z1;
     int64_t aoff, boff, coff;   // element offsets of the batch entry
 };
 
@@ -170,18 +173,18 @@ __device__ __forceinline__ WideTile wide_tile(const GemmArgs& g, uint32_t bid) {
     WideTile t;
     t.m0 = (int)(group * kGroupM + (in_group - tn * rows_here)) * kWideTile;
     t.n0 = (int)tn * kWideTile;
-    int z1 = 0, z2 = 0;
-    t.z0 = 0;
+    int z2 = 0;
+    t.z0 = t.z1 = 0;
     if (batch != 0) {
         const uint32_t b2 = (uint32_t)g.batch2, b1 = (uint32_t)g.batch1;
         const uint32_t q = batch / b2;
         z2 = (int)(batch - q * b2);
         t.z0 = (int)(q / b1);
-        z1 = (int)(q - (uint32_t)t.z0 * b1);
+        t.z1 = (int)(q - (uint32_t)t.z0 * b1);
     }
-    t.aoff = t.z0 * g.sab[0] + z1 * g.sab[1] + z2 * g.sab[2];
-    t.boff = t.z0 * g.sbb[0] + z1 * g.sbb[1] + z2 * g.sbb[2];
-    t.coff = t.z0 * g.scb[0] + z1 * g.scb[1] + z2 * g.scb[2];
+    t.aoff = t.z0 * g.sab[0] + t.z1 * g.sab[1] + z2 * g.sab[2];
+    t.boff = t.z0 * g.sbb[0] + t.z1 * g.sbb[1] + z2 * g.sbb[2];
+    t.coff = t.z0 * g.scb[0] + t.z1 * g.scb[1] + z2 * g.scb[2];
     return t;
 }
 
@@ -296,7 +299,9 @@ __device__ __forceinline__ void wide_epilogue(const GemmArgs& g, void* c_ptr, co
     });
 }
 
-template <int AKIND, int BKIND, int EPI, bool KSUM>
+// SLICED: the inner batch index z1 counts g.batch1 slices of K (its operand strides are 0); g.asum, if any, receives the partial
+// row sums [z0][z1][tile column][2][m] in fp32.
+template <int AKIND, int BKIND, int EPI, bool KSUM, bool SLICED = false>
 __global__ __launch_bounds__(kThreads) void gemm_f16_wide_kernel(const _Float16* a_ptr, const _Float16* b_ptr, void* c_ptr,
                                                                  const void* bias_ptr, const void* res_ptr, const GemmArgs g) {
 #if defined(__HIP_DEVICE_COMPILE__)   // buffer descriptors exist on the device only
@@ -313,16 +318,22 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_wide_kernel(const _Float16*
     oa.fragments(lds0, wm * 128, lane);
     ob.fragments(lds0 + 2 * kWideOperand, wn * 128, lane);
 
+    static_assert(!SLICED || (AKIND == 1 && EPI == EPI_PLAIN && !KSUM), "slices are for weight gradients");
     const int nkg = g.k / BK;                       // steps of one operand pair
-    const int nk = KSUM ? nkg * g.groups : nkg;     // steps of a tile
+    auto slice_begin = [&](int z1) { return (int)((uint32_t)nkg * (uint32_t)z1 / (uint32_t)g.batch1); };
     uint32_t bid = blockIdx.x;
     const uint32_t total = (uint32_t)g.total_blocks;
 
     // ---- what the transfers read: two steps ahead of the MFMAs, past the end of a tile the first steps of the next one
     __amdgpu_buffer_rsrc_t ra, rb;
-    int fk = 0, fgrp = 0, rows_a = 0, rows_b = 0;
+    int fk = 0, fend = nkg, fgrp = 0, rows_a = 0, rows_b = 0;
     auto point_at = [&](uint32_t at) {
         const WideTile ft = wide_tile(g, at);
+        fk = 0;
+        if constexpr (SLICED) {
+            fk = slice_begin(ft.z1);
+            fend = slice_begin(ft.z1 + 1);
+        }
         const _Float16 *a = a_ptr, *b = b_ptr;
         if constexpr (KSUM) {
             // constant indices: the table stays in the kernel-argument segment
@@ -362,8 +373,7 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_wide_kernel(const _Float16*
     };
     // the next step of this tile, or the first of the next one (of the last one: nothing is sent any more)
     auto advance = [&]() {
-        if (++fk != nkg) return;
-        fk = 0;
+        if (++fk != fend) return;
         if (KSUM && ++fgrp != g.groups) {
             point_at(bid);
             return;
@@ -392,6 +402,8 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_wide_kernel(const _Float16*
 
     floatx4 acc[T][T];
     int as = 0, bs = 0;   // stages of the step that is multiplied
+    float row_sum[SLICED ? T : 1];   // row lane % 16 of every block, the k of this lane's fragments
+    int sum_in = -1;                 // steps until this workgroup sums fragments again
     // FIRST: of a tile. FILL: the step two ahead exists and is sent. MORE: the next step exists, its first fragments are read.
     auto step = [&](auto first_c, auto fill_c, auto more_c) {
         constexpr bool FIRST = decltype(first_c)::value, FILL = decltype(fill_c)::value, MORE = decltype(more_c)::value;
@@ -422,7 +434,22 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_wide_kernel(const _Float16*
                 }
                 __builtin_amdgcn_sched_barrier(0);
             });
+            // the two wavefronts that share these rows of A take one half of the step each
+            if constexpr (SLICED) {
+                if (sum_in == 0 && wn == s) {
+                    const half2v one2 = {(_Float16)1.0f, (_Float16)1.0f};
+#pragma unroll
+                    for (int i = 0; i < T; ++i)
+#pragma unroll
+                        for (int e = 0; e < 8; e += 2) {
+                            const half2v p = {af[s][i][e], af[s][i][e + 1]};
+                            row_sum[i] = __builtin_amdgcn_fdot2(p, one2, row_sum[i], false);
+                        }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
         });
+        if constexpr (SLICED) sum_in = sum_in == 0 ? g.tiles_n - 1 : sum_in - 1;
         if constexpr (FILL) advance();
         as = an;
         bs = bn;
@@ -432,6 +459,14 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_wide_kernel(const _Float16*
     using no = std::false_type;
     for (;;) {
         const bool last = bid + gridDim.x >= total;
+        const WideTile t = wide_tile(g, bid);
+        int nk = KSUM ? nkg * g.groups : nkg;
+        if constexpr (SLICED) {
+            nk = slice_begin(t.z1 + 1) - slice_begin(t.z1);
+            sum_in = g.asum ? t.n0 / kWideTile : -1;
+#pragma unroll
+            for (int i = 0; i < T; ++i) row_sum[i] = 0.f;
+        }
         const int fills = last ? nk - 2 : nk;
         step(yes{}, yes{}, yes{});
         for (int kt = 1; kt < fills; ++kt) step(no{}, yes{}, yes{});
@@ -443,7 +478,6 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_wide_kernel(const _Float16*
         // and the next tile's first fragments are in their registers before the epilogue may use others around them
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_nop 15\n\ts_nop 3" ::: "memory");
         if (last && g.trace && threadIdx.x == 0) g.trace[4 * (size_t)blockIdx.x + 2] = wall_clock64();
-        const WideTile t = wide_tile(g, bid);
         void* c = c_ptr;
         const void* bias = bias_ptr;
         if (!KSUM && g.groups) {
@@ -453,6 +487,20 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_wide_kernel(const _Float16*
         const int mb = t.m0 + wm * 128, nb = t.n0 + wn * 128;
         if (g.out_f32) wide_epilogue<float, EPI>(g, c, res_ptr, bias, acc, mb, nb, t.coff, lane, last);
         else wide_epilogue<_Float16, EPI>(g, c, res_ptr, bias, acc, mb, nb, t.coff, lane, last);
+        if constexpr (SLICED) {
+            if (g.asum) {
+                float* const sums = reinterpret_cast<float*>(g.asum) +
+                                    ((((int64_t)t.z0 * g.batch1 + t.z1) * g.tiles_n + t.n0 / kWideTile) * 2 + wn) * g.m;
+#pragma unroll
+                for (int i = 0; i < T; ++i) {
+                    float v = row_sum[i];
+                    v += __shfl_xor(v, 16);
+                    v += __shfl_xor(v, 32);
+                    const int m = mb + i * 16 + lane;
+                    if (lane < 16 && m < g.m) sums[m] = v;
+                }
+            }
+        }
         if (last) break;
         bid += gridDim.x;
     }
@@ -461,6 +509,53 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_wide_kernel(const _Float16*
         g.trace[4 * (size_t)blockIdx.x + 3] = wall_clock64();
     }
 #endif
+}
+
+// Adds up what SLICED left: blocks of 1024 results each, behind them (asum) blocks of 64 row sums; the group in blockIdx.y.
+// Reads of 4 bytes per result and slice and the result's own: 3.3 TB/s behind the product, 80 MB in 24 us.
+struct WideSumArgs {
+    const float* part;        // [groups][slices][count]
+    const float* row_part;    // [groups][row_parts][m]
+    int slices, row_parts, m, out_f32, asum_f32;
+    int64_t count;
+    float alpha;
+    void* out[DMLHIP_GROUP_MAX];
+    void* asum[DMLHIP_GROUP_MAX];
+};
+
+__global__ __launch_bounds__(256) void wide_sum_kernel(const WideSumArgs g, int blocks) {
+    const int z = blockIdx.y;
+    if ((int)blockIdx.x < blocks) {
+        const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+        if (i >= g.count) return;
+        const float* p = g.part + (int64_t)z * g.slices * g.count + i;
+        floatx4 acc = *reinterpret_cast<const floatx4*>(p);
+#pragma unroll 4
+        for (int s = 1; s < g.slices; ++s) acc += *reinterpret_cast<const floatx4*>(p + (int64_t)s * g.count);
+        acc *= g.alpha;
+        if (g.out_f32) {
+            *reinterpret_cast<floatx4*>(reinterpret_cast<float*>(g.out[z]) + i) = acc;
+        } else {
+            const half4v h = {(_Float16)acc[0], (_Float16)acc[1], (_Float16)acc[2], (_Float16)acc[3]};
+            *reinterpret_cast<half4v*>(reinterpret_cast<_Float16*>(g.out[z]) + i) = h;
+        }
+        return;
+    }
+    __shared__ float share[256];
+    const int row = ((int)blockIdx.x - blocks) * 64 + (threadIdx.x & 63);
+    float v = 0.f;
+    if (row < g.m) {
+        const float* p = g.row_part + (int64_t)z * g.row_parts * g.m + row;
+#pragma unroll 4
+        for (int q = threadIdx.x >> 6; q < g.row_parts; q += 4) v += p[(int64_t)q * g.m];
+    }
+    share[threadIdx.x] = v;
+    __syncthreads();
+    if (threadIdx.x < 64 && row < g.m) {
+        v = (share[threadIdx.x] + share[threadIdx.x + 64]) + (share[threadIdx.x + 128] + share[threadIdx.x + 192]);
+        if (g.asum_f32) reinterpret_cast<float*>(g.asum[z])[row] = v;
+        else reinterpret_cast<_Float16*>(g.asum[z])[row] = (_Float16)v;
+    }
 }
 
 }  // namespace

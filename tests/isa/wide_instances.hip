@@ -6,9 +6,10 @@ namespace dml {
 namespace gemm16 {
 
 const void* wide_gemm_kernels[] = {
-    // A kind, B kind, epilogue, K-concatenated pairs
+    // A kind, B kind, epilogue, K-concatenated pairs, K in slices
     (const void*)gemm_f16_wide_kernel<0, 0, EPI_PLAIN, false>, (const void*)gemm_f16_wide_kernel<0, 0, EPI_GENERAL, false>,
-    (const void*)gemm_f16_wide_kernel<1, 1, EPI_PLAIN, false>, (const void*)gemm_f16_wide_kernel<0, 1, EPI_GENERAL, true>};
+    (const void*)gemm_f16_wide_kernel<1, 1, EPI_PLAIN, false>, (const void*)gemm_f16_wide_kernel<0, 1, EPI_GENERAL, true>,
+    (const void*)gemm_f16_wide_kernel<1, 1, EPI_PLAIN, false, true>};
 
 }  // namespace gemm16
 }  // namespace dml

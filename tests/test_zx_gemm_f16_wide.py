@@ -86,3 +86,47 @@ def test_several_tiles_per_workgroup(layouts, m, n, batch, lib):
     lib.dmlhip_debug_force_gemm_config(13)
     L.check(lib.dmlhip_gemm_f16(ctypes.byref(d), P(a), P(b), P(c), None, None, None, K._stream()))
     assert torch.equal(c, got.half())
+
+
+@pytest.mark.parametrize("m,n,k,groups,layout", [(8, 8, 64 * 6, 1, 1), (264, 520, 64 * 13, 3, 1), (256, 512, 64 * 50, 2, 1), (520, 136, 64 * 11, 4, 0),
+                                                 (136, 264, 64 * 70, 1, 1)])
+@pytest.mark.parametrize("sum_dtype", [torch.float32, torch.float16])
+def test_weight_gradients_in_slices(m, n, k, groups, layout, sum_dtype, lib):
+    """Products [k, m]^T [k, n] whose tiles are shared by several workgroups, with the column sums of the first operand: uneven
+    slices, more columns of tiles than steps per slice and fewer; a workspace that is too small runs the other kernels."""
+    from daceml_amd import _lib as L, kernels as K
+    r = rng(m + n + k)
+    ops = [(_operand(r, m, k, 1), _operand(r, n, k, layout)) for _ in range(groups)]
+    A, B = [o[0][1] for o in ops], [o[1][1] for o in ops]
+    code = {torch.float32: L.F32, torch.float16: L.F16}[sum_dtype]
+    eps = {torch.float32: 2.0 ** -24, torch.float16: 2.0 ** -11}
+    for dtype in (torch.float32, torch.float16):
+        d = _desc(L, m, n, k, (1, m), (k, 1) if layout == 0 else (1, n), L.F32 if dtype == torch.float32 else L.F16)
+        lib.dmlhip_debug_force_gemm_config(13)
+        need = lib.dmlhip_gemm_f16_grouped_asum_workspace_bytes(ctypes.byref(d))
+        assert need >= 2 * groups * m * n * 4
+        ws = torch.full((need, ), 255, dtype=torch.uint8, device="cuda")   # NaN wherever it is read before it is written
+        C = [torch.full((m, n), float("nan"), device="cuda", dtype=dtype) for _ in ops]
+        S = [torch.full((m, ), float("nan"), device="cuda", dtype=sum_dtype) for _ in ops]
+        L.check(lib.dmlhip_gemm_f16_grouped_asum(ctypes.byref(d), groups, _table(A), _table(B), _table(C), _table(S), code, P(ws), need, K._stream()))
+        assert lib.dmlhip_debug_last_gemm_config() == 13
+        for ((a, _, _), (b, _, _)), c, s in zip(ops, C, S):
+            exact, terms = _products([(a, b)])
+            _check(c, exact, terms, k, eps[dtype], 0, (m, n, k, dtype))
+            _check(s, a.astype(np.float64).sum(1), np.abs(a).astype(np.float64).sum(1), k, eps[sum_dtype], 0, ("sums", m, k))
+        if layout == 1:
+            lib.dmlhip_debug_force_gemm_config(-1)
+            small = [torch.full((m, n), float("nan"), device="cuda", dtype=dtype) for _ in ops]
+            L.check(lib.dmlhip_gemm_f16_grouped_asum(ctypes.byref(d), groups, _table(A), _table(B), _table(small), _table(S), code, P(ws), 16, K._stream()))
+            for ((a, _, _), (b, _, _)), c in zip(ops, small):
+                exact, terms = _products([(a, b)])
+                _check(c, exact, terms, k, eps[dtype], 0, ("small workspace", m, n, k, dtype))
+
+
+@pytest.mark.parametrize("m,n,k,groups,sliced", [(1024, 4096, 16384, 1, True), (1024, 4096, 2048, 1, False), (512, 2048, 4096, 1, True),
+                                                 (1024, 1024, 16384, 4, True), (768, 3072, 1024, 1, False)])
+def test_which_weight_gradients_are_sliced(m, n, k, groups, sliced, lib):
+    """The workspace holds the slices of a long product's results; a short one has none."""
+    from daceml_amd import _lib as L
+    d = _desc(L, m, n, k, (1, m), (1, n), L.F32)
+    assert (lib.dmlhip_gemm_f16_grouped_asum_workspace_bytes(ctypes.byref(d)) >= 2 * groups * m * n * 4) == sliced
