@@ -56,6 +56,19 @@ class AttentionDesc(Structure):
     ]
 
 
+class CallArg(Structure):
+    """struct dmlhip_call_arg"""
+    _fields_ = [("kind", ctypes.c_uint32), ("index", ctypes.c_uint32), ("value", ctypes.c_uint64)]
+
+
+class Call(Structure):
+    """struct dmlhip_call"""
+    _fields_ = [("symbol", c_int), ("argc", c_int), ("args", POINTER(CallArg))]
+
+
+CALL_VALUE, CALL_POINTER, CALL_STREAM, CALL_TABLE = range(4)
+CALL_TABLE_MAX = 16
+
 _P = c_void_p
 _I64P = POINTER(c_int64)
 
@@ -147,6 +160,8 @@ SIGNATURES = {
     "dmlhip_attention_masked_f16": (c_int, [POINTER(AttentionDesc), _P, _P, _P, _P, _I64P, _P, _P, _P]),
     "dmlhip_attention_masked_backward_f16": (c_int, [POINTER(AttentionDesc), POINTER(AttentionDesc), _P, _P, _P, _P, _I64P,
                                                      _P, _P, _P, _P, _P, _P, _P, c_size_t, _P]),
+    "dmlhip_call_symbol": (c_int, [c_char_p]),
+    "dmlhip_run_calls": (c_int, [POINTER(Call), c_int, POINTER(ctypes.c_uint64), _P, POINTER(c_int)]),
     # diagnostics (switches for tests and measurements, declared at the end of the header)
     "dmlhip_conv2d_expand_depthwise_lds_bytes": (c_size_t, [c_int64, c_int64, c_int64]),
     "dmlhip_debug_force_gemm_config": (None, [c_int]),

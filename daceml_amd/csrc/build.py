@@ -17,6 +17,7 @@ OBJ_DIR = os.path.join(HERE, "build")
 
 SOURCES = [
     "common.cpp",
+    "call_list.cpp",
     "rowwise.hip",
     "elementwise.hip",
     "reduce.hip",

@@ -7,13 +7,13 @@ transients are owned by the SDFG and allocated once, caller arrays are passed pe
 is enqueued on the caller's current stream without synchronising (the ``nosync`` states of
 ctypes_module.py:210-211).
 
-Binding is done once: each launch becomes ``(ctypes function, tuple of ctypes arguments)``. Pointers of
-caller-owned arrays live in shared mutable ``c_void_p`` objects that are updated on every call, so the
-steady state is one ctypes call per kernel and no Python-side planning.
+Binding is done once: the launches become one call list in native memory (dmlhip_run_calls), whose pointer arguments are
+numbers of arrays and byte offsets. The arrays' addresses live in one table that is updated on every call, so the steady
+state is one native call per state and no Python-side planning.
 """
 import ctypes
 import logging
-from typing import Dict, List, Optional, Sequence
+from typing import Dict, List, Optional, Sequence, Tuple
 
 import torch
 
@@ -83,10 +83,10 @@ def forwarded_transients(sdfg: SDFG, forward_states: Sequence[str], backward_sta
 
 
 class _Launch:
-    __slots__ = ("fn", "args", "label", "symbol", "flops", "bytes_moved", "kind", "state")
+    __slots__ = ("number", "args", "label", "symbol", "flops", "bytes_moved", "kind", "state")
 
-    def __init__(self, fn, args, label, symbol, flops, bytes_moved, kind, state):
-        self.fn, self.args, self.label, self.symbol = fn, args, label, symbol
+    def __init__(self, number, args, label, symbol, flops, bytes_moved, kind, state):
+        self.number, self.args, self.label, self.symbol = number, args, label, symbol
         self.flops, self.bytes_moved, self.kind, self.state = flops, bytes_moved, kind, state
 
 
@@ -125,10 +125,10 @@ class CompiledSDFG:
         if expand:
             expand_onnx_nodes(sdfg)
         self._keep = []                       # ctypes objects that must outlive the launches
-        self._ptr: Dict[str, ctypes.c_void_p] = {}
-        self._derived = []                    # (c_void_p, c_void_p of the base, byte offset)
-        self._ptr_arrays = []                 # (ctypes array, [(slot, c_void_p)])
-        self._stream = ctypes.c_void_p(0)
+        #: addresses of the arrays that are no views; array -> (number there, byte offset)
+        self.pointers = (ctypes.c_uint64 * max(len(sdfg.arrays), 1))()
+        self._place: Dict[str, Tuple[int, int]] = {}
+        self._native: Dict[Optional[tuple], tuple] = {}   # states -> call list
         self._binding = 0                     # bumped whenever a pointer may have changed
         self.buffers: Dict[str, torch.Tensor] = {}
         # [(state, node)]: the order the kernels are enqueued in
@@ -144,18 +144,27 @@ class CompiledSDFG:
         self._workspace = torch.empty(self._ws_bytes, dtype=torch.uint8, device=self.device)
         for state, node in self._order:
             self._bind_node(state, node)
+        self._calls = (L.Call * max(len(self._launches), 1))()
+        for call, l in zip(self._calls, self._launches):
+            call.symbol, call.argc, call.args = l.number, len(l.args), l.args
         # what a call has to pass, looked up once: a small program's step is bound by what the host does per call
-        self._arguments = [(name, self._ptr[name], d.dtype, d.shape, d.strides) for name, d in self.arglist().items()]
-        self._refresh()
+        self._arguments = [(name, self._place[name][0], d.dtype, d.shape, d.strides) for name, d in self.arglist().items()]
+        self.rebound()
 
     # -- memory ------------------------------------------------------------
     def _allocate(self):
+        for i, (name, desc) in enumerate(self.sdfg.arrays.items()):
+            self._place[name] = (i, 0)
         for name, desc in self.sdfg.arrays.items():
-            self._ptr[name] = ctypes.c_void_p(0)
+            at, offset = name, 0
+            while self.sdfg.arrays[at].view_of is not None:
+                offset += self.sdfg.arrays[at].view_offset * _ITEM[self.sdfg.arrays[at].dtype]
+                at = self.sdfg.arrays[at].view_of
+            self._place[name] = (self._place[at][0], offset)
         for name, desc in self.sdfg.arrays.items():
             if desc.view_of is not None:
-                self._derived.append((self._ptr[name], self._ptr[desc.view_of], desc.view_offset * _ITEM[desc.dtype]))
-            elif name in self.sdfg.constants:
+                continue
+            if name in self.sdfg.constants:
                 t = self.sdfg.constants[name].to(device=self.device, dtype=desc.dtype).contiguous()
                 if tuple(t.shape) != desc.shape:
                     raise ValueError("constant %r has shape %s, descriptor says %s" % (name, tuple(t.shape), desc.shape))
@@ -175,15 +184,23 @@ class CompiledSDFG:
             else:
                 self.buffers[name] = torch.empty(desc.shape, dtype=desc.dtype, device=self.device)
         for name, t in self.buffers.items():
-            self._ptr[name].value = t.data_ptr()
+            self.pointers[self._place[name][0]] = t.data_ptr()
 
-    def _refresh(self):
+    def slot(self, name: str) -> int:
+        """Where ``pointers`` holds the address of an array that is no view. Whoever writes it has checked the tensor
+        (``check_argument``), keeps it alive until the launches that use it have been enqueued and calls ``rebound``."""
+        if self.sdfg.arrays[name].view_of is not None:
+            raise ValueError("%r is a view" % name)
+        return self._place[name][0]
+
+    def rebound(self):
+        """An address in ``pointers`` has changed."""
         self._binding += 1
-        for obj, base, off in self._derived:
-            obj.value = (base.value or 0) + off
-        for arr, slots in self._ptr_arrays:
-            for i, ptr in slots:
-                arr[i] = ptr.value
+
+    def _address(self, name: str, offset: int) -> Tuple[int, int]:
+        """(number in ``pointers``, bytes behind that address) of an array's element."""
+        number, start = self._place[name]
+        return number, start + offset * _ITEM[self.sdfg.arrays[name].dtype]
 
     # -- binding -----------------------------------------------------------
     def _bind_node(self, state: SDFGState, node):
@@ -198,80 +215,83 @@ class CompiledSDFG:
         for e in state.out_edges(node):
             conn_to_array[e.src_conn] = e.data.data
         for call in calls:
-            fn = getattr(self.lib, call.symbol)
-            args = []
-            for a in call.args:
+            symbol = self.lib.dmlhip_call_symbol(call.symbol.encode())
+            if symbol < 0:
+                raise RuntimeError("%s cannot be part of a call list" % call.symbol)
+            args = (L.CallArg * len(call.args))()
+            for word, a in zip(args, call.args):
                 if isinstance(a, T.Ptr):
-                    name = conn_to_array[a.conn]
-                    if a.offset:
-                        obj = ctypes.c_void_p(0)
-                        self._derived.append((obj, self._ptr[name], a.offset * _ITEM[self.sdfg.arrays[name].dtype]))
-                        args.append(obj)
-                    else:
-                        args.append(self._ptr[name])
+                    word.kind = L.CALL_POINTER
+                    word.index, word.value = self._address(conn_to_array[a.conn], a.offset)
                 elif isinstance(a, T.Null):
-                    # None, not c_void_p(0): for a POINTER(c_void_p) parameter ctypes would pass the ADDRESS of a
-                    # c_void_p instance (a non-NULL pointer table with one NULL entry)
-                    args.append(None)
-                elif isinstance(a, T.I64):
-                    args.append(ctypes.c_int64(a.value))
-                elif isinstance(a, T.I32):
-                    args.append(ctypes.c_int(a.value))
+                    pass                      # a value: NULL
+                elif isinstance(a, (T.I64, T.I32, T.USize)):
+                    word.value = a.value & 0xffffffffffffffff
                 elif isinstance(a, T.F32):
-                    args.append(ctypes.c_float(a.value))
-                elif isinstance(a, T.USize):
-                    args.append(ctypes.c_size_t(a.value))
+                    word.value = ctypes.c_uint32.from_buffer(ctypes.c_float(a.value)).value
                 elif isinstance(a, T.I64Array):
                     arr = (ctypes.c_int64 * max(len(a.values), 1))(*a.values)
                     self._keep.append(arr)
-                    args.append(arr)
+                    word.value = ctypes.addressof(arr)
                 elif isinstance(a, T.PtrArray):
-                    arr = (ctypes.c_void_p * len(a.conns))()
-                    self._ptr_arrays.append((arr, [(i, self._ptr[conn_to_array[c]]) for i, c in enumerate(a.conns)]))
-                    args.append(arr)
+                    if len(a.conns) > L.CALL_TABLE_MAX:
+                        raise RuntimeError("%s: a table of %d pointers" % (call.symbol, len(a.conns)))
+                    entries = (L.CallArg * max(len(a.conns), 1))()
+                    for e, c in zip(entries, a.conns):
+                        e.index, e.value = self._address(conn_to_array[c], 0)
+                    self._keep.append(entries)
+                    word.kind, word.index, word.value = L.CALL_TABLE, len(a.conns), ctypes.addressof(entries)
                 elif isinstance(a, T.Struct):
                     self._keep.append(a.value)
-                    args.append(ctypes.byref(a.value))
+                    word.value = ctypes.addressof(a.value)
                 elif isinstance(a, T.Workspace):
-                    args.append(ctypes.c_void_p(self._workspace.data_ptr() + a.offset))
+                    word.value = self._workspace.data_ptr() + a.offset
                 elif isinstance(a, T.WorkspaceBytes):
-                    args.append(ctypes.c_size_t(self._ws_bytes - a.offset))
+                    word.value = self._ws_bytes - a.offset
                 elif isinstance(a, T.Stream):
-                    args.append(self._stream)
+                    word.kind = L.CALL_STREAM
                 else:
                     raise TypeError("unknown HIP call argument %r" % (a, ))
             # work is attributed to the node's first call only (later calls are follow-up passes)
             first = call is calls[0]
             flops = call.flops if call.flops is not None else (node.flops if first else 0)
             moved = call.bytes_moved if call.bytes_moved is not None else (node.bytes_moved if first else 0)
-            self._launches.append(_Launch(fn, tuple(args), node.label, call.symbol, flops, moved, node.kind, state.label))
+            self._launches.append(_Launch(symbol, args, node.label, call.symbol, flops, moved, node.kind, state.label))
 
     # -- execution -----------------------------------------------------------
     def _bind_arguments(self, kwargs: Dict[str, torch.Tensor], partial: bool = False):
         found = []
-        for name, ptr, dtype, shape, strides in self._arguments:
-            if name not in kwargs:
+        device = self.device
+        for name, slot, dtype, shape, strides in self._arguments:
+            t = kwargs.get(name)
+            if t is None and name not in kwargs:
                 if partial:
                     continue
                 raise TypeError("missing argument %r (arrays to pass: %s)" % (name, sorted(self.arglist())))
-            t = kwargs[name]
-            if not isinstance(t, torch.Tensor) or t.device != self.device:
-                raise ValueError("argument %r must be a tensor on %s" % (name, self.device))
-            if t.dtype != dtype or t.shape != shape:
-                raise ValueError("argument %r: expected %s %s, got %s %s" % (name, dtype, shape, t.dtype, tuple(t.shape)))
-            if t.stride() != strides and t.numel() > 1:
-                raise ValueError("argument %r must have strides %s (pass a contiguous tensor)" % (name, strides))
-            found.append((ptr, t.data_ptr()))
-        for name in kwargs:
-            if name not in self.sdfg.arrays:
-                raise TypeError("unknown argument(s) %s" % sorted(set(kwargs) - set(self.sdfg.arrays)))
-        changed = False   # a refused call has changed nothing: the derived pointers are those of the last binding
-        for ptr, address in found:
-            if (ptr.value or 0) != address:   # a c_void_p that holds NULL reads as None
-                ptr.value = address
+            if not isinstance(t, torch.Tensor) or t.device != device or t.dtype != dtype or t.shape != shape \
+                    or (t.stride() != strides and t.numel() > 1):
+                self.check_argument(name, t)
+            found.append((slot, t.data_ptr()))
+        if not kwargs.keys() <= self.sdfg.arrays.keys():
+            raise TypeError("unknown argument(s) %s" % sorted(set(kwargs) - set(self.sdfg.arrays)))
+        changed = False   # a refused call has changed nothing
+        pointers = self.pointers
+        for slot, address in found:
+            if pointers[slot] != address:
+                pointers[slot] = address
                 changed = True
         if changed:
-            self._refresh()
+            self.rebound()
+
+    def check_argument(self, name: str, t):
+        """Raises unless `t` can be bound to the array."""
+        d = self.sdfg.arrays[name]
+        if not isinstance(t, torch.Tensor) or t.device != self.device:
+            raise ValueError("argument %r must be a tensor on %s" % (name, self.device))
+        if t.dtype != d.dtype or t.shape != d.shape:
+            raise ValueError("argument %r: expected %s %s, got %s %s" % (name, d.dtype, d.shape, t.dtype, tuple(t.shape)))
+        if t.stride() != d.strides and t.numel() > 1:
+            raise ValueError("argument %r must have strides %s (pass a contiguous tensor)" % (name, d.strides))
 
     def arglist(self) -> Dict[str, Array]:
         return {k: v for k, v in self.sdfg.arrays.items()
@@ -302,22 +322,35 @@ class CompiledSDFG:
                 raise ValueError("buffer for %r must be a dense %s %s tensor on %s" % (name, desc.dtype, desc.shape,
                                                                                         self.device))
         for name, t in tensors.items():
-            self._ptr[name].value = t.data_ptr()
+            self.pointers[self._place[name][0]] = t.data_ptr()
             if release:
                 self.buffers[name] = t
         if tensors:
-            self._refresh()
+            self.rebound()
 
     def launch(self, states: Optional[Sequence[str]] = None):
         """Enqueue every kernel (of the named states) on the current stream, with the pointers of the
         last binding."""
-        self._stream.value = torch.cuda.current_stream(self.device).cuda_stream
-        for l in self._launches:
-            if states is not None and l.state not in states:
-                continue
-            status = l.fn(*l.args)
-            if status != 0:
-                raise L.HipKernelError(status, "%s (%s): %s" % (l.label, l.symbol, L.last_error()))
+        key = None if states is None else tuple(states)
+        native = self._native.get(key)
+        if native is None:
+            native = self._native[key] = self._selected(key)
+        launches, calls, count = native
+        failed = ctypes.c_int(-1)
+        status = self.lib.dmlhip_run_calls(calls, count, self.pointers, torch.cuda.current_stream(self.device).cuda_stream, failed)
+        if status != 0:
+            l = launches[failed.value]
+            raise L.HipKernelError(status, "%s (%s): %s" % (l.label, l.symbol, L.last_error()))
+
+    def _selected(self, states: Optional[tuple]):
+        """(launches, their call list, how many) of the named states."""
+        numbers = [i for i, l in enumerate(self._launches) if states is None or l.state in states]
+        if numbers == list(range(numbers[0], numbers[-1] + 1)) if numbers else True:   # one run of the program's own list
+            first = numbers[0] if numbers else 0
+            calls = ctypes.cast(ctypes.addressof(self._calls) + first * ctypes.sizeof(L.Call), ctypes.POINTER(L.Call))
+        else:
+            calls = (L.Call * len(numbers))(*[self._calls[i] for i in numbers])
+        return [self._launches[i] for i in numbers], calls, len(numbers)
 
     def capture(self, states: Optional[Sequence[str]] = None, warmup: int = 2) -> "CapturedLaunches":
         """The launches (of the named states) with the pointers of the current binding, recorded once into a HIP graph:
@@ -342,11 +375,12 @@ class CompiledSDFG:
         returns [(launch, ms)] where a launch's time runs from the event before it to the event after it - the kernel
         and its dispatch on the stream. The times add up to the time of the whole sequence between the first and the
         last event."""
-        self._stream.value = torch.cuda.current_stream(self.device).cuda_stream
+        stream = torch.cuda.current_stream(self.device).cuda_stream
         marks = [torch.cuda.Event(enable_timing=True)]
         marks[0].record()
-        for l in self._launches:
-            status = l.fn(*l.args)
+        for i, l in enumerate(self._launches):
+            call = ctypes.cast(ctypes.addressof(self._calls) + i * ctypes.sizeof(L.Call), ctypes.POINTER(L.Call))
+            status = self.lib.dmlhip_run_calls(call, 1, self.pointers, stream, None)
             e = torch.cuda.Event(enable_timing=True)
             e.record()
             marks.append(e)

@@ -237,24 +237,48 @@ class DaceModule(nn.Module):
         forwarded = compiled.forwarded_transients(forward_states, backward_states) if self.backward else []
         self.forwarded_transients = list(forwarded)
 
+        # What a call does per tensor, looked up once: a small module's step is bound by what the host does per call.
+        # (number among the module's tensors, name, number among the program's addresses, type, shape)
+        descs = sdfg.arrays
+        bound_inputs = [(i, name, compiled.slot(name), descs[name].dtype, descs[name].shape)
+                        for i, name in enumerate(in_arrays) if name in arglist]
+        bound_outputs = [(compiled.slot(name) if name in arglist else None, descs[name].dtype, descs[name].shape)
+                         for name in out_arrays]
+        kept_transients = [(name, compiled.slot(name), descs[name].dtype, descs[name].shape) for name in forwarded]
+        # a backward call's own arrays: gradients it is given and makes, and where in the tensors it saw those saved ones are
+        # that it needs (several inputs or outputs of one name: the last, as in a dictionary of them)
+        given_gradients = [(i, "gradient_" + name, compiled.slot("gradient_" + name), descs["gradient_" + name].dtype,
+                            descs["gradient_" + name].shape)
+                           for i, name in enumerate(out_arrays) if "gradient_" + name in arglist]
+        made_gradients = [None if g is None else (compiled.slot(g) if g in arglist else None, descs[g].dtype, descs[g].shape,
+                                                  descs[a].dtype) for g, a in zip(grad_of_input, in_arrays)]
+        saved_slots = [(name, slot, dtype, shape) for _, name, slot, dtype, shape in bound_inputs] + \
+            [(name, slot, dtype, shape) for name, (slot, dtype, shape) in zip(out_arrays, bound_outputs)] + kept_transients
+        pointers = compiled.pointers
+        if not all(descs[name].is_contiguous() for name, *_ in saved_slots):
+            raise ValueError("inputs, outputs and stored tensors are passed dense")
+        integer_outputs = [i for i, name in enumerate(out_arrays) if not descs[name].dtype.is_floating_point]
+
+        def checked(name, t, dtype, shape):
+            """`t`, dense and as the array says; raises where it is something else."""
+            t = t.contiguous()
+            if t.dtype != dtype or t.shape != shape or t.device != device:
+                compiled.check_argument(name, t)
+            return t
+
         def run_forward(tensors, keep=False):
-            call = {}
-            for name, t in zip(in_arrays, tensors):
-                if name in arglist:
-                    call[name] = t.detach().contiguous()
-            outs = []
-            for name in out_arrays:
-                d = sdfg.arrays[name]
-                t = torch.empty(d.shape, dtype=d.dtype, device=device)
-                call[name] = t
-                outs.append(t)
-            compiled.bind(call)
-            saved = {}
-            if keep:
-                for name in forwarded:
-                    d = sdfg.arrays[name]
-                    saved[name] = torch.empty(d.shape, dtype=d.dtype, device=device)
-                compiled.rebind_transients(saved, release=True)
+            call = [checked(name, tensors[i].detach(), dtype, shape) for i, name, _, dtype, shape in bound_inputs]
+            outs = [torch.empty(shape, dtype=dtype, device=device) for _, dtype, shape in bound_outputs]
+            saved = [torch.empty(shape, dtype=dtype, device=device) for _, _, dtype, shape in kept_transients] if keep else []
+            for (_, _, slot, _, _), t in zip(bound_inputs, call):
+                pointers[slot] = t.data_ptr()
+            for (slot, _, _), t in zip(bound_outputs, outs):
+                if slot is not None:
+                    pointers[slot] = t.data_ptr()
+            for (name, slot, _, _), t in zip(kept_transients, saved):
+                pointers[slot] = t.data_ptr()
+                compiled.buffers[name] = t   # in place of the program's own buffer
+            compiled.rebound()
             compiled.launch(forward_states)
             return tuple(outs), call, saved
 
@@ -262,37 +286,30 @@ class DaceModule(nn.Module):
             @staticmethod
             def forward(ctx, *tensors):
                 outs, call, saved = run_forward(tensors, keep=True)
-                ctx.daceml_bound_names = list(call)
-                ctx.daceml_saved_names = list(saved)
-                ctx.save_for_backward(*call.values(), *saved.values())
-                ctx.mark_non_differentiable(*[o for o in outs if not o.dtype.is_floating_point])
+                ctx.save_for_backward(*call, *outs, *saved)
+                ctx.mark_non_differentiable(*[outs[i] for i in integer_outputs])
                 return outs[0] if len(outs) == 1 else outs
 
             @staticmethod
             def backward(ctx, *grad_outputs):
-                kept = ctx.saved_tensors
-                nb = len(ctx.daceml_bound_names)
-                call = dict(zip(ctx.daceml_bound_names, kept[:nb]))
-                compiled.rebind_transients(dict(zip(ctx.daceml_saved_names, kept[nb:])))
-                for name, g in zip(out_arrays, grad_outputs):
-                    gname = "gradient_" + name
-                    if gname not in arglist:
-                        continue
-                    d = sdfg.arrays[gname]
-                    call[gname] = torch.zeros(d.shape, dtype=d.dtype, device=device) if g is None else \
-                        g.to(d.dtype).contiguous()
-                results = []
-                for gname in grad_of_input:
-                    if gname is None:
-                        results.append(None)
-                        continue
-                    d = sdfg.arrays[gname]
-                    t = torch.empty(d.shape, dtype=d.dtype, device=device)
-                    call[gname] = t
-                    results.append(t)
-                compiled.bind(call)
+                call = [checked(name, t, dtype, shape) for t, (name, _, dtype, shape) in zip(ctx.saved_tensors, saved_slots)]
+                gradients = []
+                for i, name, _, dtype, shape in given_gradients:
+                    g = grad_outputs[i]
+                    gradients.append(torch.zeros(shape, dtype=dtype, device=device) if g is None
+                                     else checked(name, g.to(dtype), dtype, shape))
+                results = [None if made is None else torch.empty(made[2], dtype=made[1], device=device) for made in made_gradients]
+                for (_, slot, _, _), t in zip(saved_slots, call):
+                    if slot is not None:
+                        pointers[slot] = t.data_ptr()
+                for (_, _, slot, _, _), t in zip(given_gradients, gradients):
+                    pointers[slot] = t.data_ptr()
+                for made, t in zip(made_gradients, results):
+                    if made is not None and made[0] is not None:
+                        pointers[made[0]] = t.data_ptr()
+                compiled.rebound()
                 compiled.launch(backward_states)
-                return tuple(None if r is None else r.to(sdfg.arrays[a].dtype) for r, a in zip(results, in_arrays))
+                return tuple(t if made is None or made[1] == made[3] else t.to(made[3]) for made, t in zip(made_gradients, results))
 
         def function(*args):
             if len(args) != n_tensor:

@@ -476,6 +476,30 @@ int dmlhip_batchnorm_backward_act_f32(const void* dy, const void* x, const void*
                                       float* dbias, int64_t n, int64_t c, int64_t hw, float eps, int act,
                                       void* workspace, size_t workspace_bytes, void* stream);
 
+/* ------------------------------------------------------------------ call lists
+ * A list of calls of the entry points above that launch kernels (int result, the stream as last parameter), run in order by
+ * one call. Nothing in the reference corresponds to it: its generated code calls the libraries from C++. */
+#define DMLHIP_CALL_VALUE 0   /* `value`: an integer, the bits of a float, the address of a descriptor or an array */
+#define DMLHIP_CALL_POINTER 1 /* pointers[index] + value */
+#define DMLHIP_CALL_STREAM 2  /* the stream of dmlhip_run_calls */
+#define DMLHIP_CALL_TABLE 3   /* a table of `index` (at most 16) pointers; `value`: address of as many dmlhip_call_arg, of which
+                               * entry e stands for pointers[entries[e].index] + entries[e].value */
+typedef struct {
+    uint32_t kind;
+    uint32_t index;
+    uint64_t value;
+} dmlhip_call_arg;
+typedef struct {
+    int symbol; /* dmlhip_call_symbol */
+    int argc;
+    const dmlhip_call_arg* args;
+} dmlhip_call;
+/* The number an entry point has in call lists of this library; -1: not one of them. */
+int dmlhip_call_symbol(const char* name);
+/* Runs calls[0 .. count) until one fails, whose status is returned and whose number is stored to *failed (-1: none; may be
+ * NULL). `pointers` is read during the call only. */
+int dmlhip_run_calls(const dmlhip_call* calls, int count, const uint64_t* pointers, void* stream, int* failed);
+
 /* ------------------------------------------------------------------ diagnostics
  * Switches for tests and measurements; nothing in the reference corresponds to them (its cuDNN expansion exposes
  * `node._algorithm`, cudnn_implementations.py:131-146, for the same purpose). The two "force" switches and the
