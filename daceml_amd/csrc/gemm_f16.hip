@@ -735,11 +735,13 @@ int dmlhip_gemm_f16_grouped(const dmlhip_gemm_desc* d, int groups, const void* c
 // 8192 / 16384 tokens 42 / 51, 79 / 75, 153 / 122; 512 x 2048 over 4096 / 16384 34 / 31, 122 / 54; three of 1024 x 1024 over 16384
 // 143 / 100.
 static int weight_gradient_slices(const dmlhip_gemm_desc* d, int groups) {
-    if (d->m <= 0 || d->n <= 0 || d->k <= 0 || d->k % BK || d->m % 8 || d->n % 8 || d->c_stride_m != d->n || !g_direct_lds) return 0;
+    if (d->m <= 0 || d->n <= 0 || d->k <= 0 || d->m % 8 || d->n % 8 || d->c_stride_m != d->n || !g_direct_lds) return 0;
     if (d->m > 65536 || d->n > 65536 || (g_force_cfg >= 0 && g_force_cfg != 13)) return 0;
     const long long t256 = ceil_div(d->m, (int64_t)kWideTile) * ceil_div(d->n, (int64_t)kWideTile) * groups;
     const long long t128 = ceil_div(d->m, (int64_t)128) * ceil_div(d->n, (int64_t)128) * groups;
-    const long long steps = d->k / BK, most = steps / 3 < kCus / t256 ? steps / 3 : kCus / t256;   // three steps each at least
+    // three steps each at least, four where the last one is ragged
+    const long long steps = ceil_div(d->k, (int64_t)BK), least = d->k % BK ? 4 : 3;
+    const long long most = steps / least < kCus / t256 ? steps / least : kCus / t256;
     if (most < 2) return 0;
     if (g_force_cfg == 13) return (int)most;
     const double mb = 4e-6 * groups * (double)d->m * (double)d->n;

@@ -26,8 +26,9 @@
 //  * SLICED (weight gradients: few tiles, a long K): the workgroups of a tile share its K steps and write fp32 partial results
 //    that wide_sum_kernel adds up, four times over for 64 tiles: 64 MB written and read, about 30 us whatever K is. The row
 //    sums of A (the bias gradient) are taken from the fragments: the workgroups of tile column c add those of every step that
-//    leaves c modulo the number of columns, so that none of them falls behind the others.
-// Requirements (checked by the host): K % 64 == 0 and at least three steps, no activation, beta == 0, n % 8 == 0, 16-byte aligned operands, column
+//    leaves c modulo the number of columns, so that none of them falls behind the others. Any K: the step with its last k is
+//    sent by a copy of the step of its own, with zeros behind them.
+// Requirements (checked by the host): K % 64 == 0 (but for SLICED) and at least three steps, no activation, beta == 0, n % 8 == 0, 16-byte aligned operands, column
 // bias and result rows, 32-bit element offsets, rows % 8 == 0 for RC operands.
 #pragma once
 
@@ -36,6 +37,8 @@
 namespace dml {
 namespace gemm16 {
 namespace {
+
+__device__ const half8 g_wide_zeros = {0, 0, 0, 0, 0, 0, 0, 0};   // what transfers past the end of K read
 
 constexpr int kWideOperand = kWideTile * kRowBytes;   // bytes of one operand's tile: 32 KB
 constexpr int kWideLds = 5 * kWideOperand;            // two of A, three of B
@@ -97,6 +100,13 @@ template <bool B> struct WideOperand<0, B> {   // K contiguous
         return (uint32_t)(((min(rows_left, kWideTile) - 1) * s_row + k) * 2);
     }
     static __device__ __forceinline__ uint32_t k_offset(int64_t, int step) { return (uint32_t)step * kRowBytes; }
+    // transfer I of a step of which only `left` < 64 k exist (a multiple of 8: so is K of such an operand)
+    template <int I>
+    __device__ __forceinline__ void send_tail(const _Float16* tile, int64_t, int step, int left, char* dst, int wave, int lane) const {
+        const char* p = reinterpret_cast<const char*>(tile) + k_offset(0, step) + (uint32_t)vo[I];
+        const int kl = ((lane & 7) ^ swz16(wave * 8 + (lane >> 3))) * 8;
+        lds_dma16(kl < left ? reinterpret_cast<const _Float16*>(p) : reinterpret_cast<const _Float16*>(&g_wide_zeros), dst);
+    }
     template <int S, int U>
     __device__ __forceinline__ half8 fragment(uint32_t stage) const {
         return lds_read_b128<U * 16 * kRowBytes>(faddr[S] + stage);
@@ -130,6 +140,12 @@ template <bool B> struct WideOperand<1, B> {   // rows contiguous
         return (uint32_t)(((k - 1) * s_k + min(rows_left, kWideTile)) * 2);
     }
     static __device__ __forceinline__ uint32_t k_offset(int64_t s_k, int step) { return (uint32_t)(step * BK * s_k * 2); }
+    // transfer I of a step of which only `left` < 64 k exist
+    template <int I>
+    __device__ __forceinline__ void send_tail(const _Float16* tile, int64_t s_k, int step, int left, char* dst, int wave, int lane) const {
+        const char* p = reinterpret_cast<const char*>(tile) + k_offset(s_k, step) + (uint32_t)vo[I];
+        lds_dma16(I * 8 + wave * 2 + (lane >> 5) < left ? reinterpret_cast<const _Float16*>(p) : reinterpret_cast<const _Float16*>(&g_wide_zeros), dst);
+    }
     template <int S, int U>
     __device__ __forceinline__ half8 fragment(uint32_t stage) const {
         const uint32_t a = faddr[U] + stage;
@@ -319,13 +335,14 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_wide_kernel(const _Float16*
     ob.fragments(lds0 + 2 * kWideOperand, wn * 128, lane);
 
     static_assert(!SLICED || (AKIND == 1 && EPI == EPI_PLAIN && !KSUM), "slices are for weight gradients");
-    const int nkg = g.k / BK;                       // steps of one operand pair
+    const int nkg = SLICED ? (g.k + BK - 1) / BK : g.k / BK;   // steps of one operand pair
     auto slice_begin = [&](int z1) { return (int)((uint32_t)nkg * (uint32_t)z1 / (uint32_t)g.batch1); };
     uint32_t bid = blockIdx.x;
     const uint32_t total = (uint32_t)g.total_blocks;
 
     // ---- what the transfers read: two steps ahead of the MFMAs, past the end of a tile the first steps of the next one
     __amdgpu_buffer_rsrc_t ra, rb;
+    const _Float16 *tile_a = nullptr, *tile_b = nullptr;   // where they begin, for the ragged step
     int fk = 0, fend = nkg, fgrp = 0, rows_a = 0, rows_b = 0;
     auto point_at = [&](uint32_t at) {
         const WideTile ft = wide_tile(g, at);
@@ -345,6 +362,10 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_wide_kernel(const _Float16*
         }
         a += ft.aoff + ft.m0 * WideOperand<AKIND, false>::row_step(g.sam);
         b += ft.boff + ft.n0 * WideOperand<BKIND, true>::row_step(g.sbn);
+        if constexpr (SLICED) {
+            tile_a = a;
+            tile_b = b;
+        }
         const int la = g.m - ft.m0, lb = g.n - ft.n0;
         // rows past the end of an operand read its last row; the descriptor ends where the operand does
         ra = __builtin_amdgcn_make_buffer_rsrc(uniform(a), 0, (int)WideOperand<AKIND, false>::extent(g.sam, g.sak, la, g.k), 0x00020000);
@@ -405,7 +426,9 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_wide_kernel(const _Float16*
     float row_sum[SLICED ? T : 1];   // row lane % 16 of every block, the k of this lane's fragments
     int sum_in = -1;                 // steps until this workgroup sums fragments again
     // FIRST: of a tile. FILL: the step two ahead exists and is sent. MORE: the next step exists, its first fragments are read.
-    auto step = [&](auto first_c, auto fill_c, auto more_c) {
+    // TAIL: what is sent is the ragged last step of K.
+    auto step = [&](auto first_c, auto fill_c, auto more_c, auto tail_c) {
+        constexpr bool TAIL = decltype(tail_c)::value;
         constexpr bool FIRST = decltype(first_c)::value, FILL = decltype(fill_c)::value, MORE = decltype(more_c)::value;
         const int an = as ^ 1, bn = bs == 2 ? 0 : bs + 1, bfill = bs == 0 ? 2 : bs - 1;
         static_for<0, 2>([&](auto sc) {
@@ -428,7 +451,11 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_wide_kernel(const _Float16*
                     if constexpr (s == 0) read(std::integral_constant<int, m / 2>{}, std::integral_constant<int, 1>{}, as * kWideOperand, bs * kWideOperand);
                     else if constexpr (MORE) read(std::integral_constant<int, m / 2>{}, std::integral_constant<int, 0>{}, an * kWideOperand, bn * kWideOperand);
                 }
-                if constexpr (FILL && m % 8 == 1) {
+                if constexpr (FILL && TAIL && m % 8 == 1) {
+                    constexpr int d = m / 8;
+                    if constexpr (s == 0) ob.template send_tail<d>(tile_b, g.sbk, fk, g.k - fk * BK, lds + (2 + bfill) * kWideOperand + (d * 4 + wave) * 1024, wave, lane);
+                    else oa.template send_tail<d>(tile_a, g.sak, fk, g.k - fk * BK, lds + as * kWideOperand + (d * 4 + wave) * 1024, wave, lane);
+                } else if constexpr (FILL && m % 8 == 1) {
                     if constexpr (s == 0) send_b(std::integral_constant<int, m / 8>{}, bfill);
                     else send_a(std::integral_constant<int, m / 8>{}, as);
                 }
@@ -468,11 +495,22 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_wide_kernel(const _Float16*
             for (int i = 0; i < T; ++i) row_sum[i] = 0.f;
         }
         const int fills = last ? nk - 2 : nk;
-        step(yes{}, yes{}, yes{});
-        for (int kt = 1; kt < fills; ++kt) step(no{}, yes{}, yes{});
+        step(yes{}, yes{}, yes{}, no{});
+        if constexpr (SLICED) {
+            // the last slice's last step may be ragged: it is sent two steps ahead (the host passes four steps then)
+            const int tail = g.k % BK != 0 && t.z1 + 1 == g.batch1 ? nk - 3 : -1;
+            int kt = 1;
+            for (; kt < fills && kt != tail; ++kt) step(no{}, yes{}, yes{}, no{});
+            if (kt == tail) {
+                step(no{}, yes{}, yes{}, yes{});
+                for (++kt; kt < fills; ++kt) step(no{}, yes{}, yes{}, no{});
+            }
+        } else {
+            for (int kt = 1; kt < fills; ++kt) step(no{}, yes{}, yes{}, no{});
+        }
         if (last) {
-            step(no{}, no{}, yes{});
-            step(no{}, no{}, no{});
+            step(no{}, no{}, yes{}, no{});
+            step(no{}, no{}, no{}, no{});
         }
         // an accumulator is read no earlier than 18 wait states behind the last MFMA (the assembly hides them from the compiler),
         // and the next tile's first fragments are in their registers before the epilogue may use others around them

@@ -936,7 +936,7 @@ def fuse_bias_gradients(sdfg: SDFG) -> int:
                 except (C.NotApplicable, ValueError):
                     continue
                 if plan.swapped or any(e != 1 for e in plan.batch) or plan.m != xd.shape[-1] \
-                        or plan.m * plan.k != xd.total_size or plan.k % 64 or b.dtype != torch.float16:
+                        or plan.m * plan.k != xd.total_size or b.dtype != torch.float16:
                     continue
                 _remove_node(state, red)
                 node.add_out_connector("InputSum")

@@ -89,7 +89,8 @@ def test_several_tiles_per_workgroup(layouts, m, n, batch, lib):
 
 
 @pytest.mark.parametrize("m,n,k,groups,layout", [(8, 8, 64 * 6, 1, 1), (264, 520, 64 * 13, 3, 1), (256, 512, 64 * 50, 2, 1), (520, 136, 64 * 11, 4, 0),
-                                                 (136, 264, 64 * 70, 1, 1)])
+                                                 (136, 264, 64 * 70, 1, 1), (264, 248, 64 * 8 - 63, 2, 1), (136, 520, 64 * 9 - 1, 1, 1), (8, 264, 64 * 37 + 33, 3, 1),
+                                                 (136, 248, 64 * 9 + 8, 2, 0)])
 @pytest.mark.parametrize("sum_dtype", [torch.float32, torch.float16])
 def test_weight_gradients_in_slices(m, n, k, groups, layout, sum_dtype, lib):
     """Products [k, m]^T [k, n] whose tiles are shared by several workgroups, with the column sums of the first operand: uneven
