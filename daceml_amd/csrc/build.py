@@ -16,6 +16,12 @@ LIB_PATH = os.path.join(HERE, LIB_NAME)
 OBJ_DIR = os.path.join(HERE, "build")
 
 SOURCES = [
+    # the ones that take minutes first
+    "gemm_f16_pipe.hip",
+    "gemm_f16_pipe_ilv.hip",
+    "gemm_f16_wide.hip",
+    "gemm_f16_pipe_ragged.hip",
+    "gemm_f16.hip",
     "common.cpp",
     "call_list.cpp",
     "rowwise.hip",
@@ -24,12 +30,8 @@ SOURCES = [
     "transpose.hip",
     "pad.hip",
     "pool.hip",
-    "gemm_f16.hip",
-    "gemm_f16_pipe.hip",
-    "gemm_f16_pipe_ilv.hip",
-    "gemm_f16_pipe_ragged.hip",
     "gemm_f16_split.hip",
-    "gemm_f16_wide.hip",
+    "gemm_f16_wide_half.hip",
     "gemm_f32.hip",
     "gemm_f32_split.hip",
     "conv.hip",

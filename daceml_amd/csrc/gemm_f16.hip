@@ -525,9 +525,10 @@ static int run_gemm_f16(const dmlhip_gemm_desc* d, const void* a, const void* b,
     if (vec) {
         auto blocks = [&](int bm, int bn) { return (long long)ceil_div(d->m, bm) * ceil_div(d->n, bn) * batch; };
         const bool sums = g.asum || (grp && g.gasum[0]);
-        // what the kernel of 256 x 256 tiles in gemm_f16_wide.h takes
-        const bool wide = pipe && !ragged && !sums && g.beta == 0.f && g.act == DMLHIP_ACT_NONE && !pre_out && g.c_vec && d->n % 8 == 0 && d->k * (g.ksum ? g.groups : 1) >= 3 * BK &&
+        // what the kernels of gemm_f16_wide.h take
+        const bool wide = pipe && !ragged && !sums && g.beta == 0.f && g.act == DMLHIP_ACT_NONE && !pre_out && g.c_vec && d->n % 8 == 0 &&
                           (!bias || g.bias_m || aligned16(bias));
+        const long long steps = (long long)(d->k / BK) * (g.ksum ? g.groups : 1);
         const bool extra = grp || asum;   // operand pairs / row sums: the 128 x 128 tile only
         const long long t256 = blocks(256, 256), t128 = blocks(128, 128);
         const long long slots256 = ceil_div(t256, (long long)kCus) * kCus, slots128 = ceil_div(t128, (long long)kCus) * kCus;
@@ -568,11 +569,13 @@ static int run_gemm_f16(const dmlhip_gemm_desc* d, const void* a, const void* b,
             }
         }
         const _Float16 *pa = (const _Float16*)a, *pb = (const _Float16*)b;
+        // The 128 x 128 tile of gemm_f16_wide.h in place of those of gemm_f16_pipe.h, from half a round of tiles and sixteen steps
+        // on (products of 144 - 192 tiles are level: 3072 x 768 x 3072 24.5 / 24.6, B row-contiguous 24.3 / 23.7).
+        if (g_force_cfg < 0 && (cfg == 5 || cfg == 9) && wide && amode == 0 && steps >= 16 && t128 * 2 >= kCus) cfg = 14;
         g_last_cfg = cfg;
-        if (cfg == 13) {
-            if (wide) return launch_wide(g, pa, pb, c, bias, residual, amode, bmode, batch, st);
-            g_last_cfg = cfg = 4;
-        }
+        if (cfg == 13 && wide && steps >= 3) return launch_wide256(g, pa, pb, c, bias, residual, amode, bmode, batch, st);
+        if (cfg == 14 && wide && steps >= 5 && amode == 0) return launch_wide128(g, pa, pb, c, bias, residual, amode, bmode, batch, st);
+        if (cfg == 13 || cfg == 14) g_last_cfg = cfg = cfg == 13 ? 4 : 5;
         if (cfg >= 10 && (!sums || amode == 1))
             return launch_split(g, pa, pb, c, bias, residual, pre_out, amode, bmode, cfg, batch, st);
         if (pipe && ragged) return launch_pipelined_ragged(g, pa, pb, c, bias, residual, pre_out, cfg, batch, st);

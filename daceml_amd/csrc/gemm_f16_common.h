@@ -260,9 +260,11 @@ int launch_pipelined_ilv(GemmArgs& g, const _Float16* a, const _Float16* b, void
 int launch_pipelined_ragged(GemmArgs& g, const _Float16* a, const _Float16* b, void* c, const void* bias, const void* residual,
                             void* pre, int cfg, long long batch, hipStream_t st);
 constexpr int kWideTile = 256;   // rows and columns of a tile of gemm_f16_wide.h
-// Configuration 13 (gemm_f16_wide.h): 256 x 256 tiles, no activation.
-int launch_wide(GemmArgs& g, const _Float16* a, const _Float16* b, void* c, const void* bias, const void* residual, int ak,
-                int bk, long long batch, hipStream_t st);
+// Configurations 13 and 14 (gemm_f16_wide.h): 256 x 256 tiles; 128 x 128 tiles, A K-contiguous. No activation.
+int launch_wide256(GemmArgs& g, const _Float16* a, const _Float16* b, void* c, const void* bias, const void* residual, int ak,
+                   int bk, long long batch, hipStream_t st);
+int launch_wide128(GemmArgs& g, const _Float16* a, const _Float16* b, void* c, const void* bias, const void* residual, int ak,
+                   int bk, long long batch, hipStream_t st);
 // Products of few 256 x 256 tiles with A row-contiguous: `slices` workgroups share the K steps of a tile (three each at least),
 // their fp32 results are summed by a second launch, as are the row sums of A where asked for. Dense results, n % 8 == 0.
 // wide_sliced_bytes: what lies in the workspace; the partial row sums begin at *row_offset.

@@ -1,5 +1,6 @@
 // fp16 GEMM for products of many 256 x 256 tiles: one workgroup of four wavefronts per compute unit that stays for all of
-// its tiles, v_mfma_f32_16x16x32_f16, both operands straight from global memory into LDS (buffer_load ... lds).
+// its tiles, v_mfma_f32_16x16x32_f16, both operands straight from global memory into LDS (buffer_load ... lds). The same with
+// 128 x 128 tiles and twice as many steps on their way, where products have fewer. What follows is about the large tile.
 //
 // What bounds it: the matrix pipe at the clock that the power limit leaves (1.4 - 1.6 GHz under this load). A 64-k step of a
 // wavefront is 128 MFMAs = 2048 clocks and takes 2240 - 2290; the 256 x 256 tile of gemm_f16_pipe.h takes 2550 - 2650 with
@@ -18,6 +19,10 @@
 //    and columns 4 (l / 16) .. + 3 of a 16 x 16 block.
 // The MFMAs are inline assembly with the accumulator tied to an accumulation register: the compiler moves 2 - 9 of the 64
 // accumulators between register files in every step otherwise (2400 against 2270 clocks).
+//
+// The 128 x 128 tile is bound by the L2s: 32 KB per 64 k and compute unit, 512 clocks of the 64 bytes that one gets at best, all
+// 256 together 18 - 19 TB/s of a step's 0.44 us (0.50 in gemm_f16_pipe.h). 4096 x 1024 x 4096 with residual 39.8 -> 36.7 us, B
+// row-contiguous 39.6 -> 36.3, three pairs of 4096 x 1024 x 1024 33.5 -> 30.2, 8192 x 1024 x 4096 75 -> 69.
 //
 // LDS tiles. KC (K contiguous): [256 rows][64 k], 128-byte rows, 16-byte chunk c of row r at slot c ^ (r & 7) ^ (r >> 3 & 1).
 // RC (rows contiguous): [64 k][256 rows], chunk c (8 rows) of K row k at slot c ^ ((k & 3) << 2) ^ ((k >> 3 & 1) << 1): the
@@ -40,8 +45,14 @@ namespace {
 
 __device__ const half8 g_wide_zeros = {0, 0, 0, 0, 0, 0, 0, 0};   // what transfers past the end of K read
 
-constexpr int kWideOperand = kWideTile * kRowBytes;   // bytes of one operand's tile: 32 KB
-constexpr int kWideLds = 5 * kWideOperand;            // two of A, three of B
+// T: 16 x 16 blocks of a wavefront in either direction; the four of a workgroup make a tile of 32 T x 32 T. AHEAD: steps that are
+// on their way or in LDS beside the one that is multiplied; so many stages for A, one more for B.
+template <int T> struct WideShape {
+    static constexpr int kTile = 32 * T;
+    static constexpr int kOperand = kTile * kRowBytes;   // bytes of one operand's tile
+    static constexpr int kAhead = T == 8 ? 2 : 4;
+    static constexpr int kLds = (2 * kAhead + 1) * kOperand;
+};
 
 template <bool FIRST>   // the first of a tile's products starts the sum
 __device__ __forceinline__ void mfma_16x16x32(floatx4& acc, half8 b, half8 a) {
@@ -69,7 +80,7 @@ __device__ __forceinline__ void trade(u32x4& p, u32x4& q) {
     }
 }
 
-template <int KIND, bool B> struct WideOperand;
+template <int T, int KIND, bool B> struct WideOperand;
 
 // Where row r of a tile lies in LDS, or r itself for A. B's 16 x 16 blocks 2 p and 2 p + 1 take turns at four columns each of
 // the 32 columns from 32 p on, so that a lane's four columns of both are eight consecutive ones.
@@ -77,14 +88,14 @@ __device__ __forceinline__ int b_row(int pos) {   // position j * 16 + 4 g + e -
     return (pos & ~31) | (pos >> 2 & 3) << 3 | (pos >> 4 & 1) << 2 | (pos & 3);
 }
 
-template <bool B> struct WideOperand<0, B> {   // K contiguous
-    int vo[8];          // byte offset of this lane's piece in transfer i of a step, from the tile's first row
+template <int T, bool B> struct WideOperand<T, 0, B> {   // K contiguous
+    int vo[T];          // byte offset of this lane's piece in transfer i of a step, from the tile's first row
     uint32_t faddr[2];  // this lane's fragment of block 0, either half of a step (stage 0)
     __device__ __forceinline__ void offsets(int64_t s_row, int64_t, int rows_left, int wave, int lane) {
         const int r0 = wave * 8 + (lane >> 3);
         const int c = (lane & 7) ^ swz16(r0);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
+        for (int i = 0; i < T; ++i) {
             const int r = i * 32 + r0;
             vo[i] = (int)((min(B ? b_row(r) : r, rows_left - 1) * s_row + c * 8) * 2);
         }
@@ -97,7 +108,7 @@ template <bool B> struct WideOperand<0, B> {   // K contiguous
     static __device__ __forceinline__ int64_t row_step(int64_t s_row) { return s_row; }
     // bytes from the tile's first element to the end of its last row
     static __device__ __forceinline__ uint32_t extent(int64_t s_row, int64_t, int rows_left, int k) {
-        return (uint32_t)(((min(rows_left, kWideTile) - 1) * s_row + k) * 2);
+        return (uint32_t)(((min(rows_left, 32 * T) - 1) * s_row + k) * 2);
     }
     static __device__ __forceinline__ uint32_t k_offset(int64_t, int step) { return (uint32_t)step * kRowBytes; }
     // transfer I of a step of which only `left` < 64 k exist (a multiple of 8: so is K of such an operand)
@@ -113,16 +124,18 @@ template <bool B> struct WideOperand<0, B> {   // K contiguous
     }
 };
 
-template <bool B> struct WideOperand<1, B> {   // rows contiguous
-    static constexpr int P = kWideTile * 2;   // bytes of a K row
-    int vo[8];
-    uint32_t faddr[8];  // this lane's first transpose read of every 16-row block (stage 0)
+template <int T, bool B> struct WideOperand<T, 1, B> {   // rows contiguous
+    static constexpr int P = 64 * T;          // bytes of a K row
+    static constexpr int KPT = 4 * 1024 / P;  // K rows of the four wavefronts' transfers of one number
+    int vo[T];
+    uint32_t faddr[T];  // this lane's first transpose read of every 16-row block (stage 0)
+    static __device__ __forceinline__ int k_of(int i, int wave, int lane) { return i * KPT + wave * (KPT / 4) + lane / (4 * T); }
     __device__ __forceinline__ void offsets(int64_t, int64_t s_k, int rows_left, int wave, int lane) {
-        const int k0 = wave * 2 + (lane >> 5);
+        const int k0 = k_of(0, wave, lane);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int k = i * 8 + k0;
-            const int c = (lane & 31) ^ ((k & 3) << 2) ^ ((i & 1) << 1);
+        for (int i = 0; i < T; ++i) {
+            const int k = i * KPT + k0;
+            const int c = (lane & (4 * T - 1)) ^ ((k & 3) << 2) ^ ((k >> 3 & 1) << 1);
             vo[i] = (int)((k * s_k + min(c * 8, rows_left - 8)) * 2);
         }
     }
@@ -130,21 +143,21 @@ template <bool B> struct WideOperand<1, B> {   // rows contiguous
         const int s = lane & 15, grp = lane >> 4;
         const int k = grp * 8 + (s >> 2);
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
+        for (int u = 0; u < T; ++u) {
             const int row = row0 + (B ? b_row(u * 16 + 4 * (s & 3)) : u * 16 + 4 * (s & 3));
             faddr[u] = tile0 + k * P + (((row >> 3) ^ ((k & 3) << 2) ^ ((grp & 1) << 1)) << 4) + (row & 7) * 2;
         }
     }
     static __device__ __forceinline__ int64_t row_step(int64_t) { return 1; }
     static __device__ __forceinline__ uint32_t extent(int64_t, int64_t s_k, int rows_left, int k) {
-        return (uint32_t)(((k - 1) * s_k + min(rows_left, kWideTile)) * 2);
+        return (uint32_t)(((k - 1) * s_k + min(rows_left, 32 * T)) * 2);
     }
     static __device__ __forceinline__ uint32_t k_offset(int64_t s_k, int step) { return (uint32_t)(step * BK * s_k * 2); }
     // transfer I of a step of which only `left` < 64 k exist
     template <int I>
     __device__ __forceinline__ void send_tail(const _Float16* tile, int64_t s_k, int step, int left, char* dst, int wave, int lane) const {
         const char* p = reinterpret_cast<const char*>(tile) + k_offset(s_k, step) + (uint32_t)vo[I];
-        lds_dma16(I * 8 + wave * 2 + (lane >> 5) < left ? reinterpret_cast<const _Float16*>(p) : reinterpret_cast<const _Float16*>(&g_wide_zeros), dst);
+        lds_dma16(k_of(I, wave, lane) < left ? reinterpret_cast<const _Float16*>(p) : reinterpret_cast<const _Float16*>(&g_wide_zeros), dst);
     }
     template <int S, int U>
     __device__ __forceinline__ half8 fragment(uint32_t stage) const {
@@ -167,6 +180,7 @@ struct WideTile {
     int64_t aoff, boff, coff;   // element offsets of the batch entry
 };
 
+template <int T>
 __device__ __forceinline__ WideTile wide_tile(const GemmArgs& g, uint32_t bid) {
     {   // contiguous runs of tiles per XCD; workgroups are dealt to the XCDs in turn
         const uint32_t total = (uint32_t)g.total_blocks;
@@ -187,8 +201,8 @@ __device__ __forceinline__ WideTile wide_tile(const GemmArgs& g, uint32_t bid) {
     const uint32_t rows_here = min((uint32_t)g.tiles_m - group * kGroupM, kGroupM);
     const uint32_t tn = in_group / rows_here;
     WideTile t;
-    t.m0 = (int)(group * kGroupM + (in_group - tn * rows_here)) * kWideTile;
-    t.n0 = (int)tn * kWideTile;
+    t.m0 = (int)(group * kGroupM + (in_group - tn * rows_here)) * WideShape<T>::kTile;
+    t.n0 = (int)tn * WideShape<T>::kTile;
     int z2 = 0;
     t.z0 = t.z1 = 0;
     if (batch != 0) {
@@ -232,18 +246,18 @@ __device__ __forceinline__ void wide_store(OutT* p, u32x4 v, bool through) {
 // The wavefront's 128 x 128 tile in strips of 16 rows and 32 columns (fp32) or 64 (fp16): lane l has columns 8 (l / 16) .. + 7
 // of every 32 of row l % 16. Lanes l and l ^ 8 trade half of a strip, so that a store instruction writes 128 bytes each of
 // eight rows: 64 bytes each of sixteen rows take twice as long (12.2 against 6.1 us for a 4096 x 4096 result).
-template <typename OutT, int EPI>
+template <int T, typename OutT, int EPI>
 __device__ __forceinline__ void wide_epilogue(const GemmArgs& g, void* c_ptr, const void* res_ptr, const void* bias_ptr,
-                                              const floatx4 (&acc)[8][8], int mb, int nb, int64_t coff, int lane, bool through) {
+                                              const floatx4 (&acc)[T][T], int mb, int nb, int64_t coff, int lane, bool through) {
     typedef typename OutVec<OutT>::type ovec;
     constexpr bool GENERAL = EPI == EPI_GENERAL;
     constexpr bool HALF = sizeof(OutT) == 2;
     OutT* C = reinterpret_cast<OutT*>(c_ptr);
     const OutT* R = reinterpret_cast<const OutT*>(res_ptr);
     const int col = (lane >> 4) * 8, row = lane & 15;
-    float bias[4][8];
+    float bias[T / 2][8];
 #pragma unroll
-    for (int p = 0; p < 4; ++p) {
+    for (int p = 0; p < T / 2; ++p) {
         const int n = min(nb + p * 32 + col, g.n - 8);
         if (!bias_ptr || g.bias_m) {
 #pragma unroll
@@ -261,9 +275,9 @@ __device__ __forceinline__ void wide_epilogue(const GemmArgs& g, void* c_ptr, co
     }
     // what has to be loaded (general variant only): four strips of 16 rows ahead of the stores of the first
     constexpr int AHEAD = GENERAL ? (HALF ? 4 : 2) : 1;
-    static_for<0, 8 / AHEAD>([&](auto hc) {
+    static_for<0, T / AHEAD>([&](auto hc) {
         constexpr int i0 = decltype(hc)::value * AHEAD;
-        ovec rv[AHEAD][4];
+        ovec rv[AHEAD][T / 2];
         float bm[AHEAD];
         if constexpr (GENERAL) {
 #pragma unroll
@@ -274,14 +288,14 @@ __device__ __forceinline__ void wide_epilogue(const GemmArgs& g, void* c_ptr, co
                     bm[i] = g.bias_f32 ? reinterpret_cast<const float*>(bias_ptr)[m]
                                        : (float)reinterpret_cast<const _Float16*>(bias_ptr)[m];
 #pragma unroll
-                for (int p = 0; p < 4; ++p)
+                for (int p = 0; p < T / 2; ++p)
                     if (R) rv[i][p] = *reinterpret_cast<const ovec*>(R + coff + (int64_t)m * g.scm + min(nb + p * 32 + col, g.n - 8));
             }
         }
         static_for<0, AHEAD>([&](auto ic) {
             constexpr int ii = decltype(ic)::value, i = i0 + ii;
             const int m = mb + i * 16 + (row & 7);
-            static_for<0, HALF ? 2 : 4>([&](auto pc) {
+            static_for<0, HALF ? T / 4 : T / 2>([&](auto pc) {
                 constexpr int p = decltype(pc)::value * (HALF ? 2 : 1);
                 u32x4 lo, hi;
                 int n;
@@ -317,22 +331,23 @@ __device__ __forceinline__ void wide_epilogue(const GemmArgs& g, void* c_ptr, co
 
 // SLICED: the inner batch index z1 counts g.batch1 slices of K (its operand strides are 0); g.asum, if any, receives the partial
 // row sums [z0][z1][tile column][2][m] in fp32.
-template <int AKIND, int BKIND, int EPI, bool KSUM, bool SLICED = false>
+template <int T, int AKIND, int BKIND, int EPI, bool KSUM, bool SLICED = false>
 __global__ __launch_bounds__(kThreads) void gemm_f16_wide_kernel(const _Float16* a_ptr, const _Float16* b_ptr, void* c_ptr,
                                                                  const void* bias_ptr, const void* res_ptr, const GemmArgs g) {
 #if defined(__HIP_DEVICE_COMPILE__)   // buffer descriptors exist on the device only
-    constexpr int T = 8, NM = T * T;   // 16 x 16 blocks of a wavefront's 128 x 128 tile
+    constexpr int NM = T * T, TILE = WideShape<T>::kTile, OPERAND = WideShape<T>::kOperand, AHEAD = WideShape<T>::kAhead;
+    constexpr int WT = TILE / 2;       // rows and columns of a wavefront
     extern __shared__ __attribute__((aligned(16))) char lds[];
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int wm = wave >> 1, wn = wave & 1;
     if (g.trace && threadIdx.x == 0) g.trace[4 * (size_t)blockIdx.x] = wall_clock64();
 
-    WideOperand<AKIND, false> oa;
-    WideOperand<BKIND, true> ob;
+    WideOperand<T, AKIND, false> oa;
+    WideOperand<T, BKIND, true> ob;
     const uint32_t lds0 = lds_addr(lds);
-    oa.fragments(lds0, wm * 128, lane);
-    ob.fragments(lds0 + 2 * kWideOperand, wn * 128, lane);
+    oa.fragments(lds0, wm * WT, lane);
+    ob.fragments(lds0 + AHEAD * OPERAND, wn * WT, lane);
 
     static_assert(!SLICED || (AKIND == 1 && EPI == EPI_PLAIN && !KSUM), "slices are for weight gradients");
     const int nkg = SLICED ? (g.k + BK - 1) / BK : g.k / BK;   // steps of one operand pair
@@ -345,7 +360,7 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_wide_kernel(const _Float16*
     const _Float16 *tile_a = nullptr, *tile_b = nullptr;   // where they begin, for the ragged step
     int fk = 0, fend = nkg, fgrp = 0, rows_a = 0, rows_b = 0;
     auto point_at = [&](uint32_t at) {
-        const WideTile ft = wide_tile(g, at);
+        const WideTile ft = wide_tile<T>(g, at);
         fk = 0;
         if constexpr (SLICED) {
             fk = slice_begin(ft.z1);
@@ -360,22 +375,22 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_wide_kernel(const _Float16*
             a = g.ga[ft.z0];
             b = g.gb[ft.z0];
         }
-        a += ft.aoff + ft.m0 * WideOperand<AKIND, false>::row_step(g.sam);
-        b += ft.boff + ft.n0 * WideOperand<BKIND, true>::row_step(g.sbn);
+        a += ft.aoff + ft.m0 * WideOperand<T, AKIND, false>::row_step(g.sam);
+        b += ft.boff + ft.n0 * WideOperand<T, BKIND, true>::row_step(g.sbn);
         if constexpr (SLICED) {
             tile_a = a;
             tile_b = b;
         }
         const int la = g.m - ft.m0, lb = g.n - ft.n0;
         // rows past the end of an operand read its last row; the descriptor ends where the operand does
-        ra = __builtin_amdgcn_make_buffer_rsrc(uniform(a), 0, (int)WideOperand<AKIND, false>::extent(g.sam, g.sak, la, g.k), 0x00020000);
-        rb = __builtin_amdgcn_make_buffer_rsrc(uniform(b), 0, (int)WideOperand<BKIND, true>::extent(g.sbn, g.sbk, lb, g.k), 0x00020000);
-        if (min(la, kWideTile) != rows_a) {
-            rows_a = min(la, kWideTile);
+        ra = __builtin_amdgcn_make_buffer_rsrc(uniform(a), 0, (int)WideOperand<T, AKIND, false>::extent(g.sam, g.sak, la, g.k), 0x00020000);
+        rb = __builtin_amdgcn_make_buffer_rsrc(uniform(b), 0, (int)WideOperand<T, BKIND, true>::extent(g.sbn, g.sbk, lb, g.k), 0x00020000);
+        if (min(la, TILE) != rows_a) {
+            rows_a = min(la, TILE);
             oa.offsets(g.sam, g.sak, rows_a, wave, lane);
         }
-        if (min(lb, kWideTile) != rows_b) {
-            rows_b = min(lb, kWideTile);
+        if (min(lb, TILE) != rows_b) {
+            rows_b = min(lb, TILE);
             ob.offsets(g.sbn, g.sbk, rows_b, wave, lane);
         }
     };
@@ -383,14 +398,14 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_wide_kernel(const _Float16*
     auto send_a = [&](auto ic, int stage) {
         constexpr int i = decltype(ic)::value;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            ra, (__attribute__((address_space(3))) void*)(lds + stage * kWideOperand + (i * 4 + wave) * 1024), 16, oa.vo[i],
-            (int)WideOperand<AKIND, false>::k_offset(g.sak, fk), 0, 0);
+            ra, (__attribute__((address_space(3))) void*)(lds + stage * OPERAND + (i * 4 + wave) * 1024), 16, oa.vo[i],
+            (int)WideOperand<T, AKIND, false>::k_offset(g.sak, fk), 0, 0);
     };
     auto send_b = [&](auto ic, int stage) {
         constexpr int i = decltype(ic)::value;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            rb, (__attribute__((address_space(3))) void*)(lds + (2 + stage) * kWideOperand + (i * 4 + wave) * 1024), 16, ob.vo[i],
-            (int)WideOperand<BKIND, true>::k_offset(g.sbk, fk), 0, 0);
+            rb, (__attribute__((address_space(3))) void*)(lds + (AHEAD + stage) * OPERAND + (i * 4 + wave) * 1024), 16, ob.vo[i],
+            (int)WideOperand<T, BKIND, true>::k_offset(g.sbk, fk), 0, 0);
     };
     // the next step of this tile, or the first of the next one (of the last one: nothing is sent any more)
     auto advance = [&]() {
@@ -403,16 +418,16 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_wide_kernel(const _Float16*
         if (bid + gridDim.x < total) point_at(bid + gridDim.x);
     };
 
-    static_for<0, 8>([&](auto i) { send_b(i, 0); });
-    static_for<0, 8>([&](auto i) { send_a(i, 0); });
-    advance();
-    static_for<0, 8>([&](auto i) { send_b(i, 1); });
-    static_for<0, 8>([&](auto i) { send_a(i, 1); });
-    advance();
-    wait_vm_lgkm0<16>();
+    for (int s = 0; s < AHEAD; ++s) {
+        static_for<0, T>([&](auto i) { send_b(i, s); });
+        static_for<0, T>([&](auto i) { send_a(i, s); });
+        advance();
+    }
+    wait_vm_lgkm0<(AHEAD - 1) * 2 * T>();
     __builtin_amdgcn_s_barrier();
     if (g.trace && threadIdx.x == 0) g.trace[4 * (size_t)blockIdx.x + 1] = wall_clock64();
 
+    constexpr int kReadEvery = T == 8 ? 2 : 1;   // MFMAs per fragment read
     half8 af[2][T], bf[2][T];   // fragments of the first and the second 32 k of a step
     auto read = [&](auto uc, auto sc, uint32_t a_stage, uint32_t b_stage) {
         constexpr int u = decltype(uc)::value, s = decltype(sc)::value;
@@ -425,19 +440,20 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_wide_kernel(const _Float16*
     int as = 0, bs = 0;   // stages of the step that is multiplied
     float row_sum[SLICED ? T : 1];   // row lane % 16 of every block, the k of this lane's fragments
     int sum_in = -1;                 // steps until this workgroup sums fragments again
-    // FIRST: of a tile. FILL: the step two ahead exists and is sent. MORE: the next step exists, its first fragments are read.
-    // TAIL: what is sent is the ragged last step of K.
-    auto step = [&](auto first_c, auto fill_c, auto more_c, auto tail_c) {
-        constexpr bool TAIL = decltype(tail_c)::value;
-        constexpr bool FIRST = decltype(first_c)::value, FILL = decltype(fill_c)::value, MORE = decltype(more_c)::value;
-        const int an = as ^ 1, bn = bs == 2 ? 0 : bs + 1, bfill = bs == 0 ? 2 : bs - 1;
+    // FIRST: of a tile. LEFT: steps that follow, AHEAD for more; with as many the step that far ahead is sent, with one the next
+    // step's first fragments are read. TAIL: what is sent is the ragged last step of K.
+    auto step = [&](auto first_c, auto left_c, auto tail_c) {
+        constexpr bool FIRST = decltype(first_c)::value, TAIL = decltype(tail_c)::value;
+        constexpr int LEFT = decltype(left_c)::value;
+        constexpr bool FILL = LEFT == AHEAD, MORE = LEFT > 0;
+        const int an = as == AHEAD - 1 ? 0 : as + 1, bn = bs == AHEAD ? 0 : bs + 1, bfill = bs == 0 ? AHEAD : bs - 1;
         static_for<0, 2>([&](auto sc) {
             constexpr int s = decltype(sc)::value;
             if constexpr (s == 1 && MORE) {
-                // this wavefront's transfers of the next step have landed (loads complete in order; with the eight of B
-                // that are younger still on their way, whatever stores are outstanding) and its last fragments of this
-                // step are in registers; behind the barrier, everybody's
-                wait_vm_lgkm0<FILL ? 8 : 0>();
+                // this wavefront's transfers of the next step have landed (loads complete in order; those of the steps behind
+                // it, B's half of a step sent so far among them, may be on their way, whatever stores are outstanding) and its
+                // last fragments of this step are in registers; behind the barrier, everybody's
+                wait_vm_lgkm0<FILL ? (AHEAD - 2) * 2 * T + T : (LEFT - 1) * 2 * T>();
                 __builtin_amdgcn_s_barrier();
             } else {
                 wait_lgkm<0>();
@@ -447,17 +463,17 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_wide_kernel(const _Float16*
                 constexpr int m = decltype(mc)::value;
                 constexpr int i = m / T, j = (i & 1) ? T - 1 - m % T : m % T;
                 mfma_16x16x32<FIRST && s == 0>(acc[i][j], bf[s][j], af[s][i]);
-                if constexpr (m % 2 == 0 && m / 2 < 2 * T) {
-                    if constexpr (s == 0) read(std::integral_constant<int, m / 2>{}, std::integral_constant<int, 1>{}, as * kWideOperand, bs * kWideOperand);
-                    else if constexpr (MORE) read(std::integral_constant<int, m / 2>{}, std::integral_constant<int, 0>{}, an * kWideOperand, bn * kWideOperand);
+                if constexpr (m % kReadEvery == 0 && m / kReadEvery < 2 * T) {
+                    if constexpr (s == 0) read(std::integral_constant<int, m / kReadEvery>{}, std::integral_constant<int, 1>{}, as * OPERAND, bs * OPERAND);
+                    else if constexpr (MORE) read(std::integral_constant<int, m / kReadEvery>{}, std::integral_constant<int, 0>{}, an * OPERAND, bn * OPERAND);
                 }
-                if constexpr (FILL && TAIL && m % 8 == 1) {
-                    constexpr int d = m / 8;
-                    if constexpr (s == 0) ob.template send_tail<d>(tile_b, g.sbk, fk, g.k - fk * BK, lds + (2 + bfill) * kWideOperand + (d * 4 + wave) * 1024, wave, lane);
-                    else oa.template send_tail<d>(tile_a, g.sak, fk, g.k - fk * BK, lds + as * kWideOperand + (d * 4 + wave) * 1024, wave, lane);
-                } else if constexpr (FILL && m % 8 == 1) {
-                    if constexpr (s == 0) send_b(std::integral_constant<int, m / 8>{}, bfill);
-                    else send_a(std::integral_constant<int, m / 8>{}, as);
+                if constexpr (FILL && TAIL && m % T == 1) {
+                    constexpr int d = m / T;
+                    if constexpr (s == 0) ob.template send_tail<d>(tile_b, g.sbk, fk, g.k - fk * BK, lds + (AHEAD + bfill) * OPERAND + (d * 4 + wave) * 1024, wave, lane);
+                    else oa.template send_tail<d>(tile_a, g.sak, fk, g.k - fk * BK, lds + as * OPERAND + (d * 4 + wave) * 1024, wave, lane);
+                } else if constexpr (FILL && m % T == 1) {
+                    if constexpr (s == 0) send_b(std::integral_constant<int, m / T>{}, bfill);
+                    else send_a(std::integral_constant<int, m / T>{}, as);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             });
@@ -484,34 +500,32 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_wide_kernel(const _Float16*
 
     using yes = std::true_type;
     using no = std::false_type;
+    using full = std::integral_constant<int, AHEAD>;
     for (;;) {
         const bool last = bid + gridDim.x >= total;
-        const WideTile t = wide_tile(g, bid);
+        const WideTile t = wide_tile<T>(g, bid);
         int nk = KSUM ? nkg * g.groups : nkg;
         if constexpr (SLICED) {
             nk = slice_begin(t.z1 + 1) - slice_begin(t.z1);
-            sum_in = g.asum ? t.n0 / kWideTile : -1;
+            sum_in = g.asum ? t.n0 / TILE : -1;
 #pragma unroll
             for (int i = 0; i < T; ++i) row_sum[i] = 0.f;
         }
-        const int fills = last ? nk - 2 : nk;
-        step(yes{}, yes{}, yes{}, no{});
+        const int fills = last ? nk - AHEAD : nk;
+        step(yes{}, full{}, no{});
         if constexpr (SLICED) {
-            // the last slice's last step may be ragged: it is sent two steps ahead (the host passes four steps then)
-            const int tail = g.k % BK != 0 && t.z1 + 1 == g.batch1 ? nk - 3 : -1;
+            // the last slice's last step may be ragged: it is sent AHEAD steps before (the host passes a step more then)
+            const int tail = g.k % BK != 0 && t.z1 + 1 == g.batch1 ? nk - 1 - AHEAD : -1;
             int kt = 1;
-            for (; kt < fills && kt != tail; ++kt) step(no{}, yes{}, yes{}, no{});
+            for (; kt < fills && kt != tail; ++kt) step(no{}, full{}, no{});
             if (kt == tail) {
-                step(no{}, yes{}, yes{}, yes{});
-                for (++kt; kt < fills; ++kt) step(no{}, yes{}, yes{}, no{});
+                step(no{}, full{}, yes{});
+                for (++kt; kt < fills; ++kt) step(no{}, full{}, no{});
             }
         } else {
-            for (int kt = 1; kt < fills; ++kt) step(no{}, yes{}, yes{}, no{});
+            for (int kt = 1; kt < fills; ++kt) step(no{}, full{}, no{});
         }
-        if (last) {
-            step(no{}, no{}, yes{}, no{});
-            step(no{}, no{}, no{}, no{});
-        }
+        if (last) static_for<1, AHEAD + 1>([&](auto lc) { step(no{}, std::integral_constant<int, AHEAD - decltype(lc)::value>{}, no{}); });
         // an accumulator is read no earlier than 18 wait states behind the last MFMA (the assembly hides them from the compiler),
         // and the next tile's first fragments are in their registers before the epilogue may use others around them
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_nop 15\n\ts_nop 3" ::: "memory");
@@ -522,13 +536,13 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_wide_kernel(const _Float16*
             c = g.gc[t.z0];
             bias = g.gbias[t.z0];
         }
-        const int mb = t.m0 + wm * 128, nb = t.n0 + wn * 128;
-        if (g.out_f32) wide_epilogue<float, EPI>(g, c, res_ptr, bias, acc, mb, nb, t.coff, lane, last);
-        else wide_epilogue<_Float16, EPI>(g, c, res_ptr, bias, acc, mb, nb, t.coff, lane, last);
+        const int mb = t.m0 + wm * WT, nb = t.n0 + wn * WT;
+        if (g.out_f32) wide_epilogue<T, float, EPI>(g, c, res_ptr, bias, acc, mb, nb, t.coff, lane, last);
+        else wide_epilogue<T, _Float16, EPI>(g, c, res_ptr, bias, acc, mb, nb, t.coff, lane, last);
         if constexpr (SLICED) {
             if (g.asum) {
                 float* const sums = reinterpret_cast<float*>(g.asum) +
-                                    ((((int64_t)t.z0 * g.batch1 + t.z1) * g.tiles_n + t.n0 / kWideTile) * 2 + wn) * g.m;
+                                    ((((int64_t)t.z0 * g.batch1 + t.z1) * g.tiles_n + t.n0 / TILE) * 2 + wn) * g.m;
 #pragma unroll
                 for (int i = 0; i < T; ++i) {
                     float v = row_sum[i];
@@ -548,6 +562,42 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_wide_kernel(const _Float16*
     }
 #endif
 }
+
+// ---------------------------------------------------------------- host side
+template <int T, int AKIND, int BKIND, int EPI, bool KSUM, bool SLICED = false>
+int launch_shape(const GemmArgs& g, const _Float16* a, const _Float16* b, void* c, const void* bias, const void* residual,
+                 hipStream_t st) {
+    auto kern = gemm_f16_wide_kernel<T, AKIND, BKIND, EPI, KSUM, SLICED>;
+    constexpr int lds = WideShape<T>::kLds;
+    const hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (e != hipSuccess) {
+        set_error("gemm_f16: cannot reserve %d bytes of LDS: %s", lds, hipGetErrorString(e));
+        return (int)e;
+    }
+    const unsigned grid = (unsigned)(g.total_blocks < kCus ? g.total_blocks : kCus);
+    hipLaunchKernelGGL(kern, grid, kThreads, lds, st, a, b, c, bias, residual, g);
+    return launch_status("gemm_f16(wide)");
+}
+
+inline int wide_unsupported(int ak, int bk) {
+    set_error("gemm_f16: no kernel with tiles that stay for operand kinds %d/%d", ak, bk);
+    return DMLHIP_ERR_UNSUPPORTED;
+}
+
+#define DML_WIDE_TILES(T)                                                                                          \
+    constexpr int tile = WideShape<T>::kTile;                                                                      \
+    g.tiles_m = (g.m + tile - 1) / tile;                                                                           \
+    g.tiles_n = (g.n + tile - 1) / tile;                                                                           \
+    const long long total = (long long)g.tiles_m * g.tiles_n * batch;                                              \
+    DML_REQUIRE(total <= 2147483647LL, DMLHIP_ERR_SHAPE, "gemm_f16: %lld workgroups exceed the grid limit", total); \
+    g.total_blocks = total;                                                                                        \
+    const int ek = epilogue_kind(g, bias, residual, nullptr);
+#define DML_WIDE_CASE(T, AK, BKD, EPI, KSUM)                    \
+    if (ak == AK && bk == BKD && ek == EPI && !!g.ksum == KSUM) \
+        return launch_shape<T, AK, BKD, EPI, KSUM>(g, a, b, c, bias, residual, st);
+#define DML_WIDE_CASES(T, AK, BKD)                                                                  \
+    DML_WIDE_CASE(T, AK, BKD, EPI_PLAIN, false) DML_WIDE_CASE(T, AK, BKD, EPI_GENERAL, false) \
+    DML_WIDE_CASE(T, AK, BKD, EPI_PLAIN, true) DML_WIDE_CASE(T, AK, BKD, EPI_GENERAL, true)
 
 // Adds up what SLICED left: blocks of 1024 results each, behind them (asum) blocks of 64 row sums; the group in blockIdx.y.
 // Reads of 4 bytes per result and slice and the result's own: 3.3 TB/s behind the product, 80 MB in 24 us.

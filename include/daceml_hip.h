@@ -513,7 +513,8 @@ int dmlhip_run_calls(const dmlhip_call* calls, int count, const uint64_t* pointe
  * only: 5 and 7 run them with the interleaved loop, 4, 6, 8 and 9 leave them on the plain one. 10 = 64x64, 12 = 32x32 tile
  * with K split over the wavefronts (products with too few 128-wide tiles for the chip; any K; operands as for the others, no
  * activation together with a residual, beta or a bias along m, row sums only of a row-contiguous A); 13 = 256x256 with
- * workgroups that stay for several tiles (what it does not take, runs as 4). */
+ * workgroups that stay for several tiles, 14 = 128x128 of the same kind, for a K-contiguous A (what they do not take, runs as 4
+ * and 5). */
 void dmlhip_debug_force_gemm_config(int cfg);
 /* Diagnostic: the configuration that the calling thread's last fp16 contraction launch ran on (of several launches, the
  * last); -1 = the kernel that stages its operands through registers. */

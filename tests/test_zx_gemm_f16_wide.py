@@ -1,4 +1,4 @@
-"""The fp16 contraction kernel of 256 x 256 tiles whose workgroups stay for several of them (configuration 13): every operand
+"""The fp16 contraction kernel whose workgroups stay for several tiles (configurations 13, 256 x 256, and 14, 128 x 128): every operand
 layout, one to many tiles per workgroup (more tiles than compute units: the steps of the next tile are on their way while a
 tile is written), edges of tiles, groups, operand pairs, both result types, residual and biases.
 
@@ -16,11 +16,13 @@ pytestmark = pytest.mark.gpu
 P = lambda t: ctypes.c_void_p(t.data_ptr()) if t is not None else None  # noqa: E731
 
 
-@pytest.mark.parametrize("layouts", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("cfg,layouts", [(13, (0, 0)), (13, (0, 1)), (13, (1, 0)), (13, (1, 1)), (14, (0, 0)), (14, (0, 1))])
 @pytest.mark.parametrize("m,n,k", [(8, 8, 192), (256, 256, 256), (264, 248, 192), (520, 768, 448), (136, 1032, 320)])
-def test_products(layouts, m, n, k, lib):
+def test_products(cfg, layouts, m, n, k, lib):
     from daceml_amd import _lib as L, kernels as K
-    lib.dmlhip_debug_force_gemm_config(13)
+    if cfg == 14:
+        k += 128   # five steps at least
+    lib.dmlhip_debug_force_gemm_config(cfg)
     r = rng(m + 7 * n + 31 * k)
     ops = [(_operand(r, m, k, layouts[0]), _operand(r, n, k, layouts[1])) for _ in range(3)]
     (a, ta, sa), (b, tb, sb) = ops[0]
@@ -43,31 +45,31 @@ def test_products(layouts, m, n, k, lib):
             rr = tres if kind == "residual" else None
             add = add + (res.astype(f) if rr is not None else 0.0)
             L.check(lib.dmlhip_gemm_f16(ctypes.byref(d), P(ta), P(tb), P(c), P(tb_), P(rr), None, K._stream()))
-            assert lib.dmlhip_debug_last_gemm_config() == 13
+            assert lib.dmlhip_debug_last_gemm_config() == cfg
             _check(c, exact + add, terms, k, eps, np.abs(add) + np.abs(exact) + np.abs(bias.astype(f)), (kind, out, layouts, m, n, k))
         d.bias_along_m = 0
         # three operand pairs along K, then three products side by side
         A, B = [o[0][1] for o in ops], [o[1][1] for o in ops]
         c = torch.full((m, n), float("nan"), device="cuda", dtype=dtype)
         L.check(lib.dmlhip_gemm_f16_ksum(ctypes.byref(d), 3, _table(A), _table(B), P(c), None, P(tres), K._stream()))
-        assert lib.dmlhip_debug_last_gemm_config() == 13
+        assert lib.dmlhip_debug_last_gemm_config() == cfg
         e3, t3 = _products([(o[0][0], o[1][0]) for o in ops])
         _check(c, e3 + res.astype(f), t3, 3 * k, eps, np.abs(res.astype(f)) + np.abs(e3), ("pairs", out, layouts, m, n, k))
         C = [torch.full((m, n), float("nan"), device="cuda", dtype=dtype) for _ in ops]
         L.check(lib.dmlhip_gemm_f16_grouped(ctypes.byref(d), 3, _table(A), _table(B), _table(C), None, None, 0, K._stream()))
-        assert lib.dmlhip_debug_last_gemm_config() == 13
+        assert lib.dmlhip_debug_last_gemm_config() == cfg
         for o, c in zip(ops, C):
             e1, t1 = _products([(o[0][0], o[1][0])])
             _check(c, e1, t1, k, eps, 0, ("groups", out, layouts, m, n, k))
 
 
-@pytest.mark.parametrize("layouts", [(0, 0), (0, 1), (1, 1)])
+@pytest.mark.parametrize("pinned,layouts", [(13, (0, 0)), (13, (0, 1)), (13, (1, 1)), (14, (0, 0)), (14, (0, 1))])
 @pytest.mark.parametrize("m,n,batch", [(16, 256 * 261, 1), (264, 512, 100), (4360, 4352, 1)])
-def test_several_tiles_per_workgroup(layouts, m, n, batch, lib):
+def test_several_tiles_per_workgroup(pinned, layouts, m, n, batch, lib):
     """More tiles than compute units, among them such of few rows behind whole ones and the other way round. Held against the
     128 x 128 tile, an fp32 result of which has its terms added in the order of K too: both are within k 2^-24 of the exact sums."""
     from daceml_amd import _lib as L, kernels as K
-    k = 192
+    k = 192 if pinned == 13 else 320
     g = torch.Generator(device="cuda").manual_seed(m + n)
     shape = lambda rows, layout: (batch, rows, k) if layout == 0 else (batch, k, rows)  # noqa: E731
     a = torch.randn(shape(m, layouts[0]), generator=g, device="cuda").half()
@@ -75,7 +77,7 @@ def test_several_tiles_per_workgroup(layouts, m, n, batch, lib):
     d = _desc(L, m, n, k, (k, 1) if layouts[0] == 0 else (1, m), (k, 1) if layouts[1] == 0 else (1, n), L.F32)
     d.batch[0], d.a_stride_batch[0], d.b_stride_batch[0], d.c_stride_batch[0] = batch, m * k, n * k, m * n
     got, want, terms = (torch.full((batch, m, n), float("nan"), device="cuda") for _ in range(3))
-    for cfg, x, y, c in ((13, a, b, got), (3, a, b, want), (3, a.abs(), b.abs(), terms)):
+    for cfg, x, y, c in ((pinned, a, b, got), (3, a, b, want), (3, a.abs(), b.abs(), terms)):
         lib.dmlhip_debug_force_gemm_config(cfg)
         L.check(lib.dmlhip_gemm_f16(ctypes.byref(d), P(x), P(y), P(c), None, None, None, K._stream()))
         assert lib.dmlhip_debug_last_gemm_config() == cfg
@@ -83,7 +85,7 @@ def test_several_tiles_per_workgroup(layouts, m, n, batch, lib):
     # fp16 results of the same tiles are these, rounded once
     d.out_dtype = L.F16
     c = torch.full((batch, m, n), float("nan"), device="cuda", dtype=torch.float16)
-    lib.dmlhip_debug_force_gemm_config(13)
+    lib.dmlhip_debug_force_gemm_config(pinned)
     L.check(lib.dmlhip_gemm_f16(ctypes.byref(d), P(a), P(b), P(c), None, None, None, K._stream()))
     assert torch.equal(c, got.half())
 
@@ -131,3 +133,13 @@ def test_which_weight_gradients_are_sliced(m, n, k, groups, sliced, lib):
     from daceml_amd import _lib as L
     d = _desc(L, m, n, k, (1, m), (1, n), L.F32)
     assert (lib.dmlhip_gemm_f16_grouped_asum_workspace_bytes(ctypes.byref(d)) >= 2 * groups * m * n * 4) == sliced
+
+
+@pytest.mark.parametrize("m,n,k,cfg", [(4096, 1024, 4096, 14), (2048, 1024, 1024, 14), (4096, 4096, 1024, 13), (4096, 1024, 960, 5)])
+def test_which_products_they_take(m, n, k, cfg, lib):
+    from daceml_amd import _lib as L, kernels as K
+    a, b = torch.zeros((m, k), device="cuda", dtype=torch.float16), torch.zeros((n, k), device="cuda", dtype=torch.float16)
+    c = torch.empty((m, n), device="cuda", dtype=torch.float16)
+    d = _desc(L, m, n, k, (k, 1), (k, 1), L.F16)
+    L.check(lib.dmlhip_gemm_f16(ctypes.byref(d), P(a), P(b), P(c), None, None, None, K._stream()))
+    assert lib.dmlhip_debug_last_gemm_config() == cfg
