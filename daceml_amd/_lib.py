@@ -80,6 +80,10 @@ SIGNATURES = {
     "dmlhip_softmax_f32": (c_int, [_P, _P, c_int64, c_int64, _P]),
     "dmlhip_softmax_backward_f16": (c_int, [_P, _P, _P, c_int64, c_int64, _P]),
     "dmlhip_softmax_backward_f32": (c_int, [_P, _P, _P, c_int64, c_int64, _P]),
+    "dmlhip_log_softmax_f16": (c_int, [_P, _P, c_int64, c_int64, _P]),
+    "dmlhip_log_softmax_f32": (c_int, [_P, _P, c_int64, c_int64, _P]),
+    "dmlhip_log_softmax_backward_f16": (c_int, [_P, _P, _P, c_int64, c_int64, _P]),
+    "dmlhip_log_softmax_backward_f32": (c_int, [_P, _P, _P, c_int64, c_int64, _P]),
     "dmlhip_layernorm_f16": (c_int, [_P, _P, _P, _P, _P, _P, _P, _P, c_int64, c_int64, c_float, _P]),
     "dmlhip_layernorm_f32": (c_int, [_P, _P, _P, _P, _P, _P, _P, _P, c_int64, c_int64, c_float, _P]),
     "dmlhip_layernorm_backward_workspace_bytes": (c_size_t, [c_int64, c_int64]),

@@ -305,7 +305,7 @@ class HipSoftmaxBackward(BackwardImplementation):
 class HipLogSoftmaxBackward(BackwardImplementation):
     """DefaultLogSoftmaxBackward (onnx_ops.py:338-373): ``dx = dy - exp(y) * ReduceSum(dy, axes=[axis], keepdims=1)``
     as the reference's own nodes - Exp, ReduceSum, Mul, Sub - with the sum over every axis the forward node made one
-    row of (from ``axis`` on)."""
+    row of (from ``axis`` on). For a forward node that the fusion passes made one pass it is one SoftmaxGrad node."""
     @staticmethod
     def backward_can_be_applied(node, state, sdfg) -> bool:
         for e in state.in_edges_by_connector(node, "input"):
@@ -321,6 +321,11 @@ class HipLogSoftmaxBackward(BackwardImplementation):
         nd = len(od.shape)
         axis = forward_node.axis % nd
         label = forward_node.label + "_backward"
+        if getattr(forward_node, "_one_pass", False):
+            sg = _new(context, "SoftmaxGrad", label, axis=axis)
+            sg._log = True
+            connect_output_from_forward(forward_node, sg, context, "output", "Y")
+            return sg, BackwardResult(required_grad_names={"input": "dX"}, given_grad_names={"output": "dY"})
         group = BackwardGroup(label)
         sums_shape = tuple(1 if i >= axis else e for i, e in enumerate(od.shape))
         probs, _ = sdfg.add_transient(label + "_exp", od.shape, od.dtype)

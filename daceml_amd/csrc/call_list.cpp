@@ -52,6 +52,10 @@ struct Entry {
     X(dmlhip_softmax_f32) \
     X(dmlhip_softmax_backward_f16) \
     X(dmlhip_softmax_backward_f32) \
+    X(dmlhip_log_softmax_f16) \
+    X(dmlhip_log_softmax_f32) \
+    X(dmlhip_log_softmax_backward_f16) \
+    X(dmlhip_log_softmax_backward_f32) \
     X(dmlhip_layernorm_f16) \
     X(dmlhip_layernorm_f32) \
     X(dmlhip_layernorm_backward_f16) \

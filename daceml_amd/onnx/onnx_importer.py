@@ -490,7 +490,9 @@ class ONNXModel:
     # ------------------------------------------------------------------ execution
     def auto_optimize(self):
         from ..transformation import fusion
-        return fusion.auto_optimize(self.sdfg, training=self.training)
+        stats = fusion.auto_optimize(self.sdfg, training=self.training)
+        fusion.fuse_log_softmax(self.sdfg)
+        return stats
 
     def compile_and_init(self, device=None):
         """Expands the library nodes and binds the kernels (daceml/onnx/onnx_importer.py:452-480)."""

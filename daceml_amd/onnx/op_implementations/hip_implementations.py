@@ -393,7 +393,8 @@ class HipLogSoftmax(ONNXForward):
     ``x - max``, ``exp``, row sum, ``log``, subtraction - with the temporaries in the workspace: the logarithm is
     taken of the row sum, never of a probability, so large negative inputs keep their finite values (a
     ``log(softmax(x))`` would turn everything below the smallest normal into ``-inf``, in fp16 everything below
-    about -16)."""
+    about -16). A private ``_one_pass`` attribute set by the fusion pass makes them one call, which holds a row in
+    registers."""
     @staticmethod
     def forward_can_be_applied(node, state, sdfg) -> bool:
         return HipSoftmax.forward_can_be_applied(node, state, sdfg)
@@ -404,6 +405,9 @@ class HipLogSoftmax(ONNXForward):
         axis = node.axis % len(x.shape)
         rows, cols = _prod(x.shape[:axis]), _prod(x.shape[axis:])
         sfx, code = _SFX[x.dtype], _CODE[x.dtype]
+        if getattr(node, "_one_pass", False):
+            call = HipCall("dmlhip_log_softmax_" + sfx, [Ptr("input"), Ptr("output"), I64(rows), I64(cols), Stream()])
+            return _tasklet(node, state, [call], bytes_moved=2 * _nbytes(x), kind="softmax")
         item = 2 if x.dtype == torch.float16 else 4
         align = lambda n: -(-n // 256) * 256  # noqa: E731
         # workspace: row maxima | x - max | row sums | their logarithms | scratch of the reductions
@@ -433,7 +437,9 @@ class HipLogSoftmax(ONNXForward):
 @op_implementation(op="SoftmaxGrad", name=IMPL)
 class HipSoftmaxGrad(ONNXForward):
     """The node DefaultSoftmaxBackward builds from ONNXMul / ONNXReduceSum / a subtraction map
-    (autodiff/implementations/onnx_ops.py:237-275), as one kernel: dx = y*dy - y*sum(y*dy)."""
+    (autodiff/implementations/onnx_ops.py:237-275), as one kernel: dx = y*dy - y*sum(y*dy). With a private ``_log``
+    attribute, set where a LogSoftmax of one pass is reversed, those of DefaultLogSoftmaxBackward (:338-373):
+    dx = dy - exp(y)*sum(dy), over the axes from ``axis`` on."""
     @staticmethod
     def forward_can_be_applied(node, state, sdfg) -> bool:
         try:
@@ -441,16 +447,16 @@ class HipSoftmaxGrad(ONNXForward):
             y, dy, dx = ins["Y"], ins["dY"], outs["dX"]
             nd = len(y.shape)
             return (_float_ok(y, dy, dx) and _dense(y, dy, dx) and y.shape == dy.shape == dx.shape
-                    and node.axis % nd == nd - 1)
+                    and (getattr(node, "_log", False) or node.axis % nd == nd - 1))
         except Exception:
             return False
 
     @staticmethod
     def forward(node, state, sdfg):
         y = in_desc_with_name(node, state, sdfg, "Y")
-        cols = y.shape[-1]
-        rows = _prod(y.shape[:-1])
-        call = HipCall("dmlhip_softmax_backward_" + _SFX[y.dtype],
+        axis = node.axis % len(y.shape)
+        rows, cols = _prod(y.shape[:axis]), _prod(y.shape[axis:])
+        call = HipCall("dmlhip_%ssoftmax_backward_%s" % ("log_" if getattr(node, "_log", False) else "", _SFX[y.dtype]),
                        [Ptr("Y"), Ptr("dY"), Ptr("dX"), I64(rows), I64(cols), Stream()])
         return _tasklet(node, state, [call], bytes_moved=3 * _nbytes(y), kind="softmax_backward")
 

@@ -190,6 +190,8 @@ class DaceModule(nn.Module):
         dummy_inputs = tuple(t.to(device) for t in dummy_inputs)
         model = self._import(dummy_inputs)
         sdfg, state = model.sdfg, model.state
+        if self.auto_optimize:
+            fusion.fuse_log_softmax(sdfg)
         params = self._exported_parameters
         tensor_inputs = [n for n in model.inputs if n not in params]
         param_inputs = [n for n in model.inputs if n in params]

@@ -12,6 +12,7 @@ expansions it replaces (that composition is the oracle of the fused kernels).
     fuse_layernorm           ReduceMean, Sub, Pow, ReduceMean, Add, Sqrt,
                              Div, Mul, Add                                -> LayerNormalization
     fuse_swish               Sigmoid, Mul                                 -> Swish
+    fuse_log_softmax         LogSoftmax of short rows                     -> one pass in place of six calls
     lower_matmul             MatMul                                       -> Einsum (PureMatMul's lowering)
     fold_views               Transpose / Reshape around an Einsum         -> operand letters / dense views
     fuse_epilogues           Einsum, [Div|Mul const], [Add bias], [Gelu],
@@ -295,6 +296,25 @@ def fuse_swish(sdfg: SDFG) -> int:
             _add_node(sdfg, state, "Swish", sig.label.replace("_sigmoid", "") + "_fused", {"X": x}, {"Y": out})
             count += 1
     _drop_unused_arrays(sdfg)
+    return count
+
+
+#: widest rows that dmlhip_log_softmax_* take
+LOG_SOFTMAX_COLS = 1024
+
+
+def fuse_log_softmax(sdfg: SDFG) -> int:
+    """LogSoftmax over rows that a wavefront holds in its registers: the six calls of its expansion become one, and the
+    Exp, ReduceSum, Mul, Sub of its reverse another. Wider rows stay with those calls, which split a row over workgroups.
+    The node keeps its kind, so the pass runs behind ``auto_optimize``, where a program is made of the graph."""
+    count = 0
+    for state in sdfg.states():
+        for node in [n for n in state.nodes() if _is_op(n, "LogSoftmax") and not getattr(n, "_one_pass", False)]:
+            x, y = (sdfg.arrays[a] for a in (_in_array(state, node, "input"), _out_array(state, node, "output")))
+            shape = x.shape
+            if shape and x.is_contiguous() and y.is_contiguous() and math.prod(shape[node.axis % len(shape):]) <= LOG_SOFTMAX_COLS:
+                node._one_pass = True
+                count += 1
     return count
 
 

@@ -66,6 +66,16 @@ int dmlhip_softmax_backward_f16(const void* y, const void* dy, void* dx, int64_t
 int dmlhip_softmax_backward_f32(const void* y, const void* dy, void* dx, int64_t rows,
                                 int64_t cols, void* stream);
 
+/* LogSoftmax "pure" (pure_implementations.py:649-656) and DefaultLogSoftmaxBackward
+ * (autodiff/implementations/onnx_ops.py:338-373), each in one pass, for rows of up to 1024 values:
+ * y = (x-max) - log(sum_row(exp(x-max))), dx = dy - exp(y)*sum_row(dy). */
+int dmlhip_log_softmax_f16(const void* x, void* y, int64_t rows, int64_t cols, void* stream);
+int dmlhip_log_softmax_f32(const void* x, void* y, int64_t rows, int64_t cols, void* stream);
+int dmlhip_log_softmax_backward_f16(const void* y, const void* dy, void* dx, int64_t rows,
+                                    int64_t cols, void* stream);
+int dmlhip_log_softmax_backward_f32(const void* y, const void* dy, void* dx, int64_t rows,
+                                    int64_t cols, void* stream);
+
 /* ------------------------------------------------------------------ LayerNormalization
  * The opset-12 export has no LayerNormalization node; the reference runs the chain
  * ReduceMean, Sub, Pow, ReduceMean, Add, Sqrt, Div, Mul, Add

@@ -342,6 +342,16 @@ class Emulator:
                 xv = x.reshape(-1)[:rows * cols].astype(np.float64).reshape(rows, cols)
                 e = np.exp(xv - xv.max(-1, keepdims=True))
                 y.reshape(-1)[:rows * cols] = (e / e.sum(-1, keepdims=True)).reshape(-1).astype(y.dtype)
+            elif call.symbol in ("dmlhip_log_softmax_f16", "dmlhip_log_softmax_f32"):
+                x, y, rows, cols = args[:4]
+                xv = x.reshape(-1)[:rows * cols].astype(np.float64).reshape(rows, cols)
+                xv = xv - xv.max(-1, keepdims=True)
+                y.reshape(-1)[:rows * cols] = (xv - np.log(np.exp(xv).sum(-1, keepdims=True))).reshape(-1).astype(y.dtype)
+            elif call.symbol in ("dmlhip_log_softmax_backward_f16", "dmlhip_log_softmax_backward_f32"):
+                yv, dy, dx, rows, cols = args[:5]
+                y64 = yv.reshape(-1)[:rows * cols].astype(np.float64).reshape(rows, cols)
+                d64 = dy.reshape(-1)[:rows * cols].astype(np.float64).reshape(rows, cols)
+                dx.reshape(-1)[:rows * cols] = (d64 - np.exp(y64) * d64.sum(-1, keepdims=True)).reshape(-1).astype(dx.dtype)
             elif call.symbol in ("dmlhip_layernorm_f16", "dmlhip_layernorm_f32"):
                 layernorm(*args[:11])
             elif call.symbol in ("dmlhip_layernorm_backward_f16", "dmlhip_layernorm_backward_f32"):
