@@ -149,6 +149,8 @@ SIGNATURES = {
     "dmlhip_conv2d_f16": (c_int, [POINTER(Conv2dDesc), _P, _P, _P, _P, _P]),
     "dmlhip_conv2d_gated_f32": (c_int, [POINTER(Conv2dDesc), _P, _P, _P, _P, _P, _P]),
     "dmlhip_conv2d_expand_depthwise_f32": (c_int, [POINTER(Conv2dDesc), POINTER(Conv2dDesc), _P, _P, _P, _P, _P, _P, _P]),
+    "dmlhip_conv2d_expand_depthwise_pool_workspace_bytes": (c_size_t, [POINTER(Conv2dDesc), POINTER(Conv2dDesc)]),
+    "dmlhip_conv2d_expand_depthwise_pool_f32": (c_int, [POINTER(Conv2dDesc), POINTER(Conv2dDesc)] + [_P] * 8 + [c_size_t, _P]),
     "dmlhip_conv2d_backward_data_f32": (c_int, [POINTER(Conv2dDesc), _P, _P, _P, _P]),
     "dmlhip_conv2d_backward_weight_workspace_bytes": (c_size_t, [POINTER(Conv2dDesc)]),
     "dmlhip_conv2d_backward_weight_f32": (c_int, [POINTER(Conv2dDesc), _P, _P, _P, _P, c_size_t, _P]),

@@ -109,6 +109,7 @@ struct Entry {
     X(dmlhip_conv2d_f16) \
     X(dmlhip_conv2d_gated_f32) \
     X(dmlhip_conv2d_expand_depthwise_f32) \
+    X(dmlhip_conv2d_expand_depthwise_pool_f32) \
     X(dmlhip_conv2d_backward_data_f32) \
     X(dmlhip_conv2d_backward_weight_f32) \
     X(dmlhip_reduce_sum_multi_f16) \

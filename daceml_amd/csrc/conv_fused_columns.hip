@@ -14,6 +14,12 @@
 // [96,32,112,112] -> 192 channels, swish / swish: stride 2 338 -> 232 us,
 // stride 1 780 -> 484 us (1.08 GB of X and results); [24,16,112,112] -> 96, stride 2 42 -> 27, stride 1 102 -> 45.
 // Every sum is added in the order of the other kernels: the results are the same bits.
+//
+// POOL: the results' mean over an image and channel too (the squeeze-excite gate's input), from the registers they are stored
+// from: a lane adds its row's results to a sum of its own, and a launch behind adds up the wavefronts' sums. Sums of rows are added
+// in fp64: a row is few values, but there are many rows and wavefronts (fp32 throughout 7.0e-8 from the mean in fp64, the
+// separate kernel 5.4e-8, so 2.7e-8). This kernel and the separate mean / with the mean, us: [96,32,112,112] -> 192, stride 2
+// 258 / 228, stride 1 667 / 485; [96,48,56,56] -> 288 241 / 190; [24,16,112,112] -> 96, stride 2 34.1 / 29.0; one image 9.8 / 9.1.
 #include "common.h"
 #include "conv_geom.h"
 
@@ -33,6 +39,7 @@ struct ColArgs {
     int seg_rows, cunits, units;     // output rows of a unit; units along a row; units of an image
     uint32_t pairs, cblocks, total;  // wavefronts per image and channel block; channel blocks; wavefronts
     uint32_t blocks;
+    float* sums;                     // POOL: [image][pair][expanded channel]
 };
 
 __device__ __forceinline__ float col_swish(float v) { return v * sigmoid_epilogue_f(v); }
@@ -49,7 +56,7 @@ __device__ __forceinline__ void col_activate(float (&v)[N], int act) {
     }
 }
 
-template <int CHUNKS, int STRIDE, bool SWISH>
+template <int CHUNKS, int STRIDE, bool SWISH, bool POOL>
 __global__ __launch_bounds__(kColWaves * 64, 3) void expand_depthwise_columns_kernel(const float* __restrict__ x,
                                                                                   const float* __restrict__ we,
                                                                                   const float* __restrict__ be,
@@ -120,6 +127,11 @@ __global__ __launch_bounds__(kColWaves * 64, 3) void expand_depthwise_columns_ke
     uint32_t soff = (uint32_t)(sch * oplane + srow * a.ow + scol) * 4u;
     const auto ybuf = __builtin_amdgcn_make_buffer_rsrc((void*)(y + ((size_t)n * a.cmid + c0) * oplane), 0,
                                                         kColCB * oplane * 4, kBufferFlags);
+    // ---- POOL: which results of this lane's channel and unit exist
+    const int pcols = hh && !second ? 0 : a.ow - (hh ? cu1 : cu0) * kOut;
+    const bool pragged = POOL && __builtin_amdgcn_ballot_w64(pcols < kOut) != 0;
+    int prow = (hh ? seg1 : seg0) * a.seg_rows;
+    double psum = 0.0;
     float* const ex_w = &exchange[wave][j * kColPitch + hh * kOut];
     const float* const ex_r = &exchange[wave][sch * kColPitch + sidx];
 
@@ -155,6 +167,18 @@ __global__ __launch_bounds__(kColWaves * 64, 3) void expand_depthwise_columns_ke
         col_activate<SWISH>(s, a.act2);
 #pragma unroll
         for (int o = 0; o < kOut; ++o) ex_w[o] = s[o];
+        if constexpr (POOL) {
+            float r = 0.f;
+            if (pragged) {
+#pragma unroll
+                for (int o = 0; o < kOut; ++o) r += o < pcols ? s[o] : 0.f;
+            } else {
+#pragma unroll
+                for (int o = 0; o < kOut; ++o) r += s[o];
+            }
+            psum += (double)(prow < a.oh ? r : 0.f);
+            ++prow;
+        }
         // LDS operations of one wavefront take effect in order: only the compiler has to keep them so
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -209,14 +233,45 @@ __global__ __launch_bounds__(kColWaves * 64, 3) void expand_depthwise_columns_ke
             stencil_row(s1, e, 0);
         }
     }
+    if constexpr (POOL) {
+        psum += __shfl_xor(psum, 32);   // both units
+        if (lane < 32) a.sums[((size_t)n * a.pairs + pair) * a.cmid + c0 + j] = (float)psum;
+    }
 }
 
-template <int CHUNKS>
+// The mean of an image's channel from its wavefronts' sums: sixteen channels of one image per workgroup, sixteen lanes each, a
+// lane's first eight loads in flight together (2 - 3 us, a launch that waits for memory once).
+__global__ __launch_bounds__(256) void pool_columns_kernel(const float* __restrict__ sums, float* __restrict__ pooled, int cmid,
+                                                           int pairs, double pixels) {
+    __shared__ double share[16][17];
+    const int c = threadIdx.x & 15, slot = threadIdx.x >> 4;
+    const uint32_t per = (uint32_t)cmid / 16u;
+    const uint32_t n = blockIdx.x / per, c0 = (blockIdx.x - n * per) * 16u;
+    const float* p = sums + (size_t)n * pairs * cmid + c0 + c;
+    double s = 0.0;
+    for (int q0 = slot; q0 < pairs; q0 += 128) {
+        float v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = p[(size_t)min(q0 + 16 * i, pairs - 1) * cmid];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) s += (double)(q0 + 16 * i < pairs ? v[i] : 0.f);
+    }
+    share[slot][c] = s;
+    __syncthreads();
+    if (slot == 0) {
+        s = 0.0;
+#pragma unroll
+        for (int q = 0; q < 16; ++q) s += share[q][c];
+        pooled[(size_t)n * cmid + c0 + c] = (float)(s / pixels);
+    }
+}
+
+template <int CHUNKS, bool POOL>
 int launch_columns(const ColArgs& a, int stride, const float* x, const float* we, const float* be, const float* wd,
                    const float* bd, float* y, hipStream_t st) {
     const bool swish = a.act1 == DMLHIP_ACT_SWISH && a.act2 == DMLHIP_ACT_SWISH;
-    const auto kern = stride == 1 ? (swish ? expand_depthwise_columns_kernel<CHUNKS, 1, true> : expand_depthwise_columns_kernel<CHUNKS, 1, false>)
-                                  : (swish ? expand_depthwise_columns_kernel<CHUNKS, 2, true> : expand_depthwise_columns_kernel<CHUNKS, 2, false>);
+    const auto kern = stride == 1 ? (swish ? expand_depthwise_columns_kernel<CHUNKS, 1, true, POOL> : expand_depthwise_columns_kernel<CHUNKS, 1, false, POOL>)
+                                  : (swish ? expand_depthwise_columns_kernel<CHUNKS, 2, true, POOL> : expand_depthwise_columns_kernel<CHUNKS, 2, false, POOL>);
     note_conv_form(16);
     hipLaunchKernelGGL(kern, a.blocks, kColWaves * 64, 0, st, x, we, be, wd, bd, y, a);
     return launch_status("conv2d_expand_depthwise");
@@ -229,21 +284,24 @@ int column_compute_units() {
     return cus > 0 ? cus : 256;
 }
 
-// *applies = false: nothing launched, the kernels with the expanded rows in LDS have to run
-int launch_expand_depthwise_columns(const dmlhip_conv2d_desc& pw, int stride, int act2, const float* x, const float* we,
-                                    const float* be, const float* wd, const float* bd, float* y, hipStream_t st, bool* applies) {
+size_t column_sums_bytes(int64_t n, int64_t cmid, int64_t pairs) { return (size_t)(n * pairs * cmid) * sizeof(float); }
+
+// How the kernel above runs a problem, with no more than `most` bytes of sums; false: the kernels with the expanded rows in LDS
+// have to run
+bool plan_columns(const dmlhip_conv2d_desc& pw, int stride, int act2, size_t most, ColArgs& a) {
     const int64_t n = pw.n, cin = pw.c, cmid = pw.m, h = pw.h, w = pw.w;
     const int act1 = pw.act;
-    *applies = false;
-    if (cin > kColMaxCin) return 0;
+    if (cin > kColMaxCin) return false;
     const bool swish = act1 == DMLHIP_ACT_SWISH || act2 == DMLHIP_ACT_SWISH, relu = act1 == DMLHIP_ACT_RELU || act2 == DMLHIP_ACT_RELU;
-    if (act1 == DMLHIP_ACT_SIGMOID || act2 == DMLHIP_ACT_SIGMOID || (swish && relu)) return 0;   // as the other kernels
-    ColArgs a;
+    if (act1 == DMLHIP_ACT_SIGMOID || act2 == DMLHIP_ACT_SIGMOID || (swish && relu)) return false;   // as the other kernels
+    // where not one row fits the other kernels' LDS the call stays refused
+    if (expand_depthwise_pinned() || dmlhip_conv2d_expand_depthwise_lds_bytes(w, cin, stride) == 0) return false;
+    a.sums = nullptr;
     a.cmid = (int)cmid; a.h = (int)h; a.w = (int)w; a.act1 = act1; a.act2 = act2;
     a.oh = (int)((h - 1) / stride + 1);
     a.ow = (int)((w - 1) / stride + 1);
     // an image's input and a channel block's output are addressed with 32-bit byte offsets
-    if (cin * h * w >= (1LL << 29) || (int64_t)kColCB * a.oh * a.ow >= (1LL << 29)) return 0;
+    if (cin * h * w >= (1LL << 29) || (int64_t)kColCB * a.oh * a.ow >= (1LL << 29)) return false;
     const int out = kColFresh / stride;
     a.cunits = (a.ow + out - 1) / out;
     a.cblocks = (uint32_t)(cmid / kColCB);
@@ -255,7 +313,7 @@ int launch_expand_depthwise_columns(const dmlhip_conv2d_desc& pw, int stride, in
     // [96,80,14,14] -> 480 50 and 56, [96,64,28,28] -> 384 102 and 110.
     const int64_t rows_of_units = n * a.cblocks * h * a.cunits;
     if (5 * w < 4LL * kColFresh * a.cunits || (w <= 42 && (cin > 32 || rows_of_units < 4000)) || (cin > 32 && rows_of_units < 8000))
-        return 0;
+        return false;
     // Output rows of a unit: each unit expands its first rows (3 - stride of them) once more and starts without loads in
     // flight, so few; but a SIMD has the throughput of about three wavefronts. Cost in image rows of the busiest SIMD.
     const long long simds = 4LL * column_compute_units();
@@ -264,7 +322,7 @@ int launch_expand_depthwise_columns(const dmlhip_conv2d_desc& pw, int stride, in
         const int rows = (a.oh + segs - 1) / segs;
         const long long units = (long long)a.cunits * ((a.oh + rows - 1) / rows);
         const long long waves = (long long)n * a.cblocks * ((units + 1) / 2);
-        if (waves > 0x3fffffffLL || units > 0x3fffffffLL) break;
+        if (waves > 0x3fffffffLL || units > 0x3fffffffLL || column_sums_bytes(n, cmid, (units + 1) / 2) > most) break;
         const long long cost = std::max(3LL, (waves + simds - 1) / simds) * ((rows - 1) * stride + 3 + 1);
         if (best < 0 || cost < best) {
             best = cost;
@@ -274,26 +332,22 @@ int launch_expand_depthwise_columns(const dmlhip_conv2d_desc& pw, int stride, in
             a.total = (uint32_t)waves;
         }
     }
-    if (best < 0) return 0;
+    if (best < 0) return false;
     a.blocks = (a.total + kColWaves - 1) / kColWaves;
-    *applies = true;
+    return true;
+}
+
+template <bool POOL>
+int launch_columns(const ColArgs& a, int64_t cin, int stride, const float* x, const float* we, const float* be, const float* wd,
+                   const float* bd, float* y, hipStream_t st) {
     switch (cin / 16) {
-        case 1: return launch_columns<1>(a, stride, x, we, be, wd, bd, y, st);
-        case 2: return launch_columns<2>(a, stride, x, we, be, wd, bd, y, st);
-        default: return launch_columns<3>(a, stride, x, we, be, wd, bd, y, st);
+        case 1: return launch_columns<1, POOL>(a, stride, x, we, be, wd, bd, y, st);
+        case 2: return launch_columns<2, POOL>(a, stride, x, we, be, wd, bd, y, st);
+        default: return launch_columns<3, POOL>(a, stride, x, we, be, wd, bd, y, st);
     }
 }
 
-}  // namespace
-}  // namespace dml
-
-using namespace dml;
-
-extern "C" {
-
-int dmlhip_conv2d_expand_depthwise_f32(const dmlhip_conv2d_desc* pw, const dmlhip_conv2d_desc* dw, const void* x,
-                                       const void* w_pw, const void* b_pw, const void* w_dw, const void* b_dw, void* y,
-                                       void* stream) {
+int check_expand_depthwise(const dmlhip_conv2d_desc* pw, const dmlhip_conv2d_desc* dw) {
     DML_REQUIRE(pw && dw, DMLHIP_ERR_NULL, "conv2d_expand_depthwise: NULL descriptor");
     DML_REQUIRE(pw->n >= 0 && pw->c > 0 && pw->h > 0 && pw->w > 0 && pw->m > 0, DMLHIP_ERR_SHAPE,
                 "conv2d_expand_depthwise: extents must be positive");
@@ -313,18 +367,54 @@ int dmlhip_conv2d_expand_depthwise_f32(const dmlhip_conv2d_desc* pw, const dmlhi
                 "conv2d_expand_depthwise: needs input channels %% 16 == 0 and expanded channels %% 32 == 0");
     DML_REQUIRE(pw->h * pw->w < (1LL << 30) && pw->w <= 4096 && pw->c * pw->h * pw->w < (1LL << 31), DMLHIP_ERR_UNSUPPORTED,
                 "conv2d_expand_depthwise: image too large");
+    return 0;
+}
+
+}  // namespace
+}  // namespace dml
+
+using namespace dml;
+
+extern "C" {
+
+int dmlhip_conv2d_expand_depthwise_f32(const dmlhip_conv2d_desc* pw, const dmlhip_conv2d_desc* dw, const void* x,
+                                       const void* w_pw, const void* b_pw, const void* w_dw, const void* b_dw, void* y,
+                                       void* stream) {
+    if (int e = check_expand_depthwise(pw, dw)) return e;
     if (pw->n == 0) return 0;
     DML_REQUIRE(x && w_pw && w_dw && y, DMLHIP_ERR_NULL, "conv2d_expand_depthwise: NULL tensor pointer");
-    hipStream_t st = (hipStream_t)stream;
-    // where not one row fits the other kernels' LDS the call stays refused
-    if (!expand_depthwise_pinned() && dmlhip_conv2d_expand_depthwise_lds_bytes(pw->w, pw->c, dw->stride_h) != 0) {
-        bool applies = false;
-        const int rc = launch_expand_depthwise_columns(*pw, (int)dw->stride_h, dw->act, (const float*)x, (const float*)w_pw,
-                                                       (const float*)b_pw, (const float*)w_dw, (const float*)b_dw, (float*)y, st,
-                                                       &applies);
-        if (applies) return rc;
+    ColArgs a;
+    if (plan_columns(*pw, (int)dw->stride_h, dw->act, SIZE_MAX, a))
+        return launch_columns<false>(a, pw->c, (int)dw->stride_h, (const float*)x, (const float*)w_pw, (const float*)b_pw,
+                                     (const float*)w_dw, (const float*)b_dw, (float*)y, (hipStream_t)stream);
+    return launch_expand_depthwise_lds(pw, dw, x, w_pw, b_pw, w_dw, b_dw, y, (hipStream_t)stream);
+}
+
+size_t dmlhip_conv2d_expand_depthwise_pool_workspace_bytes(const dmlhip_conv2d_desc* pw, const dmlhip_conv2d_desc* dw) {
+    ColArgs a;
+    if (check_expand_depthwise(pw, dw) || pw->n == 0 || !plan_columns(*pw, (int)dw->stride_h, dw->act, SIZE_MAX, a)) return 0;
+    return column_sums_bytes(pw->n, pw->m, a.pairs);
+}
+
+int dmlhip_conv2d_expand_depthwise_pool_f32(const dmlhip_conv2d_desc* pw, const dmlhip_conv2d_desc* dw, const void* x,
+                                            const void* w_pw, const void* b_pw, const void* w_dw, const void* b_dw, void* y,
+                                            void* pooled, void* workspace, size_t workspace_bytes, void* stream) {
+    if (int e = check_expand_depthwise(pw, dw)) return e;
+    if (pw->n == 0) return 0;
+    DML_REQUIRE(x && w_pw && w_dw && y && pooled, DMLHIP_ERR_NULL, "conv2d_expand_depthwise_pool: NULL tensor pointer");
+    const int stride = (int)dw->stride_h;
+    ColArgs a;
+    if (!plan_columns(*pw, stride, dw->act, workspace ? workspace_bytes : 0, a)) {
+        if (int e = dmlhip_conv2d_expand_depthwise_f32(pw, dw, x, w_pw, b_pw, w_dw, b_dw, y, stream)) return e;
+        const int64_t pixels = ((pw->h - 1) / stride + 1) * ((pw->w - 1) / stride + 1);
+        return dmlhip_reduce_f32(DMLHIP_RMEAN, y, pooled, DMLHIP_F32, pw->n * pw->m, pixels, 1, nullptr, 0, stream);
     }
-    return launch_expand_depthwise_lds(pw, dw, x, w_pw, b_pw, w_dw, b_dw, y, st);
+    a.sums = (float*)workspace;
+    if (int e = launch_columns<true>(a, pw->c, stride, (const float*)x, (const float*)w_pw, (const float*)b_pw,
+                                     (const float*)w_dw, (const float*)b_dw, (float*)y, (hipStream_t)stream)) return e;
+    hipLaunchKernelGGL(pool_columns_kernel, (unsigned)(pw->n * (a.cmid / 16)), 256, 0, (hipStream_t)stream, a.sums, (float*)pooled,
+                       a.cmid, (int)a.pairs, (double)a.oh * a.ow);
+    return launch_status("conv2d_expand_depthwise_pool");
 }
 
 }  // extern "C"

@@ -7,6 +7,7 @@ these must reproduce) and the cuDNN expansion of cudnn_implementations.py (whose
 library behind an expansion — these play). ``forward_can_be_applied`` never raises: anything outside
 what the kernels cover returns False.
 """
+import ctypes
 import math
 from typing import List, Optional, Sequence, Tuple
 
@@ -1422,8 +1423,8 @@ class HipGatedConv(ONNXForward):
 @op_implementation(op="ExpandDepthwiseConv", name=IMPL)
 class HipExpandDepthwiseConv(ONNXForward):
     """Pointwise Conv + activation + 3x3 depthwise Conv + activation (img_op_implementations.py:164-330 twice, with
-    the elementwise ops of pure_implementations.py:556-560 between) in one kernel; the expanded tensor stays in LDS.
-    fp32."""
+    the elementwise ops of pure_implementations.py:556-560 between) in one kernel; the expanded tensor stays on chip.
+    fp32. ``Pooled``, if it is connected, is the result's GlobalAveragePool (img_op_implementations.py:415-417)."""
     @staticmethod
     def _descs(node, x, w_pw, w_dw, y):
         stride = int((node.strides or [1, 1])[0])
@@ -1458,6 +1459,9 @@ class HipExpandDepthwiseConv(ONNXForward):
                 if b in ins and not (ins[b].dtype == x.dtype and ins[b].is_contiguous()
                                      and ins[b].total_size == w1.shape[0]):
                     return False
+            if "Pooled" in outs and not (_float_ok(x, outs["Pooled"]) and outs["Pooled"].is_contiguous()
+                                         and outs["Pooled"].total_size == x.shape[0] * w1.shape[0]):
+                return False
             from daceml_amd.transformation.fusion import EXPAND_DEPTHWISE_ACTIVATIONS
             if (node.act_pw, node.act_dw) not in EXPAND_DEPTHWISE_ACTIVATIONS:
                 return False
@@ -1472,11 +1476,16 @@ class HipExpandDepthwiseConv(ONNXForward):
         ins, outs = _descs(node, state, sdfg)
         x, w1, w2, y = ins["X"], ins["W_pw"], ins["W_dw"], outs["Y"]
         pw, dw, _ = HipExpandDepthwiseConv._descs(node, x, w1, w2, y)
-        call = HipCall("dmlhip_conv2d_expand_depthwise_f32",
-                       [Struct(pw, "dmlhip_conv2d_desc"), Struct(dw, "dmlhip_conv2d_desc"), Ptr("X"), Ptr("W_pw"),
-                        _opt(node, state, "B_pw"), Ptr("W_dw"), _opt(node, state, "B_dw"), Ptr("Y"), Stream()])
+        args = [Struct(pw, "dmlhip_conv2d_desc"), Struct(dw, "dmlhip_conv2d_desc"), Ptr("X"), Ptr("W_pw"),
+                _opt(node, state, "B_pw"), Ptr("W_dw"), _opt(node, state, "B_dw"), Ptr("Y")]
+        workspace = 0
+        if "Pooled" in outs:
+            workspace = L.load().dmlhip_conv2d_expand_depthwise_pool_workspace_bytes(ctypes.byref(pw), ctypes.byref(dw))
+            call = HipCall("dmlhip_conv2d_expand_depthwise_pool_f32", args + [Ptr("Pooled"), Workspace(), WorkspaceBytes(), Stream()])
+        else:
+            call = HipCall("dmlhip_conv2d_expand_depthwise_f32", args + [Stream()])
         mid = x.shape[0] * w1.shape[0] * x.shape[2] * x.shape[3]
-        return _tasklet(node, state, [call], flops=2 * mid * x.shape[1] + 18 * y.total_size,
+        return _tasklet(node, state, [call], workspace_bytes=workspace, flops=2 * mid * x.shape[1] + 18 * y.total_size,
                         bytes_moved=_nbytes(x, w1, w2, y), kind="conv")
 
 

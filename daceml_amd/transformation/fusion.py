@@ -13,6 +13,8 @@ expansions it replaces (that composition is the oracle of the fused kernels).
                              Div, Mul, Add                                -> LayerNormalization
     fuse_swish               Sigmoid, Mul                                 -> Swish
     fuse_log_softmax         LogSoftmax of short rows                     -> one pass in place of six calls
+    fuse_pool_into_expand_depthwise
+                             ExpandDepthwiseConv, GlobalAveragePool       -> the pool as that node's second result
     lower_matmul             MatMul                                       -> Einsum (PureMatMul's lowering)
     fold_views               Transpose / Reshape around an Einsum         -> operand letters / dense views
     fuse_epilogues           Einsum, [Div|Mul const], [Add bias], [Gelu],
@@ -25,6 +27,7 @@ expansions it replaces (that composition is the oracle of the fused kernels).
     fuse_conv_activation     Conv, Swish | Sigmoid | Relu                 -> Conv(_activation)
     fuse_gate_into_conv      Mul(X, gate[n,c,1,1]), Conv 1x1              -> GatedConv (inference graphs)
 """
+import ctypes
 import math
 from typing import Dict, List, Optional, Tuple
 
@@ -522,6 +525,30 @@ def fuse_expand_depthwise(sdfg: SDFG) -> int:
             count += 1
     if count:
         _drop_unused_arrays(sdfg)
+    return count
+
+
+def fuse_pool_into_expand_depthwise(sdfg: SDFG) -> int:
+    """A GlobalAveragePool of an ExpandDepthwiseConv's result becomes that node's second result where the kernel that runs it
+    sums as it stores; the library is asked for the problem's shapes, as its own choice of a kernel goes by them."""
+    from ..onnx.op_implementations.hip_implementations import HipExpandDepthwiseConv
+    count = 0
+    for state in sdfg.states():
+        for conv in [n for n in state.nodes() if _is_op(n, "ExpandDepthwiseConv")]:
+            y = _out_array(state, conv, "Y")
+            pools = [n for n, _ in _consumers(state, y) if _is_op(n, "GlobalAveragePool")]
+            if not pools or _out_array(state, conv, "Pooled") is not None:
+                continue
+            pooled = _out_array(state, pools[0], "Y")
+            xd, w1, w2, yd, pd = (sdfg.arrays[a] for a in (*(_in_array(state, conv, c) for c in ("X", "W_pw", "W_dw")), y, pooled))
+            pw, dw, _ = HipExpandDepthwiseConv._descs(conv, xd, w1, w2, yd)
+            if pd.dtype != torch.float32 or not pd.is_contiguous() or \
+                    not _lib.load().dmlhip_conv2d_expand_depthwise_pool_workspace_bytes(ctypes.byref(pw), ctypes.byref(dw)):
+                continue
+            _remove_node(state, pools[0])
+            conv.add_out_connector("Pooled")
+            state.add_edge(conv, "Pooled", state.add_write(pooled), None, sdfg.make_array_memlet(pooled))
+            count += 1
     return count
 
 
@@ -1314,6 +1341,8 @@ def auto_optimize(sdfg: SDFG, training: bool = False, attention: bool = True,
     stats["batchnorm_activation"] = fuse_batchnorm_activation(sdfg)
     stats["gated_conv"] = 0 if training else fuse_gate_into_conv(sdfg)
     stats["expand_depthwise"] = 0 if training else fuse_expand_depthwise(sdfg)
+    if stats["expand_depthwise"]:
+        fuse_pool_into_expand_depthwise(sdfg)
     stats["matmul_to_einsum"] = lower_matmul(sdfg)
     # views=False folds Transposes into the equations of the contractions next to them but keeps Reshape nodes: for
     # callers that hand the graph to a host with a view mechanism of its own (daceml_amd.dace_plugin.fuse_library_nodes)

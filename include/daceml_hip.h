@@ -364,6 +364,14 @@ int dmlhip_conv2d_gated_f32(const dmlhip_conv2d_desc* d, const void* x, const vo
 int dmlhip_conv2d_expand_depthwise_f32(const dmlhip_conv2d_desc* pw, const dmlhip_conv2d_desc* dw, const void* x,
                                        const void* w_pw, const void* b_pw, const void* w_dw, const void* b_dw,
                                        void* y, void* stream);
+/* The same, and pooled[n, m] = the mean of every image's channel of Y (GlobalAveragePool "pure",
+ * img_op_implementations.py:415-417), which a squeeze-excite gate is computed from. The workspace query gives the bytes
+ * with which the means come out of the kernel that computes Y; 0 = the problem's kernel does not sum, and it is, like any smaller
+ * workspace, the two calls one after the other. */
+size_t dmlhip_conv2d_expand_depthwise_pool_workspace_bytes(const dmlhip_conv2d_desc* pw, const dmlhip_conv2d_desc* dw);
+int dmlhip_conv2d_expand_depthwise_pool_f32(const dmlhip_conv2d_desc* pw, const dmlhip_conv2d_desc* dw, const void* x,
+                                            const void* w_pw, const void* b_pw, const void* w_dw, const void* b_dw,
+                                            void* y, void* pooled, void* workspace, size_t workspace_bytes, void* stream);
 /* LDS bytes the smallest row strip of dmlhip_conv2d_expand_depthwise_f32 needs for images `w` wide with `cin` input
  * channels and depthwise stride `stride`; 0 when no strip fits (the call would return DMLHIP_ERR_UNSUPPORTED). */
 size_t dmlhip_conv2d_expand_depthwise_lds_bytes(int64_t w, int64_t cin, int64_t stride);

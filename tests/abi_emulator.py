@@ -478,6 +478,13 @@ class Emulator:
                 mid = np.empty(pw.n * pw.m * pw.h * pw.w, dtype=np.float64)   # the expanded tensor is never rounded to memory
                 conv2d(pw, x, w_pw, b_pw, mid)
                 conv2d(dw, mid, w_dw, b_dw, y)
+            elif call.symbol == "dmlhip_conv2d_expand_depthwise_pool_f32":
+                pw, dw, x, w_pw, b_pw, w_dw, b_dw, y, pooled = args[:9]
+                mid = np.empty(pw.n * pw.m * pw.h * pw.w, dtype=np.float64)
+                conv2d(pw, x, w_pw, b_pw, mid)
+                conv2d(dw, mid, w_dw, b_dw, y)
+                out = ((dw.h - 1) // dw.stride_h + 1) * ((dw.w - 1) // dw.stride_w + 1)
+                pooled.reshape(-1)[:dw.n * dw.m] = y.reshape(-1)[:dw.n * dw.m * out].astype(np.float64).reshape(-1, out).mean(1)
             elif call.symbol in ("dmlhip_row_dot_f16", "dmlhip_row_dot_f32"):
                 a, b, y, rows, cols = args[:5]
                 av = a.reshape(-1)[:rows * cols].astype(np.float64).reshape(rows, cols)
