@@ -397,15 +397,17 @@ double estimate_small(int64_t m, int64_t n, int64_t k, long long batch, int pair
 }
 
 // Whether the workgroups that stay for several 256 x 256 tiles (gemm_f16_wide.h) beat the 128 x 128 tile, as times in us of
-// fixed + tiles per compute unit * (steps * step + what writing a tile takes); a residual is read while nothing is multiplied.
-// Over 120 products of encoder layers (1536 - 16384 tokens, 512 - 1024 wide, every operand layout, groups and operand pairs)
-// the faster of the two is missed by at most 4 % and by 0.1 % in the sum. Decided by it (us, 128-wide tiles or the 256 x 256
-// tile of gemm_f16_pipe.h / here): 4096 x 4096 x 1024 37.5 / 33.4, three of 4096 x 1024 x 1024 36.4 / 34.2, 16384 x 1024 x 4096
-// with residual 120 / 104, three pairs of 16384 x 1024 x 1024 113 / 83, 8192 x 1024 x 4096 77 / 88, 651 x 4096 x 1024 15 / 27.
-bool wide_is_faster(long long t256, long long t128, int64_t k, int pairs, bool residual) {
+// fixed + tiles per compute unit * (steps * step + what writing a tile takes). A residual is read while nothing is multiplied,
+// and the more compute units work the lower their clock. a_kc: A is K-contiguous, the 128 x 128 tile that of gemm_f16_wide.h.
+// Over 110 products (700 - 16384 tokens, 512 - 4096 wide, B in either layout, groups, operand pairs, residuals) the faster of
+// the two was missed once, by 1 %. Decided by it (us, 128 x 128 tiles / 256 x 256): 5041 x 2048 x 1024 30.3 / 28.4, three of
+// 4144 x 1024 x 1024 37.1 / 28.0, three of 5532 x 1024 x 4096 147 / 161, 4860 x 1024 x 4096 56.7 / 73, 8230 x 1024 x 3072 67 / 60.
+bool wide_is_faster(long long t256, long long t128, int64_t k, int pairs, bool residual, bool a_kc) {
     const double steps = (double)(k / BK) * pairs;
     const double t = (double)ceil_div(t256, (long long)kCus), s = (double)ceil_div(t128, (long long)kCus);
-    return 5.5 + t * (1.33 * steps + (residual ? 12.5 : 6.5)) < 4.0 + s * (0.55 * steps + (residual ? 3.5 : 2.0));
+    const double full = (double)t256 / (t * kCus);
+    return 9.0 + t * steps * (1.0 + 0.35 * full * full) + (t - 1) * 6.0 + (residual ? t * 6.0 : 0.0) <
+           4.0 + s * ((a_kc ? 0.43 : 0.55) * steps + (residual ? 3.5 : 2.0));
 }
 
 // Diagnostic switches (declared in the public header). Per calling thread, so that one thread pinning a configuration
@@ -532,8 +534,9 @@ static int run_gemm_f16(const dmlhip_gemm_desc* d, const void* a, const void* b,
         const bool extra = grp || asum;   // operand pairs / row sums: the 128 x 128 tile only
         const long long t256 = blocks(256, 256), t128 = blocks(128, 128);
         const long long slots256 = ceil_div(t256, (long long)kCus) * kCus, slots128 = ceil_div(t128, (long long)kCus) * kCus;
+        bool narrow = false;   // the estimate found the 128 x 64 tile to be the fastest
         const bool full256 = !extra && t256 * 10 >= slots256 * 9;
-        if (cfg < 0 && d->k >= 512 && wide && (full256 || wide_is_faster(t256, t128, d->k, g.ksum ? g.groups : 1, residual))) {
+        if (cfg < 0 && d->k >= 512 && wide && (full256 || wide_is_faster(t256, t128, d->k, g.ksum ? g.groups : 1, residual, amode == 0))) {
             cfg = 13;
         } else if (cfg < 0 && d->k >= 512 && full256) {
             // What the kernel above does not take (activations, beta, rows that are not stored in vectors, a ragged K). The
@@ -544,6 +547,7 @@ static int run_gemm_f16(const dmlhip_gemm_desc* d, const void* a, const void* b,
             // rows of C that are not written in vectors hide what the general kernel's longer loop costs: one round only
             const bool general = !pipe && !extra && (g.c_vec || t128 > kCus);
             estimate_small(d->m, d->n, d->k, batch, g.ksum ? g.groups : 1, g.out_f32, !extra, pipe, general, &cfg);
+            narrow = cfg == 9;
         }
         if (cfg < 0) {
             if (d->k < 512) {
@@ -554,8 +558,10 @@ static int run_gemm_f16(const dmlhip_gemm_desc* d, const void* a, const void* b,
             } else if (d->k <= 1024 && t128 >= 2 * kCus) {
                 // several rounds of short K loops (the grouped q / k / v projections: 768 tiles of 16 steps): with two
                 // LDS stages instead of four, two workgroups share a compute unit and one's epilogue and first loads
-                // overlap the other's loop - 45.3 against 46 - 49 us
-                cfg = 7;
+                // overlap the other's loop. Tiles that stay (gemm_f16_wide.h) are faster beyond one round of such pairs where K
+                // is not short or a pair would be left half empty: three of 5408 x 1024 x 1024 51 / 46 us, 12661 x 1536 x 768
+                // 42.4 / 38.3, but three of 4880 x 1024 x 512 25.7 / 26.5 and of 2633 x 1024 x 768 18.0 / 19.2
+                cfg = wide && amode == 0 && t128 > 2 * kCus && (steps >= 16 || ceil_div(t128, (long long)kCus) % 2) ? 14 : 7;
             } else if (!extra && d->k <= 1024 && t128 <= kCus && residual) {
                 // a short K loop whose epilogue also reads a residual tile (4096 x 1024 x 1024: 20.3 - 21.1 against
                 // 22.9 - 23.2 us): 128 x 64 tiles, two workgroups per compute unit, for the same overlap (without the
@@ -569,9 +575,15 @@ static int run_gemm_f16(const dmlhip_gemm_desc* d, const void* a, const void* b,
             }
         }
         const _Float16 *pa = (const _Float16*)a, *pb = (const _Float16*)b;
-        // The 128 x 128 tile of gemm_f16_wide.h in place of those of gemm_f16_pipe.h, from half a round of tiles and sixteen steps
-        // on (products of 144 - 192 tiles are level: 3072 x 768 x 3072 24.5 / 24.6, B row-contiguous 24.3 / 23.7).
-        if (g_force_cfg < 0 && (cfg == 5 || cfg == 9) && wide && amode == 0 && steps >= 16 && t128 * 2 >= kCus) cfg = 14;
+        // The 128 x 128 tile of gemm_f16_wide.h in place of those of gemm_f16_pipe.h, from sixteen steps on; not for the products
+        // that the estimate gives to 128 x 64 tiles, which are two per compute unit (960 x 2048 x 1024 9.4 us there, 11.0 here).
+        // It starts with more steps on their way and reads a residual ahead: without one, and with no other product in the
+        // launch, less than a round of tiles needs thirty-two steps and seven eighths of it (1371 x 2048 x 1024 11.3 / 11.6, B
+        // row-contiguous 2844 x 768 x 3072 22.4 / 23.6, but 4764 x 768 x 3072 26.5 / 25.6; with a residual 1280 x 2048 x 1024
+        // 13.5 / 12.7, 2432 x 1024 x 4096 30.4 / 29.3).
+        if (g_force_cfg < 0 && (cfg == 5 || (cfg == 9 && !narrow)) && wide && amode == 0 && steps >= 16 && t128 * 2 >= kCus &&
+            (residual || extra || t128 > kCus || (steps >= 32 && t128 * 8 >= kCus * 7)))
+            cfg = 14;
         g_last_cfg = cfg;
         if (cfg == 13 && wide && steps >= 3) return launch_wide256(g, pa, pb, c, bias, residual, amode, bmode, batch, st);
         if (cfg == 14 && wide && steps >= 5 && amode == 0) return launch_wide128(g, pa, pb, c, bias, residual, amode, bmode, batch, st);

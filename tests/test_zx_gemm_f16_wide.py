@@ -135,11 +135,17 @@ def test_which_weight_gradients_are_sliced(m, n, k, groups, sliced, lib):
     assert (lib.dmlhip_gemm_f16_grouped_asum_workspace_bytes(ctypes.byref(d)) >= 2 * groups * m * n * 4) == sliced
 
 
-@pytest.mark.parametrize("m,n,k,cfg", [(4096, 1024, 4096, 14), (2048, 1024, 1024, 14), (4096, 4096, 1024, 13), (4096, 1024, 960, 5)])
-def test_which_products_they_take(m, n, k, cfg, lib):
+@pytest.mark.parametrize("m,n,k,residual,cfg", [
+    (4096, 1024, 4096, False, 14), (4096, 4096, 1024, False, 13), (4096, 1024, 960, False, 5),
+    (2048, 1024, 1024, False, 9), (2048, 1024, 1024, True, 9),                    # 128 x 64 tiles, two per compute unit
+    (2560, 1024, 1024, False, 5), (2560, 1024, 1024, True, 14),                   # less than a round, a short loop
+    (2816, 1024, 4096, False, 5), (3712, 1024, 4096, False, 14),                  # ... a long one: from seven eighths of it on
+    (4352, 1024, 1024, True, 9), (4352, 1024, 4096, False, 14),                   # a little more than a round
+    (8192, 1024, 768, False, 7), (12672, 1536, 768, False, 14)])                  # short loops, two rounds and five
+def test_which_products_they_take(m, n, k, residual, cfg, lib):
     from daceml_amd import _lib as L, kernels as K
     a, b = torch.zeros((m, k), device="cuda", dtype=torch.float16), torch.zeros((n, k), device="cuda", dtype=torch.float16)
-    c = torch.empty((m, n), device="cuda", dtype=torch.float16)
+    c, r = torch.empty((m, n), device="cuda", dtype=torch.float16), torch.zeros((m, n), device="cuda", dtype=torch.float16)
     d = _desc(L, m, n, k, (k, 1), (k, 1), L.F16)
-    L.check(lib.dmlhip_gemm_f16(ctypes.byref(d), P(a), P(b), P(c), None, None, None, K._stream()))
+    L.check(lib.dmlhip_gemm_f16(ctypes.byref(d), P(a), P(b), P(c), None, P(r) if residual else None, None, K._stream()))
     assert lib.dmlhip_debug_last_gemm_config() == cfg
