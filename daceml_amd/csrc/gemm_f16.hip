@@ -748,7 +748,9 @@ int dmlhip_gemm_f16_grouped(const dmlhip_gemm_desc* d, int groups, const void* c
 // 128 x 128 tiles' 4 + rounds * (2 + steps * (0.42 + 0.14 where all compute units have one)). Fitted to 96 weight gradients with
 // row sums (1024 - 16384 tokens, 512 - 1024 wide, one product or three or four). us on those / here: 4096 x 1024 over 4096 /
 // 8192 / 16384 tokens 42 / 51, 79 / 75, 153 / 122; 512 x 2048 over 4096 / 16384 34 / 31, 122 / 54; three of 1024 x 1024 over 16384
-// 143 / 100.
+// 143 / 100. Results in fp16 may also be on the tiles with K split over the wavefronts: 1.2 of what estimate_small says of those
+// (1.13 - 1.9 measured over 2000 - 16384 tokens); 512 x 512 over 4160 15.4 / 28.8, 512 x 2048 over 4664 20.8 / 36.3, three of 512 x 512
+// over 3840 18.0 / 29.7, but 512 x 512 over 14935 45.6 / 32.1, 2048 x 512 over 14283 84.9 / 49.6.
 static int weight_gradient_slices(const dmlhip_gemm_desc* d, int groups) {
     if (d->m <= 0 || d->n <= 0 || d->k <= 0 || d->m % 8 || d->n % 8 || d->c_stride_m != d->n || !g_direct_lds) return 0;
     if (d->m > 65536 || d->n > 65536 || (g_force_cfg >= 0 && g_force_cfg != 13)) return 0;
@@ -761,6 +763,11 @@ static int weight_gradient_slices(const dmlhip_gemm_desc* d, int groups) {
     if (g_force_cfg == 13) return (int)most;
     const double mb = 4e-6 * groups * (double)d->m * (double)d->n;
     double best = 0.93 * (4.0 + (double)ceil_div(t128, (long long)kCus) * (2.0 + steps * (0.42 + 0.14 * fmin(1.0, t128 / (double)kCus))));
+    if (d->out_dtype == DMLHIP_F16 && t128 < 2 * kCus && t128 * 10 < ceil_div(t128, (long long)kCus) * kCus * 9) {
+        int cfg = -1;
+        const double us = 1.2 * estimate_small(d->m, d->n, d->k, groups, 1, false, false, true, false, &cfg);
+        if (cfg >= 10 && us < best) best = us;
+    }
     int slices = 0;
     for (int s = 2; s <= most; ++s) {
         const double us = 9.5 + 1.4 * (double)ceil_div(steps, (long long)s) + 0.3 * mb * s;

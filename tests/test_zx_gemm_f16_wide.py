@@ -135,6 +135,22 @@ def test_which_weight_gradients_are_sliced(m, n, k, groups, sliced, lib):
     assert (lib.dmlhip_gemm_f16_grouped_asum_workspace_bytes(ctypes.byref(d)) >= 2 * groups * m * n * 4) == sliced
 
 
+@pytest.mark.parametrize("m,n,k,groups,sliced", [(512, 512, 4160, 1, False), (512, 2048, 4664, 1, False), (512, 512, 3840, 3, False),
+                                                 (512, 512, 14935, 1, True), (2048, 512, 14283, 1, True), (1024, 4096, 16384, 1, True)])
+def test_which_weight_gradients_in_fp16_are_sliced(m, n, k, groups, sliced, lib):
+    """Not those that tiles with K split over the wavefronts do faster."""
+    from daceml_amd import _lib as L, kernels as K
+    d = _desc(L, m, n, k, (1, m), (1, n), L.F16)
+    a, b = (torch.zeros((k, e), device="cuda", dtype=torch.float16) for e in (m, n))
+    c = [torch.empty((m, n), device="cuda", dtype=torch.float16) for _ in range(groups)]
+    s = [torch.empty(m, device="cuda") for _ in range(groups)]
+    need = lib.dmlhip_gemm_f16_grouped_asum_workspace_bytes(ctypes.byref(d))
+    ws = torch.empty(max(need, 16), device="cuda", dtype=torch.uint8)
+    L.check(lib.dmlhip_gemm_f16_grouped_asum(ctypes.byref(d), groups, _table([a] * groups), _table([b] * groups), _table(c), _table(s),
+                                             L.F32, P(ws), need, K._stream()))
+    assert (lib.dmlhip_debug_last_gemm_config() == 13) == sliced
+
+
 @pytest.mark.parametrize("m,n,k,residual,cfg", [
     (4096, 1024, 4096, False, 14), (4096, 4096, 1024, False, 13), (4096, 1024, 960, False, 5),
     (2048, 1024, 1024, False, 9), (2048, 1024, 1024, True, 9),                    # 128 x 64 tiles, two per compute unit
