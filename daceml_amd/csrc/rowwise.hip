@@ -229,10 +229,14 @@ __global__ __launch_bounds__(kRowBlock) void log_softmax_bwd_kernel(const T* __r
         s += d[j];
     }
     s = wave_reduce<OpSum>(s);
+    // the product is rounded before it is subtracted, as where it is a launch of its own: what is left of two close terms decides
+    // gradients that cancel further on (two classes behind a LayerNorm)
 #pragma unroll
     for (int j = 0; j < N; ++j) {
+#pragma clang fp contract(off)
         const int c = lane + j * kWave;
-        if (c < cols) dx[off + c] = from_f32<T>(d[j] - expf(v[j]) * s);
+        const float p = expf(v[j]) * s;
+        if (c < cols) dx[off + c] = from_f32<T>(d[j] - p);
     }
 }
 

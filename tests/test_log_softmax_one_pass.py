@@ -111,3 +111,16 @@ def test_values_without_a_logarithm(dtype):
         # the six calls round x - max and the logarithm in the tensors' type
         tol = 2.0 ** -9 if dtype == torch.float16 else 2.0 ** -20
         assert (np.abs(a[finite] - b[finite]) <= tol * (1 + 34 * (a is out[0][1]) + np.abs(b[finite]))).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cols", [2, 10, 100, 1000])
+def test_reverse_rounds_the_product(cols, lib):
+    """dy - exp(y) * sum(dy) with each operation rounded, as by the separate launches: the same bits where the sum is exact."""
+    from daceml_amd import _lib as L, kernels as K
+    g = torch.Generator().manual_seed(cols)
+    y = torch.log_softmax(torch.randn((257, cols), generator=g), 1).cuda()
+    dy = torch.zeros((257, cols)).scatter_(1, torch.randint(0, cols, (257, 1), generator=g), torch.randn((257, 1), generator=g)).cuda()
+    dx = torch.empty_like(y)
+    L.check(lib.dmlhip_log_softmax_backward_f32(y.data_ptr(), dy.data_ptr(), dx.data_ptr(), 257, cols, K._stream()))
+    assert torch.equal(dx, dy - K.unary(L.EXP, y) * dy.sum(1, keepdim=True))
