@@ -441,16 +441,13 @@ struct GemmGroup {
     bool ksum;                 // concatenate the groups along K into one output instead of running them side by side
 };
 
-// grp != nullptr: a / b / c / bias are those of group 0 (used for the layout checks, which the caller has made sure
-// hold for every group); returns DMLHIP_ERR_UNSUPPORTED when the grouped launch is not possible.
-static int run_gemm_f16(const dmlhip_gemm_desc* d, const void* a, const void* b, void* c, const void* bias,
-                        const void* residual, void* pre_out, void* stream, const GemmGroup* grp = nullptr,
-                        void* const* asum = nullptr, int asum_f32 = 0) {
+// What is refused of a product whichever kernel would run it; the number of its batch entries in `batch`.
+static int check_gemm_f16(const dmlhip_gemm_desc* d, long long& batch) {
     DML_REQUIRE(d, DMLHIP_ERR_NULL, "gemm_f16: NULL descriptor");
     DML_REQUIRE(d->m >= 0 && d->n >= 0 && d->k >= 0, DMLHIP_ERR_SHAPE, "gemm_f16: negative extent");
     DML_REQUIRE(d->m <= 2147483647 / 2 && d->n <= 2147483647 / 2 && d->k <= 2147483647 / 2, DMLHIP_ERR_SHAPE,
                 "gemm_f16: extent exceeds 2^30");
-    long long batch = 1;
+    batch = 1;
     for (int i = 0; i < 3; ++i) {
         DML_REQUIRE(d->batch[i] >= 0 && d->batch[i] <= 2147483647, DMLHIP_ERR_SHAPE, "gemm_f16: bad batch extent");
         batch *= d->batch[i];
@@ -465,6 +462,16 @@ static int run_gemm_f16(const dmlhip_gemm_desc* d, const void* a, const void* b,
                 DMLHIP_ERR_SHAPE, "gemm_f16: negative stride");
     DML_REQUIRE(d->c_stride_m >= d->n || d->m <= 1, DMLHIP_ERR_SHAPE, "gemm_f16: rows of C overlap (stride %lld < n)",
                 (long long)d->c_stride_m);
+    return 0;
+}
+
+// grp != nullptr: a / b / c / bias are those of group 0 (used for the layout checks, which the caller has made sure
+// hold for every group); returns DMLHIP_ERR_UNSUPPORTED when the grouped launch is not possible.
+static int run_gemm_f16(const dmlhip_gemm_desc* d, const void* a, const void* b, void* c, const void* bias,
+                        const void* residual, void* pre_out, void* stream, const GemmGroup* grp = nullptr,
+                        void* const* asum = nullptr, int asum_f32 = 0) {
+    long long batch;
+    if (int e = check_gemm_f16(d, batch)) return e;
     if (d->m == 0 || d->n == 0 || batch == 0) return 0;
     DML_REQUIRE(c, DMLHIP_ERR_NULL, "gemm_f16: NULL output");
     DML_REQUIRE(d->k == 0 || (a && b), DMLHIP_ERR_NULL, "gemm_f16: NULL operand");
@@ -810,6 +817,8 @@ int dmlhip_gemm_f16_grouped_asum(const dmlhip_gemm_desc* d, int groups, const vo
     for (int i = 0; i < groups; ++i)
         DML_REQUIRE(c[i] && asum[i] && (d->k == 0 || (a[i] && b[i])), DMLHIP_ERR_NULL,
                     "gemm_f16_grouped_asum: NULL tensor in group %d", i);
+    long long batch;
+    if (int e = check_gemm_f16(d, batch)) return e;   // the products in slices below do not go through run_gemm_f16
     bool same = d->k > 0;
     for (int i = 0; i < groups && same; ++i)
         same = aligned16(a[i]) && aligned16(b[i]) && reinterpret_cast<uintptr_t>(c[i]) % 32 == 0;

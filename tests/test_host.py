@@ -668,3 +668,29 @@ def test_expand_depthwise_fusion_asks_the_library_whether_a_strip_fits(lib):
         return fusion.auto_optimize(sdfg)["expand_depthwise"]
     assert fused(1024) == 1      # 13 KB of rows + 131 KB of weights: fits
     assert fused(1200) == 0      # 154 KB of weights alone: the launch would be refused
+
+
+@pytest.mark.parametrize("tokens", [256, 16384])
+def test_argument_errors_of_weight_gradients_do_not_depend_on_their_length(tokens, lib):
+    """Products whose K steps several workgroups share are refused what every other product is, before any launch."""
+    from daceml_amd import _lib as L
+    table = (ctypes.c_void_p * 1)(64)
+
+    def status(**bad):
+        d = L.GemmDesc()
+        d.m, d.n, d.k = 512, 512, tokens
+        d.batch[0] = d.batch[1] = d.batch[2] = 1
+        d.a_stride_m, d.a_stride_k, d.b_stride_k, d.b_stride_n, d.c_stride_m = 1, 512, 512, 1, 512
+        d.alpha, d.out_dtype = 1.0, L.F32
+        need = lib.dmlhip_gemm_f16_grouped_asum_workspace_bytes(ctypes.byref(d))
+        assert (need >= 2 * 512 * 512 * 4) == (tokens == 16384)
+        for name, value in bad.items():
+            setattr(d, name, value)
+        return lib.dmlhip_gemm_f16_grouped_asum(ctypes.byref(d), 1, table, table, table, table, L.F32, 64, max(need, 1 << 24), None)
+
+    assert status(out_dtype=7) == L.ERR_ENUM and "out_dtype" in L.last_error()
+    assert status(bias_dtype=9) == L.ERR_ENUM and "bias_dtype" in L.last_error()
+    assert status(b_stride_n=-tokens, b_stride_k=1) == L.ERR_SHAPE
+    assert status(b_stride_n=1, b_stride_k=-512) == L.ERR_SHAPE
+    assert status(c_stride_m=511) == L.ERR_SHAPE
+    assert status(m=-512) == L.ERR_UNSUPPORTED and status(n=-8) == L.ERR_SHAPE and status(k=-1) == L.ERR_SHAPE
