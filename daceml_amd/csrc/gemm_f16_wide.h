@@ -33,8 +33,9 @@
 //    sums of A (the bias gradient) are taken from the fragments: the workgroups of tile column c add those of every step that
 //    leaves c modulo the number of columns, so that none of them falls behind the others. Any K: the step with its last k is
 //    sent by a copy of the step of its own, with zeros behind them.
-// Requirements (checked by the host): K % 64 == 0 (but for SLICED) and at least three steps, no activation, beta == 0, n % 8 == 0, 16-byte aligned operands, column
-// bias and result rows, 32-bit element offsets, rows % 8 == 0 for RC operands.
+// Requirements (checked by the host): K % 64 == 0 (but for SLICED), more steps than are ahead (three of the large tile, five of the
+// small one, those of all operand pairs together), no activation, beta == 0, n % 8 == 0, 16-byte aligned operands, column bias and
+// result rows, 32-bit element offsets, rows % 8 == 0 for RC operands.
 #pragma once
 
 #include "gemm_f16_common.h"
@@ -358,6 +359,7 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_wide_kernel(const _Float16*
     // ---- what the transfers read: two steps ahead of the MFMAs, past the end of a tile the first steps of the next one
     __amdgpu_buffer_rsrc_t ra, rb;
     const _Float16 *tile_a = nullptr, *tile_b = nullptr;   // where they begin, for the ragged step
+    uint32_t fbid = bid;   // the tile they belong to, which is ahead of the one that is multiplied
     int fk = 0, fend = nkg, fgrp = 0, rows_a = 0, rows_b = 0;
     auto point_at = [&](uint32_t at) {
         const WideTile ft = wide_tile<T>(g, at);
@@ -394,7 +396,7 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_wide_kernel(const _Float16*
             ob.offsets(g.sbn, g.sbk, rows_b, wave, lane);
         }
     };
-    point_at(bid);
+    point_at(fbid);
     auto send_a = [&](auto ic, int stage) {
         constexpr int i = decltype(ic)::value;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
@@ -411,11 +413,12 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_wide_kernel(const _Float16*
     auto advance = [&]() {
         if (++fk != fend) return;
         if (KSUM && ++fgrp != g.groups) {
-            point_at(bid);
+            point_at(fbid);   // a pair of few steps ends while the tile before is still being multiplied
             return;
         }
         fgrp = 0;
-        if (bid + gridDim.x < total) point_at(bid + gridDim.x);
+        fbid += gridDim.x;
+        if (fbid < total) point_at(fbid);
     };
 
     for (int s = 0; s < AHEAD; ++s) {
