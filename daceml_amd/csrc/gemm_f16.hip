@@ -751,13 +751,17 @@ int dmlhip_gemm_f16_grouped(const dmlhip_gemm_desc* d, int groups, const void* c
 }
 
 // Number of workgroups that share the K steps of a weight gradient's 256 x 256 tile (gemm_f16_wide.h); 0 = other kernels.
-// The fewest us of: both launches 9.5, a step 1.4, 0.3 per MB of partial results (written, read and summed) - against the
-// 128 x 128 tiles' 4 + rounds * (2 + steps * (0.42 + 0.14 where all compute units have one)). Fitted to 96 weight gradients with
-// row sums (1024 - 16384 tokens, 512 - 1024 wide, one product or three or four). us on those / here: 4096 x 1024 over 4096 /
-// 8192 / 16384 tokens 42 / 51, 79 / 75, 153 / 122; 512 x 2048 over 4096 / 16384 34 / 31, 122 / 54; three of 1024 x 1024 over 16384
-// 143 / 100. Results in fp16 may also be on the tiles with K split over the wavefronts: 1.2 of what estimate_small says of those
-// (1.13 - 1.9 measured over 2000 - 16384 tokens); 512 x 512 over 4160 15.4 / 28.8, 512 x 2048 over 4664 20.8 / 36.3, three of 512 x 512
-// over 3840 18.0 / 29.7, but 512 x 512 over 14935 45.6 / 32.1, 2048 x 512 over 14283 84.9 / 49.6.
+// How many: the fewest us of 9.5 + 1.4 per step + 0.3 per MB of partial results (written, read and summed). Whether at all: both
+// launches take 20.2 us, 0.78 per step and 0.70 more where all compute units have a tile, 0.109 per MB (3.9 % off in the mean over
+// 466 gradients of 256 - 4096 x 256 - 4096 over 1800 - 18500 tokens, one to four products, both result types) - against 0.94 (a second
+// round of less than 0.6: 0.86) of the 128 x 128 tiles' 4 + rounds * (2 + steps * (0.42 + 0.14 where all compute units have one)).
+// us on those / here: 4096 x 1024 over 4096 / 8192 / 16384 tokens 42 / 51, 79 / 75, 153 / 122; 512 x 2048 over 4096 / 16384 34 / 31,
+// 122 / 54; three of 1024 x 1024 over 16384 143 / 100; 896 x 896 over 3515 30.1 / 32.8, 256 x 640 over 1792 17.6 / 22.6.
+// Results in fp16 may also be on the tiles with K split over the wavefronts, whose estimate long products exceed: 32 x 32 tiles by 1.3 - 2,
+// 64 x 64 tiles by 1 - 1.2, and by 1.2 - 1.8 where the rows of A are more than those of the result are long and a multiple of 1 KB apart.
+// us there / here: 768 x 768 over 8128 tokens 31.4 / 34.2, over 10240 37.7 / 35.9; 384 x 1536 over 7872 26.6 / 36.1, 640 x 512 over 5540
+// 22.4 / 29.0; 512 x 2048 over 4664 20.8 / 36.3, 2048 x 512 over 14283 84.9 / 49.6; 512 x 512 over 4160 15.4 / 28.8, over 14935 45.6 / 32.1.
+// Of 683 gradients, most of them near the line, 553 go here; three of those are 1 - 3 % slower than there.
 static int weight_gradient_slices(const dmlhip_gemm_desc* d, int groups) {
     if (d->m <= 0 || d->n <= 0 || d->k <= 0 || d->m % 8 || d->n % 8 || d->c_stride_m != d->n || !g_direct_lds) return 0;
     if (d->m > 65536 || d->n > 65536 || (g_force_cfg >= 0 && g_force_cfg != 13)) return 0;
@@ -769,21 +773,34 @@ static int weight_gradient_slices(const dmlhip_gemm_desc* d, int groups) {
     if (most < 2) return 0;
     if (g_force_cfg == 13) return (int)most;
     const double mb = 4e-6 * groups * (double)d->m * (double)d->n;
-    double best = 0.93 * (4.0 + (double)ceil_div(t128, (long long)kCus) * (2.0 + steps * (0.42 + 0.14 * fmin(1.0, t128 / (double)kCus))));
-    if (d->out_dtype == DMLHIP_F16 && t128 < 2 * kCus && t128 * 10 < ceil_div(t128, (long long)kCus) * kCus * 9) {
-        int cfg = -1;
-        const double us = 1.2 * estimate_small(d->m, d->n, d->k, groups, 1, false, false, true, false, &cfg);
-        if (cfg >= 10 && us < best) best = us;
-    }
     int slices = 0;
+    double least_us = 1e30;
     for (int s = 2; s <= most; ++s) {
         const double us = 9.5 + 1.4 * (double)ceil_div(steps, (long long)s) + 0.3 * mb * s;
-        if (us < best) {
-            best = us;
+        if (us < least_us) {
+            least_us = us;
             slices = s;
         }
     }
-    return slices;
+    const long long rounds = ceil_div(t128, (long long)kCus);
+    const double tiles = 4.0 + (double)rounds * (2.0 + steps * (0.42 + 0.14 * fmin(1.0, t128 / (double)kCus)));
+    double split = 1e30, behind = 1.0;
+    if (d->out_dtype == DMLHIP_F16 && t128 < 2 * kCus && t128 * 10 < rounds * kCus * 9) {
+        int cfg = -1;
+        const double est = estimate_small(d->m, d->n, d->k, groups, 1, false, false, true, false, &cfg);
+        const bool far = d->m % 512 == 0 && d->m > 512 && d->m > d->n;
+        const bool many = ceil_div(d->m, (int64_t)64) * ceil_div(d->n, (int64_t)64) * groups >= 192;
+        if (cfg >= 10) {
+            split = est;
+            behind = cfg == 12 ? 1.3 : !far ? 1.05 : many ? 1.3 : 1.18;
+        }
+    }
+    const double full = (double)t256 * slices / kCus;
+    const double us = 20.2 + (double)ceil_div(steps, (long long)slices) * (0.78 + 0.70 * full) + 0.109 * mb * slices;
+    // the figures that the number of slices was chosen by have to say so too: those of many MB are the surer ones
+    const bool faster = us < tiles * (rounds > 1 && t128 * 5 < rounds * kCus * 4 ? 0.86 : 0.94) && us < split * behind &&
+                        least_us < tiles * 0.93 && least_us < split * 1.2;
+    return faster ? slices : 0;
 }
 
 size_t dmlhip_gemm_f16_grouped_asum_workspace_bytes(const dmlhip_gemm_desc* d) {

@@ -151,6 +151,23 @@ def test_which_weight_gradients_in_fp16_are_sliced(m, n, k, groups, sliced, lib)
     assert (lib.dmlhip_debug_last_gemm_config() == 13) == sliced
 
 
+@pytest.mark.parametrize("out", ["f16", "f32"])
+@pytest.mark.parametrize("m,n,k,groups,f16,f32", [(768, 768, 8128, 1, False, True), (640, 512, 5540, 1, False, True), (384, 1536, 7872, 1, False, True),
+                                                  (256, 896, 7231, 2, False, True), (896, 896, 3515, 1, False, False), (256, 640, 1792, 1, False, False),
+                                                  (768, 768, 12288, 1, True, True), (1024, 896, 6208, 1, False, True), (2048, 768, 8132, 4, True, True)])
+def test_gradients_that_other_tiles_do_faster_are_not_sliced(m, n, k, groups, f16, f32, out, lib):
+    from daceml_amd import _lib as L, kernels as K
+    dtype = torch.float16 if out == "f16" else torch.float32
+    d = _desc(L, m, n, k, (1, m), (1, n), L.F16 if out == "f16" else L.F32)
+    a, b = (torch.zeros((k, e), device="cuda", dtype=torch.float16) for e in (m, n))
+    c, s = ([torch.empty(shape, device="cuda", dtype=dtype) for _ in range(groups)] for shape in ((m, n), (m, )))
+    need = lib.dmlhip_gemm_f16_grouped_asum_workspace_bytes(ctypes.byref(d))
+    ws = torch.empty(max(need, 16), device="cuda", dtype=torch.uint8)
+    L.check(lib.dmlhip_gemm_f16_grouped_asum(ctypes.byref(d), groups, _table([a] * groups), _table([b] * groups), _table(c), _table(s),
+                                             d.out_dtype, P(ws), need, K._stream()))
+    assert (lib.dmlhip_debug_last_gemm_config() == 13) == (f16 if out == "f16" else f32)
+
+
 @pytest.mark.parametrize("m,n,k,residual,cfg", [
     (4096, 1024, 4096, False, 14), (4096, 4096, 1024, False, 13), (4096, 1024, 960, False, 5),
     (2048, 1024, 1024, False, 9), (2048, 1024, 1024, True, 9),                    # 128 x 64 tiles, two per compute unit
