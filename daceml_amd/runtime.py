@@ -218,45 +218,76 @@ class CompiledSDFG:
             symbol = self.lib.dmlhip_call_symbol(call.symbol.encode())
             if symbol < 0:
                 raise RuntimeError("%s cannot be part of a call list" % call.symbol)
+            types = getattr(self.lib, call.symbol).argtypes
+            if len(call.args) != len(types):
+                raise TypeError("%s takes %d arguments, got %d" % (call.symbol, len(types), len(call.args)))
             args = (L.CallArg * len(call.args))()
-            for word, a in zip(args, call.args):
-                if isinstance(a, T.Ptr):
-                    word.kind = L.CALL_POINTER
-                    word.index, word.value = self._address(conn_to_array[a.conn], a.offset)
-                elif isinstance(a, T.Null):
-                    pass                      # a value: NULL
-                elif isinstance(a, (T.I64, T.I32, T.USize)):
-                    word.value = a.value & 0xffffffffffffffff
-                elif isinstance(a, T.F32):
-                    word.value = ctypes.c_uint32.from_buffer(ctypes.c_float(a.value)).value
-                elif isinstance(a, T.I64Array):
-                    arr = (ctypes.c_int64 * max(len(a.values), 1))(*a.values)
-                    self._keep.append(arr)
-                    word.value = ctypes.addressof(arr)
-                elif isinstance(a, T.PtrArray):
-                    if len(a.conns) > L.CALL_TABLE_MAX:
-                        raise RuntimeError("%s: a table of %d pointers" % (call.symbol, len(a.conns)))
-                    entries = (L.CallArg * max(len(a.conns), 1))()
-                    for e, c in zip(entries, a.conns):
-                        e.index, e.value = self._address(conn_to_array[c], 0)
-                    self._keep.append(entries)
-                    word.kind, word.index, word.value = L.CALL_TABLE, len(a.conns), ctypes.addressof(entries)
-                elif isinstance(a, T.Struct):
-                    self._keep.append(a.value)
-                    word.value = ctypes.addressof(a.value)
-                elif isinstance(a, T.Workspace):
-                    word.value = self._workspace.data_ptr() + a.offset
-                elif isinstance(a, T.WorkspaceBytes):
-                    word.value = self._ws_bytes - a.offset
-                elif isinstance(a, T.Stream):
-                    word.kind = L.CALL_STREAM
-                else:
-                    raise TypeError("unknown HIP call argument %r" % (a, ))
+            for i, (word, a, type_) in enumerate(zip(args, call.args, types)):
+                try:
+                    self._bind_argument(word, a, type_, conn_to_array)
+                except TypeError as e:
+                    raise TypeError("argument %d of %s, %r: %s" % (i, call.symbol, a, e)) from None
             # work is attributed to the node's first call only (later calls are follow-up passes)
             first = call is calls[0]
             flops = call.flops if call.flops is not None else (node.flops if first else 0)
             moved = call.bytes_moved if call.bytes_moved is not None else (node.bytes_moved if first else 0)
             self._launches.append(_Launch(symbol, args, node.label, call.symbol, flops, moved, node.kind, state.label))
+
+    def _bind_argument(self, word: L.CallArg, a, type_, conn_to_array: Dict[str, str]):
+        """Fills in the word of a call list that stands for `a`. The native list takes words as they are: that `a` is what
+        the entry point's parameter takes is decided here, by what ctypes accepts for it."""
+        if isinstance(a, T.Ptr):
+            word.index, word.value = self._address(conn_to_array[a.conn], a.offset)
+            if type_ is ctypes.POINTER(ctypes.c_void_p):   # a table of the one address
+                entry = L.CallArg(L.CALL_POINTER, word.index, word.value)
+                self._keep.append(entry)
+                word.kind, word.index, word.value = L.CALL_TABLE, 1, ctypes.addressof(entry)
+            else:
+                self._takes_address(type_)
+                word.kind = L.CALL_POINTER
+        elif isinstance(a, T.Null):
+            type_.from_param(None)
+        elif isinstance(a, (T.I64, T.I32, T.USize)):
+            type_.from_param({T.I64: ctypes.c_int64, T.I32: ctypes.c_int, T.USize: ctypes.c_size_t}[type(a)](a.value))
+            word.value = a.value & 0xffffffffffffffff
+        elif isinstance(a, T.F32):
+            value = ctypes.c_float(a.value)
+            type_.from_param(value)
+            word.value = ctypes.c_uint32.from_buffer(value).value
+        elif isinstance(a, T.I64Array):
+            arr = (ctypes.c_int64 * max(len(a.values), 1))(*a.values)
+            type_.from_param(arr)
+            self._keep.append(arr)
+            word.value = ctypes.addressof(arr)
+        elif isinstance(a, T.PtrArray):
+            type_.from_param((ctypes.c_void_p * len(a.conns))())
+            if len(a.conns) > L.CALL_TABLE_MAX:
+                raise RuntimeError("a table of %d pointers" % len(a.conns))
+            entries = (L.CallArg * max(len(a.conns), 1))()
+            for e, c in zip(entries, a.conns):
+                e.index, e.value = self._address(conn_to_array[c], 0)
+            self._keep.append(entries)
+            word.kind, word.index, word.value = L.CALL_TABLE, len(a.conns), ctypes.addressof(entries)
+        elif isinstance(a, T.Struct):
+            type_.from_param(ctypes.byref(a.value))
+            self._keep.append(a.value)
+            word.value = ctypes.addressof(a.value)
+        elif isinstance(a, T.Workspace):
+            self._takes_address(type_)
+            word.value = self._workspace.data_ptr() + a.offset
+        elif isinstance(a, T.WorkspaceBytes):
+            type_.from_param(ctypes.c_size_t())
+            word.value = self._ws_bytes - a.offset
+        elif isinstance(a, T.Stream):
+            self._takes_address(type_)
+            word.kind = L.CALL_STREAM
+        else:
+            raise TypeError("unknown HIP call argument")
+
+    @staticmethod
+    def _takes_address(type_):
+        if type_ is not ctypes.c_void_p:
+            raise TypeError("expected %s" % type_.__name__)
 
     # -- execution -----------------------------------------------------------
     def _bind_arguments(self, kwargs: Dict[str, torch.Tensor], partial: bool = False):
