@@ -13,7 +13,7 @@ state is one native call per state and no Python-side planning.
 """
 import ctypes
 import logging
-from typing import Dict, List, Optional, Sequence, Tuple
+from typing import Dict, List, Optional, Sequence, Tuple, Union
 
 import torch
 
@@ -128,7 +128,7 @@ class CompiledSDFG:
         #: addresses of the arrays that are no views; array -> (number there, byte offset)
         self.pointers = (ctypes.c_uint64 * max(len(sdfg.arrays), 1))()
         self._place: Dict[str, Tuple[int, int]] = {}
-        self._native: Dict[Optional[tuple], tuple] = {}   # states -> call list
+        self._native: Dict[Union[None, str, tuple], tuple] = {}   # states -> call list
         self._binding = 0                     # bumped whenever a pointer may have changed
         self.buffers: Dict[str, torch.Tensor] = {}
         # [(state, node)]: the order the kernels are enqueued in
@@ -362,7 +362,7 @@ class CompiledSDFG:
     def launch(self, states: Optional[Sequence[str]] = None):
         """Enqueue every kernel (of the named states) on the current stream, with the pointers of the
         last binding."""
-        key = None if states is None else tuple(states)
+        key = states if states is None or isinstance(states, str) else tuple(states)
         native = self._native.get(key)
         if native is None:
             native = self._native[key] = self._selected(key)
@@ -373,7 +373,7 @@ class CompiledSDFG:
             l = launches[failed.value]
             raise L.HipKernelError(status, "%s (%s): %s" % (l.label, l.symbol, L.last_error()))
 
-    def _selected(self, states: Optional[tuple]):
+    def _selected(self, states: Union[None, str, tuple]):
         """(launches, their call list, how many) of the named states."""
         numbers = [i for i, l in enumerate(self._launches) if states is None or l.state in states]
         if numbers == list(range(numbers[0], numbers[-1] + 1)) if numbers else True:   # one run of the program's own list

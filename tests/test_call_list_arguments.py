@@ -63,3 +63,18 @@ def test_descriptors_and_tables(lib):
     entry = L.CallArg.from_address(args[0].value)
     assert (entry.index, entry.value) == (0, 4)
     assert L.SIGNATURES["dmlhip_sum_f16"][1][0] is ctypes.POINTER(ctypes.c_void_p)
+
+
+def test_states_by_name(monkeypatch, lib):
+    """One state's label selects its launches as well as a sequence of labels does."""
+    from types import SimpleNamespace
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device: SimpleNamespace(cuda_stream=0))
+    prog = object.__new__(CompiledSDFG)
+    prog._native, prog.pointers, prog.device = {}, (ctypes.c_uint64 * 1)(), None
+    prog._launches = [SimpleNamespace(state=s) for s in ("forward", "backward", "forward")]
+    prog._calls = (L.Call * 3)()
+    ran = []
+    prog.lib = SimpleNamespace(dmlhip_run_calls=lambda calls, count, *rest: ran.append(count) or 0)
+    for states, count in ((None, 3), (["forward"], 2), ("forward", 2), ("backward", 1), (("backward", "forward"), 3), ([], 0), ("other", 0)):
+        prog.launch(states)
+        assert ran.pop() == count, states
