@@ -62,3 +62,32 @@ def test_a_graph_belongs_to_its_binding():
     prog.launch()
     torch.cuda.synchronize()
     assert torch.equal(other, replayed)
+
+
+@pytest.mark.parametrize("backward", [False, True])
+def test_a_wrapper_call_with_the_same_tensors_keeps_its_graph(backward):
+    """A call that binds the addresses of the one before it leaves a graph usable; one on other tensors, or one that keeps
+    tensors for a backward call, does not."""
+    from daceml_amd.torch import DaceModule
+    net = torch.nn.Sequential(torch.nn.Linear(64, 128), torch.nn.GELU(), torch.nn.Linear(128, 32)).half().cuda()
+    w = DaceModule(net, backward=backward)
+    x = torch.randn((16, 64), device="cuda").half()
+    y = w(x)
+    place, expect = y.data_ptr(), y.detach().clone()
+    captured = w.compiled.capture([w.sdfg.states()[0].label])
+    captured.replay()
+    del y
+    y = w(x)
+    if backward:
+        with pytest.raises(RuntimeError):
+            captured.replay()
+        return
+    assert y.data_ptr() == place
+    y.fill_(float("nan"))
+    captured.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(y, expect)
+    z = w(x.clone())                             # another input, and another output beside the first
+    with pytest.raises(RuntimeError):
+        captured.replay()
+    assert torch.equal(z, expect)
