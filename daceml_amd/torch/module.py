@@ -257,8 +257,9 @@ class DaceModule(nn.Module):
         saved_slots = [(name, slot, dtype, shape) for _, name, slot, dtype, shape in bound_inputs] + \
             [(name, slot, dtype, shape) for name, (slot, dtype, shape) in zip(out_arrays, bound_outputs)] + kept_transients
         pointers = compiled.pointers
-        if not all(descs[name].is_contiguous() for name, *_ in saved_slots):
-            raise ValueError("inputs, outputs and stored tensors are passed dense")
+        bound = [name for name, *_ in saved_slots] + [name for _, name, *_ in given_gradients] + [g for g in grad_of_input if g in arglist]
+        if not all(descs[name].is_contiguous() for name in bound):
+            raise ValueError("inputs, outputs, stored tensors and gradients are passed dense")
         integer_outputs = [i for i, name in enumerate(out_arrays) if not descs[name].dtype.is_floating_point]
 
         def checked(name, t, dtype, shape):

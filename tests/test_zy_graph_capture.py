@@ -91,3 +91,49 @@ def test_a_wrapper_call_with_the_same_tensors_keeps_its_graph(backward):
     with pytest.raises(RuntimeError):
         captured.replay()
     assert torch.equal(z, expect)
+
+
+@pytest.mark.parametrize("which", ["input", "gradient given", "gradient made"])
+def test_a_wrapper_refuses_arrays_that_it_would_not_pass_as_they_are(which):
+    """Tensors go in dense: an array of another layout is an error."""
+    from daceml_amd.torch import DaceModule
+    net = torch.nn.Sequential(torch.nn.Linear(64, 128), torch.nn.GELU(), torch.nn.Linear(128, 32)).cuda()
+    w = DaceModule(net, backward=True, auto_optimize=False)
+
+    def pad_rows(name):
+        d = w.sdfg.arrays[name]
+        d.strides = (d.shape[1] + 8, 1)
+
+    def change(compiled):
+        out = list(w.dace_model.outputs)[0]
+        inp = [n for n in w.sdfg.arrays if "gradient_" + n in w.sdfg.arrays and n not in w.dace_model.outputs and
+               not w.sdfg.arrays[n].transient and w.sdfg.arrays[n].shape == (16, 64)][0]
+        pad_rows({"input": inp, "gradient given": "gradient_" + out, "gradient made": "gradient_" + inp}[which])
+
+    w.append_post_compile_hook("layout", change)
+    with pytest.raises(ValueError):
+        w(torch.randn((16, 64), device="cuda"))
+
+
+def test_transients_in_the_callers_memory():
+    from daceml_amd import graphs
+    from daceml_amd.runtime import CompiledSDFG
+    g = graphs.GraphBuilder("chain", torch.float32)
+    h = g.node("Exp", {"input": g.input("x", (5, 24))}, {"output": (5, 24)}, label="first")["output"]
+    g.output(g.node("Relu", {"X": h}, {"Y": (5, 24)}, label="second")["Y"], "y")
+    prog = CompiledSDFG(g.sdfg)
+    x, y = torch.randn((5, 24), device="cuda"), torch.empty((5, 24), device="cuda")
+    prog(x=x, y=y)
+    captured = prog.capture()
+    mine = torch.full((5, 24), float("nan"), device="cuda")
+    for name, t in (("x", mine), (h, mine[:4]), (h, mine.half()), (h, mine.t()), (h, mine.cpu())):
+        with pytest.raises(ValueError):
+            prog.rebind_transients({name: t})
+    captured.replay()
+    prog.rebind_transients({h: mine})
+    with pytest.raises(RuntimeError):
+        captured.replay()
+    y.fill_(float("nan"))
+    prog.launch()
+    torch.cuda.synchronize()
+    assert torch.equal(y, mine) and torch.equal(prog.buffers[h], mine)
