@@ -752,16 +752,17 @@ int dmlhip_gemm_f16_grouped(const dmlhip_gemm_desc* d, int groups, const void* c
 
 // Number of workgroups that share the K steps of a weight gradient's 256 x 256 tile (gemm_f16_wide.h); 0 = other kernels.
 // How many: the fewest us of 9.5 + 1.4 per step + 0.3 per MB of partial results (written, read and summed). Whether at all: both
-// launches take 20.2 us, 0.78 per step and 0.70 more where all compute units have a tile, 0.109 per MB (3.9 % off in the mean over
-// 466 gradients of 256 - 4096 x 256 - 4096 over 1800 - 18500 tokens, one to four products, both result types) - against 0.94 (a second
-// round of less than 0.6: 0.86) of the 128 x 128 tiles' 4 + rounds * (2 + steps * (0.42 + 0.14 where all compute units have one)).
+// launches take 20.6 us, 0.816 per step and 0.66 more where all compute units have a tile (0.038 more per 1024 columns beyond the
+// first), 0.098 per MB (4.4 % off in the mean over 5656 gradients of 256 - 4096 x 256 - 4096 over 1000 - 18500 tokens, one to four
+// products, both result types) - against 0.95 (a second round of less than 0.6: 0.86) of the 128 x 128 tiles' 4 + rounds * (2 + steps *
+// (0.42 + 0.14 where all compute units have one)).
 // us on those / here: 4096 x 1024 over 4096 / 8192 / 16384 tokens 42 / 51, 79 / 75, 153 / 122; 512 x 2048 over 4096 / 16384 34 / 31,
 // 122 / 54; three of 1024 x 1024 over 16384 143 / 100; 896 x 896 over 3515 30.1 / 32.8, 256 x 640 over 1792 17.6 / 22.6.
 // Results in fp16 may also be on the tiles with K split over the wavefronts, whose estimate long products exceed: 32 x 32 tiles by 1.3 - 2,
-// 64 x 64 tiles by 1 - 1.2, and by 1.2 - 1.8 where the rows of A are more than those of the result are long and a multiple of 1 KB apart.
+// 64 x 64 tiles by 1 - 1.2, and by 1.2 - 1.8 where the result has more rows than columns and a multiple of 512 of them.
 // us there / here: 768 x 768 over 8128 tokens 31.4 / 34.2, over 10240 37.7 / 35.9; 384 x 1536 over 7872 26.6 / 36.1, 640 x 512 over 5540
 // 22.4 / 29.0; 512 x 2048 over 4664 20.8 / 36.3, 2048 x 512 over 14283 84.9 / 49.6; 512 x 512 over 4160 15.4 / 28.8, over 14935 45.6 / 32.1.
-// Of 683 gradients, most of them near the line, 553 go here; three of those are 1 - 3 % slower than there.
+// Of 12 440 gradients that may be faster here 12 255 go here; 52 of those are more than 2 % slower than there, 9 % at most.
 static int weight_gradient_slices(const dmlhip_gemm_desc* d, int groups) {
     if (d->m <= 0 || d->n <= 0 || d->k <= 0 || d->m % 8 || d->n % 8 || d->c_stride_m != d->n || !g_direct_lds) return 0;
     if (d->m > 65536 || d->n > 65536 || (g_force_cfg >= 0 && g_force_cfg != 13)) return 0;
@@ -792,13 +793,14 @@ static int weight_gradient_slices(const dmlhip_gemm_desc* d, int groups) {
         const bool many = ceil_div(d->m, (int64_t)64) * ceil_div(d->n, (int64_t)64) * groups >= 192;
         if (cfg >= 10) {
             split = est;
-            behind = cfg == 12 ? 1.3 : !far ? 1.05 : many ? 1.3 : 1.18;
+            behind = cfg == 12 ? 1.3 : far ? (many ? 1.3 : 1.18) : d->n >= 3 * d->m ? 0.92 : 1.02;
         }
     }
     const double full = (double)t256 * slices / kCus;
-    const double us = 20.2 + (double)ceil_div(steps, (long long)slices) * (0.78 + 0.70 * full) + 0.109 * mb * slices;
+    const double wide_rows = d->n > 1024 ? 0.038 * (double)(d->n - 1024) / 1024 : 0.0;
+    const double us = 20.6 + (double)ceil_div(steps, (long long)slices) * (0.816 + (0.66 + wide_rows) * full) + 0.098 * mb * slices;
     // the figures that the number of slices was chosen by have to say so too: those of many MB are the surer ones
-    const bool faster = us < tiles * (rounds > 1 && t128 * 5 < rounds * kCus * 4 ? 0.86 : 0.94) && us < split * behind &&
+    const bool faster = us < tiles * (rounds > 1 && t128 * 5 < rounds * kCus * 4 ? 0.86 : 0.95) && us < split * behind &&
                         least_us < tiles * 0.93 && least_us < split * 1.2;
     return faster ? slices : 0;
 }

@@ -154,6 +154,7 @@ def test_which_weight_gradients_in_fp16_are_sliced(m, n, k, groups, sliced, lib)
 @pytest.mark.parametrize("out", ["f16", "f32"])
 @pytest.mark.parametrize("m,n,k,groups,f16,f32", [(768, 768, 8128, 1, False, True), (640, 512, 5540, 1, False, True), (384, 1536, 7872, 1, False, True),
                                                   (256, 896, 7231, 2, False, True), (896, 896, 3515, 1, False, False), (256, 640, 1792, 1, False, False),
+                                                  (256, 1536, 8960, 1, False, True), (384, 1152, 10593, 1, False, True),
                                                   (768, 768, 12288, 1, True, True), (1024, 896, 6208, 1, False, True), (2048, 768, 8132, 4, True, True)])
 def test_gradients_that_other_tiles_do_faster_are_not_sliced(m, n, k, groups, f16, f32, out, lib):
     from daceml_amd import _lib as L, kernels as K
