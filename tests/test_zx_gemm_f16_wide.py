@@ -183,3 +183,21 @@ def test_which_products_they_take(m, n, k, residual, cfg, lib):
     d = _desc(L, m, n, k, (k, 1), (k, 1), L.F16)
     L.check(lib.dmlhip_gemm_f16(ctypes.byref(d), P(a), P(b), P(c), None, P(r) if residual else None, None, K._stream()))
     assert lib.dmlhip_debug_last_gemm_config() == cfg
+
+
+@pytest.mark.parametrize("k,workspace,cfg", [(1023, True, 7), (1089, True, 4), (1089, False, 5), (1152, True, 5)])
+def test_gradients_over_a_ragged_number_of_tokens_that_fill_the_chip(k, workspace, cfg, lib):
+    """The product on 256 x 256 tiles, which make no row sums, and the sums behind it; without room for those in one launch."""
+    from daceml_amd import _lib as L, kernels as K
+    m = n = 4096
+    g = torch.Generator(device="cuda").manual_seed(k)
+    a, b = (torch.randn((k, e), generator=g, device="cuda").half() for e in (m, n))
+    d = _desc(L, m, n, k, (1, m), (1, n), L.F32)
+    c, s = torch.full((m, n), float("nan"), device="cuda"), torch.full((m, ), float("nan"), device="cuda")
+    need = lib.dmlhip_gemm_f16_grouped_asum_workspace_bytes(ctypes.byref(d)) if workspace else 0
+    ws = torch.empty(max(need, 16), device="cuda", dtype=torch.uint8)
+    L.check(lib.dmlhip_gemm_f16_grouped_asum(ctypes.byref(d), 1, _table([a]), _table([b]), _table([c]), _table([s]), L.F32, P(ws), need, K._stream()))
+    assert lib.dmlhip_debug_last_gemm_config() == cfg
+    at, b = a.double().t().contiguous(), b.double()
+    for got, exact, terms in ((c, at @ b, at.abs() @ b.abs()), (s, at.sum(1), at.abs().sum(1))):
+        assert bool(((got.double() - exact).abs() <= k * 2.0 ** -24 * terms + 3 * 2.0 ** -24 * exact.abs()).all())
