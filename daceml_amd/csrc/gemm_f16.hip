@@ -584,12 +584,15 @@ static int run_gemm_f16(const dmlhip_gemm_desc* d, const void* a, const void* b,
         const _Float16 *pa = (const _Float16*)a, *pb = (const _Float16*)b;
         // The 128 x 128 tile of gemm_f16_wide.h in place of those of gemm_f16_pipe.h, from sixteen steps on; not for the products
         // that the estimate gives to 128 x 64 tiles, which are two per compute unit (960 x 2048 x 1024 9.4 us there, 11.0 here).
-        // It starts with more steps on their way and reads a residual ahead: without one, and with no other product in the
-        // launch, less than a round of tiles needs thirty-two steps and seven eighths of it (1371 x 2048 x 1024 11.3 / 11.6, B
-        // row-contiguous 2844 x 768 x 3072 22.4 / 23.6, but 4764 x 768 x 3072 26.5 / 25.6; with a residual 1280 x 2048 x 1024
-        // 13.5 / 12.7, 2432 x 1024 x 4096 30.4 / 29.3).
-        if (g_force_cfg < 0 && (cfg == 5 || (cfg == 9 && !narrow)) && wide && amode == 0 && steps >= 16 && t128 * 2 >= kCus &&
-            (residual || extra || t128 > kCus || (steps >= 32 && t128 * 8 >= kCus * 7)))
+        // It starts with more steps on their way and reads a residual of fp16 ahead. Without one, up to a round of tiles needs
+        // thirty-two steps, and seven eighths of a round unless they are those of several operand pairs. us on 5 / 14: 1371 x 2048 x 1024
+        // 11.3 / 11.6, B row-contiguous 2844 x 768 x 3072 22.4 / 23.6, but 4764 x 768 x 3072 26.5 / 25.6; three of 317 x 2048 x 1024
+        // 11.4 / 12.5; fp32 with residual 768 x 3072 x 1024 14.4 / 15.9; with a residual 1280 x 2048 x 1024 13.5 / 12.7, 2432 x 1024 x 4096
+        // 30.4 / 29.3. (1300 products of up to a round that it takes: 0.935 of the time on 5 in the mean, three more
+        // than 1.01.)
+        const bool below = t128 <= kCus && !(residual && !g.out_f32) &&
+                           (steps < 32 || (!g.ksum && t128 * 8 < kCus * 7));
+        if (g_force_cfg < 0 && (cfg == 5 || (cfg == 9 && !narrow)) && wide && amode == 0 && steps >= 16 && t128 * 2 >= kCus && !below)
             cfg = 14;
         g_last_cfg = cfg;
         if (cfg == 13 && wide && steps >= 3) return launch_wide256(g, pa, pb, c, bias, residual, amode, bmode, batch, st);

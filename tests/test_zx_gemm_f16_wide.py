@@ -201,3 +201,26 @@ def test_gradients_over_a_ragged_number_of_tokens_that_fill_the_chip(k, workspac
     at, b = a.double().t().contiguous(), b.double()
     for got, exact, terms in ((c, at @ b, at.abs() @ b.abs()), (s, at.sum(1), at.abs().sum(1))):
         assert bool(((got.double() - exact).abs() <= k * 2.0 ** -24 * terms + 3 * 2.0 ** -24 * exact.abs()).all())
+
+
+@pytest.mark.parametrize("kind,m,n,k,count,residual,out,cfg", [
+    # up to a round of 128 x 128 tiles, no fp16 residual: long loops on nearly a round of tiles, or pairs
+    ("groups", 317, 2048, 1024, 3, False, "f16", 5), ("groups", 640, 1536, 2048, 3, False, "f16", 5), ("groups", 1280, 1024, 2048, 3, False, "f16", 14),
+    ("pairs", 755, 3072, 512, 3, True, "f32", 5), ("pairs", 755, 3072, 512, 3, True, "f16", 14), ("pairs", 755, 3072, 1024, 3, False, "f32", 14),
+    ("single", 768, 3072, 1024, 1, True, "f32", 5), ("single", 768, 3072, 1024, 1, True, "f16", 14),
+])
+def test_products_that_other_tiles_do_faster(kind, m, n, k, count, residual, out, cfg, lib):
+    from daceml_amd import _lib as L, kernels as K
+    dtype = torch.float16 if out == "f16" else torch.float32
+    d = _desc(L, m, n, k, (k, 1), (k, 1), L.F16 if out == "f16" else L.F32)
+    a, b = torch.zeros((m, k), device="cuda", dtype=torch.float16), torch.zeros((n, k), device="cuda", dtype=torch.float16)
+    c = [torch.empty((m, n), device="cuda", dtype=dtype) for _ in range(count if kind == "groups" else 1)]
+    r = torch.zeros((m, n), device="cuda", dtype=dtype) if residual else None
+    A, B = _table([a] * count), _table([b] * count)
+    if kind == "single":
+        L.check(lib.dmlhip_gemm_f16(ctypes.byref(d), P(a), P(b), P(c[0]), None, P(r), None, K._stream()))
+    elif kind == "pairs":
+        L.check(lib.dmlhip_gemm_f16_ksum(ctypes.byref(d), count, A, B, P(c[0]), None, P(r), K._stream()))
+    else:
+        L.check(lib.dmlhip_gemm_f16_grouped(ctypes.byref(d), count, A, B, _table(c), None, None, 0, K._stream()))
+    assert lib.dmlhip_debug_last_gemm_config() == cfg
