@@ -590,9 +590,12 @@ static int run_gemm_f16(const dmlhip_gemm_desc* d, const void* a, const void* b,
         // 11.4 / 12.5; fp32 with residual 768 x 3072 x 1024 14.4 / 15.9; with a residual 1280 x 2048 x 1024 13.5 / 12.7, 2432 x 1024 x 4096
         // 30.4 / 29.3. (1300 products of up to a round that it takes: 0.935 of the time on 5 in the mean, three more
         // than 1.01.)
+        // Nor for an A that the last-level cache does not hold: beyond 220 MB 0.98 in the mean, but three pairs of 11621 x 384 x 4096
+        // 175 / 189, three of 9408 x 256 x 4096 79 / 86.
         const bool below = t128 <= kCus && !(residual && !g.out_f32) &&
                            (steps < 32 || (!g.ksum && t128 * 8 < kCus * 7));
-        if (g_force_cfg < 0 && (cfg == 5 || (cfg == 9 && !narrow)) && wide && amode == 0 && steps >= 16 && t128 * 2 >= kCus && !below)
+        const bool beyond = 2e-6 * (double)d->m * (double)d->k * (grp ? grp->count : (int)batch) > 220.0;
+        if (g_force_cfg < 0 && (cfg == 5 || (cfg == 9 && !narrow)) && wide && amode == 0 && steps >= 16 && t128 * 2 >= kCus && !below && !beyond)
             cfg = 14;
         g_last_cfg = cfg;
         if (cfg == 13 && wide && steps >= 3) return launch_wide256(g, pa, pb, c, bias, residual, amode, bmode, batch, st);

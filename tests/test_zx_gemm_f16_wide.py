@@ -208,6 +208,8 @@ def test_gradients_over_a_ragged_number_of_tokens_that_fill_the_chip(k, workspac
     ("groups", 317, 2048, 1024, 3, False, "f16", 5), ("groups", 640, 1536, 2048, 3, False, "f16", 5), ("groups", 1280, 1024, 2048, 3, False, "f16", 14),
     ("pairs", 755, 3072, 512, 3, True, "f32", 5), ("pairs", 755, 3072, 512, 3, True, "f16", 14), ("pairs", 755, 3072, 1024, 3, False, "f32", 14),
     ("single", 768, 3072, 1024, 1, True, "f32", 5), ("single", 768, 3072, 1024, 1, True, "f16", 14),
+    # an A that the last-level cache does not hold
+    ("pairs", 11621, 384, 4096, 3, False, "f32", 5), ("groups", 9408, 256, 4096, 3, False, "f32", 5), ("pairs", 11621, 384, 2048, 3, False, "f32", 14),
 ])
 def test_products_that_other_tiles_do_faster(kind, m, n, k, count, residual, out, cfg, lib):
     from daceml_amd import _lib as L, kernels as K
