@@ -402,12 +402,17 @@ double estimate_small(int64_t m, int64_t n, int64_t k, long long batch, int pair
 // Over 110 products (700 - 16384 tokens, 512 - 4096 wide, B in either layout, groups, operand pairs, residuals) the faster of
 // the two was missed once, by 1 %. Decided by it (us, 128 x 128 tiles / 256 x 256): 5041 x 2048 x 1024 30.3 / 28.4, three of
 // 4144 x 1024 x 1024 37.1 / 28.0, three of 5532 x 1024 x 4096 147 / 161, 4860 x 1024 x 4096 56.7 / 73, 8230 x 1024 x 3072 67 / 60.
-bool wide_is_faster(long long t256, long long t128, int64_t k, int pairs, bool residual, bool a_kc) {
+// Short loops have to be ahead by more: those with a residual, which two workgroups per compute unit read under each other's loops
+// (16791 x 2048 x 768 80.5 / 86.7, 10647 x 2048 x 768 52.1 / 54.9, fp32 2967 x 3072 x 512 29.2 / 31.2), and eight steps with a third
+// round that is nearly empty (16512 x 2048 x 512 52.2 / 56.5). Of 1740 products that it takes from two workgroups per compute unit, 0.83
+// of the time there in the mean, none is more than 4 % slower.
+bool wide_is_faster(long long t256, long long t128, int64_t k, int pairs, bool residual, bool a_kc, bool out_f32) {
     const double steps = (double)(k / BK) * pairs;
     const double t = (double)ceil_div(t256, (long long)kCus), s = (double)ceil_div(t128, (long long)kCus);
     const double full = (double)t256 / (t * kCus);
+    const double ahead = t >= 3 && k <= 512 && !residual ? 0.9 : residual && k <= 1024 && t128 >= 2 * kCus ? (out_f32 ? 0.95 : 0.975) : 1.0;
     return 9.0 + t * steps * (1.0 + 0.35 * full * full) + (t - 1) * 6.0 + (residual ? t * 6.0 : 0.0) <
-           4.0 + s * ((a_kc ? 0.43 : 0.55) * steps + (residual ? 3.5 : 2.0));
+           ahead * (4.0 + s * ((a_kc ? 0.43 : 0.55) * steps + (residual ? 3.5 : 2.0)));
 }
 
 // Diagnostic switches (declared in the public header). Per calling thread, so that one thread pinning a configuration
@@ -543,7 +548,7 @@ static int run_gemm_f16(const dmlhip_gemm_desc* d, const void* a, const void* b,
         const long long slots256 = ceil_div(t256, (long long)kCus) * kCus, slots128 = ceil_div(t128, (long long)kCus) * kCus;
         bool narrow = false;   // the estimate found the 128 x 64 tile to be the fastest
         const bool full256 = !extra && t256 * 10 >= slots256 * 9;
-        if (cfg < 0 && d->k >= 512 && wide && (full256 || wide_is_faster(t256, t128, d->k, g.ksum ? g.groups : 1, residual, amode == 0))) {
+        if (cfg < 0 && d->k >= 512 && wide && (full256 || wide_is_faster(t256, t128, d->k, g.ksum ? g.groups : 1, residual, amode == 0, g.out_f32))) {
             cfg = 13;
         } else if (cfg < 0 && d->k >= 512 && full256) {
             // What the kernel above does not take (activations, beta, rows that are not stored in vectors, a ragged K). The

@@ -210,6 +210,9 @@ def test_gradients_over_a_ragged_number_of_tokens_that_fill_the_chip(k, workspac
     ("single", 768, 3072, 1024, 1, True, "f32", 5), ("single", 768, 3072, 1024, 1, True, "f16", 14),
     # an A that the last-level cache does not hold
     ("pairs", 11621, 384, 4096, 3, False, "f32", 5), ("groups", 9408, 256, 4096, 3, False, "f32", 5), ("pairs", 11621, 384, 2048, 3, False, "f32", 14),
+    # short loops: what two workgroups per compute unit do faster than 256 x 256 tiles
+    ("single", 10647, 2048, 768, 1, True, "f16", 7), ("single", 2967, 3072, 512, 1, True, "f32", 14), ("single", 16384, 2048, 512, 1, False, "f16", 13),
+    ("single", 8192, 2048, 768, 1, True, "f16", 13),
 ])
 def test_products_that_other_tiles_do_faster(kind, m, n, k, count, residual, out, cfg, lib):
     from daceml_amd import _lib as L, kernels as K
