@@ -570,10 +570,14 @@ static int run_gemm_f16(const dmlhip_gemm_desc* d, const void* a, const void* b,
             } else if (d->k <= 1024 && t128 >= 2 * kCus) {
                 // several rounds of short K loops (the grouped q / k / v projections: 768 tiles of 16 steps): with two
                 // LDS stages instead of four, two workgroups share a compute unit and one's epilogue and first loads
-                // overlap the other's loop. Tiles that stay (gemm_f16_wide.h) are faster beyond one round of such pairs where K
-                // is not short or a pair would be left half empty: three of 5408 x 1024 x 1024 51 / 46 us, 12661 x 1536 x 768
-                // 42.4 / 38.3, but three of 4880 x 1024 x 512 25.7 / 26.5 and of 2633 x 1024 x 768 18.0 / 19.2
-                cfg = wide && amode == 0 && t128 > 2 * kCus && (steps >= 16 || ceil_div(t128, (long long)kCus) % 2) ? 14 : 7;
+                // overlap the other's loop. Tiles that stay (gemm_f16_wide.h) are faster beyond one round of such pairs where a
+                // pair would be left half empty or the loop is not short; time of 14 over 7 with 8 / 12 / 16 steps: five rounds 0.98 / 0.93 /
+                // 0.92 (just past the fourth, 8 steps, 1.01 - 1.04), nine with a residual 1.01 / 0.95 / 0.97; four rounds with 8 - 10 / 12 / 13 / 14 / 16
+                // steps 1.05 - 1.02 / 0.98 / 0.97 / 0.97 / 0.92 - 0.98 (taken from sixteen on), of fp32 with a residual 1.05.
+                const long long rounds = ceil_div(t128, (long long)kCus);
+                const bool half = rounds % 2 && (steps >= 12 || (rounds <= 5 && (t128 - (rounds - 1) * kCus) * 6 >= kCus));
+                const bool stay = wide && amode == 0 && t128 > 2 * kCus && (half || (steps >= 16 && !(residual && g.out_f32)));
+                cfg = stay ? 14 : 7;
             } else if (!extra && d->k <= 1024 && t128 <= kCus && residual) {
                 // a short K loop whose epilogue also reads a residual tile (4096 x 1024 x 1024: 20.3 - 21.1 against
                 // 22.9 - 23.2 us): 128 x 64 tiles, two workgroups per compute unit, for the same overlap (without the

@@ -213,6 +213,8 @@ def test_gradients_over_a_ragged_number_of_tokens_that_fill_the_chip(k, workspac
     # short loops: what two workgroups per compute unit do faster than 256 x 256 tiles
     ("single", 10647, 2048, 768, 1, True, "f16", 7), ("single", 2967, 3072, 512, 1, True, "f32", 14), ("single", 16384, 2048, 512, 1, False, "f16", 13),
     ("single", 8192, 2048, 768, 1, True, "f16", 13),
+    # ... and than 128 x 128 tiles that stay: rounds in pairs, many rounds of very short loops
+    ("single", 16512, 2048, 512, 1, False, "f16", 7), ("groups", 5408, 1024, 512, 3, False, "f16", 7), ("groups", 6100, 1024, 512, 3, False, "f16", 14),
 ])
 def test_products_that_other_tiles_do_faster(kind, m, n, k, count, residual, out, cfg, lib):
     from daceml_amd import _lib as L, kernels as K
