@@ -949,6 +949,26 @@ def fuse_attention(sdfg: SDFG) -> int:
     return count
 
 
+def _row_sums_apart(sdfg: SDFG, state: SDFGState, node, plan) -> bool:
+    """Whether a weight gradient over a ragged number of rows is faster without the sums of its first operand. Only 128 x 128
+    tiles and slices of K make them; a product alone that leaves half of the chip idle also has 128 x 64 tiles, and reductions
+    share a launch. Time with the sums / without them and half of a launch for them, 12 000 single products of 24 - 18000 rows:
+    fp32 results of up to 64 tiles 0.7 - 1.0 over 700 - 1000 rows, 1.1 - 1.3 over 1400 - 3000, 0.5 - 0.9 from 5000 on (slices);
+    65 - 128 tiles 1.0, 1.04 - 1.19 over 1400 - 5000, 0.8 from 9000 on; fp16 results of up to 64 tiles 0.6 - 0.9 (tiles with K split
+    over the wavefronts, which make them too). Between 128 tiles and a round 0.8 - 1.06."""
+    tiles = -(-plan.m // 128) * -(-plan.n // 128)
+    if plan.k % 64 == 0 or tiles > 128 or not 1200 <= plan.k < 3300 + 22 * tiles:
+        return False
+    out = sdfg.arrays[_out_array(state, node, "Output")]
+    if out.dtype == torch.float16 and tiles <= 64:
+        return False
+    shapes = lambda n: [(e.dst_conn, sdfg.arrays[e.data.data].shape) for e in sorted(state.in_edges(n), key=lambda e: e.dst_conn)]  # noqa: E731
+    mine = shapes(node)
+    alike = sum(n.equation == node.equation and shapes(n) == mine for n in state.nodes() if _is_op(n, "FusedEinsum"))
+    # products that share a launch are on 128 x 128 tiles either way; four of 256 x 256 over 2545 rows 28.0 us with sums, 23.9 without
+    return alike == 1 or alike * tiles <= 32
+
+
 def fuse_bias_gradients(sdfg: SDFG) -> int:
     """A ReduceSum of dY over every axis but the last (a bias gradient; the third node DefaultEinsumBackward's
     callers emit, daceml/autodiff/implementations/onnx_ops.py:54-138) next to a contraction whose first operand is
@@ -983,7 +1003,7 @@ def fuse_bias_gradients(sdfg: SDFG) -> int:
                 except (C.NotApplicable, ValueError):
                     continue
                 if plan.swapped or any(e != 1 for e in plan.batch) or plan.m != xd.shape[-1] \
-                        or plan.m * plan.k != xd.total_size or b.dtype != torch.float16:
+                        or plan.m * plan.k != xd.total_size or b.dtype != torch.float16 or _row_sums_apart(sdfg, state, node, plan):
                     continue
                 _remove_node(state, red)
                 node.add_out_connector("InputSum")

@@ -694,3 +694,21 @@ def test_argument_errors_of_weight_gradients_do_not_depend_on_their_length(token
     assert status(b_stride_n=1, b_stride_k=-512) == L.ERR_SHAPE
     assert status(c_stride_m=511) == L.ERR_SHAPE
     assert status(m=-512) == L.ERR_UNSUPPORTED and status(n=-8) == L.ERR_SHAPE and status(k=-1) == L.ERR_SHAPE
+
+
+@pytest.mark.parametrize("batch,seq,hidden,sums,apart", [(8, 400, 512, 6, 0), (3, 217, 512, 6, 0), (8, 401, 512, 4, 2), (5, 509, 256, 0, 6), (8, 509, 1024, 6, 0),
+                                                         (29, 509, 512, 6, 0)])
+def test_bias_gradients_over_ragged_rows_come_out_of_their_products_where_that_is_faster(batch, seq, hidden, sums, apart, lib):
+    """All six of an encoder layer, but for products over some thousand ragged rows that leave half of the chip idle."""
+    from daceml_amd import graphs
+    from daceml_amd.autodiff import add_backward_pass
+    from daceml_amd.transformation import fusion
+    sdfg = graphs.bert_encoder_layer(batch, seq, hidden, hidden // 64, 4 * hidden, torch.float16, eps=1e-5)
+    fusion.auto_optimize(sdfg, training=True)
+    add_backward_pass(sdfg, sdfg.states()[0], ["y"], ["x"] + graphs.BERT_PARAM_NAMES,
+                      grad_dtypes={n: torch.float32 for n in graphs.BERT_PARAM_NAMES})
+    fusion.optimize_backward(sdfg)
+    state = sdfg.states()[1]
+    outputs = [e.src_conn for n in state.library_nodes() for e in state.out_edges(n)]
+    assert sum(c.startswith("InputSum") for c in outputs if c) == sums
+    assert sum(c.startswith("reduced") for c in outputs if c) == apart
