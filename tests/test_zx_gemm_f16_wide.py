@@ -130,9 +130,17 @@ def test_weight_gradients_in_slices(m, n, k, groups, layout, sum_dtype, lib):
                                                  (1024, 1024, 16384, 4, True), (768, 3072, 1024, 1, False)])
 def test_which_weight_gradients_are_sliced(m, n, k, groups, sliced, lib):
     """The workspace holds the slices of a long product's results; a short one has none."""
-    from daceml_amd import _lib as L
+    from daceml_amd import _lib as L, kernels as K
     d = _desc(L, m, n, k, (1, m), (1, n), L.F32)
-    assert (lib.dmlhip_gemm_f16_grouped_asum_workspace_bytes(ctypes.byref(d)) >= 2 * groups * m * n * 4) == sliced
+    need = lib.dmlhip_gemm_f16_grouped_asum_workspace_bytes(ctypes.byref(d))
+    assert (need >= 2 * groups * m * n * 4) == sliced
+    # the workspace is for any number of products: which of them are sliced is seen where they run
+    a, b = (torch.zeros((k, e), device="cuda", dtype=torch.float16) for e in (m, n))
+    c, s = ([torch.empty(shape, device="cuda") for _ in range(groups)] for shape in ((m, n), (m, )))
+    ws = torch.empty(max(need, 16), device="cuda", dtype=torch.uint8)
+    L.check(lib.dmlhip_gemm_f16_grouped_asum(ctypes.byref(d), groups, _table([a] * groups), _table([b] * groups), _table(c), _table(s), L.F32,
+                                             P(ws), need, K._stream()))
+    assert (lib.dmlhip_debug_last_gemm_config() == 13) == sliced
 
 
 @pytest.mark.parametrize("m,n,k,groups,sliced", [(512, 512, 4160, 1, False), (512, 2048, 4664, 1, False), (512, 512, 3840, 3, False),
