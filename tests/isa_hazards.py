@@ -160,3 +160,55 @@ def check_store_data(path):
             if _WIDE_STORE.match(code):
                 pending = ln
     return found
+
+
+_AREG = re.compile(r'(?<![\w\]])a\[(\d+):(\d+)\]|(?<![\w\]])a(\d+)\b')
+
+
+def check_mfma(path, read_after=18):
+    """Matrix instructions in inline assembly, whose wait states the compiler does not keep. Reports, per kernel, every
+    ``v_mfma`` that reads a vector register which a vector instruction wrote fewer than two wait states earlier, and every other
+    instruction that touches an accumulation register fewer than ``read_after`` wait states behind a ``v_mfma``. An instruction is one
+    wait state, ``s_nop N`` is N + 1. Returns {kernel: {line: instruction}}."""
+    found = {}
+    for name, body in kernels(path):
+        labels = {b[2]: i for i, b in enumerate(body) if b[1] == 'label'}
+        none = frozenset()
+        # vector registers written in the last two wait states; wait states since the last v_mfma
+        seen, work, bad = set(), [(0, (none, none), read_after)], {}
+        while work:
+            i, written, since = work.pop()
+            while i < len(body):
+                ln, kind, code = body[i]
+                if kind == 'label':
+                    if (i, written, since) in seen:
+                        break
+                    seen.add((i, written, since))
+                    i += 1
+                    continue
+                op = code.split()[0]
+                rest = code[len(op):]
+                if op == 's_endpgm':
+                    break
+                now, states = none, 1
+                if op.startswith('v_mfma'):
+                    sources = _vregs(','.join(rest.split(',')[1:]))
+                    if sources & (written[0] | written[1]):
+                        bad[ln] = code
+                elif _AREG.search(rest) and since < read_after:
+                    bad[ln] = code
+                elif op.startswith('v_') and not op.startswith('v_cmp'):
+                    now = _vregs(rest.split(',')[0])
+                elif op == 's_nop':
+                    states = int(rest.strip(), 0) + 1
+                written = (written[1], now) if states == 1 else (none, none)
+                since = 0 if op.startswith('v_mfma') else min(since + states, read_after)
+                if op == 's_branch':
+                    i = labels.get(rest.strip(), len(body))
+                    continue
+                if op.startswith('s_cbranch') and rest.strip() in labels:
+                    work.append((labels[rest.strip()], written, since))
+                i += 1
+        if bad:
+            found[name] = bad
+    return found

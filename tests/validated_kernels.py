@@ -16,7 +16,7 @@ SOURCES = [os.path.join(ROOT, "tests", "isa", "validated_instances.hip"),
            os.path.join(ROOT, "daceml_amd", "csrc", "conv_fused.hip"),
            os.path.join(ROOT, "daceml_amd", "csrc", "attention.hip")]
 #: kernels of SOURCES that are recorded
-RECORDED = re.compile(r"gemm_f16_pipe_kernel|expand_depthwise_kernel|expand_depthwise_rolling_kernel|attention_fwd_kernel|"
+RECORDED = re.compile(r"gemm_f16_pipe_kernel|gemm_f16_wide_kernel|expand_depthwise_kernel|expand_depthwise_rolling_kernel|attention_fwd_kernel|"
                       r"attention_bwd_dq_kernel|attention_bwd_dkv_kernel")
 
 
