@@ -309,7 +309,9 @@ LOG_SOFTMAX_COLS = 1024
 def fuse_log_softmax(sdfg: SDFG) -> int:
     """LogSoftmax over rows that a wavefront holds in its registers: the six calls of its expansion become one, and the
     Exp, ReduceSum, Mul, Sub of its reverse another. Wider rows stay with those calls, which split a row over workgroups.
-    The node keeps its kind, so the pass runs behind ``auto_optimize``, where a program is made of the graph."""
+    Nodes are marked, not replaced, and a mark is no attribute: a host that takes nodes over by kind and attributes (the DaCe plugin,
+    from ``auto_optimize``) would not see it, and a reverse made for a marked node would be a Softmax's there. So this is no part of
+    ``auto_optimize``; ``DaceModule`` and ``ONNXModel`` run it, and graphs that are expanded here may."""
     count = 0
     for state in sdfg.states():
         for node in [n for n in state.nodes() if _is_op(n, "LogSoftmax") and not getattr(n, "_one_pass", False)]:
