@@ -269,27 +269,20 @@ class DaceModule(nn.Module):
                 compiled.check_argument(name, t)
             return t
 
-        def point(slot, t):
-            """Where the program finds `t` from now on; whether that is another place than before."""
-            address = t.data_ptr()
-            if slot is None or pointers[slot] == address:
-                return False
-            pointers[slot] = address
-            return True
-
         def run_forward(tensors, keep=False):
             call = [checked(name, tensors[i].detach(), dtype, shape) for i, name, _, dtype, shape in bound_inputs]
             outs = [torch.empty(shape, dtype=dtype, device=device) for _, dtype, shape in bound_outputs]
             saved = [torch.empty(shape, dtype=dtype, device=device) for _, _, dtype, shape in kept_transients] if keep else []
-            changed = bool(saved)   # fresh memory, wherever it lies
+            before = None if saved else bytes(pointers)   # kept tensors are in fresh memory, wherever it lies
             for (_, _, slot, _, _), t in zip(bound_inputs, call):
-                changed |= point(slot, t)
+                pointers[slot] = t.data_ptr()
             for (slot, _, _), t in zip(bound_outputs, outs):
-                changed |= point(slot, t)
+                if slot is not None:
+                    pointers[slot] = t.data_ptr()
             for (name, slot, _, _), t in zip(kept_transients, saved):
-                point(slot, t)
+                pointers[slot] = t.data_ptr()
                 compiled.buffers[name] = t   # in place of the program's own buffer
-            if changed:
+            if bytes(pointers) != before:
                 compiled.rebound()
             compiled.launch(forward_states)
             return tuple(outs), call, saved
@@ -311,15 +304,16 @@ class DaceModule(nn.Module):
                     gradients.append(torch.zeros(shape, dtype=dtype, device=device) if g is None
                                      else checked(name, g.to(dtype), dtype, shape))
                 results = [None if made is None else torch.empty(made[2], dtype=made[1], device=device) for made in made_gradients]
-                changed = bool(kept_transients)
+                before = None if kept_transients else bytes(pointers)
                 for (_, slot, _, _), t in zip(saved_slots, call):
-                    changed |= point(slot, t)
+                    if slot is not None:
+                        pointers[slot] = t.data_ptr()
                 for (_, _, slot, _, _), t in zip(given_gradients, gradients):
-                    changed |= point(slot, t)
+                    pointers[slot] = t.data_ptr()
                 for made, t in zip(made_gradients, results):
-                    if made is not None:
-                        changed |= point(made[0], t)
-                if changed:
+                    if made is not None and made[0] is not None:
+                        pointers[made[0]] = t.data_ptr()
+                if bytes(pointers) != before:
                     compiled.rebound()
                 compiled.launch(backward_states)
                 return tuple(t if made is None or made[1] == made[3] else t.to(made[3]) for made, t in zip(made_gradients, results))
