@@ -27,7 +27,8 @@
 // LDS tiles. KC (K contiguous): [256 rows][64 k], 128-byte rows, 16-byte chunk c of row r at slot c ^ (r & 7) ^ (r >> 3 & 1).
 // RC (rows contiguous): [64 k][256 rows], chunk c (8 rows) of K row k at slot c ^ ((k & 3) << 2) ^ ((k >> 3 & 1) << 1): the
 // transpose read of 16 lanes touches four K rows, 32 bytes of each, the two groups that are read together are eight K rows
-// apart. Neither has bank conflicts.
+// apart. LDS clocks: a KC fragment 8, four of them bank conflicts (the 32-row fragments of gemm_f16_pipe.h have none), an RC one of A
+// twice 2 without conflicts, one of B, whose columns b_row moves, twice 4. All reads of a step take half as long as its MFMAs.
 //  * SLICED (weight gradients: few tiles, a long K): the workgroups of a tile share its K steps and write fp32 partial results
 //    that wide_sum_kernel adds up, four times over for 64 tiles: 64 MB written and read, about 30 us whatever K is. The row
 //    sums of A (the bias gradient) are taken from the fragments: the workgroups of tile column c add those of every step that
