@@ -695,6 +695,8 @@ int dmlhip_gemm_f16_ws(const dmlhip_gemm_desc* d, const void* a, const void* b, 
                        workspace && d->c_stride_m == d->n;
     const int s = plain ? split_k_factor(d, vector_operands(d, a, b)) : 1;
     if (s <= 1 || workspace_bytes < split_k_bytes(d, s)) return run_gemm_f16(d, a, b, c, bias, residual, pre_out, stream);
+    long long batch;
+    if (int e = check_gemm_f16(d, batch)) return e;   // the slices' own result type is another
     // stage 1: batch slot 0 enumerates the K slices; partial C tiles are dense fp32 [s][m][n]
     dmlhip_gemm_desc p = *d;
     p.k = d->k / s;

@@ -712,3 +712,20 @@ def test_bias_gradients_over_ragged_rows_come_out_of_their_products_where_that_i
     outputs = [e.src_conn for n in state.library_nodes() for e in state.out_edges(n)]
     assert sum(c.startswith("InputSum") for c in outputs if c) == sums
     assert sum(c.startswith("reduced") for c in outputs if c) == apart
+
+
+@pytest.mark.parametrize("k", [512, 16384])
+def test_argument_errors_of_products_do_not_depend_on_their_slices(k, lib):
+    """Products whose K is cut into slices have fp32 partial results, whatever type is asked for: the type is checked all the same."""
+    from daceml_amd import _lib as L
+    d = L.GemmDesc()
+    d.m, d.n, d.k = 256, 256, k
+    d.batch[0] = d.batch[1] = d.batch[2] = 1
+    d.a_stride_m, d.a_stride_k, d.b_stride_k, d.b_stride_n, d.c_stride_m = k, 1, 1, k, 256
+    d.alpha, d.out_dtype = 1.0, L.F32
+    assert (lib.dmlhip_gemm_f16_workspace_bytes(ctypes.byref(d)) > 0) == (k == 16384)
+    for name, value, error in (("out_dtype", 7, L.ERR_ENUM), ("bias_dtype", 9, L.ERR_ENUM), ("b_stride_n", -k, L.ERR_SHAPE), ("c_stride_m", 255, L.ERR_SHAPE)):
+        good = getattr(d, name)
+        setattr(d, name, value)
+        assert lib.dmlhip_gemm_f16_ws(ctypes.byref(d), 64, 64, 64, None, None, None, 64, 1 << 26, None) == error, name
+        setattr(d, name, good)
